@@ -19,6 +19,7 @@ SOURCES = [
     "sq_profile.hip",
     "sq_tiles.hip",
     "sq_ucc.hip",
+    "sq_small.hip",
     "sq_batch.hip",
     "sq_orbital.hip",
     "sq_noalloc.hip",

@@ -290,11 +290,7 @@ static void add_gate(Program& P, const sq_gate_desc& g, int n_orb) {
 // Frequencies and T^k coefficients of the multi-frequency SA doubles
 // (operator_state_algebra.py:1086-1279).  Row k-1 multiplies T^k; odd k use
 // sin(S_f th), even k use cos(S_f th) - 1.
-struct PolyTable {
-  int nf, nk;
-  double S[5];
-  double K[10][5];
-};
+using PolyTable = GatePoly;
 
 __constant__ PolyTable c_poly[4];  // index: case 2,3 -> 0; 4 -> 1; 5 -> 2; Taylor -> 3
 
@@ -355,6 +351,8 @@ static int poly_slot(const GateDev& g) {
   if (g.poly == 4) return 1;
   return 2;
 }
+
+GatePoly gate_poly(const GateDev& g) { return host_poly(poly_slot(g)); }
 
 __device__ __forceinline__ double poly_coef(const PolyTable& t, int k, double th) {
   // k is 1-based power of T
@@ -812,6 +810,7 @@ int sq_program_destroy(sq_program* pr) {
     if (pr->p.d_term_fast) (void)hipFree(pr->p.d_term_fast);
     if (pr->p.ucc_csr) ucc_csr_free(pr->p.ucc_csr);
     if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
+    if (pr->p.small) small_plan_free(pr->p.small);
     delete pr;
   });
 }
@@ -918,6 +917,10 @@ int sq_state_prep(const sq_space* sp, const sq_program* pr, const double* theta,
     const Program& p = pr->p;
     SQ_CHECK(theta || p.gates.empty(), SQ_ERR_ARG, "theta is NULL");
     hipStream_t st = as_stream(stream);
+    if (const SmallPlan* S = small_for(s, p)) {
+      small_forward(s, *S, theta, psi_in, psi_out, dagger != 0, st);
+      return;
+    }
     const TilePlan* T = tiles_for(s, p);
     if (T) {
       tiles_forward(s, p, *T, theta, psi_in, psi_out, work + 2 * s.dim, work, -1, dagger != 0, st);

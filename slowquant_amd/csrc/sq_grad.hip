@@ -71,6 +71,12 @@ static void finish(const GradBufs& b, int n, double* energy, double* grad, hipSt
 // inserts T_g after gate g.
 static void forward(const Space& s, const Program& p, const double* theta, const double* psi0, double* psi,
                     const GradBufs& b, int deriv_gate, hipStream_t st) {
+  if (deriv_gate < 0) {
+    if (const SmallPlan* S = small_for(s, p)) {
+      small_forward(s, *S, theta, psi0, psi, false, st);
+      return;
+    }
+  }
   const TilePlan* T = tiles_for(s, p);
   if (T) {
     tiles_forward(s, p, *T, theta, psi0, psi, b.s1, b.t1, deriv_gate, false, st);
@@ -92,8 +98,9 @@ void energy_grad_adjoint(const Space& s, const Program& p, const Hamiltonian& H,
   GradBufs b = carve(s, n, work);
   forward(s, p, theta, psi0, b.psi, b, -1, st);
   sigma_energy_dev(s, H, b.psi, b.lam, b.scal, b.sigw, st);
-  const TilePlan* T = tiles_for(s, p);
-  if (T) {
+  if (const SmallPlan* S = small_for(s, p)) {
+    small_reverse(s, *S, theta, b.psi, b.lam, b.grad, st);
+  } else if (const TilePlan* T = tiles_for(s, p)) {
     tiles_reverse(s, p, *T, theta, b.psi, b.lam, b.t1, b.partial, b.grad, true, st);  // matrices from forward()
   } else {
     for (int g = n - 1; g >= 0; --g) reverse_step_impl(s, p, g, theta, b.psi, b.lam, b.grad, b.t1, b.partial, st);
@@ -107,8 +114,9 @@ void adjoint_reverse(const Space& s, const Program& p, const double* theta, doub
                      double* work, hipStream_t st) {
   const int n = (int)p.gates.size();
   GradBufs b = carve(s, n, work);
-  const TilePlan* T = tiles_for(s, p);
-  if (T) {
+  if (const SmallPlan* S = small_for(s, p)) {
+    small_reverse(s, *S, theta, psi, lam, b.grad, st);
+  } else if (const TilePlan* T = tiles_for(s, p)) {
     tiles_reverse(s, p, *T, theta, psi, lam, b.t1, b.partial, b.grad, false, st);
   } else {
     for (int g = n - 1; g >= 0; --g) reverse_step_impl(s, p, g, theta, psi, lam, b.grad, b.t1, b.partial, st);
@@ -139,8 +147,9 @@ void energy_grad_reference_sweep(const Space& s, const Program& p, const Hamilto
   forward(s, p, theta, psi0, b.psi, b, -1, st);
   sigma_energy_dev(s, H, b.psi, b.lam, b.scal, b.sigw, st);
   // bra = U^+ H psi
-  const TilePlan* T = tiles_for(s, p);
-  if (T) {
+  if (const SmallPlan* S = small_for(s, p)) {
+    small_forward(s, *S, theta, b.lam, b.lam, true, st);
+  } else if (const TilePlan* T = tiles_for(s, p)) {
     tiles_forward(s, p, *T, theta, b.lam, b.lam, b.s1, b.t1, -1, true, st);
   } else {
     for (int g = n - 1; g >= 0; --g) apply_gate_impl(s, p, g, theta, true, b.lam, b.t1, st);

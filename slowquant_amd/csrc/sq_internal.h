@@ -97,6 +97,16 @@ enum GateClass : int32_t {
   GC_TAYLOR = 4      // generic: closed form 1 + sin T + (1 - cos) T^2 through T applications
 };
 
+// Frequencies S_f and T^k coefficients of a gate's closed form
+// 1 + sum_k c_k(theta) T^k: c_k = sum_f K[k-1][f] sin(S_f theta) for odd k,
+// K[k-1][f] (cos(S_f theta) - 1) for even k.
+struct GatePoly {
+  int nf, nk;
+  double S[5];
+  double K[10][5];
+};
+GatePoly gate_poly(const GateDev& g);
+
 struct Space {
   int n, na, nb;
   int nsa, nsb;
@@ -134,10 +144,15 @@ TilePlan* build_tile_plan(const Space& sp, const struct Program& P);
 void destroy_tile_plan(TilePlan* T);
 bool tile_plan_has_tiles(const TilePlan* T);
 
+struct SmallPlan;
+void small_plan_free(SmallPlan* P);
+
 struct Program {
   const Space* space;
   mutable TilePlan* tiles = nullptr;  // built on first use (sq_tiles.hip)
   mutable bool tiles_built = false;
+  mutable SmallPlan* small = nullptr;  // one-block sweep, built on first use (sq_small.hip)
+  mutable bool small_tried = false;
   int tile_target = 0;   // elements per tile (0: automatic; sq_program_set_tile_shape)
   int tile_threads = 0;  // threads per tile block, 256 or 512 (0: 512)
   int plan_gen = 0;      // bumped whenever the tile plan is dropped (batched groups check it)
@@ -208,6 +223,7 @@ enum ProfClass {
   PC_SIGMA_ROWS,
   PC_ALPHA_GEMM,
   PC_ORBITAL,
+  PC_SMALL,
   kProfClasses
 };
 bool prof_on();
@@ -252,6 +268,16 @@ void reverse_step_impl(const Space& s, const Program& p, int g, const double* th
 
 // Implemented in sq_tiles.hip
 const TilePlan* tiles_for(const Space& s, const Program& p);  // nullptr when no tiled stage applies
+
+bool tiles_cover(const Space& s, const Program& p);  // every gate runs in a tile stage
+
+// Implemented in sq_small.hip: the whole sweep of a small space in one block
+const SmallPlan* small_for(const Space& s, const Program& p);  // nullptr where it does not apply
+void small_forward(const Space& s, const SmallPlan& P, const double* theta, const double* psi_in, double* psi,
+                   bool dagger, hipStream_t st);
+// reverse sweep on (psi, lam), left as they are; dE/dtheta to grad (device)
+void small_reverse(const Space& s, const SmallPlan& P, const double* theta, const double* psi, const double* lam,
+                   double* grad, hipStream_t st);
 
 // Several instances of one (space, program) evaluated together (batched
 // groups, sq_batch.hip): the tile, gradient and row-sigma kernels run with

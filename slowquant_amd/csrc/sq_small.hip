@@ -1,0 +1,675 @@
+// Whole gate sweeps of small spaces in one workgroup (replaces the gate loop
+// of construct_ups_state and the gradient sweep, operator_state_algebra.py:
+// 963-1412, ups_wavefunction.py:1060-1142, for spaces whose state vectors fit
+// a CU's LDS).
+//
+// A gate outside the brick-wall layouts (factorised UCC: excitations between
+// any orbitals) touches a few hundred determinant pairs of a small space, far
+// too few to fill a launch: one launch per gate and direction is launch
+// latency and nothing else ((8e,8o) fUCCSD: 361 gates, 1080 launches of
+// 2-4 us, 4.0 ms per energy and gradient).  Here one block of 1024 threads
+// holds psi (and lambda in the reverse sweep) in LDS and runs every gate, one
+// barrier per gate.
+//
+//   * A rotation (GC_ROT, each half of GC_SA_SINGLE) is a list of determinant
+//     pairs, built once per program on the host: 13-bit indices i, j and the
+//     sign, one 32-bit word per pair.  The words of a gate are loaded two
+//     gates ahead into registers and the barrier waits for LDS only, so their
+//     L2 latency is off the chain.
+//   * The other gates are polynomials in T (multi-frequency spin-adapted
+//     doubles).  T couples a determinant to few others: its connected
+//     components have at most kMaxComp members.  Members are ordered by their
+//     occupation of the gate's orbitals and given signs that make the
+//     component's matrix T_c one of a handful per program, so that the gate
+//     is one small matrix-vector product per component, by one thread:
+//       M_c(theta) = 1 + sum_f sin(S_f theta) D_f + (cos(S_f theta) - 1) C_f,
+//       D_f = sum_{k odd} K_kf T_c^k,  C_f = sum_{k even} K_kf T_c^k
+//     with the polynomial's frequencies S_f and coefficients K; D_f and C_f
+//     are summed on the host in long double.  T_c is antisymmetric, so the
+//     inverse gate is the transpose.
+//     (eight to ten passes of every term over every determinant per
+//     polynomial gate and vector before).
+//   * The gradient 2 <lambda|T psi> of a gate is summed per thread, reduced
+//     in each wave and added over the waves by one of them during the next
+//     gate: no extra barrier.
+//
+// Energy and gradient, per-gate kernels -> this sweep: fUCCSD (8e,8o) 3.86 ->
+// 0.46 ms, spin-adapted fUCCSD (6e,6o) 11.1 -> 0.36 ms.
+
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+#include <map>
+#include <vector>
+
+#include "sq_internal.h"
+
+namespace sq {
+
+namespace {
+
+constexpr int kST = 1024;                 // threads of the one block
+constexpr int kSW = kST / 64;             // its waves
+constexpr int kSmallDim = 8192;           // 13-bit determinant indices
+constexpr int kMaxComp = 8;               // members of a component of T
+constexpr int kChunk = 256;               // steps (and trig slots) staged in LDS at a time
+constexpr size_t kSmallEntries = 1 << 25; // pair words per program (128 MB)
+constexpr int kDiag = 1 << 16;            // flag of a diagonal matrix element
+constexpr size_t kSmallLds = 160 * 1024 - 1024;
+
+// One step: a rotation half (nf = 0: pair words [e0, e0 + n)) or a polynomial
+// gate (components [e0, e0 + n), its matrix elements [m0, m0 + mn)).  slot:
+// first trig slot within the step's chunk.
+struct SmallStep {
+  int32_t gate, nf, e0, n, slot, m0, mn, pad;
+};
+
+struct TrigSlot {
+  double scale;
+  int32_t gate, pad;
+};
+
+struct SmallChunk {
+  int32_t s0, s1, t0, t1;  // steps [s0, s1), trig slots [t0, t1)
+};
+
+}  // namespace
+
+struct SmallPlan {
+  int nchunks = 0, maxmat = 0;
+  bool poly = false;
+  SmallStep* steps = nullptr;
+  SmallChunk* chunks = nullptr;
+  TrigSlot* slots = nullptr;
+  uint32_t* pairs = nullptr;
+  uint4* members = nullptr;  // per component kMaxComp x (index | negative << 15)
+  uint32_t* meta = nullptr;  // per component: size | matrix offset << 8
+  int2* mel = nullptr;       // per matrix element of a gate: {offset into ctab, stride | kDiag}
+  double* ctab = nullptr;    // per type: T | D_0 | C_0 | D_1 | ...
+  uint8_t* nograd = nullptr; // per gate: 1 where the generator is zero (gradient 0)
+  int ngates = 0;
+  size_t lds_fwd = 0, lds_rev = 0;
+  ~SmallPlan() {
+    for (void* p : {(void*)steps, (void*)chunks, (void*)slots, (void*)pairs, (void*)members, (void*)meta, (void*)mel,
+                    (void*)ctab, (void*)nograd})
+      if (p) (void)hipFree(p);
+  }
+};
+
+void small_plan_free(SmallPlan* P) { delete P; }
+
+namespace {
+
+template <class T>
+T* put(const std::vector<T>& v) {
+  T* d = nullptr;
+  SQ_HIP(hipMalloc(&d, sizeof(T) * std::max<size_t>(v.size(), 1)));
+  if (!v.empty()) SQ_HIP(hipMemcpy(d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+  return d;
+}
+
+size_t small_lds(int64_t dim, int maxmat, bool rev) {
+  return (size_t)(dim + 1) / 2 * 16 * (rev ? 2 : 1) + (size_t)kChunk * (sizeof(double2) + sizeof(SmallStep) + 8) +
+         (size_t)maxmat * 8 * (rev ? 4 : 2);
+}
+
+// A type of component: its size, polynomial and matrix.
+struct CompType {
+  int m, slot;
+  std::vector<double> T;
+  int off;  // into ctab
+};
+
+struct Builder {
+  const Space& sp;
+  const Program& P;
+  std::vector<SmallStep> steps;
+  std::vector<SmallChunk> chunks;
+  std::vector<TrigSlot> slots;
+  std::vector<uint32_t> pairs, meta;
+  std::vector<uint4> members;
+  std::vector<int2> mel;
+  std::vector<double> ctab;
+  std::vector<uint8_t> nograd;
+  std::vector<CompType> types;
+  std::vector<int2> lists;
+  std::map<std::pair<const void*, std::vector<int>>, std::pair<int, int>> cache;
+  int maxmat = 0;
+
+  Builder(const Space& s, const Program& p) : sp(s), P(p) {}
+
+  // (determinant, image, sign) of one operator product
+  template <class F>
+  void each(const Term& T, F&& f) {
+    int ao, al, bo, bl;
+    spin_part_list(sp.h_astr, T.a, lists, cache, ao, al);
+    spin_part_list(sp.h_bstr, T.b, lists, cache, bo, bl);
+    for (int r = 0; r < al; ++r) {
+      const int2 A = ao < 0 ? int2{r, r} : lists[ao + r];
+      for (int c = 0; c < bl; ++c) {
+        const int2 B = bo < 0 ? int2{c, c} : lists[bo + c];
+        f(A.x * sp.nsb + B.x, (A.y & 0x7fffffff) * sp.nsb + (B.y & 0x7fffffff), ((A.y ^ B.y) < 0) != (T.coef < 0));
+      }
+    }
+  }
+
+  // Opens a chunk when the running one has no room for a step of nt slots.
+  int open(int nt) {
+    if (chunks.empty() || chunks.back().s1 - chunks.back().s0 >= kChunk ||
+        chunks.back().t1 - chunks.back().t0 + nt > kChunk) {
+      const int s = (int)steps.size(), t = (int)slots.size();
+      chunks.push_back(SmallChunk{s, s, t, t});
+    }
+    SmallChunk& c = chunks.back();
+    const int slot = c.t1 - c.t0;
+    c.s1 += 1;
+    c.t1 += nt;
+    return slot;
+  }
+
+  void rotation(int g, const Term& T, double scale) {
+    const int e0 = (int)pairs.size();
+    each(T, [&](int i, int j, bool neg) { pairs.push_back((uint32_t)i | (uint32_t)j << 13 | (neg ? 0x80000000u : 0u)); });
+    const int n = (int)pairs.size() - e0;
+    const int slot = open(1);
+    slots.push_back(TrigSlot{scale, g, 0});
+    steps.push_back(SmallStep{g, 0, e0, n, slot, 0, 0, 0});
+  }
+
+  int type_of(int m, int slot, const std::vector<double>& T, const GatePoly& poly) {
+    for (size_t k = 0; k < types.size(); ++k) {
+      if (types[k].m != m || types[k].slot != slot) continue;
+      bool same = true;
+      for (int e = 0; e < m * m && same; ++e) same = std::fabs(types[k].T[e] - T[e]) < 1e-14;
+      if (same) return (int)k;
+    }
+    CompType t{m, slot, T, (int)ctab.size()};
+    const int mm = m * m;
+    ctab.insert(ctab.end(), T.begin(), T.end());
+    std::vector<long double> pw(T.begin(), T.end()), nx(mm);
+    std::vector<long double> acc((size_t)2 * poly.nf * mm, 0.0L);
+    for (int k = 1; k <= poly.nk; ++k) {
+      for (int f = 0; f < poly.nf; ++f) {
+        long double* a = acc.data() + (size_t)(2 * f + ((k & 1) ? 0 : 1)) * mm;
+        for (int e = 0; e < mm; ++e) a[e] += (long double)poly.K[k - 1][f] * pw[e];
+      }
+      for (int a = 0; a < m; ++a)
+        for (int b = 0; b < m; ++b) {
+          long double v = 0.0L;
+          for (int c = 0; c < m; ++c) v += (long double)T[a * m + c] * pw[c * m + b];
+          nx[a * m + b] = v;
+        }
+      pw.swap(nx);
+    }
+    for (long double v : acc) ctab.push_back((double)v);
+    types.push_back(std::move(t));
+    return (int)types.size() - 1;
+  }
+
+  // false: a component is too large or T is not antisymmetric
+  bool polynomial(int g) {
+    const GateDev& gd = P.gates[g];
+    const GatePoly poly = gate_poly(gd);
+    struct Ent {
+      int i, j;
+      double v;
+    };
+    std::vector<Ent> ent;
+    uint32_t orbs = 0;
+    for (int t = gd.term_begin; t < gd.term_end; ++t) {
+      const Term& T = P.terms[t];
+      for (int o = 0; o < T.a.n; ++o) orbs |= 1u << T.a.orb[o];
+      for (int o = 0; o < T.b.n; ++o) orbs |= 1u << T.b.orb[o];
+      // <j|T|i>
+      each(T, [&](int i, int j, bool neg) { ent.push_back(Ent{j, i, neg ? -std::fabs(T.coef) : std::fabs(T.coef)}); });
+    }
+    std::vector<int> root(sp.dim, -1), comp(sp.dim, -1), loc(sp.dim, 0), touched;
+    auto find = [&](int x) {
+      while (root[x] != x) x = root[x] = root[root[x]];
+      return x;
+    };
+    for (const Ent& e : ent) {
+      for (int x : {e.i, e.j})
+        if (root[x] < 0) {
+          root[x] = x;
+          touched.push_back(x);
+        }
+      const int a = find(e.i), b = find(e.j);
+      if (a != b) root[std::max(a, b)] = std::min(a, b);
+    }
+    // members of a component by their occupation of the gate's orbitals
+    auto code = [&](int x) {
+      const uint64_t a = sp.h_astr[x / sp.nsb] & orbs, b = sp.h_bstr[x % sp.nsb] & orbs;
+      return a << 32 | b;
+    };
+    std::sort(touched.begin(), touched.end(), [&](int x, int y) {
+      const int rx = find(x), ry = find(y);
+      if (rx != ry) return rx < ry;
+      return code(x) < code(y);
+    });
+    struct Comp {
+      int x0, m, type;
+      uint32_t neg;
+    };
+    std::vector<Comp> comps;
+    for (int k = 0; k < (int)touched.size(); ++k) {
+      const int x = touched[k];
+      if (k == 0 || find(touched[k - 1]) != find(x)) comps.push_back(Comp{k, 0, 0, 0});
+      Comp& c = comps.back();
+      loc[x] = c.m++;
+      comp[x] = (int)comps.size() - 1;
+      if (c.m > kMaxComp) return false;
+    }
+    std::vector<double> mats(comps.size() * kMaxComp * kMaxComp, 0.0);
+    for (const Ent& e : ent) {
+      const Comp& c = comps[comp[e.i]];
+      mats[(size_t)comp[e.i] * kMaxComp * kMaxComp + loc[e.i] * c.m + loc[e.j]] += e.v;
+    }
+    for (size_t k = 0; k < comps.size(); ++k) {
+      Comp& c = comps[k];
+      double* T = mats.data() + k * kMaxComp * kMaxComp;
+      for (int a = 0; a < c.m; ++a)
+        for (int b = 0; b <= a; ++b)
+          if (T[a * c.m + b] != -T[b * c.m + a]) return false;
+      // signs: every member positive towards the member it is first reached from
+      int order[kMaxComp], n = 0;
+      bool seen[kMaxComp] = {false};
+      for (int start = 0; start < c.m; ++start) {
+        if (seen[start]) continue;
+        seen[start] = true;
+        int at = n;
+        order[n++] = start;
+        for (; at < n; ++at)
+          for (int b = 0; b < c.m; ++b) {
+            const double v = T[b * c.m + order[at]];
+            if (seen[b] || v == 0.0) continue;
+            seen[b] = true;
+            order[n++] = b;
+            const bool neg = (v < 0) != (((c.neg >> order[at]) & 1u) != 0);
+            if (neg) c.neg |= 1u << b;
+          }
+      }
+      std::vector<double> S(c.m * c.m);
+      for (int a = 0; a < c.m; ++a)
+        for (int b = 0; b < c.m; ++b) {
+          const bool neg = (((c.neg >> a) ^ (c.neg >> b)) & 1u) != 0;
+          S[a * c.m + b] = T[a * c.m + b] == 0.0 ? 0.0 : (neg ? -T[a * c.m + b] : T[a * c.m + b]);
+        }
+      c.type = type_of(c.m, gd.kind * 16 + gd.poly, S, poly);
+    }
+    std::stable_sort(comps.begin(), comps.end(), [](const Comp& a, const Comp& b) { return a.type < b.type; });
+    const int m0 = (int)mel.size(), c0 = (int)meta.size();
+    int moff = -1, last = -1, used = 0;
+    for (const Comp& c : comps) {
+      const CompType& t = types[c.type];
+      if (c.type != last) {
+        last = c.type;
+        moff = used;
+        for (int e = 0; e < t.m * t.m; ++e)
+          mel.push_back(int2{t.off + e, t.m * t.m | (e % (t.m + 1) == 0 ? kDiag : 0)});
+        used += t.m * t.m;
+      }
+      uint16_t w[kMaxComp] = {0};
+      for (int a = 0; a < c.m; ++a)
+        w[a] = (uint16_t)((uint32_t)touched[c.x0 + a] | ((c.neg >> a) & 1u) << 15);
+      auto two = [&](int a) { return (uint32_t)w[a] | (uint32_t)w[a + 1] << 16; };
+      members.push_back(make_uint4(two(0), two(2), two(4), two(6)));
+      meta.push_back((uint32_t)c.m | (uint32_t)moff << 8);
+    }
+    maxmat = std::max(maxmat, used);
+    const int slot = open(poly.nf);
+    for (int f = 0; f < poly.nf; ++f) slots.push_back(TrigSlot{poly.S[f], g, 0});
+    steps.push_back(SmallStep{g, poly.nf, c0, (int)comps.size(), slot, m0, used, 0});
+    return true;
+  }
+
+  bool build() {
+    nograd.assign(P.gates.size(), 0);
+    for (int g = 0; g < (int)P.gates.size(); ++g) {
+      const GateDev& gd = P.gates[g];
+      if (gd.kind == GC_ROT) {
+        rotation(g, P.terms[gd.term_begin], gd.scale);
+      } else if (gd.kind == GC_SA_SINGLE) {
+        rotation(g, P.terms[gd.term_begin], 1.0);
+        rotation(g, P.terms[gd.term_begin + 2], 1.0);
+      } else if (gd.term_end == gd.term_begin) {
+        nograd[g] = 1;
+      } else if (!polynomial(g)) {
+        return false;
+      }
+      if (pairs.size() > kSmallEntries || meta.size() > kSmallEntries / 8) return false;
+    }
+    return true;
+  }
+};
+
+// ---- device ---------------------------------------------------------------------
+
+struct SmallDev {
+  const SmallStep* steps;
+  const SmallChunk* chunks;
+  const TrigSlot* slots;
+  const uint32_t* pairs;
+  const uint4* members;
+  const uint32_t* meta;
+  const int2* mel;
+  const double* ctab;
+  const uint8_t* nograd;
+  int nchunks, dim, maxmat, ngates;
+};
+
+// What a thread needs of a step, loaded ahead: the step's record and trig
+// values, and its first two pairs or its first component.
+struct Ahead {
+  int gate, nf, e0, n;
+  double c, sn, scale;
+  uint32_t p0, p1, meta;
+  uint4 mem;
+};
+
+// Waits for this wave's LDS operations only: loads issued ahead stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
+
+// Sum over each row of 16 lanes, in the row's last lane.
+__device__ __forceinline__ double row16_sum(double v) {
+  v = dpp_add<0xb1>(v);   // quad_perm [1,0,3,2]
+  v = dpp_add<0x4e>(v);   // quad_perm [2,3,0,1]
+  v = dpp_add<0x114>(v);  // row_shr:4
+  return dpp_add<0x118>(v);
+}
+
+// The matrix of one component (M: the gate, T: its generator, both m x m at
+// LDS) on its members; the transpose where inv.  Returns <lam|T psi> (REV).
+template <int m, bool REV>
+__device__ __forceinline__ double comp_apply(double* X, double* L, const double* __restrict__ M,
+                                             const double* __restrict__ T, const uint4& mem, bool inv) {
+  const uint32_t w[4] = {mem.x, mem.y, mem.z, mem.w};
+  int at[m];
+  double s[m], x[m], l[m];
+#pragma unroll
+  for (int a = 0; a < m; ++a) {
+    const uint32_t h = (w[a >> 1] >> (16 * (a & 1))) & 0xffffu;
+    at[a] = (int)(h & 0x7fffu);
+    s[a] = (h & 0x8000u) ? -1.0 : 1.0;
+    x[a] = s[a] * X[at[a]];
+    if (REV) l[a] = s[a] * L[at[a]];
+  }
+  double dot = 0.0;
+#pragma unroll
+  for (int a = 0; a < m; ++a) {
+    double vx = 0.0, vl = 0.0, vt = 0.0;
+#pragma unroll
+    for (int b = 0; b < m; ++b) {
+      const double e = inv ? M[b * m + a] : M[a * m + b];
+      vx += e * x[b];
+      if (REV) {
+        vl += e * l[b];
+        vt += T[a * m + b] * x[b];
+      }
+    }
+    X[at[a]] = s[a] * vx;
+    if (REV) {
+      L[at[a]] = s[a] * vl;
+      dot += l[a] * vt;
+    }
+  }
+  return dot;
+}
+
+template <bool REV>
+__device__ __forceinline__ double comp_any(double* X, double* L, const double* M, const double* T, uint32_t meta,
+                                           const uint4& mem, bool inv) {
+  const double* Mc = M + (meta >> 8);
+  const double* Tc = T + (meta >> 8);
+  switch (meta & 255u) {
+    case 2: return comp_apply<2, REV>(X, L, Mc, Tc, mem, inv);
+    case 3: return comp_apply<3, REV>(X, L, Mc, Tc, mem, inv);
+    case 4: return comp_apply<4, REV>(X, L, Mc, Tc, mem, inv);
+    case 5: return comp_apply<5, REV>(X, L, Mc, Tc, mem, inv);
+    case 6: return comp_apply<6, REV>(X, L, Mc, Tc, mem, inv);
+    case 7: return comp_apply<7, REV>(X, L, Mc, Tc, mem, inv);
+    case 8: return comp_apply<8, REV>(X, L, Mc, Tc, mem, inv);
+    default: return 0.0;  // a single member: T = 0
+  }
+}
+
+// REV = false: dst = U src (back: U^+ src).  REV = true: the reverse sweep on
+// (src = psi, lam), gradients to grad; back is then true.
+// Bound by the chain of barriers and LDS round trips, one per gate: the block
+// uses one CU, and a gate's arithmetic is a few hundred cycles of it.
+template <bool REV, bool POLY>
+__global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* __restrict__ theta, const double* src,
+                                                     double* dst, const double* __restrict__ lam,
+                                                     double* __restrict__ grad, int back) {
+  extern __shared__ double smem[];
+  __shared__ double red[2][kSW];
+  double* X = smem;
+  const int dimp = (S.dim + 1) & ~1;  // 16-byte alignment of what follows
+  double* L = X + (REV ? dimp : 0);
+  double2* cs = reinterpret_cast<double2*>(L + dimp);
+  SmallStep* steps = reinterpret_cast<SmallStep*>(cs + kChunk);
+  double* scales = reinterpret_cast<double*>(steps + kChunk);
+  double* mats = scales + kChunk;  // [2][maxmat] gate matrices | [2][maxmat] generators
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool inv = REV || back;
+  for (int i = tid; i < S.dim; i += kST) {
+    X[i] = src[i];
+    if (REV) L[i] = lam[i];
+  }
+  if (REV)
+    for (int g = tid; g < S.ngates; g += kST)
+      if (S.nograd[g]) grad[g] = 0.0;
+  // the running sum of the gate whose steps are being reduced
+  int par = 0;
+  int done_gate = -1;   // gate of the previous step
+  double done_sum = 0.0;
+  for (int ci = 0; ci < S.nchunks; ++ci) {
+    const SmallChunk C = S.chunks[inv ? S.nchunks - 1 - ci : ci];
+    __syncthreads();
+    for (int i = tid; i < C.s1 - C.s0; i += kST) steps[i] = S.steps[C.s0 + i];
+    for (int i = tid; i < C.t1 - C.t0; i += kST) {
+      const TrigSlot t = S.slots[C.t0 + i];
+      const double th = theta[t.gate];
+      double sn = 0.0, c = 1.0;
+      if (fabs(th) >= 1e-28) sincos(t.scale * th, &sn, &c);
+      cs[i] = double2{c, sn};
+      scales[i] = t.scale;
+    }
+    __syncthreads();
+    const int ns = C.s1 - C.s0;
+    auto step_at = [&](int k) { return inv ? ns - 1 - k : k; };
+    auto load = [&](int k, Ahead& a) {
+      if (k >= ns) return;
+      const SmallStep s = steps[step_at(k)];
+      a.gate = __builtin_amdgcn_readfirstlane(s.gate);
+      a.nf = __builtin_amdgcn_readfirstlane(s.nf);
+      a.e0 = __builtin_amdgcn_readfirstlane(s.e0);
+      a.n = __builtin_amdgcn_readfirstlane(s.n);
+      if (!POLY || a.nf == 0) {
+        const double2 x = cs[s.slot];
+        a.c = x.x;
+        a.sn = inv ? -x.y : x.y;
+        a.scale = scales[s.slot];
+        if (tid < a.n) a.p0 = S.pairs[a.e0 + tid];
+        if (tid + kST < a.n) a.p1 = S.pairs[a.e0 + tid + kST];
+      } else if (tid < a.n) {
+        a.meta = S.meta[a.e0 + tid];
+        a.mem = S.members[a.e0 + tid];
+      }
+    };
+    // the matrices of step k into buffer k & 1
+    auto matrices = [&](int k) {
+      if (!POLY || k >= ns) return;
+      const SmallStep& s = steps[step_at(k)];
+      const int nf = __builtin_amdgcn_readfirstlane(s.nf);
+      if (nf == 0) return;
+      const int mn = __builtin_amdgcn_readfirstlane(s.mn), m0 = __builtin_amdgcn_readfirstlane(s.m0);
+      const int sl = __builtin_amdgcn_readfirstlane(s.slot);
+      for (int e = tid; e < mn; e += kST) {
+        const int2 me = S.mel[m0 + e];
+        const double* c = S.ctab + me.x;
+        const int mm = me.y & (kDiag - 1);
+        double v = (me.y & kDiag) ? 1.0 : 0.0;
+        for (int f = 0; f < nf; ++f) {
+          const double2 x = cs[sl + f];
+          v += x.y * c[(2 * f + 1) * mm] + (x.x - 1.0) * c[(2 * f + 2) * mm];
+        }
+        mats[(k & 1) * S.maxmat + e] = v;
+        if (REV) mats[(2 + (k & 1)) * S.maxmat + e] = c[0];
+      }
+    };
+    auto rotate = [&](uint32_t p, double c, double sn, double& dot) {
+      const int i = (int)(p & 8191u), j = (int)((p >> 13) & 8191u);
+      const double sg = (p >> 31) ? -sn : sn;
+      const double xi = X[i], xj = X[j];
+      X[i] = c * xi - sg * xj;
+      X[j] = sg * xi + c * xj;
+      if (REV) {
+        const double li = L[i], lj = L[j];
+        L[i] = c * li - sg * lj;
+        L[j] = sg * li + c * lj;
+        const double d = lj * xi - li * xj;
+        dot += (p >> 31) ? -d : d;
+      }
+    };
+    // one wave adds the previous step's wave sums to its gate's gradient
+    auto finish = [&](int gate_now) {
+      if (!REV || done_gate < 0) return;
+      if (wave == 0) {
+        double v = lane < kSW ? red[par ^ 1][lane & (kSW - 1)] : 0.0;
+        v = row16_sum(v);
+        done_sum += v;
+        if (gate_now != done_gate) {
+          if (lane == 15) grad[done_gate] = 2.0 * done_sum;
+          done_sum = 0.0;
+        }
+      }
+    };
+    auto step = [&](int k, Ahead& cur, Ahead& fill) {
+      if (k >= ns) return;
+      lds_barrier();
+      load(k + 2, fill);
+      const int n = cur.n, gate = cur.gate, e0 = cur.e0;
+      double dot = 0.0;
+      if (!POLY || cur.nf == 0) {
+        if (tid < n) rotate(cur.p0, cur.c, cur.sn, dot);
+        if (tid + kST < n) rotate(cur.p1, cur.c, cur.sn, dot);
+        for (int i = tid + 2 * kST; i < n; i += kST) rotate(S.pairs[e0 + i], cur.c, cur.sn, dot);
+        if (REV) dot *= cur.scale;
+      } else {
+        const double* M = mats + (k & 1) * S.maxmat;
+        const double* T = mats + (2 + (k & 1)) * S.maxmat;
+        if (tid < n) dot += comp_any<REV>(X, L, M, T, cur.meta, cur.mem, inv);
+        for (int i = tid + kST; i < n; i += kST)
+          dot += comp_any<REV>(X, L, M, T, S.meta[e0 + i], S.members[e0 + i], inv);
+      }
+      matrices(k + 1);
+      if (REV) {
+        finish(gate);
+        dot = row16_sum(dot);
+        dot += __shfl_xor(dot, 16, 64);
+        dot += __shfl_xor(dot, 32, 64);
+        if (lane == 63) red[par][wave] = dot;
+        done_gate = gate;
+        par ^= 1;
+      }
+    };
+    Ahead a, b, c;
+    load(0, a);
+    load(1, b);
+    matrices(0);
+    for (int k = 0; k < ns; k += 3) {
+      step(k, a, c);
+      step(k + 1, b, a);
+      step(k + 2, c, b);
+    }
+  }
+  __syncthreads();
+  if (REV) {
+    if (done_gate >= 0 && wave == 0) {
+      double v = lane < kSW ? red[par ^ 1][lane & (kSW - 1)] : 0.0;
+      v = row16_sum(v);
+      if (lane == 15) grad[done_gate] = 2.0 * (done_sum + v);
+    }
+  } else {
+    for (int i = tid; i < S.dim; i += kST) dst[i] = X[i];
+  }
+}
+
+SmallDev device_view(const Space& s, const SmallPlan& P) {
+  return SmallDev{P.steps, P.chunks, P.slots, P.pairs, P.members, P.meta, P.mel, P.ctab, P.nograd,
+                  P.nchunks, (int)s.dim, P.maxmat, P.ngates};
+}
+
+}  // namespace
+
+// The plan of a program whose state vectors fit one block's LDS, nullptr
+// where the sweep does not apply: larger spaces, polynomial gates with larger
+// components, or programs that run in tile stages from the first gate to the
+// last (a stage spreads over many CUs and takes about 1 us per orbital pair).
+const SmallPlan* small_for(const Space& s, const Program& p) {
+  if (!p.small_tried) {
+    p.small_tried = true;
+    const char* env = getenv("SQ_SMALL_SWEEP");
+    if ((env && env[0] == '0') || s.dim == 0 || s.dim > kSmallDim || p.gates.empty()) return nullptr;
+    if (tiles_cover(s, p)) return nullptr;
+    Builder B(s, p);
+    if (!B.build()) return nullptr;
+    const size_t lds_rev = small_lds(s.dim, B.maxmat, true);
+    if (lds_rev > kSmallLds) return nullptr;
+    auto* P = new SmallPlan();
+    try {
+      P->nchunks = (int)B.chunks.size();
+      P->maxmat = B.maxmat;
+      P->poly = !B.meta.empty();
+      P->steps = put(B.steps);
+      P->chunks = put(B.chunks);
+      P->slots = put(B.slots);
+      P->pairs = put(B.pairs);
+      P->members = put(B.members);
+      P->meta = put(B.meta);
+      P->mel = put(B.mel);
+      P->ctab = put(B.ctab);
+      P->nograd = put(B.nograd);
+      P->ngates = (int)p.gates.size();
+      P->lds_fwd = small_lds(s.dim, B.maxmat, false);
+      P->lds_rev = lds_rev;
+    } catch (...) {
+      delete P;
+      throw;
+    }
+    p.small = P;
+  }
+  return p.small;
+}
+
+void small_forward(const Space& s, const SmallPlan& P, const double* theta, const double* psi_in, double* psi,
+                   bool dagger, hipStream_t st) {
+  const SmallDev D = device_view(s, P);
+  auto* kernel = P.poly ? k_small_sweep<false, true> : k_small_sweep<false, false>;
+  allow_lds(kernel, P.lds_fwd);
+  SQ_PROF(PC_SMALL, st, 16.0 * (double)s.dim, 0.0,
+          kernel<<<1, kST, P.lds_fwd, st>>>(D, theta, psi_in, psi, nullptr, nullptr, dagger ? 1 : 0));
+}
+
+void small_reverse(const Space& s, const SmallPlan& P, const double* theta, const double* psi, const double* lam,
+                   double* grad, hipStream_t st) {
+  const SmallDev D = device_view(s, P);
+  auto* kernel = P.poly ? k_small_sweep<true, true> : k_small_sweep<true, false>;
+  allow_lds(kernel, P.lds_rev);
+  SQ_PROF(PC_SMALL, st, 16.0 * (double)s.dim, 0.0,
+          kernel<<<1, kST, P.lds_rev, st>>>(D, theta, psi, nullptr, lam, grad, 1));
+}
+
+}  // namespace sq

@@ -708,6 +708,14 @@ const TilePlan* tiles_for(const Space& s, const Program& p) {
   return p.tiles;
 }
 
+bool tiles_cover(const Space& s, const Program& p) {
+  const TilePlan* T = tiles_for(s, p);
+  if (!T) return false;
+  for (const Stage& S : T->stages)
+    if (!S.tiled) return false;
+  return true;
+}
+
 // ---------------------------------------------------------------------------
 // Device kernels.
 //
