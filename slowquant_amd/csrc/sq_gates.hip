@@ -808,7 +808,7 @@ int sq_program_destroy(sq_program* pr) {
     if (pr->p.d_terms) (void)hipFree(pr->p.d_terms);
     if (pr->p.d_lists) (void)hipFree(pr->p.d_lists);
     if (pr->p.d_term_fast) (void)hipFree(pr->p.d_term_fast);
-    if (pr->p.ucc_csr) ucc_csr_free(pr->p.ucc_csr);
+    if (pr->p.ucc_t) ucc_t_free(pr->p.ucc_t);
     if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
     if (pr->p.small) small_plan_free(pr->p.small);
     delete pr;

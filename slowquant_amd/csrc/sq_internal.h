@@ -140,6 +140,7 @@ void build_row_tables(Space& s);
 void free_row_tables(Space& s);
 
 struct TilePlan;
+struct UccCsr;
 TilePlan* build_tile_plan(const Space& sp, const struct Program& P);
 void destroy_tile_plan(TilePlan* T);
 bool tile_plan_has_tiles(const TilePlan* T);
@@ -169,14 +170,13 @@ struct Program {
   // Per term, its adjoint in mask form (built on first use by the UCC
   // kernels, sq_ucc.hip).
   mutable struct TermFast* d_term_fast = nullptr;
-  // T's sparsity pattern as rows of (source determinant, term | sign) entries
-  // (built on first use by the UCC kernels, sq_ucc.hip; freed by
-  // ucc_csr_free).
-  mutable struct UccCsr* ucc_csr = nullptr;
-  mutable bool ucc_csr_tried = false;
+  // T's merged sparsity pattern (built on first use by the UCC kernels,
+  // sq_ucc.hip; freed by ucc_t_free).
+  mutable struct UccT* ucc_t = nullptr;
+  mutable bool ucc_t_tried = false;
 };
 
-void ucc_csr_free(struct UccCsr* c);
+void ucc_t_free(struct UccT* t);
 
 // Strings a spin part applies to, as (string index, image | parity << 31)
 // entries appended to lists (shared per (strings, operator) through cache);

@@ -4,19 +4,48 @@
 // gradient of ucc_wavefunction.py:1025-1098).
 //
 // T(theta) = sum_k theta_k T_k with every gate generator T_k taken from the
-// program's raw terms; exp(t T) v is applied matrix-free by a scaled Taylor
-// series: s steps of exp(t T / s) with |t| nu / s <= 2 and K terms per step
-// until (|t| nu / s)^K / K! < 2^-60, where nu bounds ||T||_2 (a power-iteration
-// estimate with margin, capped by the triangle-inequality bound).
+// program's raw terms.  T's sparsity pattern does not depend on theta: it is
+// built once per program on the device (k_csr_count / k_csr_fill, rows of
+// (source determinant, term, sign)), the entries of a row are sorted by
+// source, and those that share one are merged (k_row_sort, k_row_merge):
+// spin-adapted doubles give about five entries per matrix element.  An
+// evaluation then assembles the numbers of T(theta) once (k_assemble) and
+// every product is a plain sparse matrix-vector product over merged elements
+// (k_spmv, 12 bytes each).
+//
+// exp(t T) v is a combination of K basis vectors, kept so that one series
+// gives the state at every t in [0, 1] (k_combine).  The first kNormSteps
+// products run at once on v and on a fixed pseudo-random vector (k_spmv's two
+// columns); the latter's growth estimates ||T||_2 as a power iteration does,
+// nu = 1.5 x the estimate + 0.05, at most the largest row sum of |T(theta)|
+// (a rigorous bound the assembly yields).  Up to |t| nu = 2 the first column
+// is the head of the Taylor series (the largest term is 2: one bit), which
+// goes on to K terms with (|t| nu)^K / K! < 2^-60.  Above, the Chebyshev
+// series of the exponential takes over: T = i A with A Hermitian, so
+//   exp(t T) = sum_k (2 - delta_k0) J_k(t nu) phi_k,   phi_0 = 1,
+//   phi_1 = T / nu,  phi_{k+1} = (2 T / nu) phi_k + phi_{k-1},
+// where |phi_k v| <= |v|: no term exceeds the result and about nu / 2 times
+// fewer products are needed than in Taylor steps of radius 2.
+// Energy and gradient of UCCSD, one product per unmerged entry (8 bytes each)
+// in Taylor steps -> this: (8e,8o) 663 -> 400 us (44 products of 4-5 us: launch
+// latency), (10e,10o) 13.5 -> 2.5 ms (9.1 M merged elements of 44 M entries;
+// a product takes 31 us, 105 us before, bound by the gathers of the vector).
+// The first evaluation of a program, which builds the pattern: (10e,10o) 202
+// -> 8.9 ms.
 // The analytic gradient integrates <e^{-sT} lam | T_i | e^{-sT} psi> over
-// s in [0, 1] by composite Gauss-Legendre (lam = H psi), all gates per node.
-// T's sparsity pattern does not depend on theta: it is built once per program
-// (rows of (source determinant, term, sign)) and every T application is then
-// one weighted sparse matrix-vector product; patterns above 2^29 entries fall
-// back to kernels that rescan the terms per determinant.
+// s in [0, 1] by Gauss-Legendre (lam = H psi): the nodes of psi come from the
+// forward series, those of lam from one more series, and one pass over the
+// pattern forms the weighted sum over nodes of V_q[I] U_q[J] per merged
+// element and adds it to the gates of its entries (k_gate_dots_rows).
+//
+// Patterns above 2^29 entries, and SQ_UCC_CSR=0, keep a scaled Taylor series
+// whose products rescan the terms per determinant (tapply).
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "sq_internal.h"
@@ -211,61 +240,278 @@ __global__ __launch_bounds__(64 * kCsrRows) void k_tapply_csr(int64_t dim, const
   }
 }
 
-// Node outputs of one multi-node Taylor series: per vector, kNodes states
-// (the 8 Gauss-Legendre nodes of a subinterval and its end) at out + q * dim,
-// and the weight of the current Taylor term for each.
-constexpr int kNodes = 9;
-struct NodeW {
-  double r[kNodes];
-};
+// ---- merged pattern -------------------------------------------------------
 
-// Two vectors through the same T in one pass over the pattern:
-// nxt_v = f T cur_v (v = 0, 1) and out_v[q][I] += r_q nxt_v[I] for q < kNodes.
-// One wave per row as k_tapply_csr (same summation order); after the wave
-// sum, lanes q and 32 + q (q < kNodes) update node q of vector 0 and 1.
-__global__ __launch_bounds__(64 * kCsrRows) void k_tapply_csr2(
-    int64_t dim, const int64_t* __restrict__ rowp, const uint2* __restrict__ ent, const double* __restrict__ coef,
-    const double* __restrict__ w, const double* __restrict__ cur0, const double* __restrict__ cur1, double f,
-    double* __restrict__ nxt0, double* __restrict__ nxt1, double* __restrict__ out0, double* __restrict__ out1,
-    NodeW nw) {
-  const int lane = threadIdx.x & 63;
-  const int64_t I = (int64_t)blockIdx.x * kCsrRows + (threadIdx.x >> 6);
-  if (I >= dim) return;  // uniform per wave; no block barrier below
-  const int64_t b = rowp[I], e = rowp[I + 1];
-  double v0 = 0.0, v1 = 0.0;
-  for (int64_t k = b + lane; k < e; k += 64) {
-    const uint2 x = ent[k];
-    const uint32_t t = x.y & 0x7fffffffu;
-    const double wc = w[t] * coef[t];
-    const double c0 = wc * cur0[x.x], c1 = wc * cur1[x.x];
-    v0 += (x.y >> 31) ? -c0 : c0;
-    v1 += (x.y >> 31) ? -c1 : c1;
+// One contribution to a merged element: gate | index of |coefficient| << 24 |
+// negative << 31.
+constexpr int kGateBits = 24, kCoefBits = 7;
+constexpr int kSortRow = 8192;  // longest row sorted in LDS (64 KB of keys); longer rows merge neighbours only
+
+// Sorts row I's entries by (source, term) in place (bitonic, keys
+// source << 32 | term << 1 | sign) and counts the distinct sources.
+__global__ __launch_bounds__(kUB) void k_row_sort(const int64_t* __restrict__ rowp, uint2* __restrict__ ent,
+                                                  int32_t* __restrict__ ucnt) {
+  extern __shared__ uint64_t key[];
+  __shared__ int red[kUB / 64];
+  const int64_t b = rowp[blockIdx.x];
+  const int n = (int)(rowp[blockIdx.x + 1] - b);
+  const int tid = threadIdx.x;
+  int c = 0;
+  if (n <= kSortRow) {
+    int P = 1;
+    while (P < n) P <<= 1;
+    for (int i = tid; i < P; i += kUB) {
+      uint64_t k = ~0ull;
+      if (i < n) {
+        const uint2 e = ent[b + i];
+        k = (uint64_t)e.x << 32 | (uint64_t)(e.y & 0x7fffffffu) << 1 | (e.y >> 31);
+      }
+      key[i] = k;
+    }
+    for (int k = 2; k <= P; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        __syncthreads();
+        for (int i = tid; i < P; i += kUB) {
+          const int o = i ^ j;
+          if (o <= i) continue;
+          const uint64_t x = key[i], y = key[o];
+          if ((x > y) == ((i & k) == 0)) {
+            key[i] = y;
+            key[o] = x;
+          }
+        }
+      }
+    __syncthreads();
+    for (int i = tid; i < n; i += kUB) {
+      const uint64_t x = key[i];
+      ent[b + i] = make_uint2((uint32_t)(x >> 32), (uint32_t)(x >> 1 & 0x7fffffffu) | (uint32_t)(x & 1) << 31);
+      c += i == 0 || (uint32_t)(key[i - 1] >> 32) != (uint32_t)(x >> 32);
+    }
+  } else {
+    for (int i = tid; i < n; i += kUB) c += i == 0 || ent[b + i - 1].x != ent[b + i].x;
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    v0 += __shfl_down(v0, off, 64);
-    v1 += __shfl_down(v1, off, 64);
-  }
-  v0 = f * __shfl(v0, 0, 64);
-  v1 = f * __shfl(v1, 0, 64);
-  if (lane == 0) nxt0[I] = v0;
-  if (lane == 32) nxt1[I] = v1;
-  const int q = lane & 31;
-  if (q < kNodes) {
-    double* o = (lane < 32 ? out0 : out1) + (size_t)q * dim + I;
-    *o += nw.r[q] * (lane < 32 ? v0 : v1);
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off, 64);
+  if ((tid & 63) == 0) red[tid >> 6] = c;
+  __syncthreads();
+  if (tid == 0) {
+    int tot = 0;
+    for (int w = 0; w < kUB / 64; ++w) tot += red[w];
+    ucnt[blockIdx.x] = tot;
   }
 }
 
-// out_v[q][I] = base_v[I] for q < kNodes (the k = 0 term of every node).
-__global__ void k_nodes_init(int64_t dim, const double* __restrict__ b0, const double* __restrict__ b1,
-                             double* __restrict__ out0, double* __restrict__ out1) {
-  const int64_t I = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+// Merged elements of row I at [urow[I], urow[I + 1]): source and first
+// contribution; every entry's contribution word.  One wave per row.
+constexpr int kRows = 4;  // rows (waves) per block
+__global__ __launch_bounds__(64 * kRows) void k_row_merge(int64_t dim, const int64_t* __restrict__ rowp,
+                                                          const uint2* __restrict__ ent,
+                                                          const uint32_t* __restrict__ tword,
+                                                          const int64_t* __restrict__ urow, uint32_t* __restrict__ col,
+                                                          uint32_t* __restrict__ first, uint32_t* __restrict__ con) {
+  const int lane = threadIdx.x & 63;
+  const int64_t I = (int64_t)blockIdx.x * kRows + (threadIdx.x >> 6);
   if (I >= dim) return;
-  const double x0 = b0[I], x1 = b1[I];
-  for (int q = 0; q < kNodes; ++q) {
-    out0[(size_t)q * dim + I] = x0;
-    out1[(size_t)q * dim + I] = x1;
+  const int64_t b = rowp[I], e = rowp[I + 1];
+  int64_t u = urow[I];
+  for (int64_t k0 = b; k0 < e; k0 += 64) {
+    const int64_t k = k0 + lane;
+    uint2 x = make_uint2(0, 0);
+    bool head = false;
+    if (k < e) {
+      x = ent[k];
+      head = k == b || ent[k - 1].x != x.x;
+      con[k] = tword[x.y & 0x7fffffffu] ^ (x.y & 0x80000000u);
+    }
+    const uint64_t m = __ballot(head);
+    if (head) {
+      const int64_t at = u + __popcll(m & ((1ull << lane) - 1ull));
+      col[at] = x.x;
+      first[at] = (uint32_t)k;
+    }
+    u += __popcll(m);
   }
+}
+
+// val[u] = sum over the contributions of merged element u of sign theta[gate]
+// |coef|; rmax[block]: largest sum of |val| over the block's rows.  One wave
+// per row.  theta and the coefficients are read from LDS when theta fits
+// (ng <= kLdsGates).
+constexpr int kLdsGates = 4096;
+__global__ __launch_bounds__(64 * kRows) void k_assemble(int64_t dim, const int64_t* __restrict__ urow,
+                                                         const uint32_t* __restrict__ first,
+                                                         const uint32_t* __restrict__ con,
+                                                         const double* __restrict__ coefs, int ncoef,
+                                                         const double* __restrict__ theta, int ng,
+                                                         double* __restrict__ val, double* __restrict__ rmax) {
+  extern __shared__ double sth[];
+  __shared__ double sc[1 << kCoefBits];
+  __shared__ double red[kRows];
+  const bool lds = ng <= kLdsGates;
+  if (lds)
+    for (int i = threadIdx.x; i < ng; i += 64 * kRows) sth[i] = theta[i];
+  for (int i = threadIdx.x; i < ncoef; i += 64 * kRows) sc[i] = coefs[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double most = 0.0;
+  for (int64_t I = (int64_t)blockIdx.x * kRows + wave; I < dim; I += (int64_t)gridDim.x * kRows) {
+    const int64_t b = urow[I], e = urow[I + 1];
+    double sum = 0.0;
+    for (int64_t u = b + lane; u < e; u += 64) {
+      const uint32_t c0 = first[u], c1 = first[u + 1];
+      double v = 0.0;
+      for (uint32_t c = c0; c < c1; ++c) {
+        const uint32_t w = con[c];
+        const uint32_t g = w & ((1u << kGateBits) - 1u);
+        const double x = (lds ? sth[g] : theta[g]) * sc[(w >> kGateBits) & ((1u << kCoefBits) - 1u)];
+        v += (w >> 31) ? -x : x;
+      }
+      val[u] = v;
+      sum += fabs(v);
+    }
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    most = sum > most || sum != sum ? sum : most;
+  }
+  if (lane == 0) red[wave] = most;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kRows; ++w) most = red[w] > most || red[w] != red[w] ? red[w] : most;
+    rmax[blockIdx.x] = most;
+  }
+}
+
+// out = max of n values (NaN if one is).
+__global__ __launch_bounds__(kUB) void k_max(const double* __restrict__ x, int n, double* __restrict__ out) {
+  __shared__ double red[kUB / 64];
+  double m = 0.0;
+  for (int i = threadIdx.x; i < n; i += kUB) m = x[i] > m || x[i] != x[i] ? x[i] : m;
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_xor(m, off, 64);
+    m = o > m || o != o ? o : m;
+  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kUB / 64; ++w) m = red[w] > m || red[w] != red[w] ? red[w] : m;
+    out[0] = m;
+  }
+}
+
+// nxt[I] = f (T cur)[I] + prev[I] (prev: nullptr for none), LPR lanes per row;
+// TWO: nxt2 = f T cur2 in the same pass.  With bound, f is divided by
+// bound[0] (0 where that is 0).  A row's first four rounds of elements are
+// loaded before any is used.
+// Bound by the pattern's 12 bytes per element where it leaves the caches, by
+// launch latency below about 10^5 elements.  LPR: the smallest power of two
+// that takes an average row in two rounds (idle lanes of short rows against
+// the length of the shuffle tree).
+template <int LPR, bool TWO>
+__global__ __launch_bounds__(kUB) void k_spmv(int64_t dim, const int64_t* __restrict__ urow,
+                                              const uint32_t* __restrict__ col, const double* __restrict__ val,
+                                              const double* __restrict__ cur, const double* __restrict__ cur2,
+                                              const double* __restrict__ prev, double f,
+                                              const double* __restrict__ bound, double* __restrict__ nxt,
+                                              double* __restrict__ nxt2) {
+  constexpr int U = 4;
+  const int lane = threadIdx.x & (LPR - 1);
+  const int64_t I = (int64_t)blockIdx.x * (kUB / LPR) + threadIdx.x / LPR;
+  if (I >= dim) return;
+  if (bound) f = bound[0] > 0.0 ? f / bound[0] : 0.0;
+  const int64_t b = urow[I], e = urow[I + 1];
+  double v = 0.0, v2 = 0.0;
+  for (int64_t u0 = b + lane; u0 < e; u0 += U * LPR) {
+    double a[U];
+    uint32_t c[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int64_t u = u0 + j * LPR;
+      a[j] = u < e ? val[u] : 0.0;
+      c[j] = u < e ? col[u] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      if (u0 + j * LPR >= e) break;
+      v += a[j] * cur[c[j]];
+      if (TWO) v2 += a[j] * cur2[c[j]];
+    }
+  }
+#pragma unroll
+  for (int off = LPR / 2; off > 0; off >>= 1) {
+    v += __shfl_down(v, off, LPR);
+    if (TWO) v2 += __shfl_down(v2, off, LPR);
+  }
+  if (lane == 0) {
+    nxt[I] = f * v + (prev ? prev[I] : 0.0);
+    if (TWO) nxt2[I] = f * v2;
+  }
+}
+
+// Linear combinations of the basis vectors phi_k (k <= K, at basis + k dim):
+// node q (q < nq) to nodes[I * stride + q], output nq (if fin) to fin[I].
+constexpr int kMaxOut = 9, kMaxBasis = 44, kCB = 64;
+struct Combine {
+  double c[kMaxOut][kMaxBasis];
+};
+
+__global__ __launch_bounds__(kCB) void k_combine(int64_t dim, int K, Combine C, int nq, const double* __restrict__ basis,
+                                                 double* __restrict__ nodes, int stride, double* __restrict__ fin) {
+  const int64_t I = blockIdx.x * (int64_t)kCB + threadIdx.x;
+  if (I >= dim) return;
+  double o[kMaxOut];
+#pragma unroll
+  for (int q = 0; q < kMaxOut; ++q) o[q] = 0.0;
+#pragma unroll 4
+  for (int k = K; k >= 0; --k) {  // small terms first
+    const double x = basis[(size_t)k * dim + I];
+#pragma unroll
+    for (int q = 0; q < kMaxOut; ++q) o[q] += C.c[q][k] * x;
+  }
+#pragma unroll
+  for (int q = 0; q < kMaxOut - 1; ++q)
+    if (q < nq) nodes[(size_t)I * stride + q] = o[q];
+  if (fin) fin[I] = o[kMaxOut - 1];
+}
+
+// Gate dots: per merged element (I, J) r = sum_q V[I][q] U[J][q] over NQ
+// nodes (V carries the weights), added with sign |coef| to every
+// contribution's gate.  Gate sums in LDS per block, then to dpart[block][ng];
+// with more gates than LDS holds (lds = 0) to dpart[0][ng] by global atomics
+// (zeroed before).  One wave per row; a node row is 64 to 128 contiguous
+// bytes.
+template <int NQ>
+__global__ __launch_bounds__(64 * kRows) void k_gate_dots_rows(
+    int64_t dim, const int64_t* __restrict__ urow, const uint32_t* __restrict__ col,
+    const uint32_t* __restrict__ first, const uint32_t* __restrict__ con, const double* __restrict__ coefs, int ncoef,
+    const double* __restrict__ U, const double* __restrict__ V, int ng, int lds, double* __restrict__ dpart) {
+  extern __shared__ double sg[];
+  __shared__ double sc[1 << kCoefBits];
+  if (lds)
+    for (int i = threadIdx.x; i < ng; i += 64 * kRows) sg[i] = 0.0;
+  for (int i = threadIdx.x; i < ncoef; i += 64 * kRows) sc[i] = coefs[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int64_t I = (int64_t)blockIdx.x * kRows + wave; I < dim; I += (int64_t)gridDim.x * kRows) {
+    const int64_t e = urow[I + 1];
+    double v[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) v[q] = V[(size_t)I * NQ + q];
+    for (int64_t u = urow[I] + lane; u < e; u += 64) {
+      const double* x = U + (size_t)col[u] * NQ;
+      double r = 0.0;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) r += v[q] * x[q];
+      const uint32_t c1 = first[u + 1];
+      for (uint32_t c = first[u]; c < c1; ++c) {
+        const uint32_t w = con[c];
+        const double d = r * sc[(w >> kGateBits) & ((1u << kCoefBits) - 1u)];
+        const uint32_t g = w & ((1u << kGateBits) - 1u);
+        if (lds) atomicAdd(sg + g, (w >> 31) ? -d : d);
+        else unsafeAtomicAdd(dpart + g, (w >> 31) ? -d : d);
+      }
+    }
+  }
+  if (!lds) return;
+  __syncthreads();
+  for (int i = threadIdx.x; i < ng; i += 64 * kRows) dpart[(size_t)blockIdx.x * ng + i] = sg[i];
 }
 
 // nxt[I] = f * sum_g part[g][I]; acc[I] += nxt[I] when acc != nullptr.
@@ -323,75 +569,15 @@ __global__ void k_gate_dots(SV sv, const Term* __restrict__ terms, const TermFas
   }
 }
 
-// gsum[i] += f sum over gate i's pattern entries (I, J, t, sign) of
-// sign coef[t] v[I] u[J], i.e. f <v|T_i u>; one block per gate, its entries
-// (rows ascending) strided over the threads and summed in a fixed order.
-__global__ __launch_bounds__(kUB) void k_gate_dots_csr(const int64_t* __restrict__ gptr,
-                                                       const uint4* __restrict__ gent,
-                                                       const double* __restrict__ coef,
-                                                       const double* __restrict__ u,
-                                                       const double* __restrict__ v, double f,
-                                                       double* __restrict__ gsum) {
-  __shared__ double red[kUB / 64];
-  const int i = blockIdx.x;
-  const int64_t e = gptr[i + 1];
-  double val = 0.0;
-  for (int64_t k = gptr[i] + threadIdx.x; k < e; k += blockDim.x) {
-    const uint4 x = gent[k];
-    const double c = coef[x.z & 0x7fffffffu] * v[x.x] * u[x.y];
-    val += (x.z >> 31) ? -c : c;
-  }
-  for (int off = 32; off > 0; off >>= 1) val += __shfl_down(val, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = val;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double tot = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) tot += red[w];
-    gsum[i] += f * tot;
-  }
-}
-
-// Gate dots over the 8 nodes of one subinterval: block (s, i) takes split s
-// of gate i's pattern entries (I, J, t, sign) and writes
-// dpart[s * ng + i] = sum sign coef[t] sum_q wq[q] v_q[I] u_q[J]
-// (v_q = v + q * dim, u_q likewise), the entries strided over the threads and
-// summed in a fixed order; k_gate_accum adds the splits in order.
-__global__ __launch_bounds__(kUB) void k_gate_dots_nodes(const int64_t* __restrict__ gptr,
-                                                         const uint4* __restrict__ gent,
-                                                         const double* __restrict__ coef,
-                                                         const double* __restrict__ u, const double* __restrict__ v,
-                                                         int64_t dim, NodeW wq, int ng, double* __restrict__ dpart) {
-  __shared__ double red[kUB / 64];
-  const int i = blockIdx.x, sp = blockIdx.y, S = gridDim.y;
-  const int64_t g0 = gptr[i], g1 = gptr[i + 1];
-  const int64_t chunk = (g1 - g0 + S - 1) / S;
-  const int64_t b = g0 + sp * chunk, e = min(g1, b + chunk);
-  double val = 0.0;
-  for (int64_t k = b + threadIdx.x; k < e; k += blockDim.x) {
-    const uint4 x = gent[k];
-    double d = 0.0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) d += wq.r[q] * v[(size_t)q * dim + x.x] * u[(size_t)q * dim + x.y];
-    const double c = coef[x.z & 0x7fffffffu] * d;
-    val += (x.z >> 31) ? -c : c;
-  }
-  for (int off = 32; off > 0; off >>= 1) val += __shfl_down(val, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = val;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double tot = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) tot += red[w];
-    dpart[(size_t)sp * ng + i] = tot;
-  }
-}
-
-// gsum[i] += f * sum_b dpart[b*ng + i] (fixed order).
-__global__ void k_gate_accum(const double* __restrict__ dpart, int nb, int ng, double f, double* __restrict__ gsum) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// gsum[i] += f * sum_b dpart[b*ng + i], one wave per gate.
+__global__ __launch_bounds__(64 * kRows) void k_gate_accum(const double* __restrict__ dpart, int nb, int ng, double f,
+                                                           double* __restrict__ gsum) {
+  const int lane = threadIdx.x & 63, i = blockIdx.x * kRows + (threadIdx.x >> 6);
   if (i >= ng) return;
   double s = 0.0;
-  for (int b = 0; b < nb; ++b) s += dpart[(size_t)b * ng + i];
-  gsum[i] += f * s;
+  for (int b = lane; b < nb; b += 64) s += dpart[(size_t)b * ng + i];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+  if (lane == 0) gsum[i] += f * s;
 }
 
 // w[t] = theta[gate of term t]
@@ -483,12 +669,6 @@ struct UccCsr {
   int64_t* rowp = nullptr;  // [dim + 1]
   uint2* ent = nullptr;     // [nnz]
   double* coef = nullptr;   // [terms]
-  // The same entries grouped by gate (rows ascending inside a gate) as
-  // (I, J, t | sign << 31, 0), for the gradient's per-gate dots; nullptr
-  // above kGateMaxEntries.
-  int64_t* gptr = nullptr;  // [gates + 1]
-  uint4* gent = nullptr;    // [nnz]
-  std::vector<int64_t> host_rowp;  // row offsets on the host while the pattern is built
 };
 
 void ucc_csr_free(UccCsr* c) {
@@ -496,43 +676,33 @@ void ucc_csr_free(UccCsr* c) {
   if (c->rowp) (void)hipFree(c->rowp);
   if (c->ent) (void)hipFree(c->ent);
   if (c->coef) (void)hipFree(c->coef);
-  if (c->gptr) (void)hipFree(c->gptr);
-  if (c->gent) (void)hipFree(c->gent);
   delete c;
 }
 
-constexpr int64_t kGateMaxEntries = (int64_t)1 << 28;
-
-// Regroup the row pattern by gate on the host (stable: rows stay ascending).
-static void build_gate_major(const Space& s, const Program& p, const std::vector<int64_t>& rowp, UccCsr* c) {
-  const int ng = (int)p.gates.size();
-  if (ng == 0 || c->nnz > kGateMaxEntries) return;
-  std::vector<uint2> ent((size_t)c->nnz);
-  SQ_HIP(hipMemcpy(ent.data(), c->ent, sizeof(uint2) * ent.size(), hipMemcpyDeviceToHost));
-  std::vector<int32_t> t2g(p.terms.size(), -1);
-  for (int g = 0; g < ng; ++g)
-    for (int t = p.gates[g].term_begin; t < p.gates[g].term_end; ++t) t2g[t] = g;
-  std::vector<int64_t> gptr((size_t)ng + 1, 0);
-  for (const uint2& x : ent) {
-    const int g = t2g[x.y & 0x7fffffffu];
-    if (g >= 0) ++gptr[(size_t)g + 1];
+// T's merged pattern.  val holds the numbers of the evaluation under way: an
+// evaluation locks mu while it enqueues its work, waits on the device for the
+// last one (busy) and records busy at its end, so that evaluations on other
+// streams and threads keep to their own theta.
+struct UccT {
+  int64_t nu = 0;             // merged elements
+  int ncoef = 0;
+  int lpr = 64;               // lanes per row of k_spmv
+  int64_t* urow = nullptr;    // [dim + 1]
+  uint32_t* col = nullptr;    // [nu]
+  uint32_t* first = nullptr;  // [nu + 1]
+  uint32_t* con = nullptr;    // [entries]
+  double* coefs = nullptr;    // [ncoef]
+  double* val = nullptr;      // [nu]
+  std::mutex mu;
+  hipEvent_t busy = nullptr;
+  ~UccT() {
+    for (void* p : {(void*)urow, (void*)col, (void*)first, (void*)con, (void*)coefs, (void*)val})
+      if (p) (void)hipFree(p);
+    if (busy) (void)hipEventDestroy(busy);
   }
-  for (int g = 0; g < ng; ++g) gptr[(size_t)g + 1] += gptr[g];
-  std::vector<uint4> gent((size_t)gptr[ng]);
-  std::vector<int64_t> pos(gptr.begin(), gptr.end() - 1);
-  for (int64_t I = 0; I < s.dim; ++I)
-    for (int64_t k = rowp[I]; k < rowp[I + 1]; ++k) {
-      const uint2 x = ent[(size_t)k];
-      const int g = t2g[x.y & 0x7fffffffu];
-      if (g >= 0) gent[(size_t)pos[g]++] = make_uint4((uint32_t)I, x.x, x.y, 0u);
-    }
-  hipError_t e = hipMalloc(&c->gptr, sizeof(int64_t) * gptr.size());
-  if (e == hipSuccess) e = hipMalloc(&c->gent, sizeof(uint4) * std::max<size_t>(gent.size(), 1));
-  if (e == hipSuccess) e = hipMemcpy(c->gptr, gptr.data(), sizeof(int64_t) * gptr.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess && !gent.empty())
-    e = hipMemcpy(c->gent, gent.data(), sizeof(uint4) * gent.size(), hipMemcpyHostToDevice);
-  SQ_HIP(e);
-}
+};
+
+void ucc_t_free(UccT* t) { delete t; }
 
 // Largest pattern kept (entries of 8 bytes); above it, and with SQ_UCC_CSR=0,
 // T is applied by the term-scan kernels below.
@@ -547,7 +717,7 @@ constexpr int64_t kOpMaxEntries = (int64_t)1 << 25;
 // it is empty, above max_nnz entries, or the one-wave-per-row product would
 // not fit one grid dimension.
 static UccCsr* build_pattern(const Space& s, const std::vector<Term>& terms, const Term* d_terms,
-                             const TermFast* fast, int64_t max_nnz, hipStream_t st) {
+                             const TermFast* fast, int64_t max_nnz, hipStream_t st, int64_t* longest = nullptr) {
   const int nt = (int)terms.size();
   // k_tapply_csr runs one 64-lane wave per determinant: 64 * dim work-items
   // must stay below the 2^32 limit of one grid dimension
@@ -566,6 +736,7 @@ static UccCsr* build_pattern(const Space& s, const std::vector<Term>& terms, con
   for (size_t i = 0; i < hc.size(); ++i) rowp[i + 1] = rowp[i] + hc[i];
   const int64_t nnz = rowp.back();
   if (nnz == 0 || nnz > max_nnz) return nullptr;
+  if (longest) *longest = *std::max_element(hc.begin(), hc.end());
   UccCsr* c = new UccCsr;
   c->nnz = nnz;
   std::vector<double> coef((size_t)nt);
@@ -584,7 +755,6 @@ static UccCsr* build_pattern(const Space& s, const std::vector<Term>& terms, con
     ucc_csr_free(c);
     SQ_HIP(e);
   }
-  c->host_rowp = std::move(rowp);
   return c;
 }
 
@@ -593,24 +763,68 @@ static bool csr_enabled() {
   return !(env && env[0] == '0');
 }
 
-// The program's sparsity pattern of T on space s, built on first use
+// The program's merged pattern of T on space s, built on first use
 // (synchronous); nullptr where it is not used.
-static const UccCsr* ucc_csr(const Space& s, const Program& p, hipStream_t st) {
-  if (p.ucc_csr_tried) return p.ucc_csr;
-  p.ucc_csr_tried = true;
-  if (!csr_enabled()) return nullptr;
-  UccCsr* c = build_pattern(s, p.terms, p.d_terms, term_fast(p), kCsrMaxEntries, st);
+static UccT* ucc_t(const Space& s, const Program& p, hipStream_t st) {
+  static std::mutex mu;
+  std::lock_guard<std::mutex> lock(mu);
+  if (p.ucc_t_tried) return p.ucc_t;
+  p.ucc_t_tried = true;
+  const int ng = (int)p.gates.size();
+  if (!csr_enabled() || ng >= (1 << kGateBits)) return nullptr;
+  // the distinct |coefficients| and every term's word
+  std::vector<double> coefs;
+  std::vector<uint32_t> word(std::max<size_t>(p.terms.size(), 1), 0u);
+  for (int g = 0; g < ng; ++g)
+    for (int t = p.gates[g].term_begin; t < p.gates[g].term_end; ++t) {
+      const double c = std::fabs(p.terms[t].coef);
+      size_t k = std::find(coefs.begin(), coefs.end(), c) - coefs.begin();
+      if (k == coefs.size()) coefs.push_back(c);
+      if (k >= (1u << kCoefBits)) return nullptr;
+      word[t] = (uint32_t)g | (uint32_t)k << kGateBits | (p.terms[t].coef < 0 ? 0x80000000u : 0u);
+    }
+  int64_t longest = 0;
+  std::unique_ptr<UccCsr, void (*)(UccCsr*)> c(
+      build_pattern(s, p.terms, p.d_terms, term_fast(p), kCsrMaxEntries, st, &longest), ucc_csr_free);
   if (!c) return nullptr;
-  try {
-    build_gate_major(s, p, c->host_rowp, c);
-  } catch (...) {
-    ucc_csr_free(c);
-    throw;
-  }
-  c->host_rowp.clear();
-  c->host_rowp.shrink_to_fit();
-  p.ucc_csr = c;
-  return c;
+  std::unique_ptr<UccT> T(new UccT);
+  struct Tmp {
+    void* p = nullptr;
+    ~Tmp() { if (p) (void)hipFree(p); }
+  } ucnt, tword;
+  SQ_HIP(hipMalloc(&ucnt.p, sizeof(int32_t) * (size_t)s.dim));
+  SQ_HIP(hipMalloc(&tword.p, sizeof(uint32_t) * word.size()));
+  SQ_HIP(hipMemcpyAsync(tword.p, word.data(), sizeof(uint32_t) * word.size(), hipMemcpyHostToDevice, st));
+  int P = 1;
+  while (P < std::min<int64_t>(longest, kSortRow)) P <<= 1;
+  allow_lds(k_row_sort, (size_t)P * 8 + 1024);
+  k_row_sort<<<(unsigned)s.dim, kUB, (size_t)P * 8, st>>>(c->rowp, c->ent, (int32_t*)ucnt.p);
+  SQ_HIP(hipGetLastError());
+  std::vector<int32_t> hc((size_t)s.dim);
+  SQ_HIP(hipMemcpyAsync(hc.data(), ucnt.p, sizeof(int32_t) * hc.size(), hipMemcpyDeviceToHost, st));
+  SQ_HIP(hipStreamSynchronize(st));
+  std::vector<int64_t> urow((size_t)s.dim + 1, 0);
+  for (size_t i = 0; i < hc.size(); ++i) urow[i + 1] = urow[i] + hc[i];
+  T->nu = urow.back();
+  T->ncoef = (int)coefs.size();
+  T->lpr = T->nu <= 32 * s.dim ? 16 : T->nu <= 64 * s.dim ? 32 : 64;
+  SQ_HIP(hipMalloc(&T->urow, sizeof(int64_t) * urow.size()));
+  SQ_HIP(hipMalloc(&T->col, sizeof(uint32_t) * (size_t)T->nu));
+  SQ_HIP(hipMalloc(&T->first, sizeof(uint32_t) * ((size_t)T->nu + 1)));
+  SQ_HIP(hipMalloc(&T->con, sizeof(uint32_t) * (size_t)c->nnz));
+  SQ_HIP(hipMalloc(&T->coefs, sizeof(double) * coefs.size()));
+  SQ_HIP(hipMalloc(&T->val, sizeof(double) * (size_t)T->nu));
+  SQ_HIP(hipEventCreateWithFlags(&T->busy, hipEventDisableTiming));
+  SQ_HIP(hipMemcpyAsync(T->urow, urow.data(), sizeof(int64_t) * urow.size(), hipMemcpyHostToDevice, st));
+  SQ_HIP(hipMemcpyAsync(T->coefs, coefs.data(), sizeof(double) * coefs.size(), hipMemcpyHostToDevice, st));
+  const uint32_t end = (uint32_t)c->nnz;
+  SQ_HIP(hipMemcpyAsync(T->first + T->nu, &end, sizeof(end), hipMemcpyHostToDevice, st));
+  k_row_merge<<<(unsigned)((s.dim + kRows - 1) / kRows), 64 * kRows, 0, st>>>(
+      s.dim, c->rowp, c->ent, (const uint32_t*)tword.p, T->urow, T->col, T->first, T->con);
+  SQ_HIP(hipGetLastError());
+  SQ_HIP(hipStreamSynchronize(st));
+  p.ucc_t = T.release();
+  return p.ucc_t;
 }
 
 bool operator_apply_pattern(const Space& s, sq_operator& op, const double* in, double* out, hipStream_t st) {
@@ -619,10 +833,6 @@ bool operator_apply_pattern(const Space& s, sq_operator& op, const double* in, d
     if (!csr_enabled()) return false;
     op.d_fast = upload_term_fast(op.terms);
     op.csr = build_pattern(s, op.terms, op.d_terms, op.d_fast, kOpMaxEntries, st);
-    if (op.csr) {
-      op.csr->host_rowp.clear();
-      op.csr->host_rowp.shrink_to_fit();
-    }
   }
   const UccCsr* c = op.csr;
   if (!c) return false;
@@ -646,11 +856,9 @@ static int term_groups(const Space& s) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(64, G));
 }
 
-// Work of the UCC routines (doubles), carved in this order; A2, B2 and the
-// node states NC, ND (kNodes vectors each) serve the gradient's
-// multi-node series.
+// Work of the term-scan routines (doubles), carved in this order.
 struct UccWork {
-  double *A, *B, *C, *D, *w, *part, *dpart, *partial, *scal, *A2, *B2, *NC, *ND;
+  double *A, *B, *C, *D, *w, *part, *dpart, *partial, *scal;
 };
 
 static int64_t dot_blocks(const Space& s) { return (s.dim + kUB - 1) / kUB; }
@@ -660,10 +868,9 @@ static int gate_groups(const Space& s, int ng) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(ng, std::max<int64_t>(1, 512 / nb)));
 }
 
-int64_t ucc_work_doubles(const Space& s, const Program& p) {
+static int64_t scan_work_doubles(const Space& s, const Program& p) {
   const int64_t ng = (int64_t)std::max<size_t>(p.gates.size(), 1);
-  return 4 * s.dim + (int64_t)p.terms.size() + 64 + (int64_t)term_groups(s) * s.dim + dot_blocks(s) * ng + 1024 +
-         64 + 64 + (2 + 2 * kNodes) * s.dim;
+  return 4 * s.dim + (int64_t)p.terms.size() + 64 + (int64_t)term_groups(s) * s.dim + dot_blocks(s) * ng + 1024 + 64;
 }
 
 static UccWork carve_ucc(const Space& s, const Program& p, double* work) {
@@ -678,23 +885,59 @@ static UccWork carve_ucc(const Space& s, const Program& p, double* work) {
   u.dpart = u.part + (size_t)term_groups(s) * s.dim;
   u.partial = u.dpart + (size_t)dot_blocks(s) * ng;
   u.scal = u.partial + 1024;
-  u.A2 = u.scal + 64;
-  u.B2 = u.A2 + s.dim;
-  u.NC = u.B2 + s.dim;
-  u.ND = u.NC + (size_t)kNodes * s.dim;
   return u;
+}
+
+// Largest nu t of one series and the nodes it needs: the n-point
+// Gauss-Legendre rule on an interval of length h integrates frequencies up to
+// omega = 2 nu with an error below h (n!)^4 / ((2n+1) (2n)!^3) (h omega)^2n
+// max|f|: 1e-13 at h nu = 2, 5.5 and 9.7 for n = 8, 12 and 16.  Spaces above
+// 2^22 determinants take h nu <= 2 (24 basis vectors and 8 nodes of
+// workspace instead of 44 and 16).
+constexpr int kNormSteps = 16;  // products of the norm estimate (and head of the Taylor series)
+static double nu_limit(const Space& s) { return s.dim > ((int64_t)1 << 22) ? 2.0 : 9.7; }
+static int max_nodes(const Space& s) { return s.dim > ((int64_t)1 << 22) ? 8 : 16; }
+static int max_basis(const Space& s) { return s.dim > ((int64_t)1 << 22) ? 24 : kMaxBasis; }
+
+// Work of the merged-pattern routines (doubles): U nodes | scal | rmax |
+// basis | V nodes | C | D | dpart; from basis on it also serves sigma.
+struct ChebWork {
+  double *U, *scal, *rmax, *basis, *V, *C, *D, *dpart;
+};
+
+constexpr int kAsmBlocks = 2048;
+static int64_t row_blocks(const Space& s, int64_t cap) { return std::min<int64_t>((s.dim + kRows - 1) / kRows, cap); }
+static int64_t gate_blocks(const Space& s, int64_t ng) { return ng <= kLdsGates ? row_blocks(s, 1024) : 1; }
+
+static int64_t cheb_head(const Space& s) { return (int64_t)max_nodes(s) * s.dim + 64 + kAsmBlocks; }
+static int64_t cheb_tail(const Space& s, int64_t ng) {
+  return (int64_t)(max_basis(s) + max_nodes(s) + 2) * s.dim + gate_blocks(s, ng) * ng;
+}
+
+static ChebWork carve_cheb(const Space& s, double* work) {
+  ChebWork u;
+  u.U = work;
+  u.scal = u.U + (size_t)max_nodes(s) * s.dim;
+  u.rmax = u.scal + 64;
+  u.basis = u.rmax + kAsmBlocks;
+  u.V = u.basis + (size_t)max_basis(s) * s.dim;
+  u.C = u.V + (size_t)max_nodes(s) * s.dim;
+  u.D = u.C + s.dim;
+  u.dpart = u.D + s.dim;
+  return u;
+}
+
+static int64_t ucc_work_doubles(const Space& s, const Program& p) {
+  const int64_t ng = (int64_t)std::max<size_t>(p.gates.size(), 1);
+  int64_t n = std::max<int64_t>(scan_work_doubles(s, p), sigma_work_bytes(s) / 8);
+  if (64 * s.dim < ((int64_t)1 << 32))  // spaces the merged pattern can serve
+    n = std::max<int64_t>(n, cheb_head(s) + std::max<int64_t>(cheb_tail(s, ng), sigma_work_bytes(s) / 8));
+  return n;
 }
 
 // nxt = f T cur (w: term weights, nullptr for unit weights); acc += nxt.
 static void tapply(const Space& s, const Program& p, const double* w, const double* cur, double f, double* nxt,
                    double* acc, double* part, hipStream_t st) {
-  if (const UccCsr* c = ucc_csr(s, p, st)) {
-    SQ_PROF(PC_TAPPLY, st, 16.0 * (double)s.dim + 8.0 * (double)c->nnz, 0.0,
-            k_tapply_csr<<<(unsigned)((s.dim + kCsrRows - 1) / kCsrRows), 64 * kCsrRows, 0, st>>>(
-                s.dim, c->rowp, c->ent, c->coef, w, cur, f, nxt, acc));
-    SQ_HIP(hipGetLastError());
-    return;
-  }
   const int G = term_groups(s);
   int rows = G;  // part rows
   if (G >= kTG) {  // small space: fold kTG groups per block in LDS
@@ -830,9 +1073,264 @@ static void term_weights(const Program& p, const double* theta_dev, double* w, h
   SQ_HIP(hipGetLastError());
 }
 
+// ---- Chebyshev series over the merged pattern ------------------------------
+
+// n-point Gauss-Legendre nodes and weights on [0, 1] (Newton on P_n).
+struct GaussRule {
+  double x[16], w[16];
+};
+
+static const GaussRule& gauss_rule(int n) {
+  auto make = [](int m) {
+    GaussRule R{};
+    for (int i = 0; i < m; ++i) {
+      long double z = std::cos(3.14159265358979323846L * (i + 0.75L) / (m + 0.5L)), d = 1.0L;
+      for (int it = 0; it < 100; ++it) {
+        long double p0 = 1.0L, p1 = z;
+        for (int k = 2; k <= m; ++k) {
+          const long double p2 = ((2 * k - 1) * z * p1 - (k - 1) * p0) / k;
+          p0 = p1;
+          p1 = p2;
+        }
+        d = m * (z * p1 - p0) / (z * z - 1.0L);
+        const long double dz = p1 / d;
+        z -= dz;
+        if (std::fabs(dz) < 1e-18L) break;
+      }
+      R.x[i] = (double)(0.5L * (1.0L - z));
+      R.w[i] = (double)(1.0L / ((1.0L - z * z) * d * d));
+    }
+    return R;
+  };
+  static const GaussRule r8 = make(8), r12 = make(12), r16 = make(16);
+  return n == 8 ? r8 : n == 12 ? r12 : r16;
+}
+
+// out[k] = (2 - delta_k0) J_k(x), k <= K: Miller's downward recurrence in
+// long double, normalised by J_0 + 2 sum J_2k = 1.
+static void cheb_coefs(double x, int K, double f, double* out) {
+  const long double a = std::fabs((long double)x);
+  if (!(a > 1e-300L)) {
+    for (int k = 0; k <= K; ++k) out[k] = k == 0 ? f : 0.0;
+    return;
+  }
+  const int M = K + 30 + (int)a;
+  std::vector<long double> j(M + 2, 0.0L);
+  j[M] = 1e-300L;
+  for (int k = M; k > 0; --k) {
+    j[k - 1] = 2.0L * k / a * j[k] - j[k + 1];
+    if (std::fabs(j[k - 1]) > 1e250L)  // small arguments: rescale what is there
+      for (int i = k - 1; i <= M; ++i) j[i] *= 1e-300L;
+  }
+  long double norm = j[0];
+  for (int k = 2; k <= M; k += 2) norm += 2.0L * j[k];
+  for (int k = 0; k <= K; ++k) {
+    long double v = j[k] / norm * (k == 0 ? 1.0L : 2.0L);
+    if (x < 0 && (k & 1)) v = -v;
+    out[k] = (double)(v * f);
+  }
+}
+
+static int cheb_terms(double r, int cap) {
+  int K = 1;
+  double term = r / 2;
+  while (term > std::ldexp(1.0, -61) && K < cap) {
+    ++K;
+    term *= r / (2 * K);
+  }
+  return K;
+}
+
+// Guards a program's assembled T for one evaluation on st.
+struct UccUse {
+  UccT& T;
+  std::unique_lock<std::mutex> lock;
+  hipStream_t st;
+  UccUse(UccT& t, hipStream_t stream) : T(t), lock(t.mu), st(stream) { SQ_HIP(hipStreamWaitEvent(st, T.busy, 0)); }
+  ~UccUse() { (void)hipEventRecord(T.busy, st); }
+};
+
+static void spmv(const Space& s, const UccT& T, const double* cur, const double* prev, double f, const double* bound,
+                 double* nxt, hipStream_t st, const double* cur2 = nullptr, double* nxt2 = nullptr) {
+  auto* kernel = cur2 ? (T.lpr == 16 ? k_spmv<16, true> : T.lpr == 32 ? k_spmv<32, true> : k_spmv<64, true>)
+                      : (T.lpr == 16 ? k_spmv<16, false> : T.lpr == 32 ? k_spmv<32, false> : k_spmv<64, false>);
+  const int64_t rows = kUB / T.lpr;
+  SQ_PROF(PC_TAPPLY, st, (cur2 ? 32.0 : 16.0) * (double)s.dim + 12.0 * (double)T.nu, 0.0,
+          kernel<<<(unsigned)((s.dim + rows - 1) / rows), kUB, 0, st>>>(s.dim, T.urow, T.col, T.val, cur, cur2, prev, f,
+                                                                      bound, nxt, nxt2));
+}
+
+// A series of exp(t T): basis[k] = (T / scale)^k in (taylor) or
+// phi_k(T / scale) in, k <= K.
+struct Series {
+  bool taylor;
+  double nu;     // >= ||T||_2
+  double bound;  // largest row sum of |T|
+  int K;
+  double scale() const { return taylor ? bound : nu; }
+  void coefs(double t, double f, double* out) const {
+    if (!taylor) return cheb_coefs(nu * t, K, f, out);
+    long double c = f;
+    for (int k = 0; k <= K; ++k) {
+      out[k] = (double)c;
+      c *= (long double)t * bound / (k + 1);
+    }
+  }
+};
+
+// Basis vectors from + 1 .. K (basis[from] and, for from > 0, those before are there).
+static void series_basis(const Space& s, const UccT& T, const Series& S, int from, const ChebWork& u,
+                         hipStream_t st) {
+  for (int k = from + 1; k <= S.K; ++k) {
+    double* n = u.basis + (size_t)k * s.dim;
+    const bool three = !S.taylor && k > 1;
+    spmv(s, T, n - s.dim, three ? n - 2 * s.dim : nullptr, (three ? 2.0 : 1.0) / S.scale(), nullptr, n, st);
+  }
+}
+
+// nodes[I][q] = f_q exp(t_q T) in (q < n) and fin = exp(tfin T) in.
+static void series_combine(const Space& s, const Series& S, int n, const double* t, const double* f, double* nodes,
+                           double tfin, double* fin, const ChebWork& u, hipStream_t st) {
+  for (int q0 = 0; q0 == 0 || q0 < n; q0 += kMaxOut - 1) {
+    Combine C{};
+    const int nq = std::min(kMaxOut - 1, n - q0);
+    for (int q = 0; q < nq; ++q) S.coefs(t[q0 + q], f ? f[q0 + q] : 1.0, C.c[q]);
+    double* out = q0 == 0 ? fin : nullptr;
+    if (out) S.coefs(tfin, 1.0, C.c[kMaxOut - 1]);
+    SQ_PROF(PC_OTHER, st, 8.0 * (double)s.dim * (S.K + 1 + nq + 1), 0.0,
+            k_combine<<<(unsigned)((s.dim + kCB - 1) / kCB), kCB, 0, st>>>(s.dim, S.K, C, nq, u.basis, nodes + q0, n, out));
+  }
+}
+
+// Assembles T(theta), puts v into basis[0] and runs the first products on it
+// and on the pseudo-random vector.  Returns the series for |t| <= 1 on an
+// interval of length 1 / m; *done: basis vectors that are there.
+static Series series_start(const Space& s, const Program& p, const UccT& T, const double* theta, const double* v,
+                           double tmax, const ChebWork& u, int* m, int* done, hipStream_t st) {
+  const int ng = (int)p.gates.size();
+  const unsigned nb = (unsigned)row_blocks(s, kAsmBlocks);
+  SQ_PROF(PC_OTHER, st, 12.0 * (double)T.nu, 0.0,
+          k_assemble<<<nb, 64 * kRows, ng <= kLdsGates ? 8 * (size_t)ng : 0, st>>>(
+              s.dim, T.urow, T.first, T.con, T.coefs, T.ncoef, theta, ng, T.val, u.rmax));
+  k_max<<<1, kUB, 0, st>>>(u.rmax, (int)nb, u.scal);
+  copy_vec(v, u.basis, s.dim, st);
+  double* x = u.C;
+  double* y = u.D;
+  k_fill_pattern<<<(unsigned)((s.dim + kUB - 1) / kUB), kUB, 0, st>>>(x, s.dim);
+  SQ_HIP(hipGetLastError());
+  for (int k = 1; k <= kNormSteps; ++k) {
+    double* n = u.basis + (size_t)k * s.dim;
+    spmv(s, T, n - s.dim, nullptr, 1.0, u.scal, n, st, x, y);
+    std::swap(x, y);
+  }
+  dot_dev(y, y, s.dim, u.scal, 1, 1.0, u.rmax, st);
+  dot_dev(x, x, s.dim, u.scal, 2, 1.0, u.rmax, st);
+  double d[3];
+  SQ_HIP(hipMemcpyAsync(d, u.scal, 3 * sizeof(double), hipMemcpyDeviceToHost, st));
+  SQ_HIP(hipStreamSynchronize(st));
+  Series S{};
+  S.bound = S.nu = d[0];
+  if (!std::isfinite(d[0])) S.bound = S.nu = 1.0;  // the result is NaN whatever the series
+  else if (d[1] > 1e-200 && std::isfinite(d[2])) S.nu = std::min(d[0], 1.5 * d[0] * std::sqrt(d[2] / d[1]) + 0.05);
+  const double r = S.nu * tmax;
+  *m = std::max(1, (int)std::ceil(std::min(r / nu_limit(s), 1e9)));
+  *done = 0;
+  if (r == 0.0) {
+    S.taylor = true;
+  } else if (r <= 2.0 && S.bound < 1e6) {
+    S.taylor = true;
+    S.K = std::min(taylor_terms(r), max_basis(s) - 1);
+    *done = std::min(S.K, kNormSteps);
+  } else {
+    S.K = cheb_terms(r / *m, max_basis(s) - 1);
+  }
+  return S;
+}
+
+// out = exp(t T) in, in m steps; the first step's basis is there up to done.
+static void series_expm(const Space& s, const UccT& T, const Series& S, int m, int done, double t, double* out,
+                        const ChebWork& u, hipStream_t st) {
+  for (int k = 0; k < m; ++k) {
+    if (k > 0) copy_vec(out, u.basis, s.dim, st);
+    series_basis(s, T, S, k == 0 ? done : 0, u, st);
+    series_combine(s, S, 0, nullptr, nullptr, u.U, t / m, out, u, st);
+  }
+}
+
+static void gate_dots(const Space& s, const UccT& T, int n, int ng, const ChebWork& u, double* grad_dev,
+                      hipStream_t st) {
+  const bool lds = ng <= kLdsGates;
+  const unsigned nb = (unsigned)row_blocks(s, 1024);
+  auto* kernel = n == 8 ? k_gate_dots_rows<8> : n == 12 ? k_gate_dots_rows<12> : k_gate_dots_rows<16>;
+  if (!lds) k_zero<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(u.dpart, ng);
+  SQ_PROF(PC_OTHER, st, 12.0 * (double)T.nu, 0.0,
+          kernel<<<nb, 64 * kRows, lds ? 8 * (size_t)ng : 0, st>>>(s.dim, T.urow, T.col, T.first, T.con, T.coefs, T.ncoef,
+                                                                 u.U, u.V, ng, lds ? 1 : 0, u.dpart));
+  k_gate_accum<<<(unsigned)((ng + kRows - 1) / kRows), 64 * kRows, 0, st>>>(u.dpart, lds ? (int)nb : 1, ng, 1.0,
+                                                                          grad_dev);
+  SQ_HIP(hipGetLastError());
+}
+
+// Energy (scal[0]) and gradient (grad_dev, may be nullptr) through the merged
+// pattern.  grad_i = 2 int_0^1 <e^{-sT} lam | T_i | e^{-sT} psi> ds, and
+// e^{-sT} psi = e^{(1-s)T} psi0: one interval while nu <= the limit, with psi's
+// nodes from the forward series; else m intervals, both states propagated
+// back through them.
+static void cheb_energy_grad(const Space& s, const Program& p, UccT& T, const Hamiltonian& H, const double* theta,
+                             const double* psi0, double* psi, double* lam, double* scal, double* grad_dev,
+                             double* work, hipStream_t st) {
+  UccUse use(T, st);
+  const ChebWork u = carve_cheb(s, work);
+  const int ng = (int)p.gates.size();
+  int m, done;
+  const Series S = series_start(s, p, T, theta, psi0, 1.0, u, &m, &done, st);
+  const double r = S.nu / m;
+  const int n = r <= 2.0 ? 8 : r <= 5.5 ? 12 : 16;
+  const GaussRule& R = gauss_rule(n);
+  double t[16], f[16];
+  if (m == 1) {
+    series_basis(s, T, S, done, u, st);
+    for (int q = 0; q < n; ++q) t[q] = 1.0 - R.x[q];
+    series_combine(s, S, grad_dev ? n : 0, t, nullptr, u.U, 1.0, psi, u, st);
+  } else {
+    series_expm(s, T, S, m, done, 1.0, psi, u, st);
+  }
+  sigma_energy_dev(s, H, psi, lam, scal, u.basis, st);
+  if (!grad_dev) return;
+  k_zero<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(grad_dev, ng);
+  SQ_HIP(hipGetLastError());
+  for (int q = 0; q < n; ++q) {
+    t[q] = -R.x[q] / m;
+    f[q] = 2.0 * R.w[q] / m;
+  }
+  const double* c = psi;
+  const double* d = lam;
+  for (int j = 0; j < m; ++j) {
+    if (m > 1) {
+      copy_vec(c, u.basis, s.dim, st);
+      series_basis(s, T, S, 0, u, st);
+      series_combine(s, S, n, t, nullptr, u.U, -1.0 / m, u.C, u, st);
+      c = u.C;
+    }
+    copy_vec(d, u.basis, s.dim, st);
+    series_basis(s, T, S, 0, u, st);
+    series_combine(s, S, n, t, f, u.V, -1.0 / m, j + 1 < m ? u.D : nullptr, u, st);
+    d = u.D;
+    gate_dots(s, T, n, ng, u, grad_dev, st);
+  }
+}
+
 // out = exp(t T(theta)) in.  work: ucc_work_doubles.
 void ucc_expm_impl(const Space& s, const Program& p, const double* theta_dev, double t, const double* in,
                    double* out, double* work, hipStream_t st) {
+  if (UccT* T = ucc_t(s, p, st)) {
+    UccUse use(*T, st);
+    const ChebWork u = carve_cheb(s, work);
+    int m, done;
+    const Series S = series_start(s, p, *T, theta_dev, in, std::fabs(t), u, &m, &done, st);
+    series_expm(s, *T, S, m, done, t, out, u, st);
+    return;
+  }
   const UccWork u = carve_ucc(s, p, work);
   const std::vector<double> th = theta_host(p, theta_dev, st);
   term_weights(p, theta_dev, u.w, st);
@@ -840,108 +1338,31 @@ void ucc_expm_impl(const Space& s, const Program& p, const double* theta_dev, do
   expm_apply(s, p, u, nu, t, in, out, st);
 }
 
-// 8-point Gauss-Legendre nodes and weights on [0, 1].
-static const double kGLx[8] = {0.019855071751231856, 0.10166676129318664, 0.2372337950418355,  0.4082826787521751,
-                               0.5917173212478249,   0.7627662049581645,  0.8983332387068134,  0.9801449282487681};
-static const double kGLw[8] = {0.05061426814518813, 0.11119051722668724, 0.15685332293894363, 0.18134189168918100,
-                               0.18134189168918100, 0.15685332293894363, 0.11119051722668724, 0.05061426814518813};
-
-// Analytic dE/dtheta for E = <psi|H|psi>, psi = exp(T) psi0, lam = H psi:
-//   d psi / d theta_i = int_0^1 e^{sT} T_i e^{(1-s)T} psi0 ds, and with
-//   e^{sT}^T = e^{-sT} (T real antisymmetric)
-//   grad_i = 2 int_0^1 <e^{-sT} lam | T_i | e^{-sT} psi> ds,
-// by composite 8-point Gauss-Legendre over m subintervals of length h with
-// h * 2 nu <= 4 (the integrand is entire with frequencies bounded by
-// 2 ||T||_2 = omega; the 8-point rule's error on one subinterval is below
-// h (8!)^4 / (17 (16!)^3) (h omega)^16 max|f|, so over [0, 1] it is below
-// 1.7e-23 * 4^16 max|f| < 1e-13 max|f|).
-// Without the gate-major pattern, psi and lam are propagated from node to
-// node (C, D) and every node adds all gates' dots in one pass.
-//
-// With the gate-major pattern, each subinterval [a, a + h] runs one Taylor
-// series of exp(-h T) on psi and lam together (k_tapply_csr2: the pattern read
-// once for both), whose terms z_k = (-h)^k / k! T^k C also give every node:
-// e^{-h x_q T} C = sum_k x_q^k z_k, accumulated into the node states as the
-// terms are made (and the end of the subinterval, x = 1, starts the next);
-// h nu <= 2 bounds the series' radius.  The 8 nodes' gate dots then run in
-// one launch, split over blocks per gate.
-static void nodes_apply(const Space& s, const UccCsr* c, const UccWork& u, double nu, double h, hipStream_t st) {
-  const int K = taylor_terms(h * nu);
-  const unsigned nb = (unsigned)((s.dim + kUB - 1) / kUB);
-  k_nodes_init<<<nb, kUB, 0, st>>>(s.dim, u.C, u.D, u.NC, u.ND);
-  SQ_HIP(hipGetLastError());
-  double x[kNodes], pw[kNodes];
-  for (int q = 0; q < 8; ++q) x[q] = kGLx[q];
-  x[8] = 1.0;
-  for (int q = 0; q < kNodes; ++q) pw[q] = 1.0;
-  const double* cur0 = u.C;
-  const double* cur1 = u.D;
-  double* b0[2] = {u.A, u.B};
-  double* b1[2] = {u.A2, u.B2};
-  const unsigned rows = (unsigned)((s.dim + kCsrRows - 1) / kCsrRows);
-  for (int k = 1; k <= K; ++k) {
-    NodeW r;
-    for (int q = 0; q < kNodes; ++q) r.r[q] = pw[q] *= x[q];
-    double* n0 = b0[k & 1];
-    double* n1 = b1[k & 1];
-    SQ_PROF(PC_TAPPLY, st, 32.0 * (double)s.dim + 8.0 * (double)c->nnz + 16.0 * kNodes * (double)s.dim, 0.0,
-            k_tapply_csr2<<<rows, 64 * kCsrRows, 0, st>>>(s.dim, c->rowp, c->ent, c->coef, u.w, cur0, cur1, -h / k,
-                                                          n0, n1, u.NC, u.ND, r));
-    SQ_HIP(hipGetLastError());
-    cur0 = n0;
-    cur1 = n1;
-  }
-}
-
+// The gradient without a pattern: composite 8-point Gauss-Legendre over m
+// subintervals of length h with h * 2 nu <= 4, psi and lam propagated from
+// node to node (C, D), every node adding all gates' dots in one pass.
 static void ucc_grad_impl(const Space& s, const Program& p, const UccWork& u, double nu, const double* psi,
                           const double* lam, double* grad_dev, hipStream_t st) {
   const int ng = (int)p.gates.size();
   const int m = std::max(1, (int)std::ceil(0.5 * nu));
+  const GaussRule& R = gauss_rule(8);
   copy_vec(psi, u.C, s.dim, st);
   copy_vec(lam, u.D, s.dim, st);
   k_zero<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(grad_dev, ng);
   SQ_HIP(hipGetLastError());
   const int nb = (int)dot_blocks(s);
   const dim3 dgrid(nb, gate_groups(s, ng));
-  const UccCsr* csr = ucc_csr(s, p, st);
-  static const int nodes_env = [] {
-    const char* e = getenv("SQ_UCC_NODES");
-    return (e && e[0] == '0') ? 0 : 1;
-  }();
-  if (csr && csr->gent && nodes_env) {
-    const double h = 1.0 / m;
-    const int S = (int)std::max<int64_t>(1, std::min<int64_t>(dot_blocks(s), std::max(1, 1024 / ng)));
-    NodeW wq{};
-    for (int q = 0; q < 8; ++q) wq.r[q] = 2.0 * kGLw[q] / m;
-    for (int j = 0; j < m; ++j) {
-      nodes_apply(s, csr, u, nu, h, st);
-      k_gate_dots_nodes<<<dim3((unsigned)ng, (unsigned)S), kUB, 0, st>>>(csr->gptr, csr->gent, csr->coef, u.NC,
-                                                                        u.ND, s.dim, wq, ng, u.dpart);
-      k_gate_accum<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(u.dpart, S, ng, 1.0, grad_dev);
-      SQ_HIP(hipGetLastError());
-      if (j + 1 < m) {
-        copy_vec(u.NC + (size_t)8 * s.dim, u.C, s.dim, st);
-        copy_vec(u.ND + (size_t)8 * s.dim, u.D, s.dim, st);
-      }
-    }
-    return;
-  }
   double prev = 0.0;
   for (int j = 0; j < m; ++j) {
     for (int q = 0; q < 8; ++q) {
-      const double node = (j + kGLx[q]) / m;
+      const double node = (j + R.x[q]) / m;
       const double ds = node - prev;
       expm_apply(s, p, u, nu, -ds, u.C, u.C, st);
       expm_apply(s, p, u, nu, -ds, u.D, u.D, st);
       prev = node;
-      if (csr && csr->gent) {
-        k_gate_dots_csr<<<(unsigned)ng, kUB, 0, st>>>(csr->gptr, csr->gent, csr->coef, u.C, u.D,
-                                                     2.0 * kGLw[q] / m, grad_dev);
-      } else {
-        k_gate_dots<<<dgrid, kUB, 0, st>>>(sv(s), p.d_terms, term_fast(p), p.d_gates, ng, u.C, u.D, u.dpart);
-        k_gate_accum<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(u.dpart, nb, ng, 2.0 * kGLw[q] / m,
-                                                                       grad_dev);
-      }
+      k_gate_dots<<<dgrid, kUB, 0, st>>>(sv(s), p.d_terms, term_fast(p), p.d_gates, ng, u.C, u.D, u.dpart);
+      k_gate_accum<<<(unsigned)((ng + kRows - 1) / kRows), 64 * kRows, 0, st>>>(u.dpart, nb, ng, 2.0 * R.w[q] / m,
+                                                                             grad_dev);
       SQ_HIP(hipGetLastError());
     }
   }
@@ -980,17 +1401,21 @@ int sq_ucc_energy_grad(const sq_space* sp, const sq_program* pr, const sq_hamilt
     double* scal = lam + s.dim;            // 64
     double* gdev = scal + 64;              // ng
     double* rest = gdev + std::max(ng, 1) + 64;
-    const UccWork u = carve_ucc(s, p, rest);
-    const std::vector<double> th = theta_host(p, theta, st);
-    term_weights(p, theta, u.w, st);
-    const double nu = t_norm(s, p, th, u, st);
-    expm_apply(s, p, u, nu, 1.0, psi0, psi, st);
-    sigma_energy_dev(s, H->h, psi, lam, scal, rest, st);  // reuses the UCC work area
-    if (grad && ng) {
+    if (UccT* T = ucc_t(s, p, st)) {
+      cheb_energy_grad(s, p, *T, H->h, theta, psi0, psi, lam, scal, grad && ng ? gdev : nullptr, rest, st);
+    } else {
+      const UccWork u = carve_ucc(s, p, rest);
+      const std::vector<double> th = theta_host(p, theta, st);
       term_weights(p, theta, u.w, st);
-      ucc_grad_impl(s, p, u, nu, psi, lam, gdev, st);
-      SQ_HIP(hipMemcpyAsync(grad, gdev, sizeof(double) * ng, hipMemcpyDeviceToHost, st));
+      const double nu = t_norm(s, p, th, u, st);
+      expm_apply(s, p, u, nu, 1.0, psi0, psi, st);
+      sigma_energy_dev(s, H->h, psi, lam, scal, rest, st);  // reuses the UCC work area
+      if (grad && ng) {
+        term_weights(p, theta, u.w, st);
+        ucc_grad_impl(s, p, u, nu, psi, lam, gdev, st);
+      }
     }
+    if (grad && ng) SQ_HIP(hipMemcpyAsync(grad, gdev, sizeof(double) * ng, hipMemcpyDeviceToHost, st));
     SQ_HIP(hipMemcpyAsync(energy, scal, sizeof(double), hipMemcpyDeviceToHost, st));
     SQ_HIP(hipStreamSynchronize(st));
   });
@@ -1000,8 +1425,7 @@ int64_t sq_ucc_work_bytes(const sq_space* sp, const sq_program* pr) {
   if (!sp || !pr) return -1;
   const Space& s = sp->s;
   const int64_t ng = (int64_t)pr->p.gates.size() + 1;
-  const int64_t body = std::max<int64_t>(ucc_work_doubles(s, pr->p), sigma_work_bytes(s) / 8);
-  return 8 * (2 * s.dim + 64 + ng + 64 + body);
+  return 8 * (2 * s.dim + 64 + ng + 64 + ucc_work_doubles(s, pr->p));
 }
 
 }  // extern "C"
