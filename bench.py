@@ -138,7 +138,7 @@ def rotation_profile(sp, lay, prog, theta, psi0):
             "sweep_ms": pg_ms,
         },
         "fused_stages": {
-            "kernel": "k_stage_fwd",
+            "kernel": "k_win_fwd",
             "launches_per_sweep": tf.get("launches_per_call"),
             "avg_us": tf.get("avg_us"),
             "achieved_GBs": tf.get("achieved_GBs"),

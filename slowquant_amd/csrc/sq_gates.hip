@@ -810,6 +810,7 @@ int sq_program_destroy(sq_program* pr) {
     if (pr->p.d_term_fast) (void)hipFree(pr->p.d_term_fast);
     if (pr->p.ucc_t) ucc_t_free(pr->p.ucc_t);
     if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
+    if (pr->p.group_tiles) destroy_tile_plan(pr->p.group_tiles);
     if (pr->p.small) small_plan_free(pr->p.small);
     delete pr;
   });
@@ -823,9 +824,11 @@ int sq_program_set_tile_shape(sq_program* pr, int target, int threads) {
              "tile target must be >= 0 and threads 0, 256 or 512");
     if (pr->p.tile_target == target && pr->p.tile_threads == threads) return;
     SQ_HIP(hipDeviceSynchronize());  // the old plan's buffers may be in use by queued kernels
-    if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
-    pr->p.tiles = nullptr;
-    pr->p.tiles_built = false;
+    for (TilePlan** t : {&pr->p.tiles, &pr->p.group_tiles}) {
+      if (*t) destroy_tile_plan(*t);
+      *t = nullptr;
+    }
+    pr->p.tiles_built = pr->p.group_tiles_built = false;
     ++pr->p.plan_gen;
     pr->p.tile_target = target;
     pr->p.tile_threads = threads;

@@ -133,7 +133,10 @@ struct Space {
   // row sigma shape (sq_sigma_configure): 0 / -1 = automatic
   int sig_R = 0, sig_nsplit = 0, sig_det = -1;
   std::vector<uint32_t> h_astr, h_bstr;
+  mutable struct WinCache* win = nullptr;  // window tables of the tile stages (sq_tiles.hip), built on first use
 };
+
+void win_cache_free(struct WinCache* c);
 
 void build_gemm_tables(Space& s);
 void build_row_tables(Space& s);
@@ -141,9 +144,7 @@ void free_row_tables(Space& s);
 
 struct TilePlan;
 struct UccCsr;
-TilePlan* build_tile_plan(const Space& sp, const struct Program& P);
 void destroy_tile_plan(TilePlan* T);
-bool tile_plan_has_tiles(const TilePlan* T);
 
 struct SmallPlan;
 void small_plan_free(SmallPlan* P);
@@ -152,6 +153,8 @@ struct Program {
   const Space* space;
   mutable TilePlan* tiles = nullptr;  // built on first use (sq_tiles.hip)
   mutable bool tiles_built = false;
+  mutable TilePlan* group_tiles = nullptr;  // the plan of batched groups
+  mutable bool group_tiles_built = false;
   mutable SmallPlan* small = nullptr;  // one-block sweep, built on first use (sq_small.hip)
   mutable bool small_tried = false;
   int tile_target = 0;   // elements per tile (0: automatic; sq_program_set_tile_shape)

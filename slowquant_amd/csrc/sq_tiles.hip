@@ -1,23 +1,32 @@
-// Fused brick-column passes for gate layouts made of adjacent-pair gates
+// Fused brick-wall sweeps for gate layouts made of adjacent-pair gates
 // (tUPS / QNP brick walls: sa_single(p,p+1), double(2p,2p+1,2p+2,2p+3)).
 //
-// A "stage" is a run of consecutive gates acting on a set of disjoint orbital
-// pairs (p, p+1).  Under all gates of a stage a determinant can only move
-// within the set of strings that keep, for every pair, the electron count
-// c_j = n_p + n_{p+1}, and keep every unpaired orbital: per spin, strings
-// group into hypercubes {p, p+1}^m over the m singly occupied pairs.  A tile
-// = (one alpha group) x (a run of whole beta groups) is closed under the
-// stage, so one launch loads each tile into LDS once, applies every gate of
-// the stage there, and writes it back: one HBM pass per stage instead of one
-// per rotation.  Tiles gather their columns from the canonical order through
-// a position -> column table, so state vectors never change layout.
+// Consecutive gates on one orbital pair (p, p+1) merge into a pair op.  Under
+// the pair ops inside a window of w consecutive orbitals a determinant keeps
+// its occupation outside the window and its electron count inside it, per
+// spin: strings fall into groups of C(w, k) strings, in the canonical order of
+// their window occupations.  A tile = (one alpha group) x (one beta group) is
+// closed under every gate of the window, so one launch (a stage) loads each
+// tile into LDS once, applies all the pair ops that are ready inside the
+// window, whatever their depth in the brick wall, and writes it back.  The
+// stages of a program are chosen greedily: the window position that takes
+// the most pair ops next.  (12e,12o) tUPS with 4 layers has 8 brick columns
+// and takes 3 stages of up to 22 pair ops at w = 8; (14e,14o) with 6 layers
+// 12 columns and 5 stages.  Tiles gather rows and columns through tables, so
+// state vectors never change layout.
 //
-// Gates on different pairs commute, so the stage runs pair by pair.  For one
-// pair j the gates only mix the <= 4 members of an "orbit" {alpha bit of j}
-// x {beta bit of j} (other indices fixed), and their whole product is one
-// small matrix per orbit type; a thread owns an orbit and applies it.  Signs
-// come from the pair-local bits only: the environment parity cancels for
-// number-conserving spin parts.  One barrier per pair.
+// For one pair the gates only mix the <= 4 members of an "orbit" {alpha bit}
+// x {beta bit} (other indices fixed), and their whole product is one small
+// matrix per orbit type; a thread owns an orbit and applies it.  Signs come
+// from the pair-local bits only: the environment parity cancels for
+// number-conserving spin parts.  One barrier per pair op.
+//
+// The orbits of a tile depend on (w, electrons of both groups, pair position)
+// only.  They are listed once per space as 32-bit words of LDS offsets, type
+// after type; a thread loads its words two pair ops ahead into registers and
+// the barriers wait for LDS only, so a pair op is LDS reads, the small matrix
+// and LDS writes.  (Indices computed in the kernel from per-spin lists cost
+// more than the matrices: 37 against 24 us for a (12e,12o) stage of 22 ops.)
 //
 // Per rotation string and orbit type (alpha part of the pair empty / doubly
 // occupied / single, same for beta) the host precomputes a 12-bit code: for
@@ -25,12 +34,12 @@
 // string rotates it and with which sign.
 //
 // Kernels:
-//   k_stage_mats    per stage, pair and orbit type: the product of the pair's
-//                   gates (optionally with T_g inserted) from theta
-//   k_stage_fwd     one stage on one vector; dagger runs U^+
-//   k_stage_rev     reverse stage on (psi, lambda): antisymmetric orbit
-//                   products, then un-apply the pair matrices
-//   k_stage_grad    grad[g] from the orbit products summed over tiles
+//   k_op_mats      per pair op and orbit type: the product of the op's gates
+//                  (optionally with T_g inserted) from theta
+//   k_win_fwd      one stage on one vector; dagger runs U^+
+//   k_win_rev      reverse stage on (psi, lambda): antisymmetric orbit
+//                  products, then un-apply the op matrices
+//   k_op_grad      grad[g] from the orbit products summed over blocks
 
 #include <algorithm>
 #include <cmath>
@@ -43,15 +52,11 @@
 
 namespace sq {
 
-constexpr int kMaxPairs = 6;        // hypercubes of at most 64 strings per spin
-constexpr int kTileMax = 4096;      // doubles per vector per tile
-constexpr int kTileMaxCols = 1024;  // columns per tile
-constexpr int kDenseCols = 256;     // columns per tile of a split stage's main launch
-constexpr int kTB = 256;            // threads per block of the reductions
-constexpr int kNT = 512;            // threads per block of the tile kernels
-constexpr int kMaxStageGates = 48;  // stage entries (sa_single counts twice)
-constexpr int kMaxPairEntries = 8;  // entries per pair within a stage
+constexpr int kMaxWin = 8;          // orbitals per window: at most C(8,4)^2 = 4900 amplitudes per tile
+constexpr int kMaxPairEntries = 8;  // entries per pair op (sa_single counts twice)
+constexpr int kMaxOps = 64;         // pair ops per stage
 constexpr int kTypes = 9;           // orbit types (alpha kind x beta kind)
+constexpr int kTB = 256;            // threads per block of the gradient kernel
 
 struct LocalOps {
   int8_t n;
@@ -61,12 +66,11 @@ struct LocalOps {
 
 struct StageEntry {
   int32_t gate;   // program gate index
-  int32_t pair;   // pair index within the stage
   double scale;   // angle multiplier (|coefficient|)
   uint32_t code[kTypes];
 };
 
-// Per pair of a stage, the gates act on orbits of <= 4 amplitudes (member
+// Per pair op, the gates act on orbits of <= 4 amplitudes (member
 // o = alpha bit | beta bit << 1).  Their combined action is one matrix per
 // orbit type, stored compactly in kPairVals doubles:
 //   [0..15]  type (alpha single, beta single): 4x4, row-major M[a][b]
@@ -76,116 +80,140 @@ struct StageEntry {
 //   [28..31] type (alpha double, beta single): 2x2 on members {0, 2}
 // (types without a single pair are left alone by every gate).  A gate's
 // gradient is sum over orbits of <lam|W T W^T|psi> with W the product of the
-// pair's later gates; W T W^T is antisymmetric, so the reverse sweep only
+// op's later gates; W T W^T is antisymmetric, so the reverse sweep only
 // accumulates Q[a<b] = sum (lam_a psi_b - lam_b psi_a):
 //   Q[0..5]  type (single, single): pairs (0,1),(0,2),(0,3),(1,2),(1,3),(2,3)
 //   Q[6..9]  the four two-member types, (member 0, second member)
 constexpr int kPairVals = 32;
 constexpr int kQVals = 10;
-// Pair matrices carry one more value, [32]: the factor for orbits of types
+// Op matrices carry one more value, [32]: the factor for orbits of types
 // without a single pair (1, or 0 when a derivative T_g is inserted on the
-// pair: T_g annihilates them); padded to 36.
+// op: T_g annihilates them); padded to 36.
 constexpr int kMatVals = 36;
 
-// Per pair j of a stage, a 5-bit field (bits 5j..5j+4) of a string's
-// descriptor: kind (2 bits: 0 pair empty, 1 pair doubly occupied, 2 singly
-// occupied with hypercube bit 0, 3 singly occupied with hypercube bit 1) and
-// the hypercube bit index (3 bits).
-// One dispatch slot: alpha rows arows[r0, r0+R), beta stage positions
-// [c0, c1), the alpha group's pair descriptor, the tile's column run and that
-// run's table offset, and the tile's index among the stage's tiles (its
-// gradient partials).  R = 0 marks an empty slot.
+// One dispatch slot: alpha group rows arows[r0, r0 + R), beta group columns
+// bcol[c0, c0 + W), electrons in the window, the orbit words of (ka, kb).
+// R = 0 marks an empty slot.
 struct TileRec {
-  int32_t r0, R, c0, c1;
-  uint32_t adesc;
-  int32_t run, toff, tile;
+  int32_t r0, R, c0, W, ka, kb, items, pad;
 };
 
-// Orbit column lists of one run of beta stage positions [c0, c1), shared by
-// every tile over that run.  Per pair j the run's table holds W = c1 - c0
-// 16-bit entries at ctab[toff + j*W]: first the columns whose beta pair j is
-// singly occupied with hypercube bit 0 (cnt[0][j] of them: 4-member orbits,
-// or 2-member beta orbits when the alpha pair is not single), then the
-// columns with beta pair j empty (cnt[1][j]), then doubly occupied
-// (cnt[2][j]).  inv[t][j] = 1 / max(cnt[t][j], 1) and inv[3][j] =
-// 1 / max(cnt[1][j] + cnt[2][j], 1) (float) split work items into (row,
-// list entry) without a division in the kernels.  Entry = column within the run (10 bits) | hypercube bit of
-// the pair << 10.  Columns holding the upper member of a single beta pair are
-// reached from their lower member and listed nowhere.  The counts are 32-bit
-// so that the tile kernels read them with uniform (scalar) loads.
-struct ColRun {
-  int32_t c0, c1, toff, pad;
-  int32_t cnt[3][8];
-  float inv[4][8];
+// Local strings of k electrons in the window: n4 have a given pair singly
+// occupied (lower member; as many the upper one), ne have it empty, nd doubly
+// occupied, at every pair position.
+struct KInfo {
+  int32_t n4, ne, nd;
+};
+
+// Orbit words of one pair position: five ranges and a sixth (alpha list x
+// beta list), each filled up to whole waves of 64 words with kNone, so that a
+// wave's 64 words are of one type: the type is a scalar branch and every
+// matrix value a scalar operand.
+//   [0, c1)  alpha and beta single: 4 members, m0 | dr << 13 | dc << 26
+//   [c1, c2) alpha single, beta empty    [c2, c3) alpha single, beta double
+//   [c3, c4) alpha empty, beta single    [c4, c5) alpha double, beta single:
+//            2 members, m0 | d << 13
+//   [c5, c6) neither single: m0
+// (in waves; m0: first member, in doubles from the tile's first, which is
+// preceded by a zero that kNone points to; dr, dc, d: distance of the others;
+// swapping neighbouring orbitals moves a string by at most C(6, 3) = 20
+// places).
+struct OpItems {
+  int c1, c2, c3, c4, c5, c6;
+};
+__host__ __device__ inline OpItems op_items(const KInfo& A, const KInfo& B) {
+  auto waves = [](int n) { return (n + 63) / 64; };
+  OpItems o;
+  o.c1 = waves(A.n4 * B.n4);
+  o.c2 = o.c1 + waves(A.n4 * B.ne);
+  o.c3 = o.c2 + waves(A.n4 * B.nd);
+  o.c4 = o.c3 + waves(A.ne * B.n4);
+  o.c5 = o.c4 + waves(A.nd * B.n4);
+  o.c6 = o.c5 + waves((A.ne + A.nd) * (B.ne + B.nd));
+  return o;
+}
+constexpr uint32_t kNone = 0u;  // the zero before the tile
+constexpr int kMaxWaves = 27;   // c5 at most: k = 4 of 8 on both sides
+
+struct OpRef {
+  int32_t op, pos;  // program-wide pair op, pair position within the window
+  int64_t poff;     // its gradient partials
 };
 
 struct StageDev {
-  int npairs;
-  int nsb;
-  int nt;                    // tiles
-  int nb;                    // dispatch slots (the tiles in XCD-aware order, and empty slots)
-  int64_t poff;              // this stage's block of the gradient partials
-  const double* mats;        // this stage's pair matrices [npairs][kMatVals]
-  const int32_t* arows;      // concatenated alpha rows (canonical alpha index), groups sorted by hypercube index
-  const int32_t* bcol;       // per beta stage position: canonical beta column
-  const struct TileRec* tiles;  // [nb]: slot b's tile
-  const ColRun* runs;        // column runs of the stage's tiles
-  const uint16_t* ctab;      // their orbit column tables (runs start 16-byte aligned)
+  int nops, nsb, w, nb;  // nb: dispatch slots
+  const int32_t* arows;
+  const int32_t* bcol;
+  const TileRec* tiles;
+  const uint32_t* items;
+  const OpRef* ops;      // program order
+  KInfo k[kMaxWin + 1];
 };
 
-// Dynamic LDS of one tile, carved in this order (16-byte aligned parts):
-// X[E] (| L[E] in the reverse sweep) | orbit column table [npairs][W]
-// (16-bit) | canonical columns [W] | alpha rows [R].
+struct OpInfo {
+  int32_t e0, e1;   // entries
+  int32_t nblk;     // blocks of the reverse launch
+  int32_t pad;
+  int64_t poff;     // gradient partials [kQVals][nblk]
+};
+
 __host__ __device__ constexpr size_t align16(size_t b) { return (b + 15) / 16 * 16; }
-__host__ __device__ constexpr size_t tab_entries(int npairs, int W) { return ((size_t)npairs * W + 7) / 8 * 8; }
-__host__ __device__ constexpr size_t tile_lds(int E, int W, int R, int npairs, int nvec) {
-  return align16((size_t)E * 8 * nvec) + align16(tab_entries(npairs, W) * 2) + align16((size_t)W * 4) + (size_t)R * 4;
+// Dynamic LDS of one tile: zero, X (| zero, L) | rows | columns.  Two reverse tiles of
+// 70 x 70 amplitudes fit a CU.
+__host__ __device__ constexpr size_t tile_lds(int R, int W, int nvec) {
+  return align16((size_t)R * W * 8 + 8) * nvec + align16(4 * (size_t)(R + W));
 }
-
-// Per tiled stage, what the matrix and gradient kernels need.
-struct StageInfo {
-  int npairs, nentries, ntiles, pad;
-  int pe[kMaxPairs + 1];     // entries of pair j: [pe[j], pe[j+1]) (entries sorted by pair)
-  int64_t poff;              // gradient partials: [npairs][kQVals][ntiles]
-  const StageEntry* entries;
-};
 
 struct Stage {
   bool tiled = false;
-  int g0 = 0, g1 = 0;  // program gates [g0, g1)
-  int npairs = 0;
-  int pp[kMaxPairs];
-  std::vector<StageEntry> entries;
-  int pe[kMaxPairs + 1];
-  int ntiles = 0;
-  int index = -1;              // position among the tiled stages
-  StageDev dev{};              // launch descriptor
-  size_t lds_fwd = 0, lds_rev = 0;  // dynamic LDS of the forward / reverse launches (largest tile)
-  StageDev dev_big{};          // tiles above the target when they run as a side launch (nb = 0: none)
-  size_t lds_fwd_big = 0, lds_rev_big = 0;
-  const StageEntry* d_entries = nullptr;
-  std::vector<void*> allocs;
+  int g0 = 0;                // program gate of an untiled stage
+  StageDev dev{};
+  int rev_blocks = 0;        // grid of the reverse launch
+  size_t lds_fwd = 0, lds_rev = 0;
 };
+
+// Rows, columns and tiles of one window position.
+struct Window {
+  int32_t *arows = nullptr, *bcol = nullptr;
+  TileRec* tiles = nullptr;
+  int nb = 0;
+  int maxR = 0, maxW = 0;
+};
+
+// What the windows of one width need on one space: the orbit words of the
+// (ka, kb) that occur, and the window positions used so far.
+struct WidthTables {
+  KInfo k[kMaxWin + 1] = {};
+  uint32_t* items = nullptr;
+  std::map<std::pair<int, int>, int> off;
+  std::map<int, Window> at;
+};
+
+// Kept by the space (a space's programs share them) and freed with it.
+struct WinCache {
+  std::map<int, WidthTables> width;
+  std::vector<void*> allocs;
+  ~WinCache() {
+    for (void* p : allocs) (void)hipFree(p);
+  }
+};
+
+void win_cache_free(WinCache* c) { delete c; }
 
 struct TilePlan {
   std::vector<Stage> stages;
-  int ntiled = 0;
-  int nt = kNT;  // threads per block of the stage kernels (256 or 512)
-  double* d_partial = nullptr;  // gradient partials of all tiled stages
+  int nops = 0;
+  int nt = 512;                 // threads per block of the stage kernels
+  double* d_partial = nullptr;  // gradient partials of all ops
   int64_t partial_len = 0;
-  double* d_mats = nullptr;     // [ntiled][kMaxPairs][kMatVals]
-  StageInfo* d_info = nullptr;  // [ntiled]
-  hipStream_t side = nullptr;   // side launches of large tiles (default priority, non-blocking)
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  double* d_mats = nullptr;     // [nops][kMatVals]
+  OpInfo* d_info = nullptr;     // [nops]
+  StageEntry* d_entries = nullptr;
+  std::vector<void*> allocs;
   ~TilePlan() {
-    if (ev_fork) (void)hipEventDestroy(ev_fork);
-    if (ev_join) (void)hipEventDestroy(ev_join);
-    if (side) (void)hipStreamDestroy(side);
-    for (auto& s : stages)
-      for (void* p : s.allocs) (void)hipFree(p);
+    for (void* p : allocs) (void)hipFree(p);
     if (d_partial) (void)hipFree(d_partial);
     if (d_mats) (void)hipFree(d_mats);
-    if (d_info) (void)hipFree(d_info);
   }
 };
 
@@ -285,79 +313,6 @@ static bool tile_entries(const Program& P, int g, int& p_out, std::vector<StageE
   return true;
 }
 
-struct GroupInfo {
-  std::vector<int32_t> order;  // strings sorted by (key, h)
-  std::vector<int32_t> start;  // group start per sorted position
-  std::vector<int32_t> goff;   // group offsets
-  std::vector<uint32_t> gocc, gbit;
-  std::vector<uint32_t> occ, bit;  // per sorted position
-};
-
-static GroupInfo group_strings(const std::vector<uint32_t>& strs, int npairs, const int* pp) {
-  uint32_t paired = 0;
-  for (int j = 0; j < npairs; ++j) paired |= 3u << pp[j];
-  const size_t n = strs.size();
-  std::vector<std::pair<std::vector<uint32_t>, int32_t>> keyed(n);
-  std::vector<uint32_t> hyper(n);
-  for (size_t i = 0; i < n; ++i) {
-    uint32_t s = strs[i];
-    std::vector<uint32_t> key;
-    uint32_t h = 0;
-    int b = 0;
-    for (int j = 0; j < npairs; ++j) {
-      uint32_t loc = (s >> pp[j]) & 3u;
-      int c = __builtin_popcount(loc);
-      key.push_back((uint32_t)c);
-      if (c == 1) {
-        if (loc == 2u) h |= 1u << b;
-        ++b;
-      }
-    }
-    key.push_back(s & ~paired);
-    hyper[i] = h;
-    keyed[i] = {key, (int32_t)i};
-  }
-  std::vector<int32_t> idx(n);
-  std::iota(idx.begin(), idx.end(), 0);
-  std::sort(idx.begin(), idx.end(), [&](int32_t x, int32_t y) {
-    if (keyed[x].first != keyed[y].first) return keyed[x].first < keyed[y].first;
-    return hyper[x] < hyper[y];
-  });
-  GroupInfo G;
-  G.order = idx;
-  G.start.resize(n);
-  G.occ.resize(n);
-  G.bit.resize(n);
-  for (size_t k = 0; k < n; ++k) {
-    if (k == 0 || keyed[idx[k]].first != keyed[idx[k - 1]].first) {
-      G.goff.push_back((int32_t)k);
-      uint32_t s = strs[idx[k]];
-      uint32_t gocc = 0, gbit = 0;
-      int b = 0;
-      for (int j = 0; j < npairs; ++j) {
-        uint32_t loc = (s >> pp[j]) & 3u;
-        if (__builtin_popcount(loc) == 1) {
-          gbit |= (uint32_t)b << (4 * j);
-          ++b;
-        } else {
-          gbit |= 0xFu << (4 * j);
-          gocc |= loc << (2 * j);
-        }
-      }
-      G.gocc.push_back(gocc);
-      G.gbit.push_back(gbit);
-    }
-    G.start[k] = G.goff.back();
-    uint32_t s = strs[idx[k]];
-    uint32_t occ = 0;
-    for (int j = 0; j < npairs; ++j) occ |= ((s >> pp[j]) & 3u) << (2 * j);
-    G.occ[k] = occ;
-    G.bit[k] = G.gbit.back();
-  }
-  G.goff.push_back((int32_t)n);
-  return G;
-}
-
 template <class T>
 static T* upload(std::vector<void*>& allocs, const std::vector<T>& v) {
   T* d = nullptr;
@@ -367,316 +322,381 @@ static T* upload(std::vector<void*>& allocs, const std::vector<T>& v) {
   return d;
 }
 
-// Elements per tile that runs of beta groups are filled up to (SQ_TILE_TARGET
-// overrides); a single group pair above it still makes one tile.
-static int tile_target(int64_t dim, int program_target) {
-  if (program_target > 0) return std::min(std::max(program_target, 16), kTileMax);
-  const char* env = getenv("SQ_TILE_TARGET");
-  if (env) return std::min(std::max(atoi(env), 16), kTileMax);
-  // 256..2048 elements, about 400 tiles or more per stage (measured fastest at
-  // (12e,12o) and (14e,14o); the autotuner also tries 4096)
-  int t = 256;
-  while (t < 2048 && (int64_t)t * 2 * 384 <= dim) t *= 2;
-  return t;
+// Local strings of k of w orbitals, lexicographic by occupied orbitals, as the
+// space orders its strings.
+static std::vector<uint32_t> local_strings(int w, int k) {
+  std::vector<uint32_t> strs;
+  std::vector<int> c(k);
+  std::iota(c.begin(), c.end(), 0);
+  for (;;) {
+    uint32_t s = 0;
+    for (int p : c) s |= 1u << p;
+    strs.push_back(s);
+    int i = k - 1;
+    while (i >= 0 && c[i] == w - k + i) --i;
+    if (i < 0) break;
+    ++c[i];
+    for (int j = i + 1; j < k; ++j) c[j] = c[j - 1] + 1;
+  }
+  return strs;
 }
 
-// 5-bit pair fields of a string given its local occupancies (2 bits per pair)
-// and hypercube bit indices (4 bits per pair, 0xF if the pair is not single).
-static uint32_t pair_desc(uint32_t occ, uint32_t bits, int npairs) {
-  uint32_t d = 0;
-  for (int j = 0; j < npairs; ++j) {
-    const uint32_t loc = (occ >> (2 * j)) & 3u;
-    const uint32_t b = (bits >> (4 * j)) & 0xFu;
-    uint32_t f;
-    if (b == 0xFu) f = loc == 0 ? 0u : 1u;
-    else f = (loc == 2u ? 3u : 2u) | (b << 2);
-    d |= f << (5 * j);
-  }
-  return d;
+// Per pair position: lower members, their upper partners, empty, double.
+struct PairLists {
+  std::vector<int> lo, up, em, db;
+};
+static std::vector<PairLists> pair_lists(int w, int k) {
+  const std::vector<uint32_t> strs = local_strings(w, k);
+  std::vector<int> rank((size_t)1 << w, -1);
+  for (size_t i = 0; i < strs.size(); ++i) rank[strs[i]] = (int)i;
+  std::vector<PairLists> out(w - 1);
+  for (int j = 0; j + 1 < w; ++j)
+    for (size_t i = 0; i < strs.size(); ++i) {
+      const uint32_t loc = (strs[i] >> j) & 3u;
+      if (loc == 0u) out[j].em.push_back((int)i);
+      else if (loc == 3u) out[j].db.push_back((int)i);
+      else if (loc == 1u) {
+        out[j].lo.push_back((int)i);
+        out[j].up.push_back(rank[strs[i] ^ (3u << j)]);
+      }
+    }
+  return out;
 }
 
-static void finalize_stage(const Space& sp, Stage& S, int program_target) {
-  // entries grouped by pair, program order kept within a pair
-  std::stable_sort(S.entries.begin(), S.entries.end(),
-                   [](const StageEntry& a, const StageEntry& b) { return a.pair < b.pair; });
-  int* pe = S.pe;
-  for (int j = 0, k = 0; j <= kMaxPairs; ++j) {
-    while (k < (int)S.entries.size() && S.entries[k].pair < j) ++k;
-    pe[j] = k;
+// Orders the words items[from..] so that the 16 lanes which reach LDS together
+// (8-byte accesses, 32 banks of 8 bytes) fall into different banks with every
+// member of their orbits: each group of 16 takes the first words among the
+// next 64 that still fit.  (By this model list order takes 1.9 times the
+// conflict-free cycles and this order 1.04; the counters go from 2.2 to 1.8,
+// a reverse stage from 37.6 to 36.0 us at 12 orbitals, 404 to 393 at 14.)
+static void spread_banks(std::vector<uint32_t>& items, size_t from, bool four) {
+  constexpr int kLook = 64;
+  std::vector<uint32_t> out;
+  out.reserve(items.size() - from);
+  uint32_t look[kLook];
+  int n = 0;
+  size_t next = from;
+  while (n > 0 || next < items.size()) {
+    while (n < kLook && next < items.size()) look[n++] = items[next++];
+    uint32_t used[4] = {0, 0, 0, 0};
+    int taken = 0, kept = 0;
+    uint32_t rest[kLook];
+    for (int i = 0; i < n; ++i) {
+      const uint32_t x = look[i], m0 = x & 8191u;
+      const uint32_t d = four ? (x >> 13) & 8191u : x >> 13, dc = four ? x >> 26 : 0u;
+      const uint32_t bit[4] = {1u << (m0 & 31u), 1u << ((m0 + d) & 31u), 1u << ((m0 + dc) & 31u),
+                               1u << ((m0 + d + dc) & 31u)};
+      bool fits = taken < 16;
+      for (int a = 0; a < (four ? 4 : 2) && fits; ++a) fits = !(used[a] & bit[a]);
+      if (fits) {
+        for (int a = 0; a < (four ? 4 : 2); ++a) used[a] |= bit[a];
+        out.push_back(x);
+        ++taken;
+      } else {
+        rest[kept++] = x;
+      }
+    }
+    // a group that found fewer takes the oldest of the others
+    int i = 0;
+    for (; taken < 16 && i < kept; ++i, ++taken) out.push_back(rest[i]);
+    n = kept - i;
+    std::copy(rest + i, rest + kept, look);
   }
-  GroupInfo A = group_strings(sp.h_astr, S.npairs, S.pp);
-  GroupInfo B = group_strings(sp.h_bstr, S.npairs, S.pp);
-  // tiles: each alpha group x runs of whole beta groups, up to the target
-  // size and maxcols columns; a beta group that alone exceeds the target gets
-  // its own tile
-  const int target = tile_target(sp.dim, program_target);
-  const int nag = (int)A.goff.size() - 1;
-  const int nbg = (int)B.goff.size() - 1;
-  auto build_tiles = [&](int maxcols) {
-    std::vector<int4> out;
-    for (int ga = 0; ga < nag; ++ga) {
-      const int R = A.goff[ga + 1] - A.goff[ga];
-      SQ_CHECK(R <= 64, SQ_ERR_ARG, "tile does not fit: alpha hypercube too large");
-      int gb = 0;
-      while (gb < nbg) {
-        const int c0 = B.goff[gb];
-        int c1 = B.goff[gb + 1];
-        ++gb;
-        while (gb < nbg && (int64_t)R * (B.goff[gb + 1] - c0) <= target && B.goff[gb + 1] - c0 <= maxcols) {
-          c1 = B.goff[gb + 1];
-          ++gb;
+  std::copy(out.begin(), out.end(), items.begin() + from);
+}
+
+// Orbit words of the electron counts that occur in windows of width w.
+static void build_width(const Space& sp, int w, WidthTables& T, std::vector<void*>& allocs) {
+  std::vector<std::vector<PairLists>> L(w + 1);
+  for (int k = 0; k <= w; ++k) {
+    L[k] = pair_lists(w, k);
+    T.k[k] = KInfo{(int)L[k][0].lo.size(), (int)L[k][0].em.size(), (int)L[k][0].db.size()};
+  }
+  auto occurs = [&](int k, int ne) { return k <= ne && ne - k <= sp.n - w; };
+  std::vector<uint32_t> items;
+  for (int ka = 0; ka <= w; ++ka)
+    for (int kb = 0; kb <= w; ++kb) {
+      if (!occurs(ka, sp.na) || !occurs(kb, sp.nb)) continue;
+      T.off[{ka, kb}] = (int)items.size();
+      const int W = (int)local_strings(w, kb).size();
+      for (int j = 0; j + 1 < w; ++j) {
+        const PairLists &A = L[ka][j], &B = L[kb][j];
+        auto at = [&](int r, int c) { return (uint32_t)(1 + r * W + c); };
+        size_t from = items.size();
+        auto fill = [&](bool four) {
+          spread_banks(items, from, four);
+          items.resize((items.size() + 63) / 64 * 64, kNone);
+          from = items.size();
+        };
+        for (size_t r = 0; r < A.lo.size(); ++r)
+          for (size_t c = 0; c < B.lo.size(); ++c)
+            items.push_back(at(A.lo[r], B.lo[c]) | (uint32_t)((A.up[r] - A.lo[r]) * W) << 13 |
+                            (uint32_t)(B.up[c] - B.lo[c]) << 26);
+        fill(true);
+        for (const std::vector<int>* q : {&B.em, &B.db}) {
+          for (size_t r = 0; r < A.lo.size(); ++r)
+            for (int c : *q) items.push_back(at(A.lo[r], c) | (uint32_t)((A.up[r] - A.lo[r]) * W) << 13);
+          fill(false);
         }
-        const int64_t E = (int64_t)R * (c1 - c0);
-        SQ_CHECK(E <= kTileMax && c1 - c0 <= kTileMaxCols, SQ_ERR_ARG, "tile does not fit: hypercube groups too large");
-        out.push_back(int4{ga, c0, c1, (int)E});
+        for (const std::vector<int>* q : {&A.em, &A.db}) {
+          for (int r : *q)
+            for (size_t c = 0; c < B.lo.size(); ++c)
+              items.push_back(at(r, B.lo[c]) | (uint32_t)(B.up[c] - B.lo[c]) << 13);
+          fill(false);
+        }
+        for (const std::vector<int>* q : {&A.em, &A.db})
+          for (int r : *q)
+            for (const std::vector<int>* x : {&B.em, &B.db})
+              for (int c : *x) items.push_back(at(r, c));
+        items.resize((items.size() + 63) / 64 * 64, kNone);
       }
     }
-    return out;
-  };
-  std::vector<int4> tiles = build_tiles(kTileMaxCols);
-  // Occupancy.  Every block of a launch reserves the LDS of the launch's
-  // largest tile.  When the stage has more tiles than the CUs hold at once at
-  // that footprint, the stage runs as two launches side by side: the tiles
-  // above the target (alpha and beta groups that are both large hypercubes,
-  // up to twice the target) in a side launch, the others in the main launch,
-  // rebuilt with at most kDenseCols columns so that their column tables stay
-  // small too (SQ_TILE_SPLIT=0 keeps one launch of the tiles above).
-  bool split = false;
-  {
-    size_t lmax = 0;
-    for (const int4& t : tiles)
-      lmax = std::max(lmax, tile_lds(t.w, t.z - t.y, A.goff[t.x + 1] - A.goff[t.x], S.npairs, 2));
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const int64_t resident = (int64_t)std::max(1, cus) * std::max<int64_t>(1, (int64_t)(160 * 1024) / (int64_t)lmax);
-    const char* senv = getenv("SQ_TILE_SPLIT");
-    split = !(senv && senv[0] == '0') && (int64_t)tiles.size() > resident;
-    if (split) tiles = build_tiles(kDenseCols);
-  }
-  // largest tiles first: they start in the first dispatch round
-  std::stable_sort(tiles.begin(), tiles.end(), [](const int4& a, const int4& b) { return a.w > b.w; });
-  S.ntiles = (int)tiles.size();
-  std::vector<uint32_t> adesc(nag), bdesc(sp.nsb);
-  for (int ga = 0; ga < nag; ++ga) {
-    // kind 2 (single, bit 0) for single pairs; the row's own bit is its hypercube index
-    uint32_t d = 0;
-    for (int j = 0; j < S.npairs; ++j) {
-      const uint32_t b = (A.gbit[ga] >> (4 * j)) & 0xFu;
-      const uint32_t loc = (A.gocc[ga] >> (2 * j)) & 3u;
-      const uint32_t f = b == 0xFu ? (loc == 0 ? 0u : 1u) : (2u | (b << 2));
-      d |= f << (5 * j);
-    }
-    adesc[ga] = d;
-  }
-  for (int k = 0; k < sp.nsb; ++k) bdesc[k] = pair_desc(B.occ[k], B.bit[k], S.npairs);
-  // column runs (distinct [c0, c1)) and their orbit column tables
-  std::map<std::pair<int, int>, int> run_of;
-  std::vector<ColRun> runs;
-  std::vector<uint16_t> ctab;
-  auto run_index = [&](int c0, int c1) {
-    auto it = run_of.find({c0, c1});
-    if (it != run_of.end()) return it->second;
-    ColRun r{};
-    r.c0 = c0;
-    r.c1 = c1;
-    r.toff = (int)ctab.size();
-    const int W = c1 - c0;
-    for (int j = 0; j < S.npairs; ++j) {
-      std::vector<uint16_t> lists[3];
-      for (int k = c0; k < c1; ++k) {
-        const uint32_t f = (bdesc[k] >> (5 * j)) & 31u;
-        const uint32_t kind = f & 3u;
-        const uint16_t e = (uint16_t)((uint32_t)(k - c0) | ((f >> 2) << 10));
-        if (kind == 2u) lists[0].push_back(e);
-        else if (kind == 0u) lists[1].push_back(e);
-        else if (kind == 1u) lists[2].push_back(e);
-      }
-      for (int t = 0; t < 3; ++t) {
-        r.cnt[t][j] = (int32_t)lists[t].size();
-        r.inv[t][j] = 1.0f / (float)std::max<int32_t>(r.cnt[t][j], 1);
-        ctab.insert(ctab.end(), lists[t].begin(), lists[t].end());
-      }
-      r.inv[3][j] = 1.0f / (float)std::max<int32_t>(r.cnt[1][j] + r.cnt[2][j], 1);
-      ctab.resize((size_t)r.toff + (size_t)(j + 1) * W, 0);
-    }
-    ctab.resize((ctab.size() + 7) / 8 * 8, 0);  // next run 16-byte aligned
-    runs.push_back(r);
-    run_of[{c0, c1}] = (int)runs.size() - 1;
-    return (int)runs.size() - 1;
-  };
-  std::vector<TileRec> recs(tiles.size());
-  for (size_t t = 0; t < tiles.size(); ++t) {
-    const int ga = tiles[t].x;
-    const int run = run_index(tiles[t].y, tiles[t].z);
-    recs[t] = TileRec{A.goff[ga], A.goff[ga + 1] - A.goff[ga], tiles[t].y, tiles[t].z, adesc[ga], run,
-                      runs[run].toff, (int32_t)t};
-  }
-  StageDev d{};
-  d.npairs = S.npairs;
-  d.nsb = sp.nsb;
-  d.arows = upload(S.allocs, A.order);
-  d.bcol = upload(S.allocs, B.order);
-  d.runs = upload(S.allocs, runs);
-  d.ctab = upload(S.allocs, ctab);
-  S.d_entries = upload(S.allocs, S.entries);
-  d.nt = S.ntiles;
-  S.dev = d;
-  auto lds_of = [&](const TileRec& r, int nvec) {
-    const int W = r.c1 - r.c0;
-    return tile_lds(r.R * W, W, r.R, S.npairs, nvec);
-  };
-  // the tiles of the side launch (split stages only)
-  std::vector<char> big(tiles.size(), 0);
-  {
-    int nbig = 0;
-    if (split)
-      for (size_t t = 0; t < tiles.size(); ++t) nbig += (big[t] = tiles[t].w > target) ? 1 : 0;
-    if (nbig == (int)tiles.size()) std::fill(big.begin(), big.end(), 0);
-  }
-  // Dispatch order of one launch.  Workgroups go to the XCDs round robin
-  // (slot b on XCD b % 8), each XCD with its own L2.  Tiles of one alpha
-  // group read the same rows of the state, so whole groups are given to one
-  // XCD (groups largest first, each to the XCD with the fewest elements so
-  // far) and run there back to back; SQ_TILE_XCD=0 keeps the plain
-  // largest-first order.  The slots hold the tile records themselves (empty
-  // slots: R = 0).
-  auto make_launch = [&](bool want_big, StageDev& out, size_t& lds_fwd, size_t& lds_rev) {
-    constexpr int kXcds = 8;
-    std::vector<int32_t> mine;
-    for (size_t t = 0; t < tiles.size(); ++t)
-      if ((big[t] != 0) == want_big) mine.push_back((int32_t)t);
-    out = d;
-    out.nb = 0;
-    out.tiles = nullptr;
-    lds_fwd = lds_rev = 0;
-    if (mine.empty()) return;
-    std::vector<int32_t> order;
-    const char* xenv = getenv("SQ_TILE_XCD");
-    if (xenv && xenv[0] == '0') {
-      order = mine;
-    } else {
-      std::vector<std::vector<int32_t>> of_group(nag);
-      std::vector<int64_t> gsize(nag, 0);
-      for (int32_t t : mine) {
-        of_group[tiles[t].x].push_back(t);
-        gsize[tiles[t].x] += tiles[t].w;
-      }
-      std::vector<int> gorder(nag);
-      std::iota(gorder.begin(), gorder.end(), 0);
-      std::stable_sort(gorder.begin(), gorder.end(), [&](int a, int b) { return gsize[a] > gsize[b]; });
-      std::vector<std::vector<int32_t>> bins(kXcds);
-      std::vector<int64_t> load(kXcds, 0);
-      for (int ga : gorder) {
-        if (of_group[ga].empty()) continue;
-        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        load[x] += gsize[ga];
-        bins[x].insert(bins[x].end(), of_group[ga].begin(), of_group[ga].end());
-      }
-      size_t len = 0;
-      for (auto& b : bins) len = std::max(len, b.size());
-      order.assign(len * kXcds, -1);
-      for (int x = 0; x < kXcds; ++x)
-        for (size_t k = 0; k < bins[x].size(); ++k) order[k * kXcds + x] = bins[x][k];
-    }
-    std::vector<TileRec> slots(order.size(), TileRec{0, 0, 0, 0, 0u, 0, 0, -1});
-    for (size_t b = 0; b < order.size(); ++b)
-      if (order[b] >= 0) slots[b] = recs[order[b]];
-    out.nb = (int)slots.size();
-    out.tiles = upload(S.allocs, slots);
-    for (int32_t t : mine) {
-      lds_fwd = std::max(lds_fwd, lds_of(recs[t], 1));
-      lds_rev = std::max(lds_rev, lds_of(recs[t], 2));
-    }
-  };
-  make_launch(false, S.dev, S.lds_fwd, S.lds_rev);
-  make_launch(true, S.dev_big, S.lds_fwd_big, S.lds_rev_big);
+  T.items = upload(allocs, items);
 }
 
-TilePlan* build_tile_plan(const Space& sp, const Program& P) {
+struct Group {
+  int k;
+  std::vector<int32_t> str;
+};
+
+// Strings by occupation outside [lo, lo + w) and electrons inside; canonical
+// order within a group.
+static std::vector<Group> window_groups(const std::vector<uint32_t>& strs, int lo, int w) {
+  const uint32_t in = ((1u << w) - 1u) << lo;
+  std::map<uint64_t, Group> g;
+  for (size_t i = 0; i < strs.size(); ++i) {
+    const int k = __builtin_popcount(strs[i] & in);
+    Group& G = g[(uint64_t)(strs[i] & ~in) << 8 | (uint64_t)k];
+    G.k = k;
+    G.str.push_back((int32_t)i);
+  }
+  std::vector<Group> out;
+  for (auto& x : g) out.push_back(std::move(x.second));
+  return out;
+}
+
+// Tables and dispatch order of one window position.  Workgroups go to the
+// XCDs round robin (slot b on XCD b % 8), each XCD with its own L2: tiles of
+// one alpha group read the same rows of the state, so whole groups are given
+// to one XCD (largest first, each to the XCD with the fewest elements so
+// far), largest tiles first there.  Empty slots have R = 0.
+static Window make_window(const Space& sp, int lo, int w, const WidthTables& T, std::vector<void*>& allocs) {
+  const std::vector<Group> A = window_groups(sp.h_astr, lo, w), B = window_groups(sp.h_bstr, lo, w);
+  Window W;
+  std::vector<int32_t> arows, bcol;
+  std::vector<int> a0, b0;
+  for (const Group& g : A) {
+    a0.push_back((int)arows.size());
+    arows.insert(arows.end(), g.str.begin(), g.str.end());
+    W.maxR = std::max(W.maxR, (int)g.str.size());
+  }
+  for (const Group& g : B) {
+    b0.push_back((int)bcol.size());
+    bcol.insert(bcol.end(), g.str.begin(), g.str.end());
+    W.maxW = std::max(W.maxW, (int)g.str.size());
+  }
+  constexpr int kXcds = 8;
+  std::vector<int> ao(A.size()), bo(B.size());
+  std::iota(ao.begin(), ao.end(), 0);
+  std::iota(bo.begin(), bo.end(), 0);
+  std::stable_sort(ao.begin(), ao.end(), [&](int x, int y) { return A[x].str.size() > A[y].str.size(); });
+  std::stable_sort(bo.begin(), bo.end(), [&](int x, int y) { return B[x].str.size() > B[y].str.size(); });
+  std::vector<std::vector<TileRec>> bins(kXcds);
+  std::vector<int64_t> load(kXcds, 0);
+  // few alpha groups: single tiles are spread instead
+  const bool whole = A.size() >= 2 * kXcds;
+  for (int a : ao) {
+    int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    for (int b : bo) {
+      if (!whole) x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      bins[x].push_back(TileRec{a0[a], (int)A[a].str.size(), b0[b], (int)B[b].str.size(), A[a].k, B[b].k, T.off.at({A[a].k, B[b].k}), 0});
+      load[x] += (int64_t)A[a].str.size() * (int64_t)B[b].str.size();
+    }
+  }
+  size_t len = 0;
+  for (auto& b : bins) {
+    std::stable_sort(b.begin(), b.end(), [](const TileRec& x, const TileRec& y) {
+      return (int64_t)x.R * x.W > (int64_t)y.R * y.W;
+    });
+    len = std::max(len, b.size());
+  }
+  std::vector<TileRec> slots(len * kXcds, TileRec{});
+  for (int x = 0; x < kXcds; ++x)
+    for (size_t k = 0; k < bins[x].size(); ++k) slots[k * kXcds + x] = bins[x][k];
+  while (!slots.empty() && slots.back().R == 0) slots.pop_back();
+  W.nb = (int)slots.size();
+  W.arows = upload(allocs, arows);
+  W.bcol = upload(allocs, bcol);
+  W.tiles = upload(allocs, slots);
+  return W;
+}
+
+struct PairOp {
+  int p;
+  std::vector<StageEntry> entries;
+};
+
+// The order in which stages of width w take the ops of one run: per stage its
+// window position and the ops (indices into ops), program order kept.
+static std::vector<std::pair<int, std::vector<int>>> schedule(const std::vector<PairOp>& ops, int n, int w) {
+  std::vector<std::pair<int, std::vector<int>>> out;
+  std::vector<char> done(ops.size(), 0);
+  size_t left = ops.size();
+  while (left > 0) {
+    int best = -1;
+    std::vector<int> take;
+    for (int lo = 0; lo + w <= n; ++lo) {
+      uint32_t blocked = ~(((1u << w) - 1u) << lo);
+      std::vector<int> t;
+      for (size_t i = 0; i < ops.size() && t.size() < kMaxOps; ++i) {
+        if (done[i]) continue;
+        const uint32_t m = 3u << ops[i].p;
+        if (blocked & m) blocked |= m;
+        else t.push_back((int)i);
+      }
+      if (t.size() > take.size()) {
+        take = t;
+        best = lo;
+      }
+    }
+    for (int i : take) done[i] = 1;
+    left -= take.size();
+    out.push_back({best, take});
+  }
+  return out;
+}
+
+// Window width.  A program's tile target (or SQ_TILE_TARGET) gives the widest
+// window whose mean tile stays below it.  Otherwise the cheapest by a model of the sweep fitted
+// to launches at 8 to 14 orbitals (us, mean of forward and reverse): a stage
+// costs 8 and 0.3 per round of 256 tiles; a pair op 0.55 and 1 more per 9400
+// amplitudes of a tile, or 1 per 3000 amplitudes that a CU has to work through
+// where there are many tiles.  Narrow windows need more stages, wide ones
+// leave small spaces with fewer tiles than CUs.  Measured, energy and
+// gradient with w = 6, 7, 8: (8e,8o) 125, 118, 123; (10e,10o) 142, 134, 147;
+// (11e,11o) 370, 224, 240; (12e,12o) 1536, 674, 496 us; 256 instances of
+// (4e,4o)..(10e,10o) 3.41, 2.19, 1.83 ms.
+static int window_width(const Space& sp, const std::vector<PairOp>& ops, int target, int instances) {
+  const int most = std::min(kMaxWin, sp.n);
+  if (target <= 0)
+    if (const char* env = getenv("SQ_TILE_TARGET")) target = atoi(env);
+  auto groups = [&](int w) {
+    auto count = [&](int k) {
+      int64_t c = 0, b = 1;  // outside strings that leave 0..w electrons inside
+      for (int o = 0; o <= sp.n - w; ++o) {
+        if (k - o >= 0 && k - o <= w) c += b;
+        b = b * (sp.n - w - o) / (o + 1);
+      }
+      return std::max<int64_t>(c, 1);
+    };
+    return count(sp.na) * count(sp.nb);
+  };
+  if (target > 0) {
+    int w = 2;
+    while (w < most && sp.dim <= groups(w + 1) * (int64_t)target) ++w;
+    return w;
+  }
+  int best = most;
+  double cost = -1.0;
+  for (int w = std::min(4, most); w <= most; ++w) {
+    const double tiles = (double)groups(w) * instances;
+    const double tile = (double)sp.dim / (double)groups(w), rounds = std::ceil(tiles / 256.0);
+    const double op = std::max(0.55 + tile / 9400.0, rounds * tile / 3000.0);
+    double c = 0.0;
+    for (auto& st : schedule(ops, sp.n, w)) c += 8.0 + 0.3 * rounds + (double)st.second.size() * op;
+    if (cost < 0.0 || c < cost) {
+      cost = c;
+      best = w;
+    }
+  }
+  return best;
+}
+
+TilePlan* build_tile_plan(const Space& sp, const Program& P, int instances) {
   auto* T = new TilePlan();
   try {
     const int n = (int)P.gates.size();
-    int g = 0;
-    std::vector<StageEntry> ent;
-    while (g < n) {
+    std::vector<StageEntry> ent, all;
+    std::vector<OpInfo> info;
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lock(mu);  // the space's tables are shared
+    if (!sp.win) sp.win = new WinCache;
+    for (int g = 0; g < n;) {
       int p;
       if (!tile_entries(P, g, p, ent)) {
         Stage S;
-        S.tiled = false;
-        S.g0 = g;
-        S.g1 = g + 1;
-        T->stages.push_back(std::move(S));
-        ++g;
+        S.g0 = g++;
+        T->stages.push_back(S);
         continue;
       }
-      Stage S;
-      S.tiled = true;
-      S.g0 = g;
-      S.npairs = 0;
-      int per_pair[kMaxPairs] = {0};
-      while (g < n) {
-        if (!tile_entries(P, g, p, ent)) break;
-        int j = -1;
-        bool clash = false;
-        for (int k = 0; k < S.npairs; ++k) {
-          if (S.pp[k] == p) j = k;
-          else if (std::abs(S.pp[k] - p) < 2) clash = true;
+      // the run of tileable gates from g, merged into pair ops
+      std::vector<PairOp> ops;
+      std::vector<int> last(sp.n, -1);  // latest op on each orbital
+      for (; g < n && tile_entries(P, g, p, ent); ++g) {
+        const int o = last[p];
+        if (o >= 0 && o == last[p + 1] && ops[o].p == p &&
+            ops[o].entries.size() + ent.size() <= (size_t)kMaxPairEntries) {
+          ops[o].entries.insert(ops[o].entries.end(), ent.begin(), ent.end());
+        } else {
+          last[p] = last[p + 1] = (int)ops.size();
+          ops.push_back(PairOp{p, ent});
         }
-        if (clash) break;
-        if (j < 0 && S.npairs == kMaxPairs) break;
-        if ((int)(S.entries.size() + ent.size()) > kMaxStageGates) break;
-        if (j >= 0 && per_pair[j] + (int)ent.size() > kMaxPairEntries) break;
-        if (j < 0) {
-          j = S.npairs;
-          S.pp[S.npairs++] = p;
-        }
-        per_pair[j] += (int)ent.size();
-        for (auto& e : ent) {
-          e.pair = j;
-          S.entries.push_back(e);
-        }
-        ++g;
       }
-      S.g1 = g;
-      T->stages.push_back(std::move(S));
+      const int w = window_width(sp, ops, P.tile_target, instances);
+      auto wt = sp.win->width.find(w);
+      if (wt == sp.win->width.end()) {
+        WidthTables t;
+        build_width(sp, w, t, sp.win->allocs);
+        wt = sp.win->width.emplace(w, std::move(t)).first;
+      }
+      WidthTables& wide = wt->second;
+      for (auto& st : schedule(ops, sp.n, w)) {
+        const int lo = st.first;
+        auto it = wide.at.find(lo);
+        if (it == wide.at.end()) it = wide.at.emplace(lo, make_window(sp, lo, w, wide, sp.win->allocs)).first;
+        const Window& W = it->second;
+        Stage S;
+        S.tiled = true;
+        S.rev_blocks = std::min(W.nb, 1024);
+        std::vector<OpRef> refs;
+        for (int i : st.second) {
+          OpInfo I{};
+          I.e0 = (int)all.size();
+          all.insert(all.end(), ops[i].entries.begin(), ops[i].entries.end());
+          I.e1 = (int)all.size();
+          I.nblk = S.rev_blocks;
+          I.poff = T->partial_len;
+          T->partial_len += (int64_t)kQVals * I.nblk;
+          refs.push_back(OpRef{(int)info.size(), ops[i].p - lo, I.poff});
+          info.push_back(I);
+        }
+        StageDev d{};
+        d.nops = (int)refs.size();
+        d.nsb = sp.nsb;
+        d.w = w;
+        d.nb = W.nb;
+        d.arows = W.arows;
+        d.bcol = W.bcol;
+        d.tiles = W.tiles;
+        d.items = wide.items;
+        d.ops = upload(T->allocs, refs);
+        for (int k = 0; k <= w; ++k) d.k[k] = wide.k[k];
+        S.dev = d;
+        S.lds_fwd = tile_lds(W.maxR, W.maxW, 1);
+        S.lds_rev = tile_lds(W.maxR, W.maxW, 2);
+        T->stages.push_back(S);
+      }
     }
-    int64_t off = 0;
-    std::vector<StageInfo> info;
-    for (auto& S : T->stages) {
-      if (!S.tiled) continue;
-      finalize_stage(sp, S, P.tile_target);
-      S.index = (int)info.size();
-      StageInfo I{};
-      I.npairs = S.npairs;
-      I.nentries = (int)S.entries.size();
-      I.ntiles = S.ntiles;
-      for (int j = 0; j <= kMaxPairs; ++j) I.pe[j] = S.pe[j];
-      I.poff = off;
-      I.entries = S.d_entries;
-      info.push_back(I);
-      S.dev.poff = off;
-      S.dev_big.poff = off;
-      off += (int64_t)S.ntiles * S.npairs * kQVals;
-    }
-    T->ntiled = (int)info.size();
-    T->nt = P.tile_threads == 256 ? 256 : kNT;
-    SQ_HIP(hipMalloc(&T->d_partial, sizeof(double) * std::max<int64_t>(off, 1)));
-    T->partial_len = off;
-    SQ_HIP(hipMalloc(&T->d_mats, sizeof(double) * std::max<int64_t>((int64_t)T->ntiled * kMaxPairs * kMatVals, 1)));
-    for (auto& S : T->stages) {
-      if (!S.tiled) continue;
-      S.dev.mats = T->d_mats + (size_t)S.index * kMaxPairs * kMatVals;
-      S.dev_big.mats = S.dev.mats;
-    }
-    std::vector<void*> tmp;
-    T->d_info = upload(tmp, info);
-    bool any_big = false;
-    for (auto& S : T->stages) any_big = any_big || (S.tiled && S.dev_big.nb > 0);
-    if (any_big) {
-      SQ_HIP(hipStreamCreateWithFlags(&T->side, hipStreamNonBlocking));
-      SQ_HIP(hipEventCreateWithFlags(&T->ev_fork, hipEventDisableTiming));
-      SQ_HIP(hipEventCreateWithFlags(&T->ev_join, hipEventDisableTiming));
-    }
+    T->nops = (int)info.size();
+    // one block per CU and tile: more threads shorten every pair op; more
+    // tiles than that keep the CUs full with smaller blocks
+    int most = 0;
+    for (auto& S : T->stages) most = std::max(most, S.dev.nb);
+    T->nt = P.tile_threads ? P.tile_threads : (int64_t)most * instances <= 256 ? 1024 : 512;
+    T->d_entries = upload(T->allocs, all);
+    T->d_info = upload(T->allocs, info);
+    SQ_HIP(hipMalloc(&T->d_partial, sizeof(double) * std::max<int64_t>(T->partial_len, 1)));
+    SQ_HIP(hipMalloc(&T->d_mats, sizeof(double) * std::max<int64_t>((int64_t)T->nops * kMatVals, 1)));
   } catch (...) {
     delete T;
     throw;
@@ -686,26 +706,29 @@ TilePlan* build_tile_plan(const Space& sp, const Program& P) {
 
 void destroy_tile_plan(TilePlan* T) { delete T; }
 
-bool tile_plan_has_tiles(const TilePlan* T) {
-  if (!T) return false;
-  for (auto& S : T->stages)
-    if (S.tiled) return true;
-  return false;
-}
+static bool usable(const TilePlan* T) { return T && T->nops > 0; }
 
-// Tiled stages are used unless SQ_TILES=0 (column tables hold 16-bit indices).
-const TilePlan* tiles_for(const Space& s, const Program& p) {
-  if (!p.tiles_built) {
-    p.tiles_built = true;
+// Tiled stages are used unless SQ_TILES=0.  Groups of instances (sq_batch.hip)
+// have a plan of their own: with many instances per launch the widest window
+// is the best one.
+static const TilePlan* plan_of(const Space& s, const Program& p, TilePlan*& slot, bool& built, int instances) {
+  if (!built) {
+    built = true;
     const char* env = getenv("SQ_TILES");
     bool enabled = !(env && env[0] == '0');
-    if (enabled && s.dim > 0 && s.nsb <= 65535) p.tiles = build_tile_plan(s, p);
-    if (p.tiles && !tile_plan_has_tiles(p.tiles)) {
-      destroy_tile_plan(p.tiles);
-      p.tiles = nullptr;
+    if (enabled && s.dim > 0 && s.nsb <= 65535) slot = build_tile_plan(s, p, instances);
+    if (slot && !usable(slot)) {
+      destroy_tile_plan(slot);
+      slot = nullptr;
     }
   }
-  return p.tiles;
+  return slot;
+}
+
+const TilePlan* tiles_for(const Space& s, const Program& p) { return plan_of(s, p, p.tiles, p.tiles_built, 1); }
+
+static const TilePlan* group_tiles_for(const Space& s, const Program& p) {
+  return plan_of(s, p, p.group_tiles, p.group_tiles_built, 64);
 }
 
 bool tiles_cover(const Space& s, const Program& p) {
@@ -718,90 +741,22 @@ bool tiles_cover(const Space& s, const Program& p) {
 
 // ---------------------------------------------------------------------------
 // Device kernels.
-//
-// k_stage_mats   per tiled stage and pair, the product of the pair's gates
-//                (optionally with T_g inserted after gate g) per orbit type
-// k_stage_fwd    one stage on one vector: per pair, orbit matrix-vector
-//                products (transposed for U^+)
-// k_stage_rev    reverse stage on (psi, lam): per pair, accumulate the orbit
-//                outer products, then un-apply the pair matrix on both
-// k_stage_grad   per stage and pair, sum the outer products over tiles and
-//                contract them with each gate's conjugated generator
-//
-// Tile kernels run kNT threads per block, one block per tile, one launch per
-// stage; tiles are sorted largest first so that they start in the first
-// dispatch round.  LDS is dynamic and carved per tile (tile_lds); the
-// launch requests the largest tile's footprint.  Pair matrices are read from
-// global memory with uniform (scalar) loads.
-
-// ---- 4x4 orbit algebra (matrix kernels) ------------------------------------
-
-// R M for the rotation of one entry code (disjoint member planes).
-__device__ __forceinline__ void rot_rows(uint32_t code, double c, double s, double (&M)[16]) {
-#pragma unroll
-  for (int sl = 0; sl < 6; ++sl) {
-    const uint32_t f = (code >> (2 * sl)) & 3u;
-    if (!(f & 1u)) continue;
-    const int a = kSlotA[sl], b = kSlotB[sl];
-    const double sg = (f & 2u) ? -s : s;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const double x = M[a * 4 + q], y = M[b * 4 + q];
-      M[a * 4 + q] = c * x - sg * y;
-      M[b * 4 + q] = sg * x + c * y;
-    }
-  }
-}
-
-// M R^T (columns), the other half of a conjugation.
-__device__ __forceinline__ void rot_cols(uint32_t code, double c, double s, double (&M)[16]) {
-#pragma unroll
-  for (int sl = 0; sl < 6; ++sl) {
-    const uint32_t f = (code >> (2 * sl)) & 3u;
-    if (!(f & 1u)) continue;
-    const int a = kSlotA[sl], b = kSlotB[sl];
-    const double sg = (f & 2u) ? -s : s;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const double x = M[q * 4 + a], y = M[q * 4 + b];
-      M[q * 4 + a] = c * x - sg * y;
-      M[q * 4 + b] = sg * x + c * y;
-    }
-  }
-}
-
-// out += scale * T M (rows), T|a> = sg|b>, T|b> = -sg|a> per active plane.
-__device__ __forceinline__ void t_rows(uint32_t code, double scale, const double (&M)[16], double (&out)[16]) {
-#pragma unroll
-  for (int sl = 0; sl < 6; ++sl) {
-    const uint32_t f = (code >> (2 * sl)) & 3u;
-    if (!(f & 1u)) continue;
-    const int a = kSlotA[sl], b = kSlotB[sl];
-    const double sg = (f & 2u) ? -scale : scale;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      out[b * 4 + q] += sg * M[a * 4 + q];
-      out[a * 4 + q] -= sg * M[b * 4 + q];
-    }
-  }
-}
 
 // Orbit-type classes of the compact layout: type index (alpha kind * 3 +
 // beta kind), offset, second member.
 __device__ __constant__ int c_cls_type[5] = {8, 6, 7, 2, 5};
 __device__ __constant__ int c_cls_off[5] = {0, 16, 20, 24, 28};
 
-// Stage entries [e0, e0 + n) staged in LDS with their rotation cosine/sine
-// (one thread per entry), so the products below run on LDS values instead of
-// chains of dependent global loads.
+// An op's entries in LDS with their rotation cosine/sine.
 struct EntryLds {
-  int gate[kMaxStageGates];
-  double scale[kMaxStageGates], c[kMaxStageGates], s[kMaxStageGates];
-  uint32_t code[kMaxStageGates][kTypes];
+  int gate[kMaxPairEntries];
+  double scale[kMaxPairEntries], c[kMaxPairEntries], s[kMaxPairEntries];
+  uint32_t code[kMaxPairEntries][kTypes];
 };
 
-__device__ __forceinline__ void stage_entries(const StageEntry* __restrict__ entries, int e0, int n,
-                                              const double* __restrict__ theta, EntryLds& E) {
+__device__ __forceinline__ void load_entries(const StageEntry* __restrict__ entries, int e0, int n,
+                                             const double* __restrict__ theta, EntryLds& E) {
+  for (int x = threadIdx.x; x < n * kTypes; x += blockDim.x) E.code[x / kTypes][x % kTypes] = entries[e0 + x / kTypes].code[x % kTypes];
   for (int e = threadIdx.x; e < n; e += blockDim.x) {
     const StageEntry& en = entries[e0 + e];
     const double th = theta[en.gate];
@@ -811,132 +766,168 @@ __device__ __forceinline__ void stage_entries(const StageEntry* __restrict__ ent
     E.scale[e] = en.scale;
     E.c[e] = c;
     E.s[e] = s;
-#pragma unroll
-    for (int t = 0; t < kTypes; ++t) E.code[e][t] = en.code[t];
   }
 }
 
-// One thread per (stage, pair, class): the pair's gate product in forward
-// order, with T_g inserted after gate g when deriv_gate is on this pair.
-__global__ __launch_bounds__(64) void k_stage_mats(const StageInfo* __restrict__ info, const double* __restrict__ theta, int deriv_gate,
-                             double* __restrict__ mats, int64_t th_stride, int64_t mats_stride) {
+// v = R v for the rotation of one entry code (disjoint member planes).
+__device__ __forceinline__ void rot_vec(uint32_t code, double c, double s, double (&v)[4]) {
+#pragma unroll
+  for (int sl = 0; sl < 6; ++sl) {
+    const uint32_t f = (code >> (2 * sl)) & 3u;
+    const int a = kSlotA[sl], b = kSlotB[sl];
+    const double cc = (f & 1u) ? c : 1.0, sg = (f & 1u) ? ((f & 2u) ? -s : s) : 0.0;
+    const double x = v[a], y = v[b];
+    v[a] = cc * x - sg * y;
+    v[b] = sg * x + cc * y;
+  }
+}
+
+// out += scale * T v, T|a> = sg|b>, T|b> = -sg|a> per active plane.
+__device__ __forceinline__ void t_vec(uint32_t code, double scale, const double (&v)[4], double (&out)[4]) {
+#pragma unroll
+  for (int sl = 0; sl < 6; ++sl) {
+    const uint32_t f = (code >> (2 * sl)) & 3u;
+    const int a = kSlotA[sl], b = kSlotB[sl];
+    const double sg = (f & 1u) ? ((f & 2u) ? -scale : scale) : 0.0;
+    out[b] += sg * v[a];
+    out[a] -= sg * v[b];
+  }
+}
+
+// One block per pair op: the op's gate product in forward order, with T_g
+// inserted after gate g when deriv_gate is in this op.  A thread carries one
+// column of one class's matrix through the rotations.
+__global__ __launch_bounds__(64) void k_op_mats(const OpInfo* __restrict__ info, const StageEntry* __restrict__ entries,
+                                                const double* __restrict__ theta, int deriv_gate,
+                                                double* __restrict__ mats, int64_t th_stride, int64_t mats_stride) {
   __shared__ EntryLds E;
   theta += blockIdx.y * th_stride;
   mats += blockIdx.y * mats_stride;
-  const StageInfo* __restrict__ I = info + blockIdx.x;
-  stage_entries(I->entries, 0, I->nentries, theta, E);
+  const OpInfo I = info[blockIdx.x];
+  const int n = I.e1 - I.e0;
+  load_entries(entries, I.e0, n, theta, E);
   __syncthreads();
-  const int j = threadIdx.x / 5, cls = threadIdx.x % 5;
-  if (j >= I->npairs) return;
+  const int cls = threadIdx.x >> 2, q = threadIdx.x & 3;
+  if (cls >= 5) return;
   const int t = c_cls_type[cls];
-  double M[16];
-  #pragma unroll
-  for (int q = 0; q < 16; ++q) M[q] = (q % 5 == 0) ? 1.0 : 0.0;
-  const int k0 = I->pe[j], k1 = I->pe[j + 1];
+  double v[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) v[a] = a == q ? 1.0 : 0.0;
   bool has_deriv = false;
-  for (int k = k0; k < k1; ++k) {
-    rot_rows(E.code[k][t], E.c[k], E.s[k], M);
-    if (E.gate[k] == deriv_gate && (k + 1 == k1 || E.gate[k + 1] != deriv_gate)) {
+  for (int k = 0; k < n; ++k) {
+    rot_vec(E.code[k][t], E.c[k], E.s[k], v);
+    if (E.gate[k] == deriv_gate && (k + 1 == n || E.gate[k + 1] != deriv_gate)) {
       has_deriv = true;
-      double o[16];
-      #pragma unroll
-      for (int q = 0; q < 16; ++q) o[q] = 0.0;
-      for (int q = k; q >= k0 && E.gate[q] == deriv_gate; --q) t_rows(E.code[q][t], E.scale[q], M, o);
-      #pragma unroll
-      for (int q = 0; q < 16; ++q) M[q] = o[q];
+      double o[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int x = k; x >= 0 && E.gate[x] == deriv_gate; --x) t_vec(E.code[x][t], E.scale[x], v, o);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) v[a] = o[a];
     }
   }
-  double* base = mats + ((size_t)blockIdx.x * kMaxPairs + j) * kMatVals;
-  if (cls == 0) base[kPairVals] = has_deriv ? 0.0 : 1.0;
+  double* base = mats + (size_t)blockIdx.x * kMatVals;
+  if (threadIdx.x == 0) base[kPairVals] = has_deriv ? 0.0 : 1.0;
   double* out = base + c_cls_off[cls];
   if (cls == 0) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) out[q] = M[q];
+    for (int a = 0; a < 4; ++a) out[a * 4 + q] = v[a];
   } else {
-    const bool a = cls <= 2;  // second member 1 (alpha pair) or 2 (beta pair)
-    out[0] = M[0];
-    out[1] = a ? M[1] : M[2];
-    out[2] = a ? M[4] : M[8];
-    out[3] = a ? M[5] : M[10];
+    const int m1 = cls <= 2 ? 1 : 2;  // second member: alpha pair or beta pair
+    if (q == 0 || q == m1) {
+      out[q ? 1 : 0] = v[0];
+      out[q ? 3 : 2] = m1 == 1 ? v[1] : v[2];
+    }
   }
 }
 
-// One block per (stage, pair): Q summed over the stage's tiles, then for every
-// entry k of the pair dot_k = sum_{a<b} (W T_k W^T)[a][b] Q[a<b] per class, W
-// the product of the pair's entries after k; grad[gate] = 2 sum over its
-// entries of scale * dot.
+// One block per pair op: Q summed over the blocks of the reverse launch, then
+// for every entry k of the op dot_k = sum_{a<b} (W T_k W^T)[a][b] Q[a<b] per
+// class, W the product of the op's entries after k; grad[gate] = 2 sum over
+// its entries of scale * dot.  A thread carries column q of W and of W T_k
+// through the rotations: (W T_k W^T)[a][b] = sum_q (W T_k)[a][q] W[b][q].
 constexpr int kQa[6] = {0, 0, 0, 1, 1, 2};
 constexpr int kQb[6] = {1, 2, 3, 2, 3, 3};
 
-__global__ __launch_bounds__(kTB) void k_stage_grad(const StageInfo* __restrict__ info, const double* __restrict__ theta,
-                             const double* __restrict__ partial, double* __restrict__ grad, int64_t th_stride,
-                             int64_t part_stride, int64_t grad_stride) {
+__global__ __launch_bounds__(kTB) void k_op_grad(const OpInfo* __restrict__ info, const StageEntry* __restrict__ entries,
+                                                 const double* __restrict__ theta, const double* __restrict__ partial,
+                                                 double* __restrict__ grad, int64_t th_stride, int64_t part_stride,
+                                                 int64_t grad_stride) {
   theta += blockIdx.y * th_stride;
   partial += blockIdx.y * part_stride;
   grad += blockIdx.y * grad_stride;
   __shared__ double Q[kQVals];
+  __shared__ double wt[kMaxPairEntries * 5 * 4][8];
   __shared__ double dots[kMaxPairEntries * 5];
-  __shared__ double red[kQVals * (kTB / 64)];
+  __shared__ double red[kQVals][kTB / 64];
   __shared__ EntryLds E;
-  const StageInfo I = info[blockIdx.x / kMaxPairs];
-  const int j = blockIdx.x % kMaxPairs;
-  if (j >= I.npairs) return;
+  const OpInfo I = info[blockIdx.x];
+  const int n = I.e1 - I.e0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int k0 = I.pe[j], k1 = I.pe[j + 1];
-  const int nent = k1 - k0;
-  stage_entries(I.entries, k0, nent, theta, E);  // entries of this pair, indexed from 0
-  {
-    const double* src = partial + I.poff + (size_t)j * kQVals * I.ntiles;
-    double acc[kQVals];
+  double acc[kQVals];
 #pragma unroll
-    for (int v = 0; v < kQVals; ++v) acc[v] = 0.0;
-    for (int tile = threadIdx.x; tile < I.ntiles; tile += blockDim.x) {
+  for (int v = 0; v < kQVals; ++v) acc[v] = 0.0;
+  const double* src = partial + I.poff;
+  for (int b = threadIdx.x; b < I.nblk; b += kTB)
 #pragma unroll
-      for (int v = 0; v < kQVals; ++v) acc[v] += src[(size_t)v * I.ntiles + tile];
-    }
-#pragma unroll
-    for (int v = 0; v < kQVals; ++v) {
-      double a = acc[v];
-      for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
-      if (lane == 0) red[v * (kTB / 64) + wave] = a;
-    }
-    __syncthreads();
-    if (threadIdx.x < kQVals) {
-      double tot = 0.0;
-      for (int w = 0; w < kTB / 64; ++w) tot += red[threadIdx.x * (kTB / 64) + w];
-      Q[threadIdx.x] = tot;
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < nent * 5) {
-    const int k = threadIdx.x / 5, cls = threadIdx.x % 5;
+    for (int v = 0; v < kQVals; ++v) acc[v] += src[(size_t)v * I.nblk + b];
+  load_entries(entries, I.e0, n, theta, E);
+  __syncthreads();
+  if (threadIdx.x < n * 20) {
+    const int k = threadIdx.x / 20, cls = (threadIdx.x % 20) >> 2, q = threadIdx.x & 3;
     const int t = c_cls_type[cls];
-    double M[16];
-    #pragma unroll
-    for (int q = 0; q < 16; ++q) M[q] = 0.0;
-    double I4[16];
-    #pragma unroll
-    for (int q = 0; q < 16; ++q) I4[q] = (q % 5 == 0) ? 1.0 : 0.0;
-    t_rows(E.code[k][t], 1.0, I4, M);  // M = T_k
-    for (int e = k + 1; e < nent; ++e) {
-      rot_rows(E.code[e][t], E.c[e], E.s[e], M);
-      rot_cols(E.code[e][t], E.c[e], E.s[e], M);
+    double w[4], x[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int a = 0; a < 4; ++a) w[a] = a == q ? 1.0 : 0.0;
+    t_vec(E.code[k][t], 1.0, w, x);
+    for (int e = k + 1; e < n; ++e) {
+      rot_vec(E.code[e][t], E.c[e], E.s[e], w);
+      rot_vec(E.code[e][t], E.c[e], E.s[e], x);
     }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      wt[threadIdx.x][a] = w[a];
+      wt[threadIdx.x][4 + a] = x[a];
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < kQVals; ++v) {
+    double a = acc[v];
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
+    if (lane == 0) red[v][wave] = a;
+  }
+  __syncthreads();
+  if (threadIdx.x < kQVals) {
+    double tot = 0.0;
+    for (int w = 0; w < kTB / 64; ++w) tot += red[threadIdx.x][w];
+    Q[threadIdx.x] = tot;
+  }
+  __syncthreads();
+  if (threadIdx.x < n * 5) {
+    const int k = threadIdx.x / 5, cls = threadIdx.x % 5;
+    const double(*c)[8] = wt + k * 20 + cls * 4;
     double d = 0.0;
     if (cls == 0) {
 #pragma unroll
-      for (int q = 0; q < 6; ++q) d += M[kQa[q] * 4 + kQb[q]] * Q[q];
+      for (int x = 0; x < 6; ++x) {
+        double m = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) m += c[q][4 + kQa[x]] * c[q][kQb[x]];
+        d += m * Q[x];
+      }
     } else {
-      d = (cls <= 2 ? M[1] : M[2]) * Q[5 + cls];  // M[0][m1], m1 = 1 (alpha pair) or 2 (beta pair)
+      const int m1 = cls <= 2 ? 1 : 2;
+      double m = 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) m += c[q][4] * c[q][m1];
+      d = m * Q[5 + cls];
     }
     dots[threadIdx.x] = d * E.scale[k];
   }
   __syncthreads();
   // one thread per gate: the first entry of each run of equal gates sums the run
-  if (threadIdx.x < nent && (threadIdx.x == 0 || E.gate[threadIdx.x - 1] != E.gate[threadIdx.x])) {
+  if (threadIdx.x < n && (threadIdx.x == 0 || E.gate[threadIdx.x - 1] != E.gate[threadIdx.x])) {
     const int g = E.gate[threadIdx.x];
     double tot = 0.0;
-    for (int q = threadIdx.x; q < nent && E.gate[q] == g; ++q)
+    for (int q = threadIdx.x; q < n && E.gate[q] == g; ++q)
       for (int cls = 0; cls < 5; ++cls) tot += dots[q * 5 + cls];
     grad[g] = 2.0 * tot;
   }
@@ -944,76 +935,91 @@ __global__ __launch_bounds__(kTB) void k_stage_grad(const StageInfo* __restrict_
 
 // ---- tile kernels -----------------------------------------------------------
 
-struct TileView {
-  int R, W, E, c0;
-  float invW;
-  uint32_t adesc;
-  int tile;  // index among the stage's tiles
-  const ColRun* run;
-};
-
 struct TileLds {
   double* X;
   double* L;
-  uint16_t* tab;  // the run's orbit column table, [npairs][W]
-  uint32_t* ccol;
   int32_t* rows;
+  int32_t* cols;
 };
 
-// LDS parts of one tile (layout of tile_lds).
-__device__ __forceinline__ TileLds carve_lds(double* smem, int E, int W, int npairs, bool rev) {
+__device__ __forceinline__ TileLds carve_lds(double* smem, int R, int W, bool rev) {
   TileLds m;
   char* p = reinterpret_cast<char*>(smem);
+  const size_t v = align16((size_t)R * W * 8 + 8);
   m.X = smem;
-  m.L = rev ? m.X + E : nullptr;
-  p += align16((size_t)E * 8 * (rev ? 2 : 1));
-  m.tab = reinterpret_cast<uint16_t*>(p);
-  p += align16(tab_entries(npairs, W) * 2);
-  m.ccol = reinterpret_cast<uint32_t*>(p);
-  p += align16((size_t)W * 4);
+  p += v;
+  m.L = reinterpret_cast<double*>(p);
+  if (rev) p += v;
+  if (threadIdx.x == 0) {
+    m.X[0] = 0.0;
+    if (rev) m.L[0] = 0.0;
+  }
   m.rows = reinterpret_cast<int32_t*>(p);
+  m.cols = m.rows + R;
   return m;
 }
 
-// Tile descriptors into LDS: alpha rows, the columns' canonical indices and
-// the run's orbit column table (16-byte copies).
+// A tile's canonical rows and columns into LDS.
 template <int NT>
-__device__ __forceinline__ TileView tile_setup(const StageDev& S, double* smem, bool rev, const TileRec& T,
-                                               TileLds& m) {
-  TileView t;
-  t.R = T.R;
-  t.W = T.c1 - T.c0;
-  t.E = t.R * t.W;
-  t.c0 = T.c0;
-  t.invW = 1.0f / (float)t.W;
-  t.adesc = T.adesc;
-  t.tile = T.tile;
-  t.run = S.runs + T.run;
-  m = carve_lds(smem, t.E, t.W, S.npairs, rev);
-  for (int r = threadIdx.x; r < t.R; r += NT) m.rows[r] = S.arows[T.r0 + r];
-  for (int c = threadIdx.x; c < t.W; c += NT) m.ccol[c] = (uint32_t)S.bcol[T.c0 + c];
-  const uint4* src = reinterpret_cast<const uint4*>(S.ctab + T.toff);
-  uint4* dst = reinterpret_cast<uint4*>(m.tab);
-  const int n16 = (int)(tab_entries(S.npairs, t.W) / 8);
-  for (int i = threadIdx.x; i < n16; i += NT) dst[i] = src[i];
+__device__ __forceinline__ void tile_setup(const StageDev& S, const TileRec& T, const TileLds& m) {
+  for (int r = threadIdx.x; r < T.R; r += NT) m.rows[r] = S.arows[T.r0 + r];
+  for (int c = threadIdx.x; c < T.W; c += NT) m.cols[c] = S.bcol[T.c0 + c];
   __syncthreads();
-  return t;
+}
+
+// Data that no kernel in flight writes, read through the constant address
+// space: uniform reads become scalar loads, also past the barriers' memory
+// clobbers (which otherwise turn them into vector loads with a full wait).
+template <class T>
+using ConstPtr = const T __attribute__((address_space(4)))*;
+template <class T>
+__device__ __forceinline__ ConstPtr<T> as_const(const T* p) {
+  return (ConstPtr<T>)(uintptr_t)p;
+}
+
+// Waits for this wave's LDS operations only: orbit words loaded ahead stay in
+// flight.
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+}
+
+// A thread's orbit words of one pair op: wave v takes the wave-sized groups
+// v, v + NT / 64, ...
+template <int NT>
+struct Words {
+  static constexpr int P = (kMaxWaves + NT / 64 - 1) / (NT / 64);
+  uint32_t w[P];
+};
+
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
+template <int NT>
+__device__ __forceinline__ void load_words(const uint32_t* __restrict__ items, int n, Words<NT>& x) {
+#pragma unroll
+  for (int u = 0; u < Words<NT>::P; ++u) {
+    const int g = wave_id() + u * (NT / 64);
+    if (g < n) x.w[u] = items[g * 64 + (threadIdx.x & 63)];
+  }
 }
 
 // Global <-> LDS copies of a tile for NV vectors (psi | lam), gathered
-// through the row and column tables, eight loads per vector in flight.
+// through the row and column tables, U loads per vector in flight.
 template <int NT, int NV>
-__device__ __forceinline__ void tile_load(const StageDev& S, const TileView& t, const TileLds& m,
+__device__ __forceinline__ void tile_load(const StageDev& S, const TileRec& T, const TileLds& m,
                                           const double* __restrict__ g0, const double* __restrict__ g1) {
-  constexpr int U = 8;
-  for (int e0 = threadIdx.x; e0 < t.E; e0 += NT * U) {
+  constexpr int U = NT >= 1024 ? 5 : 8;
+  const int E = T.R * T.W;
+  const float invW = 1.0f / (float)T.W;
+  for (int e0 = threadIdx.x; e0 < E; e0 += NT * U) {
     double v[NV][U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int e = e0 + u * NT;
-      if (e < t.E) {
-        const int r = (int)(((float)e + 0.5f) * t.invW);
-        const size_t idx = (size_t)m.rows[r] * S.nsb + m.ccol[e - r * t.W];
+      if (e < E) {
+        const int r = (int)(((float)e + 0.5f) * invW);
+        const size_t idx = (size_t)m.rows[r] * S.nsb + m.cols[e - r * T.W];
         v[0][u] = g0[idx];
         if (NV > 1) v[NV - 1][u] = g1[idx];
       }
@@ -1021,34 +1027,26 @@ __device__ __forceinline__ void tile_load(const StageDev& S, const TileView& t, 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int e = e0 + u * NT;
-      if (e < t.E) {
-        m.X[e] = v[0][u];
-        if (NV > 1) m.L[e] = v[NV - 1][u];
+      if (e < E) {
+        m.X[1 + e] = v[0][u];
+        if (NV > 1) m.L[1 + e] = v[NV - 1][u];
       }
     }
   }
 }
 
 template <int NT, int NV>
-__device__ __forceinline__ void tile_store(const StageDev& S, const TileView& t, const TileLds& m, double* g0,
+__device__ __forceinline__ void tile_store(const StageDev& S, const TileRec& T, const TileLds& m, double* g0,
                                            double* g1) {
-  for (int e = threadIdx.x; e < t.E; e += NT) {
-    const int r = (int)(((float)e + 0.5f) * t.invW);
-    const size_t idx = (size_t)m.rows[r] * S.nsb + m.ccol[e - r * t.W];
-    g0[idx] = m.X[e];
-    if (NV > 1) g1[idx] = m.L[e];
+  const int E = T.R * T.W;
+  const float invW = 1.0f / (float)T.W;
+  for (int e = threadIdx.x; e < E; e += NT) {
+    const int r = (int)(((float)e + 0.5f) * invW);
+    const int c = e - r * T.W;
+    const size_t idx = (size_t)m.rows[r] * S.nsb + m.cols[c];
+    g0[idx] = m.X[1 + e];
+    if (NV > 1) g1[idx] = m.L[1 + e];
   }
-}
-
-// Work item i over (rows) x (n list entries): row rr and list index k (inv = 1/n).
-__device__ __forceinline__ void split_item(int i, int n, float inv, int& rr, int& k) {
-  rr = (int)(((float)i + 0.5f) * inv);
-  k = i - rr * n;
-}
-
-// Row of the lower alpha member of hypercube row rr: a zero bit inserted at abit.
-__device__ __forceinline__ int ins0(int rr, int abit) {
-  return ((rr >> abit) << (abit + 1)) | (rr & ((1 << abit) - 1));
 }
 
 // o = M v (TR: M^T v), M row-major 4x4.
@@ -1063,85 +1061,53 @@ __device__ __forceinline__ void mat4(const double (&M)[16], const double (&v)[4]
   }
 }
 
-// One pair pass of a forward stage on the tile in LDS.  Orbits come from the
-// run's column lists, so every work item is one orbit and a wave runs one
-// orbit type except where two lists meet.  Orbit members: 0 = (alpha lower,
-// beta lower) at m0, 1 = alpha upper (+ dr), 2 = beta upper (+ dc), 3 = both.
-// The pair's matrix values are read into registers before the orbit loops,
-// and the 2-member orbits of beta-empty and beta-double columns run as
-// separate item ranges, so every matrix value stays a wave-uniform (scalar)
-// operand.
 template <bool TR>
-__device__ __forceinline__ void orbit2(double* X, int m0, int d, const double (&B)[4]) {
-  const double v0 = X[m0], v1 = X[m0 + d];
+__device__ __forceinline__ void orbit2(double* X, uint32_t w, const double (&B)[4]) {
+  const int m0 = (int)(w & 8191u), m1 = m0 + (int)(w >> 13);
+  const double v0 = X[m0], v1 = X[m1];
   X[m0] = B[0] * v0 + (TR ? B[2] : B[1]) * v1;
-  X[m0 + d] = (TR ? B[1] : B[2]) * v0 + B[3] * v1;
+  X[m1] = (TR ? B[1] : B[2]) * v0 + B[3] * v1;
 }
 
 template <int NT, bool TR>
-__device__ __forceinline__ void fwd_pair(const TileView& t, const TileLds& m, const double* __restrict__ Mp, int j) {
-  const uint32_t fa = (t.adesc >> (5 * j)) & 31u;
-  const int n4 = t.run->cnt[0][j], n2e = t.run->cnt[1][j], n2d = t.run->cnt[2][j];
-  const uint16_t* tab = m.tab + j * t.W;
-  double* X = m.X;
-  const int W = t.W;
-  if ((fa & 3u) >= 2u) {  // alpha pair single: 4-member orbits, then 2-member alpha orbits
-    const int abit = (int)(fa >> 2);
-    const int Rh = t.R >> 1, dr = W << abit;
-    const int nA = Rh * n4, nE = nA + Rh * n2e, nT = nE + Rh * n2d;
-    const float iA = t.run->inv[0][j], iE = t.run->inv[1][j], iD = t.run->inv[2][j];
-    double M[16], be[4], bd[4];
+__device__ __forceinline__ void fwd_op(const OpItems& o, const Words<NT>& x, double* X, ConstPtr<double> Mp,
+                                       const uint32_t* __restrict__ items) {
+  double M[16], be[4], bd[4], ae[4], ad[4];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) M[q] = Mp[q];
+  for (int q = 0; q < 16; ++q) M[q] = Mp[q];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      be[q] = Mp[16 + q];
-      bd[q] = Mp[20 + q];
-    }
-    for (int i = threadIdx.x; i < nT; i += NT) {
-      int rr, k;
-      if (i < nA) {
-        split_item(i, n4, iA, rr, k);
-        const uint32_t e = tab[k];
-        const int m0 = ins0(rr, abit) * W + (int)(e & 1023u);
-        const int m2 = m0 + (1 << (e >> 10));
-        const double v[4] = {X[m0], X[m0 + dr], X[m2], X[m2 + dr]};
-        double o[4];
-        mat4<TR>(M, v, o);
-        X[m0] = o[0];
-        X[m0 + dr] = o[1];
-        X[m2] = o[2];
-        X[m2 + dr] = o[3];
-      } else if (i < nE) {  // beta pair empty
-        split_item(i - nA, n2e, iE, rr, k);
-        orbit2<TR>(X, ins0(rr, abit) * W + (int)(tab[n4 + k] & 1023u), dr, be);
-      } else {  // beta pair doubly occupied
-        split_item(i - nE, n2d, iD, rr, k);
-        orbit2<TR>(X, ins0(rr, abit) * W + (int)(tab[n4 + n2e + k] & 1023u), dr, bd);
-      }
-    }
-  } else {  // alpha pair empty or double: 2-member beta orbits; other amplitudes stay
-    const double* Bp = Mp + ((fa & 3u) == 0u ? 24 : 28);
-    const double B[4] = {Bp[0], Bp[1], Bp[2], Bp[3]};
-    const bool deriv = Mp[kPairVals] == 0.0;
-    const int nA = t.R * n4;
-    const float iA = t.run->inv[0][j];
-    for (int i = threadIdx.x; i < nA; i += NT) {
-      int rr, k;
-      split_item(i, n4, iA, rr, k);
-      const uint32_t e = tab[k];
-      orbit2<TR>(X, rr * W + (int)(e & 1023u), 1 << (e >> 10), B);
-    }
-    if (deriv) {  // derivative pair: T_g annihilates the amplitudes no gate moves
-      const int n2 = n2e + n2d, nB = t.R * n2;
-      const float iB = t.run->inv[3][j];
-      for (int i = threadIdx.x; i < nB; i += NT) {
-        int rr, k;
-        split_item(i, n2, iB, rr, k);
-        X[rr * W + (int)(tab[n4 + k] & 1023u)] = 0.0;
-      }
+  for (int q = 0; q < 4; ++q) {
+    be[q] = Mp[16 + q];
+    bd[q] = Mp[20 + q];
+    ae[q] = Mp[24 + q];
+    ad[q] = Mp[28 + q];
+  }
+  const bool deriv = Mp[kPairVals] == 0.0;
+#pragma unroll
+  for (int u = 0; u < Words<NT>::P; ++u) {
+    const int g = wave_id() + u * (NT / 64);
+    const uint32_t w = x.w[u];
+    if (g < o.c1) {
+      const int m0 = (int)(w & 8191u), dr = (int)((w >> 13) & 8191u), dc = (int)(w >> 26);
+      const double v[4] = {X[m0], X[m0 + dr], X[m0 + dc], X[m0 + dr + dc]};
+      double y[4];
+      mat4<TR>(M, v, y);
+      X[m0] = y[0];
+      X[m0 + dr] = y[1];
+      X[m0 + dc] = y[2];
+      X[m0 + dr + dc] = y[3];
+    } else if (g < o.c2) {
+      orbit2<TR>(X, w, be);
+    } else if (g < o.c3) {
+      orbit2<TR>(X, w, bd);
+    } else if (g < o.c4) {
+      orbit2<TR>(X, w, ae);
+    } else if (g < o.c5) {
+      orbit2<TR>(X, w, ad);
     }
   }
+  if (deriv)  // T_g annihilates the amplitudes no gate moves
+    for (int i = o.c5 * 64 + threadIdx.x; i < o.c6 * 64; i += NT) X[items[i]] = 0.0;
 }
 
 // DPP lane moves of a double (bound_ctrl: lanes without a source read 0).
@@ -1152,216 +1118,221 @@ __device__ __forceinline__ double dpp_move(double v) {
   return __hiloint2double(hi, lo);
 }
 
-// Row sums (16 lanes) of 8 per-lane values with halving exchanges inside
-// each quad (xor 1, xor 2) and row shifts by 4 and 8: lane l with
-// l % 16 >= 12 ends with the row sums of values
-// q = (l & 1) * 4 + ((l >> 1) & 1) * 2 + {0, 1} in w[0], w[1].
-// Every lane of the wave must be active.
-__device__ __forceinline__ void row_fold8(const double (&Q)[8], double (&w)[2], int lane) {
-  const bool o1 = lane & 1, o2 = lane & 2;
-  double w1[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const double keep = o1 ? Q[4 + i] : Q[i], send = o1 ? Q[i] : Q[4 + i];
-    w1[i] = keep + dpp_move<0xb1, 0xf>(send);  // quad_perm [1,0,3,2]
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const double keep = o2 ? w1[2 + i] : w1[i], send = o2 ? w1[i] : w1[2 + i];
-    w[i] = keep + dpp_move<0x4e, 0xf>(send);  // quad_perm [2,3,0,1]
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    w[i] += dpp_move<0x114, 0xf>(w[i]);  // row_shr:4
-    w[i] += dpp_move<0x118, 0xf>(w[i]);  // row_shr:8
-  }
-}
-
-// Row sum of one value; lane l with l % 16 == 15 holds it.
+// Sum over each row of 16 lanes, in the row's last lane.
 __device__ __forceinline__ double row_sum(double v) {
-  v += dpp_move<0xb1, 0xf>(v);
-  v += dpp_move<0x4e, 0xf>(v);
-  v += dpp_move<0x114, 0xf>(v);
-  v += dpp_move<0x118, 0xf>(v);
+  v += dpp_move<0xb1, 0xf>(v);   // quad_perm [1,0,3,2]
+  v += dpp_move<0x4e, 0xf>(v);   // quad_perm [2,3,0,1]
+  v += dpp_move<0x114, 0xf>(v);  // row_shr:4
+  v += dpp_move<0x118, 0xf>(v);  // row_shr:8
   return v;
 }
 
-// Gates of one stage on one vector (canonical order, in place).
-// dagger: U^+ (transposed pair matrices).  src may be dst (in place) or the
-// sweep's input vector (first stage).
-template <int NT>
-__global__ __launch_bounds__(NT) void k_stage_fwd(StageDev S, const double* __restrict__ mats, int dagger,
-                                                  const double* src, double* dst, int64_t mats_stride,
-                                                  int64_t vec_stride) {
+// Wave sums of four values on the matrix cores.  v_mfma_f64_4x4x4 contracts
+// over the four rows of 16 lanes: A[i][k] at lane i + 4 b + 16 k, B[k][j] at
+// lane j + 4 b + 16 k, D[i][j] at lane j + 4 b + 16 i.  With A[i][k] = 1 for
+// i = q only, value q's sum over the rows lands in row q of D; the four
+// products add into one register, whose rows are then summed.  Row q's last
+// lane ends with the sum of value q.  (Four MFMAs and 12 vector instructions
+// for four values, against about 44 with lane exchanges.)
+__device__ __forceinline__ double rows_of(double acc, double one, double v) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(one, v, acc, 0, 0, 0);
+}
+
+// The pair ops of one stage on one vector (canonical order, in place).
+// dagger: U^+ (transposed matrices, ops in reverse).  src may be dst (in
+// place) or the sweep's input vector (first stage).
+template <int NT, bool DAGGER>
+__global__ __launch_bounds__(NT) void k_win_fwd(StageDev S, const double* __restrict__ mats, const double* src, double* dst, int64_t mats_stride,
+                                                int64_t vec_stride) {
   extern __shared__ double smem[];
   mats += blockIdx.y * mats_stride;
   src += blockIdx.y * vec_stride;
   dst += blockIdx.y * vec_stride;
-  // block b walks slots b, b + grid, ... (tiles are sorted largest first)
   for (int slot = blockIdx.x; slot < S.nb; slot += gridDim.x) {
-    const TileRec T = S.tiles[slot];
+    const ConstPtr<TileRec> tp = as_const(S.tiles) + slot;
+    const TileRec T{tp->r0, tp->R, tp->c0, tp->W, tp->ka, tp->kb, tp->items, 0};
     if (T.R == 0) continue;
-    TileLds m;
-    const TileView t = tile_setup<NT>(S, smem, false, T, m);
-    tile_load<NT, 1>(S, t, m, src, nullptr);
-    __syncthreads();
-    for (int j = 0; j < S.npairs; ++j) {
-      if (dagger) fwd_pair<NT, true>(t, m, mats + j * kMatVals, j);
-      else fwd_pair<NT, false>(t, m, mats + j * kMatVals, j);
-      __syncthreads();
+    const TileLds m = carve_lds(smem, T.R, T.W, false);
+    const OpItems o = op_items(S.k[T.ka], S.k[T.kb]);
+    const uint32_t* items = S.items + T.items;
+    auto at = [&](int j) { return as_const(S.ops) + (DAGGER ? S.nops - 1 - j : j); };
+    auto load = [&](int j, Words<NT>& x) {
+      if (j < S.nops) load_words<NT>(items + at(j)->pos * o.c6 * 64, o.c5, x);
+    };
+    auto step = [&](int j, const Words<NT>& cur, Words<NT>& fill) {
+      if (j >= S.nops) return;
+      lds_barrier();
+      load(j + 2, fill);
+      const int op = at(j)->op, pos = at(j)->pos;
+      fwd_op<NT, DAGGER>(o, cur, m.X, as_const(mats) + op * kMatVals, items + pos * o.c6 * 64);
+    };
+    tile_setup<NT>(S, T, m);
+    Words<NT> a, b, c;
+    load(0, a);
+    load(1, b);
+    tile_load<NT, 1>(S, T, m, src, nullptr);
+    for (int j = 0; j < S.nops; j += 3) {
+      step(j, a, c);
+      step(j + 1, b, a);
+      step(j + 2, c, b);
     }
-    tile_store<NT, 1>(S, t, m, dst, nullptr);
+    __syncthreads();
+    tile_store<NT, 1>(S, T, m, dst, nullptr);
     __syncthreads();  // the next tile overwrites the LDS tables
   }
 }
 
-// One 2-member orbit of the reverse sweep at (m0, m0 + d): returns its
-// product lam_0 psi_1 - lam_1 psi_0 and, with wb, un-applies the matrix (B^T)
-// on both vectors.
-__device__ __forceinline__ double rev_orbit2(double* X, double* L, int m0, int d, const double (&B)[4], bool wb) {
-  const double v0 = X[m0], v1 = X[m0 + d], w0 = L[m0], w1 = L[m0 + d];
-  if (wb) {
-    X[m0] = B[0] * v0 + B[2] * v1;
-    X[m0 + d] = B[1] * v0 + B[3] * v1;
-    L[m0] = B[0] * w0 + B[2] * w1;
-    L[m0 + d] = B[1] * w0 + B[3] * w1;
-  }
+// One 2-member orbit of the reverse sweep: returns its product
+// lam_0 psi_1 - lam_1 psi_0 and un-applies the matrix (B^T) on both vectors.
+__device__ __forceinline__ double rev_orbit2(double* X, double* L, uint32_t w, const double (&B)[4]) {
+  const int m0 = (int)(w & 8191u), m1 = m0 + (int)(w >> 13);
+  const double v0 = X[m0], v1 = X[m1], w0 = L[m0], w1 = L[m1];
+  X[m0] = B[0] * v0 + B[2] * v1;
+  X[m1] = B[1] * v0 + B[3] * v1;
+  L[m0] = B[0] * w0 + B[2] * w1;
+  L[m1] = B[1] * w0 + B[3] * w1;
   return w0 * v1 - w1 * v0;
 }
 
-// Reverse stage on (psi, lam), in place: per pair, the antisymmetric orbit
-// products Q[a<b] += lam_a psi_b - lam_b psi_a before un-applying the pair
-// matrix (M^T) on both; per-tile sums go to partial[poff + (j*10 + v)*ntiles + tile].
-// Per pair the wave sums land in red[j][.][wave] (8 values when the alpha
-// pair is single, else one: the beta orbit type of the alpha occupation).
+// Reverse stage on (psi, lam), in place: per pair op, the antisymmetric orbit
+// products Q[a<b] += lam_a psi_b - lam_b psi_a before un-applying the op's
+// matrix (M^T) on both.  The wave sums of an op are added up by one wave
+// during the next op and go to partial[poff + v * blocks + block], which a
+// block that walks several tiles accumulates.
 template <int NT>
-__global__ __launch_bounds__(NT) void k_stage_rev(StageDev S, const double* __restrict__ mats,
-                                                  double* __restrict__ psi, double* __restrict__ lam,
-                                                  double* __restrict__ partial, int write_back, int64_t mats_stride,
-                                                  int64_t vec_stride, int64_t part_stride) {
+__global__ __launch_bounds__(NT) void k_win_rev(StageDev S, const double* __restrict__ mats, double* __restrict__ psi,
+                                                double* __restrict__ lam, double* __restrict__ partial, int write_back,
+                                                int64_t mats_stride, int64_t vec_stride, int64_t part_stride) {
   mats += blockIdx.y * mats_stride;
   psi += blockIdx.y * vec_stride;
   lam += blockIdx.y * vec_stride;
   partial += blockIdx.y * part_stride;
   constexpr int kWaves = NT / 64;
   extern __shared__ double smem[];
-  __shared__ double red[kMaxPairs][8][kWaves];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool wb = write_back != 0;
+  __shared__ double red[2][kQVals][kWaves];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  double sel[4];  // rows_of's selectors
+#pragma unroll
+  for (int q = 0; q < 4; ++q) sel[q] = (lane & 3) == q ? 1.0 : 0.0;
+  bool first = true;
   for (int slot = blockIdx.x; slot < S.nb; slot += gridDim.x) {
-    const TileRec T = S.tiles[slot];
+    const ConstPtr<TileRec> tp = as_const(S.tiles) + slot;
+    const TileRec T{tp->r0, tp->R, tp->c0, tp->W, tp->ka, tp->kb, tp->items, 0};
     if (T.R == 0) continue;
-    TileLds m;
-    const TileView t = tile_setup<NT>(S, smem, true, T, m);
-    tile_load<NT, 2>(S, t, m, psi, lam);
-    __syncthreads();
-    const int W = t.W;
+    const TileLds m = carve_lds(smem, T.R, T.W, true);
+    const OpItems o = op_items(S.k[T.ka], S.k[T.kb]);
+    const uint32_t* items = S.items + T.items;
     double* X = m.X;
     double* L = m.L;
-    for (int j = 0; j < S.npairs; ++j) {
-      const double* __restrict__ Mp = mats + j * kMatVals;
-      const uint32_t fa = (t.adesc >> (5 * j)) & 31u;
-      const int n4 = t.run->cnt[0][j], n2e = t.run->cnt[1][j], n2d = t.run->cnt[2][j];
-      const uint16_t* tab = m.tab + j * W;
-      double Q[8];
+    auto load = [&](int j, Words<NT>& x) {
+      if (j >= 0) load_words<NT>(items + as_const(S.ops)[j].pos * o.c6 * 64, o.c5, x);
+    };
+    auto finish = [&](int j) {  // op j's wave sums to the block's partial
+      if (wave == (j & (kWaves - 1)) && lane < kQVals) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) v += red[j & 1][lane][w];
+        double* dst = partial + as_const(S.ops)[j].poff + (size_t)lane * gridDim.x + blockIdx.x;
+        *dst = first ? v : *dst + v;
+      }
+    };
+    auto step = [&](int j, const Words<NT>& cur, Words<NT>& fill) {
+      if (j < 0) return;
+      lds_barrier();
+      load(j - 2, fill);
+      const ConstPtr<double> Mp = as_const(mats) + as_const(S.ops)[j].op * kMatVals;
+      double M[16], be[4], bd[4], ae[4], ad[4];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) M[q] = Mp[q];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        be[q] = Mp[16 + q];
+        bd[q] = Mp[20 + q];
+        ae[q] = Mp[24 + q];
+        ad[q] = Mp[28 + q];
+      }
+      double Q[8], Qe = 0.0, Qd = 0.0;
 #pragma unroll
       for (int q = 0; q < 8; ++q) Q[q] = 0.0;
-      if ((fa & 3u) >= 2u) {
-        const int abit = (int)(fa >> 2);
-        const int Rh = t.R >> 1, dr = W << abit;
-        const int nA = Rh * n4, nE = nA + Rh * n2e, nT = nE + Rh * n2d;
-        const float iA = t.run->inv[0][j], iE = t.run->inv[1][j], iD = t.run->inv[2][j];
-        double M[16], be[4], bd[4];  // pair matrix in registers (see fwd_pair)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) M[q] = Mp[q];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          be[q] = Mp[16 + q];
-          bd[q] = Mp[20 + q];
+      for (int u = 0; u < Words<NT>::P; ++u) {
+        const int g = wave_id() + u * (NT / 64);
+        const uint32_t x = cur.w[u];
+        if (g < o.c1) {
+          const int m0 = (int)(x & 8191u), dr = (int)((x >> 13) & 8191u), dc = (int)(x >> 26);
+          const double v[4] = {X[m0], X[m0 + dr], X[m0 + dc], X[m0 + dr + dc]};
+          const double w[4] = {L[m0], L[m0 + dr], L[m0 + dc], L[m0 + dr + dc]};
+          Q[0] += w[0] * v[1] - w[1] * v[0];
+          Q[1] += w[0] * v[2] - w[2] * v[0];
+          Q[2] += w[0] * v[3] - w[3] * v[0];
+          Q[3] += w[1] * v[2] - w[2] * v[1];
+          Q[4] += w[1] * v[3] - w[3] * v[1];
+          Q[5] += w[2] * v[3] - w[3] * v[2];
+          double y[4];
+          mat4<true>(M, v, y);
+          X[m0] = y[0];
+          X[m0 + dr] = y[1];
+          X[m0 + dc] = y[2];
+          X[m0 + dr + dc] = y[3];
+          mat4<true>(M, w, y);
+          L[m0] = y[0];
+          L[m0 + dr] = y[1];
+          L[m0 + dc] = y[2];
+          L[m0 + dr + dc] = y[3];
+        } else if (g < o.c2) {
+          Q[6] += rev_orbit2(X, L, x, be);
+        } else if (g < o.c3) {
+          Q[7] += rev_orbit2(X, L, x, bd);
+        } else if (g < o.c4) {
+          Qe += rev_orbit2(X, L, x, ae);
+        } else if (g < o.c5) {
+          Qd += rev_orbit2(X, L, x, ad);
         }
-        for (int i = threadIdx.x; i < nT; i += NT) {
-          if (i < nA) {
-            int rr, k;
-            split_item(i, n4, iA, rr, k);
-            const uint32_t e = tab[k];
-            const int m0 = ins0(rr, abit) * W + (int)(e & 1023u);
-            const int m2 = m0 + (1 << (e >> 10));
-            const double v[4] = {X[m0], X[m0 + dr], X[m2], X[m2 + dr]};
-            const double w[4] = {L[m0], L[m0 + dr], L[m2], L[m2 + dr]};
-            Q[0] += w[0] * v[1] - w[1] * v[0];
-            Q[1] += w[0] * v[2] - w[2] * v[0];
-            Q[2] += w[0] * v[3] - w[3] * v[0];
-            Q[3] += w[1] * v[2] - w[2] * v[1];
-            Q[4] += w[1] * v[3] - w[3] * v[1];
-            Q[5] += w[2] * v[3] - w[3] * v[2];
-            if (wb) {
-              double ov[4], ow[4];
-              mat4<true>(M, v, ov);
-              mat4<true>(M, w, ow);
-              X[m0] = ov[0];
-              X[m0 + dr] = ov[1];
-              X[m2] = ov[2];
-              X[m2 + dr] = ov[3];
-              L[m0] = ow[0];
-              L[m0 + dr] = ow[1];
-              L[m2] = ow[2];
-              L[m2 + dr] = ow[3];
-            }
-          } else if (i < nE) {  // beta pair empty
-            int rr, k;
-            split_item(i - nA, n2e, iE, rr, k);
-            Q[6] += rev_orbit2(X, L, ins0(rr, abit) * W + (int)(tab[n4 + k] & 1023u), dr, be, wb);
-          } else {  // beta pair doubly occupied
-            int rr, k;
-            split_item(i - nE, n2d, iD, rr, k);
-            Q[7] += rev_orbit2(X, L, ins0(rr, abit) * W + (int)(tab[n4 + n2e + k] & 1023u), dr, bd, wb);
-          }
-        }
-        double w2[2];
-        row_fold8(Q, w2, lane);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {  // across the rows of the wave
-          w2[i] += __shfl_xor(w2[i], 16, 64);
-          w2[i] += __shfl_xor(w2[i], 32, 64);
-        }
-        if (lane >= 60) {
-          const int q = (lane & 1) * 4 + ((lane >> 1) & 1) * 2;
-          red[j][q][wave] = w2[0];
-          red[j][q + 1][wave] = w2[1];
-        }
-      } else {
-        const double* Bp = Mp + ((fa & 3u) == 0u ? 24 : 28);
-        const double B[4] = {Bp[0], Bp[1], Bp[2], Bp[3]};
-        const int nA = t.R * n4;
-        const float iA = t.run->inv[0][j];
-        for (int i = threadIdx.x; i < nA; i += NT) {
-          int rr, k;
-          split_item(i, n4, iA, rr, k);
-          const uint32_t e = tab[k];
-          Q[0] += rev_orbit2(X, L, rr * W + (int)(e & 1023u), 1 << (e >> 10), B, wb);
-        }
-        double s = row_sum(Q[0]);
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
-        if (lane == 63) red[j][0][wave] = s;
       }
-      __syncthreads();
+      // a wave's groups are wave, wave + kWaves, ...: the types it has
+      const bool four = wave < o.c1;
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+      if (four) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s0 = rows_of(s0, sel[q], Q[q]);
+        s1 = rows_of(s1, sel[0], Q[4]);
+        s1 = rows_of(s1, sel[1], Q[5]);
+        s0 = row_sum(s0);
+      }
+      s1 = rows_of(s1, sel[2], Q[6]);
+      s1 = rows_of(s1, sel[3], Q[7]);
+      s2 = rows_of(s2, sel[0], Qe);
+      s2 = rows_of(s2, sel[1], Qd);
+      s1 = row_sum(s1);
+      s2 = row_sum(s2);
+      if ((lane & 15) == 15) {
+        const int q = lane >> 4;
+        red[j & 1][q][wave] = s0;
+        red[j & 1][4 + q][wave] = s1;
+        if (q < 2) red[j & 1][8 + q][wave] = s2;
+      }
+      if (j + 1 < S.nops) finish(j + 1);
+    };
+    tile_setup<NT>(S, T, m);
+    Words<NT> a, b, c;
+    load(S.nops - 1, a);
+    load(S.nops - 2, b);
+    tile_load<NT, 2>(S, T, m, psi, lam);
+    for (int j = S.nops - 1; j >= 0; j -= 3) {
+      step(j, a, c);
+      step(j - 1, b, a);
+      step(j - 2, c, b);
     }
-    for (int x = threadIdx.x; x < S.npairs * kQVals; x += NT) {
-      const int j = x / kQVals, q = x - j * kQVals;
-      const uint32_t fa = (t.adesc >> (5 * j)) & 31u;
-      int src = -1;
-      if ((fa & 3u) >= 2u) src = q < 8 ? q : -1;
-      else src = q == ((fa & 3u) == 0u ? 8 : 9) ? 0 : -1;
-      double v = 0.0;
-      if (src >= 0)
-        for (int w = 0; w < kWaves; ++w) v += red[j][src][w];
-      partial[S.poff + (size_t)x * S.nt + t.tile] = v;
-    }
-    if (wb)  // not for the first stage of the program: the un-applied states are not needed
-      tile_store<NT, 2>(S, t, m, psi, lam);
+    __syncthreads();
+    finish(0);
+    first = false;
+    if (write_back)  // not for the first stage of the program: the un-applied states are not needed
+      tile_store<NT, 2>(S, T, m, psi, lam);
     __syncthreads();  // the next tile overwrites the LDS tables and red
   }
+  if (first)  // no tile: empty sums
+    for (int x = threadIdx.x; x < S.nops * kQVals; x += NT)
+      partial[S.ops[x / kQVals].poff + (size_t)(x % kQVals) * gridDim.x + blockIdx.x] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1369,68 +1340,38 @@ __global__ __launch_bounds__(NT) void k_stage_rev(StageDev S, const double* __re
 
 static double stage_bytes(const Space& s, int vectors) { return 16.0 * (double)s.dim * vectors; }
 
-// Tile grids: one block per dispatch slot up to blocks_per_cu blocks per CU
-// (more slots are walked by the same blocks; 256 * blocks_per_cu is a
-// multiple of 8, so a block stays on one XCD's share of the slots).
-static unsigned tile_grid(int nslots, int blocks_per_cu) {
-  return (unsigned)std::max(1, std::min(nslots, 256 * blocks_per_cu));
-}
-
-static void launch_mats(const TilePlan& T, const double* theta, int deriv_gate, hipStream_t st) {
+static void launch_mats(const TilePlan& T, const double* theta, int deriv_gate, double* mats, const Multi& M,
+                        hipStream_t st) {
   SQ_PROF(PC_OTHER, st, 0.0, 0.0,
-          k_stage_mats<<<T.ntiled, 64, 0, st>>>(T.d_info, theta, deriv_gate, T.d_mats, 0, 0));
+          k_op_mats<<<dim3(T.nops, M.n), 64, 0, st>>>(T.d_info, T.d_entries, theta, deriv_gate, mats, M.theta, M.mats));
 }
 
-static void launch_fwd1(const StageDev& D, size_t lds, int nt, bool dagger, const double* src, double* dst,
+// One block per dispatch slot, up to 2048 (more slots are walked by the same
+// blocks; 2048 is a multiple of 8, so a block stays on one XCD's slots).
+static void launch_fwd(const TilePlan& T, const Stage& S, const double* mats, bool dagger, const double* src,
+                       double* dst, const Multi& M, hipStream_t st) {
+  auto* kernel = dagger ? (T.nt == 256 ? k_win_fwd<256, true> : T.nt == 512 ? k_win_fwd<512, true> : k_win_fwd<1024, true>)
+                        : (T.nt == 256 ? k_win_fwd<256, false> : T.nt == 512 ? k_win_fwd<512, false> : k_win_fwd<1024, false>);
+  allow_lds(kernel, S.lds_fwd + 1024);
+  const dim3 grid((unsigned)std::max(1, std::min(S.dev.nb, 2048)), (unsigned)M.n);
+  kernel<<<grid, T.nt, S.lds_fwd, st>>>(S.dev, mats, src, dst, M.mats, M.vec);
+  SQ_HIP(hipGetLastError());
+}
+
+static void launch_rev(const TilePlan& T, const Stage& S, const double* mats, double* psi, double* lam,
+                       double* partial, int wb, const Multi& M, hipStream_t st) {
+  auto* kernel = T.nt == 256 ? k_win_rev<256> : T.nt == 512 ? k_win_rev<512> : k_win_rev<1024>;
+  allow_lds(kernel, S.lds_rev + 4096);
+  const dim3 grid((unsigned)std::max(1, S.rev_blocks), (unsigned)M.n);
+  kernel<<<grid, T.nt, S.lds_rev, st>>>(S.dev, mats, psi, lam, partial, wb, M.mats, M.vec, M.part);
+  SQ_HIP(hipGetLastError());
+}
+
+static void launch_grad(const TilePlan& T, const double* theta, const double* partial, double* grad, const Multi& M,
                         hipStream_t st) {
-  if (nt == 256) {
-    allow_lds(k_stage_fwd<256>, lds);
-    k_stage_fwd<256><<<tile_grid(D.nb, 16), 256, lds, st>>>(D, D.mats, dagger ? 1 : 0, src, dst, 0, 0);
-    return;
-  }
-  allow_lds(k_stage_fwd<kNT>, lds);
-  k_stage_fwd<kNT><<<tile_grid(D.nb, 8), kNT, lds, st>>>(D, D.mats, dagger ? 1 : 0, src, dst, 0, 0);
-}
-
-static void launch_rev1(const StageDev& D, size_t lds, int nt, double* psi, double* lam, double* partial, int wb,
-                        hipStream_t st) {
-  if (nt == 256) {
-    allow_lds(k_stage_rev<256>, lds);
-    k_stage_rev<256><<<tile_grid(D.nb, 16), 256, lds, st>>>(D, D.mats, psi, lam, partial, wb, 0, 0, 0);
-    return;
-  }
-  allow_lds(k_stage_rev<kNT>, lds);
-  k_stage_rev<kNT><<<tile_grid(D.nb, 8), kNT, lds, st>>>(D, D.mats, psi, lam, partial, wb, 0, 0, 0);
-}
-
-// A stage's launches: with a large-tile side launch, it runs on the plan's
-// side stream between a fork and a join event, concurrently with the main
-// launch on st (the two write disjoint amplitudes).
-template <class F>
-static void stage_launches(const TilePlan& T, const Stage& S, hipStream_t st, F&& launch) {
-  if (S.dev_big.nb == 0) {
-    launch(S.dev, false, st);
-    return;
-  }
-  SQ_HIP(hipEventRecord(T.ev_fork, st));
-  SQ_HIP(hipStreamWaitEvent(T.side, T.ev_fork, 0));
-  launch(S.dev_big, true, T.side);
-  launch(S.dev, false, st);
-  SQ_HIP(hipEventRecord(T.ev_join, T.side));
-  SQ_HIP(hipStreamWaitEvent(st, T.ev_join, 0));
-}
-
-static void launch_fwd(const TilePlan& T, const Stage& S, bool dagger, const double* src, double* dst, hipStream_t st) {
-  stage_launches(T, S, st, [&](const StageDev& D, bool big, hipStream_t s) {
-    launch_fwd1(D, big ? S.lds_fwd_big : S.lds_fwd, T.nt, dagger, src, dst, s);
-  });
-}
-
-static void launch_rev(const TilePlan& T, const Stage& S, double* psi, double* lam, double* partial, int wb,
-                       hipStream_t st) {
-  stage_launches(T, S, st, [&](const StageDev& D, bool big, hipStream_t s) {
-    launch_rev1(D, big ? S.lds_rev_big : S.lds_rev, T.nt, psi, lam, partial, wb, s);
-  });
+  SQ_PROF(PC_REDUCE, st, 8.0 * (double)T.partial_len * M.n, 0.0,
+          k_op_grad<<<dim3(T.nops, M.n), kTB, 0, st>>>(T.d_info, T.d_entries, theta, partial, grad, M.theta, M.part,
+                                                      M.grad));
 }
 
 // Forward sweep (dagger: U^+, gates reversed with -theta) over the whole
@@ -1442,7 +1383,8 @@ static void launch_rev(const TilePlan& T, const Stage& S, double* psi, double* l
 // deriv_gate >= 0 inserts T_g right after gate g (plain gradient; forward only).
 void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const double* theta, const double* psi_in,
                    double* psi, double* scratch, double* gwork, int deriv_gate, bool dagger, hipStream_t st) {
-  launch_mats(T, theta, dagger ? -1 : deriv_gate, st);
+  const Multi one;
+  launch_mats(T, theta, dagger ? -1 : deriv_gate, T.d_mats, one, st);
   const int ns = (int)T.stages.size();
   const double* src = psi_in;
   for (int ii = 0; ii < ns; ++ii) {
@@ -1458,7 +1400,7 @@ void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const do
       }
       continue;
     }
-    SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1), 0.0, launch_fwd(T, S, dagger, src, psi, st));
+    SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1), 0.0, launch_fwd(T, S, T.d_mats, dagger, src, psi, one, st));
     src = psi;
   }
   if (src != psi) copy_vec(src, psi, s.dim, st);
@@ -1466,11 +1408,12 @@ void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const do
 
 // Reverse sweep on (psi, lam) with gradient dots into grad_dev[g] (device).
 // gwork >= 2*dim; partial: reduction scratch of the per-gate kernels.
-// mats_ready: the pair matrices of theta (no derivative insertion) are still
+// mats_ready: the op matrices of theta (no derivative insertion) are still
 // in place from a forward sweep on this stream.
 void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const double* theta, double* psi, double* lam,
                    double* gwork, double* partial, double* grad_dev, bool mats_ready, hipStream_t st) {
-  if (!mats_ready) launch_mats(T, theta, -1, st);
+  const Multi one;
+  if (!mats_ready) launch_mats(T, theta, -1, T.d_mats, one, st);
   for (int i = (int)T.stages.size() - 1; i >= 0; --i) {
     const Stage& S = T.stages[i];
     if (!S.tiled) {
@@ -1478,88 +1421,52 @@ void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const do
       continue;
     }
     const int wb = i > 0 ? 1 : 0;
-    SQ_PROF(PC_TILE_REV, st, stage_bytes(s, wb ? 2 : 1), 0.0, launch_rev(T, S, psi, lam, T.d_partial, wb, st));
+    SQ_PROF(PC_TILE_REV, st, stage_bytes(s, wb ? 2 : 1), 0.0,
+            launch_rev(T, S, T.d_mats, psi, lam, T.d_partial, wb, one, st));
   }
-  if (T.ntiled > 0)
-    SQ_PROF(PC_REDUCE, st, 8.0 * (double)T.partial_len, 0.0,
-            k_stage_grad<<<T.ntiled * kMaxPairs, kTB, 0, st>>>(T.d_info, theta, T.d_partial, grad_dev, 0, 0, 0));
+  if (T.nops > 0) launch_grad(T, theta, T.d_partial, grad_dev, one, st);
 }
 
 // ---- groups of instances of one program ------------------------------------
 
 bool tiles_group_ok(const Space& s, const Program& p) {
-  const TilePlan* T = tiles_for(s, p);
-  if (!T || T->ntiled == 0) return false;
+  const TilePlan* T = group_tiles_for(s, p);
+  if (!T) return false;
   for (const Stage& S : T->stages)
-    if (!S.tiled || S.dev_big.nb != 0) return false;
+    if (!S.tiled) return false;
   return true;
 }
 
 int64_t tiles_mats_doubles(const Space& s, const Program& p) {
-  const TilePlan* T = tiles_for(s, p);
-  return T ? (int64_t)T->ntiled * kMaxPairs * kMatVals : 0;
+  const TilePlan* T = group_tiles_for(s, p);
+  return T ? (int64_t)T->nops * kMatVals : 0;
 }
 
 int64_t tiles_partial_doubles(const Space& s, const Program& p) {
-  const TilePlan* T = tiles_for(s, p);
+  const TilePlan* T = group_tiles_for(s, p);
   return T ? std::max<int64_t>(T->partial_len, 1) : 0;
-}
-
-// The launches of one stage over M.n instances (grid y), each stage's pair
-// matrices at mats + stage index * kMaxPairs * kMatVals of every instance.
-static void launch_fwd_group(const TilePlan& T, const Stage& S, const double* mats, double* psi, const Multi& M,
-                             hipStream_t st) {
-  const StageDev& D = S.dev;
-  const double* sm = mats + (size_t)S.index * kMaxPairs * kMatVals;
-  if (T.nt == 256) {
-    allow_lds(k_stage_fwd<256>, S.lds_fwd);
-    k_stage_fwd<256><<<dim3(tile_grid(D.nb, 16), M.n), 256, S.lds_fwd, st>>>(D, sm, 0, psi, psi, M.mats, M.vec);
-  } else {
-    allow_lds(k_stage_fwd<kNT>, S.lds_fwd);
-    k_stage_fwd<kNT><<<dim3(tile_grid(D.nb, 8), M.n), kNT, S.lds_fwd, st>>>(D, sm, 0, psi, psi, M.mats, M.vec);
-  }
-  SQ_HIP(hipGetLastError());
-}
-
-static void launch_rev_group(const TilePlan& T, const Stage& S, const double* mats, double* psi, double* lam,
-                             double* partial, int wb, const Multi& M, hipStream_t st) {
-  const StageDev& D = S.dev;
-  const double* sm = mats + (size_t)S.index * kMaxPairs * kMatVals;
-  if (T.nt == 256) {
-    allow_lds(k_stage_rev<256>, S.lds_rev);
-    k_stage_rev<256><<<dim3(tile_grid(D.nb, 16), M.n), 256, S.lds_rev, st>>>(D, sm, psi, lam, partial, wb, M.mats,
-                                                                            M.vec, M.part);
-  } else {
-    allow_lds(k_stage_rev<kNT>, S.lds_rev);
-    k_stage_rev<kNT><<<dim3(tile_grid(D.nb, 8), M.n), kNT, S.lds_rev, st>>>(D, sm, psi, lam, partial, wb, M.mats,
-                                                                          M.vec, M.part);
-  }
-  SQ_HIP(hipGetLastError());
 }
 
 void tiles_forward_group(const Space& s, const Program& p, const double* theta, double* psi, double* mats,
                          const Multi& M, hipStream_t st) {
-  const TilePlan* T = tiles_for(s, p);
+  const TilePlan* T = group_tiles_for(s, p);
   SQ_CHECK(T && tiles_group_ok(s, p) && M.n > 0 && M.n <= 65535, SQ_ERR_ARG, "program has no group tile path");
-  SQ_PROF(PC_OTHER, st, 0.0, 0.0,
-          k_stage_mats<<<dim3(T->ntiled, M.n), 64, 0, st>>>(T->d_info, theta, -1, mats, M.theta, M.mats));
+  launch_mats(*T, theta, -1, mats, M, st);
   for (const Stage& S : T->stages)
-    SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1) * M.n, 0.0, launch_fwd_group(*T, S, mats, psi, M, st));
+    SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1) * M.n, 0.0, launch_fwd(*T, S, mats, false, psi, psi, M, st));
 }
 
 void tiles_reverse_group(const Space& s, const Program& p, const double* theta, double* psi, double* lam,
                          const double* mats, double* partial, double* grad, const Multi& M, hipStream_t st) {
-  const TilePlan* T = tiles_for(s, p);
+  const TilePlan* T = group_tiles_for(s, p);
   SQ_CHECK(T && tiles_group_ok(s, p) && M.n > 0 && M.n <= 65535, SQ_ERR_ARG, "program has no group tile path");
   for (int i = (int)T->stages.size() - 1; i >= 0; --i) {
     const Stage& S = T->stages[i];
     const int wb = i > 0 ? 1 : 0;
     SQ_PROF(PC_TILE_REV, st, stage_bytes(s, wb ? 2 : 1) * M.n, 0.0,
-            launch_rev_group(*T, S, mats, psi, lam, partial, wb, M, st));
+            launch_rev(*T, S, mats, psi, lam, partial, wb, M, st));
   }
-  SQ_PROF(PC_REDUCE, st, 8.0 * (double)T->partial_len * M.n, 0.0,
-          k_stage_grad<<<dim3(T->ntiled * kMaxPairs, M.n), kTB, 0, st>>>(T->d_info, theta, partial, grad, M.theta,
-                                                                        M.part, M.grad));
+  launch_grad(*T, theta, partial, grad, M, st);
 }
 
 }  // namespace sq
