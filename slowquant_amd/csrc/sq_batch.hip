@@ -328,11 +328,11 @@ struct BatchGroup {
   const Space* space = nullptr;
   const Program* prog = nullptr;
   int n = 0, ng = 0;
-  int64_t dim = 0, A_stride = 0, Ma_stride = 0, mats_stride = 0, tpart_stride = 0, spart_stride = 0;
+  int64_t dim = 0, A_stride = 0, Ma_stride = 0, Mb_stride = 0, mats_stride = 0, tpart_stride = 0, spart_stride = 0;
   double hf = 1.0;  // the HF determinant's amplitude in the engine's sign convention
   int plan_gen = 0;  // the program's tile-plan generation the buffers are sized for
   int32_t *d_inst = nullptr, *d_theta0 = nullptr, *d_out0 = nullptr;  // per member
-  double *theta = nullptr, *A = nullptr, *Ma = nullptr, *psi = nullptr, *lam = nullptr, *mats = nullptr,
+  double *theta = nullptr, *A = nullptr, *Ma = nullptr, *Mb = nullptr, *psi = nullptr, *lam = nullptr, *mats = nullptr,
          *tpart = nullptr, *spart = nullptr, *grad = nullptr;
 };
 
@@ -495,6 +495,8 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
     G.theta = balloc<double>(B, n * G.ng);
     G.A = balloc<double>(B, n * G.A_stride);
     G.Ma = balloc<double>(B, n * G.Ma_stride);
+    G.Mb_stride = H0.d_Mb ? (int64_t)s.nsb * s.nsb : G.Ma_stride;
+    G.Mb = H0.d_Mb ? balloc<double>(B, n * G.Mb_stride) : G.Ma;
     G.psi = balloc<double>(B, n * G.dim);
     G.lam = balloc<double>(B, n * G.dim);
     G.mats = balloc<double>(B, n * G.mats_stride);
@@ -503,9 +505,11 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
     G.grad = balloc<double>(B, n * G.ng);
     for (size_t m = 0; m < n; ++m) {
       const Hamiltonian& H = hams[mem[m]]->h;
-      SQ_CHECK(H.kpad == H0.kpad && H.d_Ma, SQ_ERR_ARG, "group Hamiltonians differ in shape");
+      SQ_CHECK(H.kpad == H0.kpad && H.d_Ma && !H.d_Mb == !H0.d_Mb, SQ_ERR_ARG, "group Hamiltonians differ in shape");
       SQ_HIP(hipMemcpy(G.A + m * G.A_stride, H.d_A, sizeof(double) * G.A_stride, hipMemcpyDeviceToDevice));
       SQ_HIP(hipMemcpy(G.Ma + m * G.Ma_stride, H.d_Ma, sizeof(double) * G.Ma_stride, hipMemcpyDeviceToDevice));
+      if (H.d_Mb)
+        SQ_HIP(hipMemcpy(G.Mb + m * G.Mb_stride, H.d_Mb, sizeof(double) * G.Mb_stride, hipMemcpyDeviceToDevice));
     }
   }
 }
@@ -544,7 +548,7 @@ static void group_launch(const Batch& B, const BatchGroup& G, hipStream_t st) {
   k_group_init<<<dim3(ib, (unsigned)G.n), 256, 0, st>>>(B.dev.psi0, G.d_inst, G.dim, G.hf, G.psi);
   SQ_HIP(hipGetLastError());
   tiles_forward_group(s, *G.prog, G.theta, G.psi, G.mats, M, st);
-  row_sigma_group(s, G.A, G.A_stride, G.Ma, G.Ma_stride, G.psi, G.lam, G.spart, G.n, st);
+  row_sigma_group(s, G.A, G.A_stride, G.Ma, G.Ma_stride, G.Mb, G.Mb_stride, G.psi, G.lam, G.spart, G.n, st);
   tiles_reverse_group(s, *G.prog, G.theta, G.psi, G.lam, G.mats, G.tpart, G.grad, M, st);
   k_group_out<<<(unsigned)G.n, 256, 0, st>>>(G.spart, G.spart_stride, G.grad, G.ng, G.d_inst, G.d_out0,
                                              B.dev.energy, B.dev.grad);

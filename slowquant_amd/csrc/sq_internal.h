@@ -126,6 +126,8 @@ struct Space {
   // row sigma tables (sq_rowsigma.hip): operand rows [K8 + 16][nsa], [K8 + 32][nsb],
   // beta neighbour lists by partner column with per-tile offsets
   int2* d_rta = nullptr;
+  int32_t* d_rtc = nullptr;  // beta partners, packed
+  int2* d_alist = nullptr;  // nonvanishing alpha excitations per string
   int2* d_rtb = nullptr;
   uint32_t* d_nbr = nullptr;
   int32_t* d_nbr_off = nullptr;
@@ -194,14 +196,16 @@ struct Hamiltonian {
   int kpad;            // padded K (= M) of the packed GEMM, multiple of 16
   double e_core;
   double* d_A = nullptr;  // [kpad][kpad] transposed coefficient matrix (see sq_sigma.hip)
-  double* d_Ma = nullptr;  // [nsa][nsa] alpha-string Hamiltonian + e_core (sq_rowsigma.hip)
+  double* d_Ma = nullptr;  // [nsa][nsa] alpha-string Hamiltonian + e_core / 2 (sq_rowsigma.hip)
+  double* d_Mb = nullptr;  // [nsb][nsb] the beta one; null: d_Ma serves both or only Ma is needed
 };
 
 // Row sigma (sq_rowsigma.hip)
 bool row_sigma_applies(const Space& s);
 int64_t row_sigma_work_doubles(const Space& s);
 int64_t row_sigma_used_doubles(const Space& s);
-void build_alpha_ham(const Space& s, Hamiltonian& H);
+void build_string_hams(const Space& s, Hamiltonian& H);
+void free_string_hams(Hamiltonian& H);
 // allow_library = false keeps every step in this library's own kernels (no
 // library call that may allocate).
 int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* work,
@@ -300,13 +304,14 @@ void tiles_forward_group(const Space& s, const Program& p, const double* theta, 
 // reverse sweep on (psi, lam) with dE/dtheta into grad (n x gates)
 void tiles_reverse_group(const Space& s, const Program& p, const double* theta, double* psi, double* lam,
                          const double* mats, double* partial, double* grad, const Multi& M, hipStream_t st);
-// sigma = H psi for n instances of one space (row form with its alpha GEMM
-// tiles in the launch); A and Ma per instance at the given strides; energy
+// sigma = H psi for n instances of one space (row form with the string
+// products' tiles in the launch); A, Ma and Mb per instance at the given strides; energy
 // partials per instance (row_sigma_group_partials of them) at partial.
 bool row_sigma_group_ok(const Space& s);
 int64_t row_sigma_group_partials(const Space& s);
 void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
-                     const double* psi, double* sigma, double* partial, int n, hipStream_t st);
+                     const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
+                     hipStream_t st);
 void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const double* theta, const double* psi_in,
                    double* psi, double* scratch, double* gwork, int deriv_gate, bool dagger, hipStream_t st);
 void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const double* theta, double* psi, double* lam,

@@ -2,7 +2,7 @@
 // whose scratch memory is a file-scope device array instead of a caller's
 // workspace, for callers that cannot allocate.
 //
-// The row sigma's alpha GEMM partials and block energy partials live in
+// The row sigma's string product partials and block energy partials live in
 // `scratch`, kScratchDoubles doubles (64 MiB) that every GPU the library runs
 // on holds until the process ends.  Host code never passes the array's name
 // to a kernel: at the first call on a device, hipGetSymbolAddress gives that

@@ -43,7 +43,7 @@ static SigmaDims sigma_dims(const Space& s) {
 }
 
 // Work layout (doubles): D [K4*dim] | G [npair*dim] | partials [nsa*ceil(nsb/256)] | scalars [8];
-// the row path (sq_rowsigma.hip) needs only its alpha GEMM partials and block partials.
+// the row path (sq_rowsigma.hip) needs only its string product partials and block partials.
 int64_t sigma_work_bytes(const Space& s) {
   if (row_sigma_applies(s)) return 8 * row_sigma_work_doubles(s);
   SigmaDims d = sigma_dims(s);
@@ -878,9 +878,9 @@ int sq_hamiltonian_create(const sq_space* sp, const double* h, const double* g, 
       throw Error{SQ_ERR_HIP, hipGetErrorString(e)};
     }
     try {
-      if (row_sigma_applies(s)) build_alpha_ham(s, ho->h);
+      if (row_sigma_applies(s)) build_string_hams(s, ho->h);
     } catch (...) {
-      if (ho->h.d_Ma) (void)hipFree(ho->h.d_Ma);
+      free_string_hams(ho->h);
       (void)hipFree(ho->h.d_A);
       delete ho;
       throw;
@@ -893,7 +893,7 @@ int sq_hamiltonian_destroy(sq_hamiltonian* H) {
   return guarded([&] {
     if (!H) return;
     if (H->h.d_A) (void)hipFree(H->h.d_A);
-    if (H->h.d_Ma) (void)hipFree(H->h.d_Ma);
+    free_string_hams(H->h);
     delete H;
   });
 }
