@@ -162,6 +162,11 @@ int sq_sigma_noalloc(const sq_space* s, const sq_hamiltonian* H, const double* p
 int sq_energy_grad_adjoint(const sq_space* s, const sq_program* p, const sq_hamiltonian* H,
                            const double* theta, const double* psi0, double* energy, double* grad,
                            double* work, void* stream);
+/* The same with theta in host memory (n_gates doubles, read before the call
+ * returns). */
+int sq_energy_grad_adjoint_host(const sq_space* s, const sq_program* p, const sq_hamiltonian* H,
+                                const double* theta, const double* psi0, double* energy, double* grad,
+                                double* work, void* stream);
 /* Same quantities by per-parameter derivative propagation (O(N^2) gate
  * applications): d_i psi = U_N..U_{i+1} U_i T_i U_{i-1}..U_1 psi0. */
 int sq_energy_grad_plain(const sq_space* s, const sq_program* p, const sq_hamiltonian* H,

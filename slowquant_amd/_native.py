@@ -84,6 +84,7 @@ _SIGNATURES = {
     "sq_sigma_noalloc": ([vp, vp, dp, dp, dp, vp], i32),
     "sq_sigma_configure": ([vp, i32, i32, i32], i32),
     "sq_energy_grad_adjoint": ([vp, vp, vp, dp, dp, vp, vp, dp, vp], i32),
+    "sq_energy_grad_adjoint_host": ([vp, vp, vp, vp, dp, vp, vp, dp, vp], i32),
     "sq_energy_grad_plain": ([vp, vp, vp, dp, dp, vp, vp, dp, vp], i32),
     "sq_energy_grad_reference_sweep": ([vp, vp, vp, dp, dp, vp, vp, dp, vp], i32),
     "sq_adjoint_reverse": ([vp, vp, dp, dp, dp, vp, dp, vp], i32),

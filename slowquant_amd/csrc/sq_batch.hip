@@ -547,8 +547,8 @@ static void group_launch(const Batch& B, const BatchGroup& G, hipStream_t st) {
   const unsigned ib = (unsigned)std::min<int64_t>((G.dim + 255) / 256, 64);
   k_group_init<<<dim3(ib, (unsigned)G.n), 256, 0, st>>>(B.dev.psi0, G.d_inst, G.dim, G.hf, G.psi);
   SQ_HIP(hipGetLastError());
-  tiles_forward_group(s, *G.prog, G.theta, G.psi, G.mats, M, st);
-  row_sigma_group(s, G.A, G.A_stride, G.Ma, G.Ma_stride, G.Mb, G.Mb_stride, G.psi, G.lam, G.spart, G.n, st);
+  tiles_forward_group(s, *G.prog, G.theta, G.psi, G.mats, M, G.lam, st);
+  row_sigma_group(s, G.A, G.A_stride, G.Ma, G.Ma_stride, G.Mb, G.Mb_stride, G.psi, G.lam, G.spart, G.n, true, st);
   tiles_reverse_group(s, *G.prog, G.theta, G.psi, G.lam, G.mats, G.tpart, G.grad, M, st);
   k_group_out<<<(unsigned)G.n, 256, 0, st>>>(G.spart, G.spart_stride, G.grad, G.ng, G.d_inst, G.d_out0,
                                              B.dev.energy, B.dev.grad);

@@ -812,6 +812,7 @@ int sq_program_destroy(sq_program* pr) {
     if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
     if (pr->p.group_tiles) destroy_tile_plan(pr->p.group_tiles);
     if (pr->p.small) small_plan_free(pr->p.small);
+    host_slots_free(pr->p);
     delete pr;
   });
 }

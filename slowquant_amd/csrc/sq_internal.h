@@ -179,7 +179,14 @@ struct Program {
   // sq_ucc.hip; freed by ucc_t_free).
   mutable struct UccT* ucc_t = nullptr;
   mutable bool ucc_t_tried = false;
+  // Host-visible parameter and result blocks of the energy and gradient calls
+  // (sq_grad.hip): one per concurrent call, kept for the next, freed with the
+  // program.
+  mutable std::mutex slot_mu;
+  mutable std::vector<struct HostSlot*> slots;
 };
+
+void host_slots_free(const Program& p);
 
 void ucc_t_free(struct UccT* t);
 
@@ -209,7 +216,9 @@ void free_string_hams(Hamiltonian& H);
 // allow_library = false keeps every step in this library's own kernels (no
 // library call that may allocate).
 int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* work,
-                  double** partial_out, hipStream_t st, bool allow_library = true);
+                  double** partial_out, hipStream_t st, bool allow_library = true, bool zeroed = false);
+// Whether row_sigma adds into a zeroed sigma (and zeroes it unless told it is).
+bool row_sigma_wants_zero(const Space& s);
 
 // Kernel timing classes (sq_profile.hip).
 enum ProfClass {
@@ -253,6 +262,11 @@ int64_t sigma_work_bytes(const Space& s);
 // Implemented in sq_sigma.hip
 void sigma_impl(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* energy_host,
                 double* work, hipStream_t st);
+// sigma = H psi and the block partials of <psi|sigma> (*partial, the count is
+// returned); zeroed: sigma is already zero (sigma_wants_zero).
+bool sigma_wants_zero(const Space& s, const Hamiltonian& H);
+int64_t sigma_partials_dev(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* work,
+                           double** partial, bool zeroed, hipStream_t st);
 void sigma_energy_dev(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* e_dev,
                       double* work, hipStream_t st);
 void dot_dev(const double* x, const double* y, int64_t n, double* out_dev, int slot, double factor, double* partial,
@@ -300,7 +314,7 @@ int64_t tiles_mats_doubles(const Space& s, const Program& p);     // pair matric
 int64_t tiles_partial_doubles(const Space& s, const Program& p);  // gradient partials per instance
 // psi (in place, start states already there) = U(theta) psi for every instance
 void tiles_forward_group(const Space& s, const Program& p, const double* theta, double* psi, double* mats,
-                         const Multi& M, hipStream_t st);
+                         const Multi& M, double* zero, hipStream_t st);
 // reverse sweep on (psi, lam) with dE/dtheta into grad (n x gates)
 void tiles_reverse_group(const Space& s, const Program& p, const double* theta, double* psi, double* lam,
                          const double* mats, double* partial, double* grad, const Multi& M, hipStream_t st);
@@ -311,11 +325,18 @@ bool row_sigma_group_ok(const Space& s);
 int64_t row_sigma_group_partials(const Space& s);
 void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
                      const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
-                     hipStream_t st);
+                     bool zeroed, hipStream_t st);
+// tiles_whole: every stage is tiled, so theta is read by the first and last
+// launch only.  zero: dim doubles the first launch clears.  theta_out: theta is
+// host memory; the first launch copies it there.
+bool tiles_whole(const TilePlan& T);
 void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const double* theta, const double* psi_in,
-                   double* psi, double* scratch, double* gwork, int deriv_gate, bool dagger, hipStream_t st);
+                   double* psi, double* scratch, double* gwork, int deriv_gate, bool dagger, hipStream_t st,
+                   double* zero = nullptr, double* theta_out = nullptr);
+// epart, n_epart, e_out: energy partials the last launch sums into e_out[0].
 void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const double* theta, double* psi, double* lam,
-                   double* gwork, double* partial, double* grad_dev, bool mats_ready, hipStream_t st);
+                   double* gwork, double* partial, double* grad_dev, bool mats_ready, hipStream_t st,
+                   const double* epart = nullptr, int64_t n_epart = 0, double* e_out = nullptr);
 
 // Dynamic LDS above 64 KB must be enabled per kernel; the request covers
 // exactly what a launch needs (raised only, kept per kernel).

@@ -1280,11 +1280,11 @@ rocblas_handle blas_handle() {
 }
 
 // k_sigma_rows_list for n instances at the given strides (fused: sigma zeroed
-// here and the string products' tiles in the launch; else the nsplit products
+// here unless it is already, and the string products' tiles in the launch; else the nsplit products
 // at sin added).
 void rows_list_launch(const Space& s, const RowPlan& pl, const double* A, int64_t A_stride, int kpad, const double* Ma,
                       int64_t Ma_stride, const double* Mb, int64_t Mb_stride, const double* psi, const double* sin,
-                      int nsplit, double* sigma, double* partial, int n, hipStream_t st) {
+                      int nsplit, double* sigma, double* partial, int n, bool zeroed, hipStream_t st) {
   static const int xcd = env_int("SQ_ROWS_XCD", 1) != 0 ? 1 : 0;
   RowArgs P{};
   P.At = A, P.psi = psi, P.sin = sin, P.Ma = Ma, P.Mb = Mb, P.sigma = sigma, P.partial = partial;
@@ -1297,7 +1297,7 @@ void rows_list_launch(const Space& s, const RowPlan& pl, const double* A, int64_
   const double rows = 2.0 * (double)s.npair * 4.0 * list_steps(s) * (double)s.dim;
   const double flops = n * (rows + (pl.fused ? 2.0 * (double)s.dim * (s.nsa + s.nsb) : 0.0));
   const double bytes = 8.0 * (double)s.dim * n * (pl.fused ? 3 : 2 + nsplit);
-  if (pl.fused) {
+  if (pl.fused && !zeroed) {
     const int64_t total = (int64_t)n * s.dim;
     k_zero<<<(unsigned)std::min<int64_t>((total + 255) / 256, 16384), 256, 0, st>>>(sigma, total);
     SQ_HIP(hipGetLastError());
@@ -1326,7 +1326,7 @@ void rows_list_launch(const Space& s, const RowPlan& pl, const double* A, int64_
 // rocBLAS unless allow_library is false (the no-allocation entry point) or
 // SQ_ALPHA_GEMM_LIB=0: 66.5 TFLOP/s on 3432^3 against 62 for k_string_gemm.
 int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* work,
-                  double** partial_out, hipStream_t st, bool allow_library) {
+                  double** partial_out, hipStream_t st, bool allow_library, bool zeroed) {
   RowPlan pl;
   SQ_CHECK(row_plan(s, &pl) && H.d_Ma, SQ_ERR_ARG, "row sigma does not apply to this space");
   SQ_CHECK(pl.nsplit <= kMaxSplit && pl.ngroups <= s.nsa, SQ_ERR_ARG, "row sigma shape exceeds its workspace");
@@ -1336,7 +1336,7 @@ int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, doubl
   const double* Mb = H.d_Mb ? H.d_Mb : H.d_Ma;
   if (pl.fused) {
     *partial_out = work;
-    rows_list_launch(s, pl, H.d_A, 0, H.kpad, H.d_Ma, 0, Mb, 0, psi, nullptr, 0, sigma, work, 1, st);
+    rows_list_launch(s, pl, H.d_A, 0, H.kpad, H.d_Ma, 0, Mb, 0, psi, nullptr, 0, sigma, work, 1, zeroed, st);
     return (int64_t)pl.ngroups + pl.ngemm_a + pl.ngemm_b;
   }
   double* sinp = work;
@@ -1376,7 +1376,7 @@ int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, doubl
     }
   }
   if (pl.list) {
-    rows_list_launch(s, pl, H.d_A, 0, H.kpad, H.d_Ma, 0, Mb, 0, psi, sinp, nsplit, sigma, partial, 1, st);
+    rows_list_launch(s, pl, H.d_A, 0, H.kpad, H.d_Ma, 0, Mb, 0, psi, sinp, nsplit, sigma, partial, 1, false, st);
     return pl.ngroups;
   }
   const int K8 = row_k8(s);
@@ -1431,6 +1431,11 @@ int64_t row_sigma_used_doubles(const Space& s) {
   return (int64_t)std::max(pl.nsplit, least) * s.dim + pl.ngroups;
 }
 
+bool row_sigma_wants_zero(const Space& s) {
+  RowPlan pl;
+  return row_plan(s, &pl) && pl.fused;
+}
+
 bool row_sigma_group_ok(const Space& s) {
   RowPlan pl;
   return rows_enabled() && s.d_rtb != nullptr && row_plan(s, &pl) && pl.scatter && pl.fused;
@@ -1444,12 +1449,12 @@ int64_t row_sigma_group_partials(const Space& s) {
 
 void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
                      const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
-                     hipStream_t st) {
+                     bool zeroed, hipStream_t st) {
   RowPlan pl;
   SQ_CHECK(row_sigma_group_ok(s) && row_plan(s, &pl) && n > 0 && n <= 65535, SQ_ERR_ARG,
            "the grouped row sigma does not apply to this space");
   rows_list_launch(s, pl, A, A_stride, rup(s.npair + 1, 16), Ma, Ma_stride, Mb, Mb_stride, psi, nullptr, 0, sigma,
-                   partial, n, st);
+                   partial, n, zeroed, st);
 }
 
 }  // namespace sq

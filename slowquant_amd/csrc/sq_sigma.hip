@@ -432,22 +432,20 @@ void sigma_impl(const Space& s, const Hamiltonian& H, const double* psi, double*
   }
 }
 
-// Device-resident energy: same as sigma_impl but leaves <psi|sigma> in e_dev[0].
-void sigma_energy_dev(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* e_dev,
-                      double* work, hipStream_t st) {
+bool sigma_wants_zero(const Space& s, const Hamiltonian& H) {
+  return H.d_Ma && row_sigma_applies(s) && row_sigma_wants_zero(s);
+}
+
+int64_t sigma_partials_dev(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* work,
+                           double** partial_out, bool zeroed, hipStream_t st) {
   SigmaDims d = sigma_dims(s);
-  if (H.d_Ma && row_sigma_applies(s)) {
-    double* partial = nullptr;
-    const int64_t nb = row_sigma(s, H, psi, sigma, work, &partial, st);
-    reduce_impl(partial, nb, e_dev, 0, false, 1.0, st);
-    return;
-  }
+  if (H.d_Ma && row_sigma_applies(s)) return row_sigma(s, H, psi, sigma, work, partial_out, st, true, zeroed);
   const int32_t* ae = s.d_aexc;
   const int32_t* be = s.d_bexc;
   double* D = work;
   double* G = D + (size_t)d.K4 * d.dim;
   double* partial = G + (size_t)d.npair * d.dim;
-  int64_t nb = (int64_t)s.nsa * ((s.nsb + kB - 1) / kB);
+  *partial_out = partial;
   dim3 grid((s.nsb + kB - 1) / kB, s.nsa);
   const double d8 = 8.0 * (double)d.dim;
   const int gth = gather_threads(s);
@@ -462,7 +460,15 @@ void sigma_energy_dev(const Space& s, const Hamiltonian& H, const double* psi, d
   }
   SQ_PROF(PC_SIGMA_GATHER, st, d8 * (d.npair + 2), 0.0,
           k_sigma_gather<<<ggrid, gth, 0, st>>>(s.n, s.nsa, s.nsb, ae, be, G, psi, H.e_core, sigma, partial));
-  reduce_impl(partial, gnb, e_dev, 0, false, 1.0, st);
+  return gnb;
+}
+
+// Device-resident energy: same as sigma_impl but leaves <psi|sigma> in e_dev[0].
+void sigma_energy_dev(const Space& s, const Hamiltonian& H, const double* psi, double* sigma, double* e_dev,
+                      double* work, hipStream_t st) {
+  double* partial = nullptr;
+  const int64_t nb = sigma_partials_dev(s, H, psi, sigma, work, &partial, false, st);
+  reduce_impl(partial, nb, e_dev, 0, false, 1.0, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -755,11 +755,13 @@ struct EntryLds {
 };
 
 __device__ __forceinline__ void load_entries(const StageEntry* __restrict__ entries, int e0, int n,
-                                             const double* __restrict__ theta, EntryLds& E) {
+                                             const double* __restrict__ theta, EntryLds& E,
+                                             double* __restrict__ theta_out = nullptr) {
   for (int x = threadIdx.x; x < n * kTypes; x += blockDim.x) E.code[x / kTypes][x % kTypes] = entries[e0 + x / kTypes].code[x % kTypes];
   for (int e = threadIdx.x; e < n; e += blockDim.x) {
     const StageEntry& en = entries[e0 + e];
     const double th = theta[en.gate];
+    if (theta_out) theta_out[en.gate] = th;
     double s = 0.0, c = 1.0;
     if (fabs(th) >= 1e-28) sincos(en.scale * th, &s, &c);
     E.gate[e] = en.gate;
@@ -794,18 +796,28 @@ __device__ __forceinline__ void t_vec(uint32_t code, double scale, const double 
   }
 }
 
-// One block per pair op: the op's gate product in forward order, with T_g
+// One block per pair op (the blocks after them clear nzero doubles at zero, the
+// target of the sigma that follows): the op's gate product in forward order,
+// with T_g
 // inserted after gate g when deriv_gate is in this op.  A thread carries one
 // column of one class's matrix through the rotations.
 __global__ __launch_bounds__(64) void k_op_mats(const OpInfo* __restrict__ info, const StageEntry* __restrict__ entries,
                                                 const double* __restrict__ theta, int deriv_gate,
-                                                double* __restrict__ mats, int64_t th_stride, int64_t mats_stride) {
+                                                double* __restrict__ mats, int64_t th_stride, int64_t mats_stride,
+                                                int nops, double* __restrict__ theta_out, double* __restrict__ zero,
+                                                int64_t nzero) {
   __shared__ EntryLds E;
+  if ((int)blockIdx.x >= nops) {
+    zero += blockIdx.y * nzero;
+    const int64_t step = (int64_t)(gridDim.x - nops) * blockDim.x;
+    for (int64_t i = (int64_t)(blockIdx.x - nops) * blockDim.x + threadIdx.x; i < nzero; i += step) zero[i] = 0.0;
+    return;
+  }
   theta += blockIdx.y * th_stride;
   mats += blockIdx.y * mats_stride;
   const OpInfo I = info[blockIdx.x];
   const int n = I.e1 - I.e0;
-  load_entries(entries, I.e0, n, theta, E);
+  load_entries(entries, I.e0, n, theta, E, theta_out);
   __syncthreads();
   const int cls = threadIdx.x >> 2, q = threadIdx.x & 3;
   if (cls >= 5) return;
@@ -850,7 +862,22 @@ constexpr int kQb[6] = {1, 2, 3, 2, 3, 3};
 __global__ __launch_bounds__(kTB) void k_op_grad(const OpInfo* __restrict__ info, const StageEntry* __restrict__ entries,
                                                  const double* __restrict__ theta, const double* __restrict__ partial,
                                                  double* __restrict__ grad, int64_t th_stride, int64_t part_stride,
-                                                 int64_t grad_stride) {
+                                                 int64_t grad_stride, int nops, const double* __restrict__ epart,
+                                                 int64_t n_epart, double* __restrict__ e_out) {
+  if ((int)blockIdx.x == nops) {  // the energy from the partials of the sigma
+    __shared__ double ered[kTB / 64];
+    double e = 0.0;
+    for (int64_t i = threadIdx.x; i < n_epart; i += kTB) e += epart[i];
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_down(e, off, 64);
+    if ((threadIdx.x & 63) == 0) ered[threadIdx.x >> 6] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double tot = 0.0;
+      for (int w = 0; w < kTB / 64; ++w) tot += ered[w];
+      e_out[0] = tot;
+    }
+    return;
+  }
   theta += blockIdx.y * th_stride;
   partial += blockIdx.y * part_stride;
   grad += blockIdx.y * grad_stride;
@@ -1341,9 +1368,11 @@ __global__ __launch_bounds__(NT) void k_win_rev(StageDev S, const double* __rest
 static double stage_bytes(const Space& s, int vectors) { return 16.0 * (double)s.dim * vectors; }
 
 static void launch_mats(const TilePlan& T, const double* theta, int deriv_gate, double* mats, const Multi& M,
-                        hipStream_t st) {
-  SQ_PROF(PC_OTHER, st, 0.0, 0.0,
-          k_op_mats<<<dim3(T.nops, M.n), 64, 0, st>>>(T.d_info, T.d_entries, theta, deriv_gate, mats, M.theta, M.mats));
+                        hipStream_t st, double* theta_out = nullptr, double* zero = nullptr, int64_t nzero = 0) {
+  const int zb = zero ? (int)std::min<int64_t>((nzero + 1023) / 1024, 512) : 0;
+  SQ_PROF(PC_OTHER, st, 8.0 * (double)(zero ? nzero : 0) * M.n, 0.0,
+          k_op_mats<<<dim3(T.nops + zb, M.n), 64, 0, st>>>(T.d_info, T.d_entries, theta, deriv_gate, mats, M.theta,
+                                                          M.mats, T.nops, theta_out, zero, nzero));
 }
 
 // One block per dispatch slot, up to 2048 (more slots are walked by the same
@@ -1368,10 +1397,18 @@ static void launch_rev(const TilePlan& T, const Stage& S, const double* mats, do
 }
 
 static void launch_grad(const TilePlan& T, const double* theta, const double* partial, double* grad, const Multi& M,
-                        hipStream_t st) {
-  SQ_PROF(PC_REDUCE, st, 8.0 * (double)T.partial_len * M.n, 0.0,
-          k_op_grad<<<dim3(T.nops, M.n), kTB, 0, st>>>(T.d_info, T.d_entries, theta, partial, grad, M.theta, M.part,
-                                                      M.grad));
+                        hipStream_t st, const double* epart = nullptr, int64_t n_epart = 0, double* e_out = nullptr) {
+  SQ_PROF(PC_REDUCE, st, 8.0 * ((double)T.partial_len * M.n + (double)n_epart), 0.0,
+          k_op_grad<<<dim3(T.nops + (e_out ? 1 : 0), M.n), kTB, 0, st>>>(T.d_info, T.d_entries, theta, partial, grad,
+                                                                        M.theta, M.part, M.grad, T.nops, epart,
+                                                                        n_epart, e_out));
+}
+
+bool tiles_whole(const TilePlan& T) {
+  if (T.nops == 0) return false;
+  for (const Stage& S : T.stages)
+    if (!S.tiled) return false;
+  return true;
 }
 
 // Forward sweep (dagger: U^+, gates reversed with -theta) over the whole
@@ -1382,9 +1419,10 @@ static void launch_grad(const TilePlan& T, const double* theta, const double* pa
 // gwork >= 2*dim doubles for gates that run through the per-gate kernels.
 // deriv_gate >= 0 inserts T_g right after gate g (plain gradient; forward only).
 void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const double* theta, const double* psi_in,
-                   double* psi, double* scratch, double* gwork, int deriv_gate, bool dagger, hipStream_t st) {
+                   double* psi, double* scratch, double* gwork, int deriv_gate, bool dagger, hipStream_t st,
+                   double* zero, double* theta_out) {
   const Multi one;
-  launch_mats(T, theta, dagger ? -1 : deriv_gate, T.d_mats, one, st);
+  launch_mats(T, theta, dagger ? -1 : deriv_gate, T.d_mats, one, st, theta_out, zero, zero ? s.dim : 0);
   const int ns = (int)T.stages.size();
   const double* src = psi_in;
   for (int ii = 0; ii < ns; ++ii) {
@@ -1411,7 +1449,8 @@ void tiles_forward(const Space& s, const Program& p, const TilePlan& T, const do
 // mats_ready: the op matrices of theta (no derivative insertion) are still
 // in place from a forward sweep on this stream.
 void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const double* theta, double* psi, double* lam,
-                   double* gwork, double* partial, double* grad_dev, bool mats_ready, hipStream_t st) {
+                   double* gwork, double* partial, double* grad_dev, bool mats_ready, hipStream_t st,
+                   const double* epart, int64_t n_epart, double* e_out) {
   const Multi one;
   if (!mats_ready) launch_mats(T, theta, -1, T.d_mats, one, st);
   for (int i = (int)T.stages.size() - 1; i >= 0; --i) {
@@ -1424,17 +1463,14 @@ void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const do
     SQ_PROF(PC_TILE_REV, st, stage_bytes(s, wb ? 2 : 1), 0.0,
             launch_rev(T, S, T.d_mats, psi, lam, T.d_partial, wb, one, st));
   }
-  if (T.nops > 0) launch_grad(T, theta, T.d_partial, grad_dev, one, st);
+  if (T.nops > 0) launch_grad(T, theta, T.d_partial, grad_dev, one, st, epart, n_epart, e_out);
 }
 
 // ---- groups of instances of one program ------------------------------------
 
 bool tiles_group_ok(const Space& s, const Program& p) {
   const TilePlan* T = group_tiles_for(s, p);
-  if (!T) return false;
-  for (const Stage& S : T->stages)
-    if (!S.tiled) return false;
-  return true;
+  return T && tiles_whole(*T);
 }
 
 int64_t tiles_mats_doubles(const Space& s, const Program& p) {
@@ -1448,10 +1484,10 @@ int64_t tiles_partial_doubles(const Space& s, const Program& p) {
 }
 
 void tiles_forward_group(const Space& s, const Program& p, const double* theta, double* psi, double* mats,
-                         const Multi& M, hipStream_t st) {
+                         const Multi& M, double* zero, hipStream_t st) {
   const TilePlan* T = group_tiles_for(s, p);
   SQ_CHECK(T && tiles_group_ok(s, p) && M.n > 0 && M.n <= 65535, SQ_ERR_ARG, "program has no group tile path");
-  launch_mats(*T, theta, -1, mats, M, st);
+  launch_mats(*T, theta, -1, mats, M, st, nullptr, zero, s.dim);
   for (const Stage& S : T->stages)
     SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1) * M.n, 0.0, launch_fwd(*T, S, mats, false, psi, psi, M, st));
 }

@@ -18,7 +18,9 @@ from . import _native as N
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle of torch's current stream (a torch.cuda.Stream object for
+    # every call costs 3 us)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -180,16 +182,25 @@ class Program:
         return out
 
     def energy_grad(self, H: "Hamiltonian", theta, psi0: torch.Tensor, method: str = "adjoint"):
-        th = self.theta_tensor(theta)
-        e = ctypes.c_double()
-        g = np.zeros(max(self.n_gates, 1))
         fn = {
             "adjoint": N.lib().sq_energy_grad_adjoint,
             "plain": N.lib().sq_energy_grad_plain,
             "reference": N.lib().sq_energy_grad_reference_sweep,
         }[method]
+        if method == "adjoint" and not isinstance(theta, torch.Tensor):
+            # host values go to the entry point that takes them (its first
+            # launch reads them from pinned memory)
+            th = np.ascontiguousarray(theta, dtype=np.float64).ravel()
+            if th.size != self.n_gates:
+                raise ValueError(f"Expected {self.n_gates} theta values got {th.size}")
+            fn, th_ptr = N.lib().sq_energy_grad_adjoint_host, th.ctypes.data
+        else:
+            th = self.theta_tensor(theta)
+            th_ptr = _ptr(th)
+        e = ctypes.c_double()
+        g = np.zeros(max(self.n_gates, 1))
         N.check(
-            fn(self.space.handle, self._h, H.handle, _ptr(th), _ptr(psi0), ctypes.byref(e), g.ctypes.data,
+            fn(self.space.handle, self._h, H.handle, th_ptr, _ptr(psi0), ctypes.byref(e), g.ctypes.data,
                _ptr(self.space.work(2)), _stream())
         )
         return e.value, g[: self.n_gates].copy()
