@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <numeric>
 #include <string>
@@ -371,6 +372,18 @@ __global__ void k_group_out(const double* __restrict__ spart, int64_t nblk, cons
   for (int g = threadIdx.x; g < ng; g += blockDim.x) grad[out0[m] + g] = grad_g[(size_t)m * ng + g];
 }
 
+// Instances this large go to groups (the persistent launch keeps the rest):
+// one workgroup runs a 3-layer (8e,8o) evaluation in 967 us and then bounds the
+// whole batch, a 2-layer (6e,6o) one in 173, less than the launches of another
+// group.  256 instances of 4 to 10 orbitals with groups from 16384 (10
+// orbitals), 4096 (8) and 300 (6) determinants: 1524, 1206, 1358 us.
+constexpr int64_t kGroupMinDim = 4096;
+
+// Streams the groups run on: one group's short kernels and the ends of its long
+// ones leave CUs idle that another group's fill (256 instances as above on 1,
+// 3 and 4: 1549, 1329, 1206 us; there are four hardware queues).
+constexpr int kGroupLanes = 4;
+
 struct Batch {
   std::vector<BatchInstance> inst;
   int nwg = 0;
@@ -386,8 +399,12 @@ struct Batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::vector<int32_t> grad_off;
-  hipStream_t side = nullptr;  // the persistent launch beside the groups (default priority)
+  double* host_out = nullptr;  // pinned: energies | gradients on their way to the caller
+  mutable std::mutex host_mu;
+  hipStream_t side = nullptr;  // the persistent launch beside the groups (default priority, as the lanes)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipStream_t lane[kGroupLanes] = {};  // [0] unused: the caller's stream
+  hipEvent_t ev_lane[kGroupLanes] = {};
   int rot_pairs = 2;    // rotation pairs per thread in flight (1, 2, 4)
   int gemm_tiles = 1;   // sigma GEMM column tiles per wave (1, 2)
   void drop_graph() {
@@ -399,9 +416,14 @@ struct Batch {
   ~Batch() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
+    if (host_out) (void)hipHostFree(host_out);
+    if (side) (void)hipStreamDestroy(side);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
-    if (side) (void)hipStreamDestroy(side);
+    for (hipStream_t l : lane)
+      if (l) (void)hipStreamDestroy(l);
+    for (hipEvent_t e : ev_lane)
+      if (e) (void)hipEventDestroy(e);
     for (void* p : allocs) (void)hipFree(p);
   }
 };
@@ -414,12 +436,6 @@ static T* bupload(Batch& B, const std::vector<T>& v) {
   B.allocs.push_back(d);
   return d;
 }
-
-
-// Instances this large go to groups (the persistent launch keeps the rest):
-// at (10e,10o) one workgroup per instance runs a 3-layer evaluation in
-// 14.5 ms against 0.25 ms through the single-instance kernels.
-constexpr int64_t kGroupMinDim = 16384;
 
 // Bytes of a program's gate layout (kinds, pairs, scales and generator
 // terms): equal keys on one space give identical tile plans.
@@ -475,7 +491,7 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
     G.plan_gen = G.prog->plan_gen;
     G.mats_stride = tiles_mats_doubles(s, *G.prog);
     G.tpart_stride = tiles_partial_doubles(s, *G.prog);
-    G.spart_stride = row_sigma_group_partials(s);
+    G.spart_stride = row_sigma_group_partials(s, G.n);
     SQ_CHECK(G.mats_stride > 0 && G.tpart_stride > 0 && G.spart_stride > 0, SQ_ERR_ARG, "group path unavailable");
     {
       const uint32_t a = s.h_astr[0], b = s.h_bstr[0];
@@ -522,7 +538,7 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
 static void check_group(const BatchGroup& G) {
   SQ_CHECK(G.prog->plan_gen == G.plan_gen, SQ_ERR_ARG,
            "a batched program's tile shape changed after the batch was created; create the batch again");
-  SQ_CHECK(row_sigma_group_partials(*G.space) == G.spart_stride, SQ_ERR_ARG,
+  SQ_CHECK(row_sigma_group_partials(*G.space, G.n) == G.spart_stride, SQ_ERR_ARG,
            "a batched space's sigma shape changed after the batch was created; create the batch again");
 }
 
@@ -723,24 +739,29 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
       SQ_HIP(hipMalloc(&scratch, sizeof(double) * std::max<size_t>((size_t)B.slot * nwg, 1)));
       B.allocs.push_back(scratch);
       B.dev.scratch = scratch;
+      // energies | gradients, one copy to the host
       double* en = nullptr;
-      SQ_HIP(hipMalloc(&en, sizeof(double) * n_inst));
+      SQ_HIP(hipMalloc(&en, sizeof(double) * ((size_t)n_inst + grad_off)));
       B.allocs.push_back(en);
       B.dev.energy = en;
-      double* gr = nullptr;
-      SQ_HIP(hipMalloc(&gr, sizeof(double) * std::max<int64_t>(grad_off, 1)));
-      B.allocs.push_back(gr);
-      B.dev.grad = gr;
+      B.dev.grad = en + n_inst;
+      SQ_HIP(hipHostMalloc(reinterpret_cast<void**>(&B.host_out), sizeof(double) * ((size_t)n_inst + grad_off),
+                           hipHostMallocDefault));
       SQ_HIP(hipMalloc(&B.d_theta, sizeof(double) * std::max(theta_off, 1)));
       B.allocs.push_back(B.d_theta);
       B.dev.theta = B.d_theta;
       B.d_psi0 = bupload(B, std::vector<const double*>(n_inst, nullptr));
       B.dev.psi0 = B.d_psi0;
       build_groups(B, hams, spaces);
-      if (!B.groups.empty() && n_small > 0) {
+      const int nl = std::min<int>(kGroupLanes, (int)B.groups.size());
+      if (nl > 1 || (nl > 0 && nwg > 0)) SQ_HIP(hipEventCreateWithFlags(&B.ev_fork, hipEventDisableTiming));
+      if (nl > 0 && nwg > 0) {
         SQ_HIP(hipStreamCreateWithFlags(&B.side, hipStreamNonBlocking));
-        SQ_HIP(hipEventCreateWithFlags(&B.ev_fork, hipEventDisableTiming));
         SQ_HIP(hipEventCreateWithFlags(&B.ev_join, hipEventDisableTiming));
+      }
+      for (int l = 1; l < nl; ++l) {
+        SQ_HIP(hipStreamCreateWithFlags(&B.lane[l], hipStreamNonBlocking));
+        SQ_HIP(hipEventCreateWithFlags(&B.ev_lane[l], hipEventDisableTiming));
       }
     } catch (...) {
       delete bo;
@@ -790,21 +811,46 @@ static BatchKernel batch_kernel(const Batch& B) {
   return table[u][B.gemm_tiles - 1];
 }
 
-// The persistent launch and the groups write disjoint outputs; with both,
-// the persistent launch runs on the batch's side stream between a fork and
-// a join event, beside the groups' kernels on st.
+// The persistent launch and the groups write disjoint outputs: between a fork
+// and join events the persistent launch runs on the batch's side stream, first
+// (last, or in a lane of the groups: 955 -> 980 to 1100 us), and the groups on
+// the lanes (the first is st), the longest first, each on the lane with the
+// least work.
 static void batch_launch(Batch& B, hipStream_t st) {
-  if (B.nwg > 0 && !B.groups.empty()) {
-    SQ_HIP(hipEventRecord(B.ev_fork, st));
-    SQ_HIP(hipStreamWaitEvent(B.side, B.ev_fork, 0));
-    SQ_PROF(PC_BATCH, B.side, B.bytes, B.flops, batch_kernel(B)<<<B.nwg, kBT, B.lds, B.side>>>(B.dev));
-    for (const BatchGroup& G : B.groups) group_launch(B, G, st);
-    SQ_HIP(hipEventRecord(B.ev_join, B.side));
-    SQ_HIP(hipStreamWaitEvent(st, B.ev_join, 0));
+  const int nl = std::min<int>(kGroupLanes, (int)B.groups.size());
+  if (nl == 0) {
+    if (B.nwg > 0) SQ_PROF(PC_BATCH, st, B.bytes, B.flops, batch_kernel(B)<<<B.nwg, kBT, B.lds, st>>>(B.dev));
     return;
   }
-  if (B.nwg > 0) SQ_PROF(PC_BATCH, st, B.bytes, B.flops, batch_kernel(B)<<<B.nwg, kBT, B.lds, st>>>(B.dev));
-  for (const BatchGroup& G : B.groups) group_launch(B, G, st);
+  if (B.ev_fork) SQ_HIP(hipEventRecord(B.ev_fork, st));
+  if (B.nwg > 0) {
+    SQ_HIP(hipStreamWaitEvent(B.side, B.ev_fork, 0));
+    SQ_PROF(PC_BATCH, B.side, B.bytes, B.flops, batch_kernel(B)<<<B.nwg, kBT, B.lds, B.side>>>(B.dev));
+  }
+  for (int l = 1; l < nl; ++l) SQ_HIP(hipStreamWaitEvent(B.lane[l], B.ev_fork, 0));
+  // about how long a group takes (us): its chain of launches and its work
+  // (29 instances of (10e,10o) with three layers: 800)
+  auto us = [&](int i) {
+    const BatchGroup& G = B.groups[i];
+    return 100.0 + 1.3e-6 * (double)G.n * (double)G.dim * (G.ng + 4.0 * G.space->npair);
+  };
+  std::vector<int> order(B.groups.size());
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return us(a) > us(b); });
+  double load[kGroupLanes] = {};
+  for (int i : order) {
+    const int l = (int)(std::min_element(load, load + nl) - load);
+    load[l] += us(i);
+    group_launch(B, B.groups[i], l == 0 ? st : B.lane[l]);
+  }
+  for (int l = 1; l < nl; ++l) {
+    SQ_HIP(hipEventRecord(B.ev_lane[l], B.lane[l]));
+    SQ_HIP(hipStreamWaitEvent(st, B.ev_lane[l], 0));
+  }
+  if (B.nwg > 0) {
+    SQ_HIP(hipEventRecord(B.ev_join, B.side));
+    SQ_HIP(hipStreamWaitEvent(st, B.ev_join, 0));
+  }
 }
 
 /* Kernel shape: rotation pairs per thread in flight (1, 2 or 4) and sigma
@@ -874,9 +920,12 @@ int sq_batch_results(const sq_batch* bo, double* energies, double* grads, void* 
     SQ_CHECK(bo && energies && grads, SQ_ERR_ARG, "NULL argument");
     const Batch& B = bo->b;
     hipStream_t st = as_stream(stream);
-    SQ_HIP(hipMemcpyAsync(energies, B.dev.energy, sizeof(double) * B.inst.size(), hipMemcpyDeviceToHost, st));
-    SQ_HIP(hipMemcpyAsync(grads, B.dev.grad, sizeof(double) * B.ngrad, hipMemcpyDeviceToHost, st));
+    const size_t n = B.inst.size();
+    std::lock_guard<std::mutex> lock(B.host_mu);
+    SQ_HIP(hipMemcpyAsync(B.host_out, B.dev.energy, sizeof(double) * (n + (size_t)B.ngrad), hipMemcpyDeviceToHost, st));
     SQ_HIP(hipStreamSynchronize(st));
+    std::memcpy(energies, B.host_out, sizeof(double) * n);
+    std::memcpy(grads, B.host_out + n, sizeof(double) * (size_t)B.ngrad);
   });
 }
 

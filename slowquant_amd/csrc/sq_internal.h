@@ -322,7 +322,7 @@ void tiles_reverse_group(const Space& s, const Program& p, const double* theta, 
 // products' tiles in the launch); A, Ma and Mb per instance at the given strides; energy
 // partials per instance (row_sigma_group_partials of them) at partial.
 bool row_sigma_group_ok(const Space& s);
-int64_t row_sigma_group_partials(const Space& s);
+int64_t row_sigma_group_partials(const Space& s, int n);
 void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
                      const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
                      bool zeroed, hipStream_t st);

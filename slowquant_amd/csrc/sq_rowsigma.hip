@@ -1052,8 +1052,12 @@ int string_gemm_split(const Space& s) {
 // (one block per CU).  Scatter form: the smallest R that gives every wave a
 // tile (more, smaller blocks).  List form: two rows at least, which halves the
 // staging of A per row: 10 orbitals in groups 1600 -> 1506 us, (11e,11o) 205 ->
-// 186, (12e,12o) 437 -> 424 (energy and gradient); more rows gain no more.
-bool row_plan(const Space& s, RowPlan* out) {
+// 186, (12e,12o) 437 -> 424 (energy and gradient); more rows gain no more.  A
+// launch of many instances has blocks enough: four rows and the string products
+// unsplit (a quarter of the atomic adds), 256 instances 1283 -> 1206 us.
+constexpr int kManyInst = 8;
+
+bool row_plan(const Space& s, RowPlan* out, int n = 1) {
   if (s.dim == 0 || s.nsb > 16384 || s.npair + 1 > 255 || s.dim >= ((int64_t)1 << 31)) return false;
   const bool scatter = !row_deterministic(s);
   const int kpad = rup(s.npair + 1, 16);
@@ -1067,7 +1071,7 @@ bool row_plan(const Space& s, RowPlan* out) {
   const int tpr = (s.nsb + 15) / 16;
   int bestR = 0;
   if (scatter) {
-    bestR = std::max(list ? 2 : 1, (kRowWaves + tpr - 1) / tpr);
+    bestR = std::max(list ? (n >= kManyInst ? 4 : 2) : 1, (kRowWaves + tpr - 1) / tpr);
     bestR = std::max(1, std::min(s.nsa, bestR));
     while (bestR > 1 && row_lds(s, mt, bestR, true, list) > kLdsMax) --bestR;
   } else {
@@ -1118,7 +1122,7 @@ bool row_plan(const Space& s, RowPlan* out) {
   out->fused = list && fuse_env != 0 && 2 * out->lds <= kLdsMax && mt <= kMaxFusedMt;
   out->ngemm_a = out->ngemm_b = out->kchunk_b = 0;
   if (out->fused) {
-    const int split = s.sig_nsplit > 0 ? s.sig_nsplit : 4;
+    const int split = s.sig_nsplit > 0 ? s.sig_nsplit : n >= kManyInst ? 1 : 4;
     out->kchunk = chunk(s.nsa, split);
     out->kchunk_b = chunk(s.nsb, split);
     const int tiles = ((s.nsa + kGemmRows - 1) / kGemmRows) * ((s.nsb + kGemmCols - 1) / kGemmCols);
@@ -1441,9 +1445,9 @@ bool row_sigma_group_ok(const Space& s) {
   return rows_enabled() && s.d_rtb != nullptr && row_plan(s, &pl) && pl.scatter && pl.fused;
 }
 
-int64_t row_sigma_group_partials(const Space& s) {
+int64_t row_sigma_group_partials(const Space& s, int n) {
   RowPlan pl;
-  if (!row_plan(s, &pl) || !pl.fused) return 0;
+  if (!row_plan(s, &pl, n) || !pl.fused) return 0;
   return (int64_t)pl.ngroups + pl.ngemm_a + pl.ngemm_b;
 }
 
@@ -1451,7 +1455,7 @@ void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const do
                      const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
                      bool zeroed, hipStream_t st) {
   RowPlan pl;
-  SQ_CHECK(row_sigma_group_ok(s) && row_plan(s, &pl) && n > 0 && n <= 65535, SQ_ERR_ARG,
+  SQ_CHECK(row_sigma_group_ok(s) && row_plan(s, &pl, n) && n > 0 && n <= 65535, SQ_ERR_ARG,
            "the grouped row sigma does not apply to this space");
   rows_list_launch(s, pl, A, A_stride, rup(s.npair + 1, 16), Ma, Ma_stride, Mb, Mb_stride, psi, nullptr, 0, sigma,
                    partial, n, zeroed, st);

@@ -434,7 +434,7 @@ SHAPES = tuple((u, ct) for u in (1, 2, 4) for ct in (1, 2))
 # Instances of this many determinants or more run in the library's batched
 # groups (sq_batch.hip, kGroupMinDim): through the tile-stage kernels, whose
 # tile shape (elements per tile, threads per block) is the program's.
-BATCH_GROUP_MIN_DIM = 16384
+BATCH_GROUP_MIN_DIM = 4096
 GROUP_TILE_SHAPES = ((0, 0), (1024, 256), (2048, 256), (4096, 512))
 
 

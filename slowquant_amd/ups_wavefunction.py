@@ -278,7 +278,7 @@ class WaveFunctionUPS(WaveFunctionBase):
         one batch).  All shifted instances run in one batched launch when the
         layout allows it (rotation gates, at most 12 active orbitals: the
         persistent kernel for small spaces, the tile-stage and row-sigma
-        kernels over the group of copies from 16384 determinants), else one
+        kernels over the group of copies from 4096 determinants), else one
         engine energy per shift."""
         th = np.asarray(parameters, dtype=np.float64)
         thetas = np.repeat(th[None, :], len(theta_diffs), axis=0)
