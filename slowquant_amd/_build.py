@@ -15,6 +15,7 @@ SOURCES = [
     "sq_gates.hip",
     "sq_sigma.hip",
     "sq_rowsigma.hip",
+    "sq_rdm.hip",
     "sq_grad.hip",
     "sq_profile.hip",
     "sq_tiles.hip",

@@ -42,7 +42,7 @@ static GradBufs carve(const Space& s, int n_gates, double* work) {
 
 // Device -> host copy of n doubles through a pinned staging buffer: one DMA
 // and no pageable bounce buffer; synchronizes the stream.
-static void copy_to_host_pinned(double* host, const double* dev, size_t n, hipStream_t st) {
+void copy_to_host_pinned(double* host, const double* dev, size_t n, hipStream_t st) {
   static std::mutex mu;
   static double* buf = nullptr;
   static size_t cap = 0;
@@ -285,7 +285,7 @@ int64_t sq_work_bytes(const sq_space* sp, int what) {
     case 2:  // gradients, for programs of up to 65536 gates
       return 8 * grad_doubles(s, 65536);
     case 3:  // RDMs
-      return rdm_work_bytes(s, nullptr, nullptr, nullptr);
+      return rdm_work_bytes(s);
     default:
       return -1;
   }

@@ -135,6 +135,10 @@ struct Space {
   // row sigma shape (sq_sigma_configure): 0 / -1 = automatic
   int sig_R = 0, sig_nsplit = 0, sig_det = -1;
   std::vector<uint32_t> h_astr, h_bstr;
+  // RDM tables (sq_rdm.hip), built on first use
+  mutable std::mutex rdm_mu;
+  mutable int2* d_rdm_alist = nullptr;
+  mutable int32_t* d_rdm_btab = nullptr;
   mutable struct WinCache* win = nullptr;  // window tables of the tile stages (sq_tiles.hip), built on first use
 };
 
@@ -143,6 +147,7 @@ void win_cache_free(struct WinCache* c);
 void build_gemm_tables(Space& s);
 void build_row_tables(Space& s);
 void free_row_tables(Space& s);
+void rdm_tables_free(Space& s);
 
 struct TilePlan;
 struct UccCsr;
@@ -271,8 +276,14 @@ void sigma_energy_dev(const Space& s, const Hamiltonian& H, const double* psi, d
                       double* work, hipStream_t st);
 void dot_dev(const double* x, const double* y, int64_t n, double* out_dev, int slot, double factor, double* partial,
              hipStream_t st);
-int64_t rdm_work_bytes(const Space& s, int* rt_out, int* nchunks_out, int64_t* chunk_out);
+// RDMs (sq_rdm.hip)
+int64_t rdm_work_bytes(const Space& s);
 void rdm_impl(const Space& s, const double* psi, double* rdm1, double* rdm2, double* work, hipStream_t st);
+// rho_a = C C^T and rho_b = C^T C (upper tiles only) for C nsa x nsb and its
+// transpose Ct (sq_rowsigma.hip).
+void string_grams(const double* C, const double* Ct, double* rho_a, double* rho_b, int nsa, int nsb, hipStream_t st);
+// n doubles to the host through pinned memory; synchronizes the stream.
+void copy_to_host_pinned(double* host, const double* dev, size_t n, hipStream_t st);
 
 // Implemented in sq_gates.hip
 void apply_gate_impl(const Space& s, const Program& p, int g, const double* theta_dev, bool negate, double* psi,

@@ -238,16 +238,11 @@ struct GemmArgs {
 };
 
 template <int T>
-__global__ __launch_bounds__(256, 2) void k_string_gemm(GemmArgs P) {
+__device__ __forceinline__ void string_gemm_block(const GemmArgs& P, int i0, int j0, int z) {
   constexpr int F = T / 32;  // MFMA tiles per wave and side
   constexpr int LJ = T / 16;
   __shared__ double sL[2][16][T];
   __shared__ double sR[2][16][T];
-  const int tn = (P.n + T - 1) / T, tm = (P.m + T - 1) / T, nt = tm * tn;
-  int id = blockIdx.x;
-  if (id < (nt & ~7)) id = (id & 7) * (nt >> 3) + (id >> 3);
-  const int strip = id / (8 * tn), sr = min(8, tm - strip * 8), rem = id - strip * 8 * tn;
-  const int i0 = (strip * 8 + rem % sr) * T, j0 = (rem / sr) * T;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63, kq = lane >> 4, li = lane & 15;
   const int wi = (wave >> 1) * (T / 2), wj = (wave & 1) * (T / 2);
   double4_t acc[F][F];
@@ -268,7 +263,7 @@ __global__ __launch_bounds__(256, 2) void k_string_gemm(GemmArgs P) {
   // the slice's uniform base
   uint32_t lofs[LJ], rofs[LJ];
   double pl[LJ], pr[LJ];
-  const int zb = blockIdx.y * P.kchunk, ze = min(P.k0n + P.k1n, zb + P.kchunk);
+  const int zb = z * P.kchunk, ze = min(P.k0n + P.k1n, zb + P.kchunk);
   for (int phase = 0; phase < 2; ++phase) {
     const double* __restrict__ L = phase ? P.L1 : P.L0;
     const double* __restrict__ R = phase ? P.R1 : P.R0;
@@ -339,7 +334,7 @@ __global__ __launch_bounds__(256, 2) void k_string_gemm(GemmArgs P) {
       lds_barrier();
     }
   }
-  double* o = P.out + (size_t)blockIdx.y * P.m * P.n;
+  double* o = P.out + (size_t)z * P.m * P.n;
 #pragma unroll
   for (int x = 0; x < F; ++x)
 #pragma unroll
@@ -349,6 +344,27 @@ __global__ __launch_bounds__(256, 2) void k_string_gemm(GemmArgs P) {
         const int I = i0 + wi + x * 16 + kq + 4 * r, J = j0 + wj + y * 16 + li;
         if (I < P.m && J < P.n) o[(size_t)I * P.n + J] = acc[x][y][r];
       }
+}
+
+template <int T>
+__global__ __launch_bounds__(256, 2) void k_string_gemm(GemmArgs P) {
+  const int tn = (P.n + T - 1) / T, tm = (P.m + T - 1) / T, nt = tm * tn;
+  int id = blockIdx.x;
+  if (id < (nt & ~7)) id = (id & 7) * (nt >> 3) + (id >> 3);
+  const int strip = id / (8 * tn), sr = min(8, tm - strip * 8), rem = id - strip * 8 * tn;
+  const int i0 = (strip * 8 + rem % sr) * T, j0 = (rem / sr) * T;
+  string_gemm_block<T>(P, i0, j0, blockIdx.y);
+}
+
+// L0 R0 of two symmetric products (blockIdx.y: which), their tiles i <= j only.
+template <int T>
+__global__ __launch_bounds__(256, 2) void k_string_grams(GemmArgs A, GemmArgs B) {
+  const GemmArgs& P = blockIdx.y ? B : A;
+  const int tn = (P.n + T - 1) / T;
+  int i = 0, id = blockIdx.x;
+  while (i < tn && id >= tn - i) id -= tn - i++;
+  if (i >= tn) return;
+  string_gemm_block<T>(P, i * T, (i + id) * T, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1142,6 +1158,16 @@ bool rows_enabled() {
 }
 
 }  // namespace
+
+void string_grams(const double* C, const double* Ct, double* rho_a, double* rho_b, int nsa, int nsb, hipStream_t st) {
+  const GemmArgs A{C, Ct, nullptr, nullptr, rho_a, nsa, nsa, nsb, 0, nsb};
+  const GemmArgs B{Ct, C, nullptr, nullptr, rho_b, nsb, nsb, nsa, 0, nsa};
+  const double flops = (double)nsa * nsb * (nsa + nsb);
+  const double bytes = 8.0 * ((double)nsa * nsb + (double)nsa * nsa + (double)nsb * nsb);
+  const int t = (std::max(nsa, nsb) + 63) / 64;
+  SQ_PROF(PC_ALPHA_GEMM, st, bytes, flops,
+          (k_string_grams<64><<<dim3(t * (t + 1) / 2, 2), 256, 0, st>>>(A, B)));
+}
 
 bool row_sigma_applies(const Space& s) {
   RowPlan pl;

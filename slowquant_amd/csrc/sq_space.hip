@@ -218,6 +218,7 @@ int sq_space_destroy(sq_space* sp) {
     if (!sp) return;
     Space& s = sp->s;
     free_row_tables(s);
+    rdm_tables_free(s);
     if (s.win) win_cache_free(s.win);
     for (void* p : {(void*)s.d_astr, (void*)s.d_bstr, (void*)s.d_arank, (void*)s.d_brank, (void*)s.d_aexc,
                     (void*)s.d_bexc, (void*)s.d_aexc_full, (void*)s.d_bexc_full, (void*)s.d_gta, (void*)s.d_gtb})
