@@ -283,120 +283,52 @@ __device__ __forceinline__ double full_rdm2_elem(int p, int q, int r, int s, int
   return v;
 }
 
-// G1[p][q] (N x o, rows >= o zero) and the compact G2c[p][q][r][s] (o^4).
-__global__ void k_full_rdm1(int N, int ni, int na, const double* __restrict__ rdm1, double* __restrict__ G1) {
-  const int o = ni + na;
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= N * o) return;
-  const int p = x / o, q = x % o;
-  G1[x] = p < o ? full_rdm1_elem(p, q, ni, na, rdm1) : 0.0;
-}
-
-__global__ void k_full_rdm2(int ni, int na, const double* __restrict__ rdm1, const double* __restrict__ rdm2,
-                            double* __restrict__ G2) {
-  const int o = ni + na;
-  const int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t o4 = (int64_t)o * o * o * o;
-  if (x >= o4) return;
-  const int s = (int)(x % o), r = (int)((x / o) % o), q = (int)((x / ((int64_t)o * o)) % o),
-            p = (int)(x / ((int64_t)o * o * o));
-  G2[x] = full_rdm2_elem(p, q, r, s, ni, na, rdm1, rdm2);
-}
-
-// The whole orbital gradient in one block for o <= kSmallGradO: Gamma1 and
-// Gamma2 over the o orbitals in LDS; one wave per kappa element (m, n), its
-// lanes splitting the o^3 index triples of the four sums Z(n,m), W(m,n),
-// Z(m,n), W(n,m) of k_kappa_grad (and the o terms of Y and V), summed by a
-// fixed-order shuffle reduction; g is read from global memory.
-constexpr int kSmallGradO = 8;
-
-__global__ __launch_bounds__(256) void k_kappa_grad_small(int N, int ni, int na, const double* __restrict__ h,
+// Orbital gradient: one block per kappa element (m, n), its threads splitting
+// the o^3 index triples of
+//   grad = 2 Y(n,m) - 2 V(m,n) + Z(n,m) - W(m,n) - Z(m,n) + W(n,m),
+//   Z(a,b) = sum_pqr g[a][p][q][r] G2[b][p][q][r], W(a,b) = sum_pqr g[p][a][q][r] G2[p][b][q][r],
+//   Y(a,b) = sum_p h[a][p] G1[b][p], V(a,b) = sum_p h[p][a] G1[p][b]
+// (p, q, r < o; terms with an index b >= o vanish with Gamma), summed in a fixed
+// order.  The elements of Gamma1 and Gamma2 are formed where they are used.
+// Latency bound: a few dependent loads per triple, o^3 / 256 triples a thread.
+// 12 orbitals, 2 + 6 of them inactive and active: 7 us against 56 for one block
+// with both matrices in LDS; larger ones with the contractions as GEMMs over
+// copies of g and Gamma2 took 247 us a gradient at 20 orbitals (4 + 6) and 8.1 ms
+// at 100 (30 + 10), against 79 us and 1.0 ms.
+__global__ __launch_bounds__(256) void k_kappa_grad(int N, int ni, int na, const double* __restrict__ h,
                                                           const double* __restrict__ g,
                                                           const double* __restrict__ rdm1,
-                                                          const double* __restrict__ rdm2, int nk,
+                                                          const double* __restrict__ rdm2,
                                                           const int32_t* __restrict__ idx, double* __restrict__ grad) {
-  __shared__ double sG1[kSmallGradO * kSmallGradO];
-  __shared__ double sG2[kSmallGradO * kSmallGradO * kSmallGradO * kSmallGradO];
-  const int o = ni + na, o2 = o * o, o3 = o2 * o, o4 = o3 * o;
-  for (int x = threadIdx.x; x < o2; x += blockDim.x) sG1[x] = full_rdm1_elem(x / o, x % o, ni, na, rdm1);
-  for (int x = threadIdx.x; x < o4; x += blockDim.x)
-    sG2[x] = full_rdm2_elem(x / o3, (x / o2) % o, (x / o) % o, x % o, ni, na, rdm1, rdm2);
-  __syncthreads();
+  __shared__ double red[4];
+  const int o = ni + na, o2 = o * o, o3 = o2 * o;
   const int64_t N2 = (int64_t)N * N, N3 = N2 * N;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (int)(blockDim.x >> 6);
-  for (int i = wave; i < nk; i += nw) {
-    const int m = idx[2 * i], n = idx[2 * i + 1];
-    double t = 0.0;
-    // grad = 2 Y[n][m] - 2 V[m][n] + Z(n,m) - W(m,n) - Z(m,n) + W(n,m), with
-    // Z(a,b) = sum_pqr g[a][p][q][r] G2[b][p][q][r], W(a,b) = sum_pqr g[p][a][q][r] G2[p][b][q][r]
-    // (terms with an index b >= o vanish with Gamma)
-    for (int x = lane; x < o3; x += 64) {
-      const int p = x / o2, q = (x / o) % o, r = x % o;
-      const int64_t qr = (int64_t)q * N + r;
-      const int pqr = p * o2 + q * o + r;  // = x
-      if (m < o)
-        t += g[n * N3 + p * N2 + qr] * sG2[m * o3 + pqr] + g[p * N3 + n * N2 + qr] * sG2[p * o3 + m * o2 + q * o + r];
-      if (n < o)
-        t -= g[m * N3 + p * N2 + qr] * sG2[n * o3 + pqr] + g[p * N3 + m * N2 + qr] * sG2[p * o3 + n * o2 + q * o + r];
-    }
-    if (lane < o) {
-      if (m < o) t += 2.0 * h[(int64_t)n * N + lane] * sG1[m * o + lane];
-      if (n < o) t -= 2.0 * h[(int64_t)lane * N + m] * sG1[lane * o + n];
-    }
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
-    if (lane == 0) grad[i] = t;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = idx[2 * blockIdx.x], n = idx[2 * blockIdx.x + 1];
+  auto G1 = [&](int p, int q) { return full_rdm1_elem(p, q, ni, na, rdm1); };
+  auto G2 = [&](int p, int q, int r, int s) { return full_rdm2_elem(p, q, r, s, ni, na, rdm1, rdm2); };
+  double t = 0.0;
+  for (int x = threadIdx.x; x < o3; x += 256) {
+    const int p = x / o2, q = (x / o) % o, r = x % o;
+    const int64_t qr = (int64_t)q * N + r;
+    if (m < o) t += g[n * N3 + p * N2 + qr] * G2(m, p, q, r) + g[p * N3 + n * N2 + qr] * G2(p, m, q, r);
+    if (n < o) t -= g[m * N3 + p * N2 + qr] * G2(n, p, q, r) + g[p * N3 + m * N2 + qr] * G2(p, n, q, r);
   }
-}
-
-// gc[a][pqr] = g[a][p][q][r] and gt[a][pqr] = g[p][a][q][r] over p, q, r < o.
-__global__ void k_g_blocks(int N, int o, const double* __restrict__ g, double* __restrict__ gc,
-                           double* __restrict__ gt) {
-  const int64_t o3 = (int64_t)o * o * o;
-  const int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (x >= (int64_t)N * o3) return;
-  const int a = (int)(x / o3);
-  const int64_t rem = x % o3;
-  const int p = (int)(rem / ((int64_t)o * o)), q = (int)((rem / o) % o), r = (int)(rem % o);
-  const int64_t N2 = (int64_t)N * N;
-  gc[x] = g[((int64_t)a * N + p) * N2 + (int64_t)q * N + r];
-  gt[x] = g[((int64_t)p * N + a) * N2 + (int64_t)q * N + r];
-}
-
-// G2t[b][pqr] = G2c[p][b][q][r]
-__global__ void k_perm01(int o, const double* __restrict__ G2, double* __restrict__ G2t) {
-  const int64_t o3 = (int64_t)o * o * o;
-  const int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (x >= (int64_t)o * o3) return;
-  const int b = (int)(x / o3);
-  const int64_t rem = x % o3;
-  const int p = (int)(rem / ((int64_t)o * o));
-  const int64_t qr = rem % ((int64_t)o * o);
-  G2t[x] = G2[((int64_t)p * o + b) * o * o + qr];
-}
-
-// grad[i] = 2 Y[n][m] - 2 V[m][n] + Z[n][m] - W[m][n] - Z[m][n] + W[n][m]
-// with Y = h G1^T (N x N) and V = h^T G1, Z = gc G2c^T, W = gt G2t^T stored
-// N x o (their columns >= o vanish with Gamma outside the o orbitals).
-__global__ void k_kappa_grad(int N, int o, int nk, const int32_t* __restrict__ idx, const double* __restrict__ Y,
-                             const double* __restrict__ V, const double* __restrict__ Z,
-                             const double* __restrict__ W, double* __restrict__ grad) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nk) return;
-  const int m = idx[2 * i], n = idx[2 * i + 1];
-  auto z = [&](const double* M, int a, int b) { return b < o ? M[(int64_t)a * o + b] : 0.0; };
-  grad[i] = 2.0 * Y[(int64_t)n * N + m] - 2.0 * z(V, m, n) + z(Z, n, m) - z(W, m, n) - z(Z, m, n) + z(W, n, m);
+  if ((int)threadIdx.x < o) {
+    const int p = threadIdx.x;
+    if (m < o) t += 2.0 * h[(int64_t)n * N + p] * G1(m, p);
+    if (n < o) t -= 2.0 * h[(int64_t)p * N + m] * G1(p, n);
+  }
+  for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
+  if (lane == 0) red[wave] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) grad[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 int64_t ao2mo_work_doubles(int nao, int nmo) {
   const int64_t a = nao, m = nmo;
   const int64_t t = std::max({m * a * a * a, m * m * a * a, m * m * m * a});
   return 2 * t + m * a;
-}
-
-int64_t grad_work_doubles(int N, int o, int nk) {
-  const int64_t o3 = (int64_t)o * o * o;
-  return (int64_t)N * o + o * o3 + o * o3 + 2 * (int64_t)N * o3 + 2 * (int64_t)N * N + 2 * (int64_t)N * o + nk +
-         2 * (int64_t)nk + 64;
 }
 
 }  // namespace
@@ -411,7 +343,8 @@ int64_t sq_orbital_work_bytes(int n_ao, int n_mo, int n_inactive, int n_active, 
   if (n_ao <= 0 || n_mo <= 0 || n_inactive < 0 || n_active < 0 || n_inactive + n_active > n_mo || n_kappa < 0)
     return -1;
   const int64_t rot = 3 * (int64_t)n_mo * n_mo;
-  return 8 * std::max({rot, ao2mo_work_doubles(n_ao, n_mo), grad_work_doubles(n_mo, n_inactive + n_active, n_kappa)});
+  const int64_t grad = 2 * (int64_t)n_kappa;  // gradient | index pairs
+  return 8 * std::max({rot, ao2mo_work_doubles(n_ao, n_mo), grad});
 }
 
 int sq_orbital_rotation(int n, int n_ao, const double* c_old, const double* kappa, double* c_new, double* work,
@@ -515,42 +448,10 @@ int sq_orbital_gradient(int n_orb, int n_inactive, int n_active, const double* h
       SQ_CHECK(kappa_idx[i] >= 0 && kappa_idx[i] < N, SQ_ERR_ARG, "kappa index out of range");
     if (n_kappa == 0) return;
     hipStream_t st = as_stream(stream);
-    const int64_t o3 = (int64_t)o * o * o;
-    double* G1 = work;                 // N x o
-    double* G2 = G1 + (int64_t)N * o;  // o^4 (compact)
-    double* G2t = G2 + o * o3;         // o x o^3
-    double* gc = G2t + o * o3;         // N x o^3
-    double* gt = gc + (int64_t)N * o3;
-    double* Y = gt + (int64_t)N * o3;  // N x N
-    double* V = Y + (int64_t)N * N;    // N x o
-    double* Z = V + (int64_t)N * o;    // N x o
-    double* W = Z + (int64_t)N * o;
-    double* dgrad = W + (int64_t)N * o;
+    double* dgrad = work;
     int32_t* didx = reinterpret_cast<int32_t*>(dgrad + n_kappa);
     SQ_HIP(hipMemcpyAsync(didx, kappa_idx, sizeof(int32_t) * 2 * n_kappa, hipMemcpyHostToDevice, st));
-    if (o <= kSmallGradO) {
-      k_kappa_grad_small<<<1, 256, 0, st>>>(N, ni, na, h_mo, g_mo, rdm1, rdm2, n_kappa, didx, dgrad);
-      SQ_HIP(hipGetLastError());
-      SQ_HIP(hipMemcpyAsync(grad, dgrad, sizeof(double) * n_kappa, hipMemcpyDeviceToHost, st));
-      SQ_HIP(hipStreamSynchronize(st));
-      return;
-    }
-    k_full_rdm1<<<(unsigned)((N * o + 255) / 256), 256, 0, st>>>(N, ni, na, rdm1, G1);
-    SQ_HIP(hipGetLastError());
-    k_full_rdm2<<<(unsigned)((o * o3 + 255) / 256), 256, 0, st>>>(ni, na, rdm1, rdm2, G2);
-    SQ_HIP(hipGetLastError());
-    k_perm01<<<(unsigned)((o * o3 + 255) / 256), 256, 0, st>>>(o, G2, G2t);
-    SQ_HIP(hipGetLastError());
-    k_g_blocks<<<(unsigned)(((int64_t)N * o3 + 255) / 256), 256, 0, st>>>(N, o, g_mo, gc, gt);
-    SQ_HIP(hipGetLastError());
-    // Y[n][m] = sum_{p<o} h[n][p] G1[m][p]
-    gemm(N, N, o, 1.0, rowmaj(h_mo, N), trans(G1, o), 0.0, Y, N, 1, 0, 1, st);
-    // V[m][n] = sum_{p<o} h[p][m] G1[p][n] for n < o (Gamma1 vanishes for n >= o)
-    gemm(N, o, o, 1.0, trans(h_mo, N), rowmaj(G1, o), 0.0, V, o, 1, 0, 1, st);
-    // Z[a][b] = sum_{pqr} g[a][pqr] G2[b][pqr];  W[a][b] = sum_{pqr} g[p][a][qr] G2[p][b][qr]
-    gemm(N, o, (int)o3, 1.0, rowmaj(gc, o3), trans(G2, o3), 0.0, Z, o, 1, 0, 1, st);
-    gemm(N, o, (int)o3, 1.0, rowmaj(gt, o3), trans(G2t, o3), 0.0, W, o, 1, 0, 1, st);
-    k_kappa_grad<<<(unsigned)((n_kappa + 255) / 256), 256, 0, st>>>(N, o, n_kappa, didx, Y, V, Z, W, dgrad);
+    k_kappa_grad<<<n_kappa, 256, 0, st>>>(N, ni, na, h_mo, g_mo, rdm1, rdm2, didx, dgrad);
     SQ_HIP(hipGetLastError());
     SQ_HIP(hipMemcpyAsync(grad, dgrad, sizeof(double) * n_kappa, hipMemcpyDeviceToHost, st));
     SQ_HIP(hipStreamSynchronize(st));
