@@ -27,9 +27,9 @@
 // where |phi_k v| <= |v|: no term exceeds the result and about nu / 2 times
 // fewer products are needed than in Taylor steps of radius 2.
 // Energy and gradient of UCCSD, one product per unmerged entry (8 bytes each)
-// in Taylor steps -> this: (8e,8o) 663 -> 400 us (44 products of 4-5 us: launch
-// latency), (10e,10o) 13.5 -> 2.5 ms (9.1 M merged elements of 44 M entries;
-// a product takes 31 us, 105 us before, bound by the gathers of the vector).
+// in Taylor steps -> this: (8e,8o) 663 -> 310 us (44 products of 4-5 us: launch
+// latency), (10e,10o) 13.5 -> 2.1 ms (9.1 M merged elements of 44 M entries;
+// a product takes 25 us, 105 us before).
 // The first evaluation of a program, which builds the pattern: (10e,10o) 202
 // -> 8.9 ms.
 // The analytic gradient integrates <e^{-sT} lam | T_i | e^{-sT} psi> over
@@ -44,6 +44,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -53,6 +54,15 @@
 namespace sq {
 
 constexpr int kUB = 256;
+
+// A fixed pseudo-random vector in [-1, 1) (integer hash of the index).
+__device__ __forceinline__ double pattern_at(int64_t i) {
+  uint64_t h = (uint64_t)i * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
+  h ^= h >> 31;
+  h *= 0xBF58476D1CE4E5B9ull;
+  h ^= h >> 29;
+  return (double)(h >> 11) * (2.0 / 9007199254740992.0) - 1.0;
+}
 
 struct SV {
   int nsa, nsb;
@@ -333,19 +343,26 @@ __global__ __launch_bounds__(64 * kRows) void k_row_merge(int64_t dim, const int
 }
 
 // val[u] = sum over the contributions of merged element u of sign theta[gate]
-// |coef|; rmax[block]: largest sum of |val| over the block's rows.  One wave
-// per row.  theta and the coefficients are read from LDS when theta fits
-// (ng <= kLdsGates).
+// |coef|; rmax[block]: largest sum of |val| over the block's rows.  One wave per
+// row.  theta and the coefficients are read from LDS when theta fits (ng <=
+// kLdsGates).  Also v = v0 and x = the pseudo-random vector, for the products
+// that follow.
 constexpr int kLdsGates = 4096;
 __global__ __launch_bounds__(64 * kRows) void k_assemble(int64_t dim, const int64_t* __restrict__ urow,
                                                          const uint32_t* __restrict__ first,
                                                          const uint32_t* __restrict__ con,
                                                          const double* __restrict__ coefs, int ncoef,
                                                          const double* __restrict__ theta, int ng,
-                                                         double* __restrict__ val, double* __restrict__ rmax) {
+                                                         double* __restrict__ val, double* __restrict__ rmax,
+                                                         const double* __restrict__ v0, double* __restrict__ v,
+                                                         double* __restrict__ x) {
   extern __shared__ double sth[];
   __shared__ double sc[1 << kCoefBits];
   __shared__ double red[kRows];
+  for (int64_t i = blockIdx.x * (int64_t)(64 * kRows) + threadIdx.x; i < dim; i += (int64_t)gridDim.x * 64 * kRows) {
+    v[i] = v0[i];
+    x[i] = pattern_at(i);
+  }
   const bool lds = ng <= kLdsGates;
   if (lds)
     for (int i = threadIdx.x; i < ng; i += 64 * kRows) sth[i] = theta[i];
@@ -396,14 +413,73 @@ __global__ __launch_bounds__(kUB) void k_max(const double* __restrict__ x, int n
   }
 }
 
+// out[0..2] = bound[0], |y|^2, |x|^2 (out in pinned host memory), summed in a
+// fixed order by the last block.
+// The blocks' sums pass between them by agent-scope stores and loads; a fence
+// would write back the caches' other lines first (9 us against 5).
+__global__ __launch_bounds__(kUB) void k_norms(const double* __restrict__ y, const double* __restrict__ x, int64_t n,
+                                               const double* __restrict__ bound, double* __restrict__ part,
+                                               int* __restrict__ count, double* __restrict__ out) {
+  __shared__ double red[2][kUB / 64];
+  __shared__ int last;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto sums = [&](double a, double b) {
+    for (int off = 32; off > 0; off >>= 1) {
+      a += __shfl_down(a, off, 64);
+      b += __shfl_down(b, off, 64);
+    }
+    if (lane == 0) {
+      red[0][wave] = a;
+      red[1][wave] = b;
+    }
+    __syncthreads();
+  };
+  double a = 0.0, b = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)kUB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kUB) {
+    a += y[i] * y[i];
+    b += x[i] * x[i];
+  }
+  sums(a, b);
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kUB / 64; ++w) {
+      red[0][0] += red[0][w];
+      red[1][0] += red[1][w];
+    }
+    __hip_atomic_store(part + 2 * blockIdx.x, red[0][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(part + 2 * blockIdx.x + 1, red[1][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the sums have arrived before the count says so
+    last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  a = b = 0.0;
+  for (int i = threadIdx.x; i < (int)gridDim.x; i += kUB) {
+    a += __hip_atomic_load(part + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    b += __hip_atomic_load(part + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  sums(a, b);
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kUB / 64; ++w) {
+      red[0][0] += red[0][w];
+      red[1][0] += red[1][w];
+    }
+    out[0] = bound[0];
+    out[1] = red[0][0];
+    out[2] = red[1][0];
+    *count = 0;
+  }
+}
+
 // nxt[I] = f (T cur)[I] + prev[I] (prev: nullptr for none), LPR lanes per row;
 // TWO: nxt2 = f T cur2 in the same pass.  With bound, f is divided by
-// bound[0] (0 where that is 0).  A row's first four rounds of elements are
-// loaded before any is used.
-// Bound by the pattern's 12 bytes per element where it leaves the caches, by
-// launch latency below about 10^5 elements.  LPR: the smallest power of two
-// that takes an average row in two rounds (idle lanes of short rows against
-// the length of the shuffle tree).
+// bound[0] (0 where that is 0).  U rounds of a row's elements are loaded before
+// any is used, the next U during the gathers of those.
+// Bound by the chain row pointer -> elements -> gathers -> sum of a row, some
+// 3 us that the waves of a SIMD overlap, not by bytes ((10e,10o): 9.1 M
+// elements of 12 bytes; without the gathers' misses or the 8-byte numbers it
+// takes as long), and by launch latency below about 10^5 elements.  So a row
+// gets half a wave: 64, 32 and 16 lanes 2464, 2140 and 2200 us an energy and
+// gradient of (10e,10o) UCCSD (U = 6); U = 1, 2, 4, 6: 2448, 2236, 2180, 2140
 template <int LPR, bool TWO>
 __global__ __launch_bounds__(kUB) void k_spmv(int64_t dim, const int64_t* __restrict__ urow,
                                               const uint32_t* __restrict__ col, const double* __restrict__ val,
@@ -411,27 +487,39 @@ __global__ __launch_bounds__(kUB) void k_spmv(int64_t dim, const int64_t* __rest
                                               const double* __restrict__ prev, double f,
                                               const double* __restrict__ bound, double* __restrict__ nxt,
                                               double* __restrict__ nxt2) {
-  constexpr int U = 4;
+  constexpr int U = 6;
   const int lane = threadIdx.x & (LPR - 1);
   const int64_t I = (int64_t)blockIdx.x * (kUB / LPR) + threadIdx.x / LPR;
   if (I >= dim) return;
   if (bound) f = bound[0] > 0.0 ? f / bound[0] : 0.0;
-  const int64_t b = urow[I], e = urow[I + 1];
-  double v = 0.0, v2 = 0.0;
-  for (int64_t u0 = b + lane; u0 < e; u0 += U * LPR) {
-    double a[U];
-    uint32_t c[U];
+  const int64_t e = urow[I + 1];
+  int64_t u0 = urow[I] + lane;
+  double a[U], v = 0.0, v2 = 0.0;
+  uint32_t c[U];
+  auto load = [&] {
 #pragma unroll
     for (int j = 0; j < U; ++j) {
       const int64_t u = u0 + j * LPR;
       a[j] = u < e ? val[u] : 0.0;
       c[j] = u < e ? col[u] : 0u;
     }
+  };
+  load();
+  for (bool more = true; more;) {
+    double m[U], x[U], x2[U];
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-      if (u0 + j * LPR >= e) break;
-      v += a[j] * cur[c[j]];
-      if (TWO) v2 += a[j] * cur2[c[j]];
+      m[j] = a[j];
+      x[j] = cur[c[j]];
+      if (TWO) x2[j] = cur2[c[j]];
+    }
+    u0 += U * LPR;
+    more = u0 - lane < e;
+    if (more) load();
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      v += m[j] * x[j];
+      if (TWO) v2 += m[j] * x2[j];
     }
   }
 #pragma unroll
@@ -446,14 +534,16 @@ __global__ __launch_bounds__(kUB) void k_spmv(int64_t dim, const int64_t* __rest
 }
 
 // Linear combinations of the basis vectors phi_k (k <= K, at basis + k dim):
-// node q (q < nq) to nodes[I * stride + q], output nq (if fin) to fin[I].
+// node q (q < nq) to nodes[I * stride + q], the last output (if fin) to fin[I];
+// zero (if given; it may be a basis vector) is cleared.
 constexpr int kMaxOut = 9, kMaxBasis = 44, kCB = 64;
 struct Combine {
   double c[kMaxOut][kMaxBasis];
 };
 
-__global__ __launch_bounds__(kCB) void k_combine(int64_t dim, int K, Combine C, int nq, const double* __restrict__ basis,
-                                                 double* __restrict__ nodes, int stride, double* __restrict__ fin) {
+__global__ __launch_bounds__(kCB) void k_combine(int64_t dim, int K, Combine C, int nq, const double* basis,
+                                                 double* __restrict__ nodes, int stride, double* __restrict__ fin,
+                                                 double* zero) {
   const int64_t I = blockIdx.x * (int64_t)kCB + threadIdx.x;
   if (I >= dim) return;
   double o[kMaxOut];
@@ -469,6 +559,7 @@ __global__ __launch_bounds__(kCB) void k_combine(int64_t dim, int K, Combine C, 
   for (int q = 0; q < kMaxOut - 1; ++q)
     if (q < nq) nodes[(size_t)I * stride + q] = o[q];
   if (fin) fin[I] = o[kMaxOut - 1];
+  if (zero) zero[I] = 0.0;
 }
 
 // Gate dots: per merged element (I, J) r = sum_q V[I][q] U[J][q] over NQ
@@ -569,15 +660,20 @@ __global__ void k_gate_dots(SV sv, const Term* __restrict__ terms, const TermFas
   }
 }
 
-// gsum[i] += f * sum_b dpart[b*ng + i], one wave per gate.
+// gsum[i] = f * sum_b dpart[b*ng + i] (+ gsum[i] with add), one wave per gate;
+// also to host (if given).
 __global__ __launch_bounds__(64 * kRows) void k_gate_accum(const double* __restrict__ dpart, int nb, int ng, double f,
-                                                           double* __restrict__ gsum) {
+                                                           int add, double* __restrict__ gsum,
+                                                           double* __restrict__ host) {
   const int lane = threadIdx.x & 63, i = blockIdx.x * kRows + (threadIdx.x >> 6);
   if (i >= ng) return;
   double s = 0.0;
   for (int b = lane; b < nb; b += 64) s += dpart[(size_t)b * ng + i];
   for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) gsum[i] += f * s;
+  if (lane != 0) return;
+  s = f * s + (add ? gsum[i] : 0.0);
+  gsum[i] = s;
+  if (host) host[i] = s;
 }
 
 // w[t] = theta[gate of term t]
@@ -593,15 +689,9 @@ __global__ void k_zero(double* __restrict__ x, int64_t n) {
   if (i < n) x[i] = 0.0;
 }
 
-// A fixed pseudo-random start vector in [-1, 1) (integer hash of the index).
 __global__ void k_fill_pattern(double* __restrict__ x, int64_t n) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint64_t h = (uint64_t)i * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
-  h ^= h >> 31;
-  h *= 0xBF58476D1CE4E5B9ull;
-  h ^= h >> 29;
-  x[i] = (double)(h >> 11) * (2.0 / 9007199254740992.0) - 1.0;
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < n) x[i] = pattern_at(i);
 }
 
 __global__ void k_scale(double* __restrict__ x, int64_t n, const double* __restrict__ s, int slot) {
@@ -686,17 +776,20 @@ void ucc_csr_free(UccCsr* c) {
 struct UccT {
   int64_t nu = 0;             // merged elements
   int ncoef = 0;
-  int lpr = 64;               // lanes per row of k_spmv
+  int lpr = 32;               // lanes per row of k_spmv
   int64_t* urow = nullptr;    // [dim + 1]
   uint32_t* col = nullptr;    // [nu]
   uint32_t* first = nullptr;  // [nu + 1]
   uint32_t* con = nullptr;    // [entries]
   double* coefs = nullptr;    // [ncoef]
   double* val = nullptr;      // [nu]
+  int* count = nullptr;       // blocks done of k_norms, zero between launches
+  double* host = nullptr;     // pinned: norms [3] | energy | gradient
   std::mutex mu;
   hipEvent_t busy = nullptr;
   ~UccT() {
-    for (void* p : {(void*)urow, (void*)col, (void*)first, (void*)con, (void*)coefs, (void*)val})
+    if (host) (void)hipHostFree(host);
+    for (void* p : {(void*)count, (void*)urow, (void*)col, (void*)first, (void*)con, (void*)coefs, (void*)val})
       if (p) (void)hipFree(p);
     if (busy) (void)hipEventDestroy(busy);
   }
@@ -807,13 +900,18 @@ static UccT* ucc_t(const Space& s, const Program& p, hipStream_t st) {
   for (size_t i = 0; i < hc.size(); ++i) urow[i + 1] = urow[i] + hc[i];
   T->nu = urow.back();
   T->ncoef = (int)coefs.size();
-  T->lpr = T->nu <= 32 * s.dim ? 16 : T->nu <= 64 * s.dim ? 32 : 64;
+  T->lpr = T->nu <= 32 * s.dim ? 16 : 32;
   SQ_HIP(hipMalloc(&T->urow, sizeof(int64_t) * urow.size()));
   SQ_HIP(hipMalloc(&T->col, sizeof(uint32_t) * (size_t)T->nu));
   SQ_HIP(hipMalloc(&T->first, sizeof(uint32_t) * ((size_t)T->nu + 1)));
   SQ_HIP(hipMalloc(&T->con, sizeof(uint32_t) * (size_t)c->nnz));
   SQ_HIP(hipMalloc(&T->coefs, sizeof(double) * coefs.size()));
   SQ_HIP(hipMalloc(&T->val, sizeof(double) * (size_t)T->nu));
+  SQ_HIP(hipMalloc(&T->count, sizeof(double)));
+  k_zero<<<1, 1, 0, st>>>(reinterpret_cast<double*>(T->count), 1);
+  SQ_HIP(hipGetLastError());
+  SQ_HIP(hipHostMalloc(reinterpret_cast<void**>(&T->host), sizeof(double) * (4 + (size_t)ng),
+                       hipHostMallocPortable | hipHostMallocCoherent));
   SQ_HIP(hipEventCreateWithFlags(&T->busy, hipEventDisableTiming));
   SQ_HIP(hipMemcpyAsync(T->urow, urow.data(), sizeof(int64_t) * urow.size(), hipMemcpyHostToDevice, st));
   SQ_HIP(hipMemcpyAsync(T->coefs, coefs.data(), sizeof(double) * coefs.size(), hipMemcpyHostToDevice, st));
@@ -1152,8 +1250,8 @@ struct UccUse {
 
 static void spmv(const Space& s, const UccT& T, const double* cur, const double* prev, double f, const double* bound,
                  double* nxt, hipStream_t st, const double* cur2 = nullptr, double* nxt2 = nullptr) {
-  auto* kernel = cur2 ? (T.lpr == 16 ? k_spmv<16, true> : T.lpr == 32 ? k_spmv<32, true> : k_spmv<64, true>)
-                      : (T.lpr == 16 ? k_spmv<16, false> : T.lpr == 32 ? k_spmv<32, false> : k_spmv<64, false>);
+  auto* kernel = cur2 ? (T.lpr == 16 ? k_spmv<16, true> : k_spmv<32, true>)
+                      : (T.lpr == 16 ? k_spmv<16, false> : k_spmv<32, false>);
   const int64_t rows = kUB / T.lpr;
   SQ_PROF(PC_TAPPLY, st, (cur2 ? 32.0 : 16.0) * (double)s.dim + 12.0 * (double)T.nu, 0.0,
           kernel<<<(unsigned)((s.dim + rows - 1) / rows), kUB, 0, st>>>(s.dim, T.urow, T.col, T.val, cur, cur2, prev, f,
@@ -1188,9 +1286,10 @@ static void series_basis(const Space& s, const UccT& T, const Series& S, int fro
   }
 }
 
-// nodes[I][q] = f_q exp(t_q T) in (q < n) and fin = exp(tfin T) in.
+// nodes[I][q] = f_q exp(t_q T) in (q < n) and fin = exp(tfin T) in; the last
+// launch clears zero.
 static void series_combine(const Space& s, const Series& S, int n, const double* t, const double* f, double* nodes,
-                           double tfin, double* fin, const ChebWork& u, hipStream_t st) {
+                           double tfin, double* fin, const ChebWork& u, hipStream_t st, double* zero = nullptr) {
   for (int q0 = 0; q0 == 0 || q0 < n; q0 += kMaxOut - 1) {
     Combine C{};
     const int nq = std::min(kMaxOut - 1, n - q0);
@@ -1198,7 +1297,8 @@ static void series_combine(const Space& s, const Series& S, int n, const double*
     double* out = q0 == 0 ? fin : nullptr;
     if (out) S.coefs(tfin, 1.0, C.c[kMaxOut - 1]);
     SQ_PROF(PC_OTHER, st, 8.0 * (double)s.dim * (S.K + 1 + nq + 1), 0.0,
-            k_combine<<<(unsigned)((s.dim + kCB - 1) / kCB), kCB, 0, st>>>(s.dim, S.K, C, nq, u.basis, nodes + q0, n, out));
+            k_combine<<<(unsigned)((s.dim + kCB - 1) / kCB), kCB, 0, st>>>(s.dim, S.K, C, nq, u.basis, nodes + q0, n, out,
+                                                                       q0 + kMaxOut - 1 >= n ? zero : nullptr));
   }
 }
 
@@ -1211,23 +1311,21 @@ static Series series_start(const Space& s, const Program& p, const UccT& T, cons
   const unsigned nb = (unsigned)row_blocks(s, kAsmBlocks);
   SQ_PROF(PC_OTHER, st, 12.0 * (double)T.nu, 0.0,
           k_assemble<<<nb, 64 * kRows, ng <= kLdsGates ? 8 * (size_t)ng : 0, st>>>(
-              s.dim, T.urow, T.first, T.con, T.coefs, T.ncoef, theta, ng, T.val, u.rmax));
+              s.dim, T.urow, T.first, T.con, T.coefs, T.ncoef, theta, ng, T.val, u.rmax, v, u.basis, u.C));
   k_max<<<1, kUB, 0, st>>>(u.rmax, (int)nb, u.scal);
-  copy_vec(v, u.basis, s.dim, st);
+  SQ_HIP(hipGetLastError());
   double* x = u.C;
   double* y = u.D;
-  k_fill_pattern<<<(unsigned)((s.dim + kUB - 1) / kUB), kUB, 0, st>>>(x, s.dim);
-  SQ_HIP(hipGetLastError());
   for (int k = 1; k <= kNormSteps; ++k) {
     double* n = u.basis + (size_t)k * s.dim;
     spmv(s, T, n - s.dim, nullptr, 1.0, u.scal, n, st, x, y);
     std::swap(x, y);
   }
-  dot_dev(y, y, s.dim, u.scal, 1, 1.0, u.rmax, st);
-  dot_dev(x, x, s.dim, u.scal, 2, 1.0, u.rmax, st);
-  double d[3];
-  SQ_HIP(hipMemcpyAsync(d, u.scal, 3 * sizeof(double), hipMemcpyDeviceToHost, st));
+  k_norms<<<(unsigned)std::min<int64_t>((s.dim + kUB - 1) / kUB, 256), kUB, 0, st>>>(y, x, s.dim, u.scal, u.rmax,
+                                                                                  T.count, T.host);
+  SQ_HIP(hipGetLastError());
   SQ_HIP(hipStreamSynchronize(st));
+  const double* d = T.host;
   Series S{};
   S.bound = S.nu = d[0];
   if (!std::isfinite(d[0])) S.bound = S.nu = 1.0;  // the result is NaN whatever the series
@@ -1257,8 +1355,8 @@ static void series_expm(const Space& s, const UccT& T, const Series& S, int m, i
   }
 }
 
-static void gate_dots(const Space& s, const UccT& T, int n, int ng, const ChebWork& u, double* grad_dev,
-                      hipStream_t st) {
+static void gate_dots(const Space& s, const UccT& T, int n, int ng, const ChebWork& u, bool add, double* grad_dev,
+                      double* grad_host, hipStream_t st) {
   const bool lds = ng <= kLdsGates;
   const unsigned nb = (unsigned)row_blocks(s, 1024);
   auto* kernel = n == 8 ? k_gate_dots_rows<8> : n == 12 ? k_gate_dots_rows<12> : k_gate_dots_rows<16>;
@@ -1267,57 +1365,67 @@ static void gate_dots(const Space& s, const UccT& T, int n, int ng, const ChebWo
           kernel<<<nb, 64 * kRows, lds ? 8 * (size_t)ng : 0, st>>>(s.dim, T.urow, T.col, T.first, T.con, T.coefs, T.ncoef,
                                                                  u.U, u.V, ng, lds ? 1 : 0, u.dpart));
   k_gate_accum<<<(unsigned)((ng + kRows - 1) / kRows), 64 * kRows, 0, st>>>(u.dpart, lds ? (int)nb : 1, ng, 1.0,
-                                                                          grad_dev);
+                                                                          add ? 1 : 0, grad_dev, grad_host);
   SQ_HIP(hipGetLastError());
 }
 
-// Energy (scal[0]) and gradient (grad_dev, may be nullptr) through the merged
+// Energy and gradient (grad may be nullptr; gdev: ng doubles) through the merged
 // pattern.  grad_i = 2 int_0^1 <e^{-sT} lam | T_i | e^{-sT} psi> ds, and
 // e^{-sT} psi = e^{(1-s)T} psi0: one interval while nu <= the limit, with psi's
 // nodes from the forward series; else m intervals, both states propagated
-// back through them.
+// back through them.  With one interval and a sigma that adds into a zeroed
+// vector, the last launch of the forward series clears basis[0] and sigma
+// writes lam there.
 static void cheb_energy_grad(const Space& s, const Program& p, UccT& T, const Hamiltonian& H, const double* theta,
-                             const double* psi0, double* psi, double* lam, double* scal, double* grad_dev,
+                             const double* psi0, double* psi, double* lam, double* gdev, double* energy, double* grad,
                              double* work, hipStream_t st) {
   UccUse use(T, st);
   const ChebWork u = carve_cheb(s, work);
   const int ng = (int)p.gates.size();
+  double *e_host = T.host + 3, *g_host = T.host + 4;
   int m, done;
   const Series S = series_start(s, p, T, theta, psi0, 1.0, u, &m, &done, st);
   const double r = S.nu / m;
   const int n = r <= 2.0 ? 8 : r <= 5.5 ? 12 : 16;
   const GaussRule& R = gauss_rule(n);
   double t[16], f[16];
+  const bool direct = m == 1 && sigma_wants_zero(s, H);
   if (m == 1) {
     series_basis(s, T, S, done, u, st);
     for (int q = 0; q < n; ++q) t[q] = 1.0 - R.x[q];
-    series_combine(s, S, grad_dev ? n : 0, t, nullptr, u.U, 1.0, psi, u, st);
+    series_combine(s, S, grad ? n : 0, t, nullptr, u.U, 1.0, psi, u, st, direct ? u.basis : nullptr);
   } else {
     series_expm(s, T, S, m, done, 1.0, psi, u, st);
   }
-  sigma_energy_dev(s, H, psi, lam, scal, u.basis, st);
-  if (!grad_dev) return;
-  k_zero<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(grad_dev, ng);
-  SQ_HIP(hipGetLastError());
-  for (int q = 0; q < n; ++q) {
-    t[q] = -R.x[q] / m;
-    f[q] = 2.0 * R.w[q] / m;
-  }
-  const double* c = psi;
-  const double* d = lam;
-  for (int j = 0; j < m; ++j) {
-    if (m > 1) {
-      copy_vec(c, u.basis, s.dim, st);
-      series_basis(s, T, S, 0, u, st);
-      series_combine(s, S, n, t, nullptr, u.U, -1.0 / m, u.C, u, st);
-      c = u.C;
+  if (direct) lam = u.basis;
+  double* epart = nullptr;
+  // sigma's work: from the nodes of lam on where lam is basis[0]
+  const int64_t ne = sigma_partials_dev(s, H, psi, lam, direct ? u.V : u.basis, &epart, direct, st);
+  reduce_impl(epart, ne, e_host, 0, false, 1.0, st);
+  if (grad) {
+    for (int q = 0; q < n; ++q) {
+      t[q] = -R.x[q] / m;
+      f[q] = 2.0 * R.w[q] / m;
     }
-    copy_vec(d, u.basis, s.dim, st);
-    series_basis(s, T, S, 0, u, st);
-    series_combine(s, S, n, t, f, u.V, -1.0 / m, j + 1 < m ? u.D : nullptr, u, st);
-    d = u.D;
-    gate_dots(s, T, n, ng, u, grad_dev, st);
+    const double* c = psi;
+    const double* d = lam;
+    for (int j = 0; j < m; ++j) {
+      if (m > 1) {
+        copy_vec(c, u.basis, s.dim, st);
+        series_basis(s, T, S, 0, u, st);
+        series_combine(s, S, n, t, nullptr, u.U, -1.0 / m, u.C, u, st);
+        c = u.C;
+      }
+      copy_vec(d, u.basis, s.dim, st);
+      series_basis(s, T, S, 0, u, st);
+      series_combine(s, S, n, t, f, u.V, -1.0 / m, j + 1 < m ? u.D : nullptr, u, st);
+      d = u.D;
+      gate_dots(s, T, n, ng, u, j > 0, gdev, j + 1 == m ? g_host : nullptr, st);
+    }
   }
+  SQ_HIP(hipStreamSynchronize(st));
+  *energy = *e_host;
+  if (grad) std::memcpy(grad, g_host, sizeof(double) * ng);
 }
 
 // out = exp(t T(theta)) in.  work: ucc_work_doubles.
@@ -1361,8 +1469,8 @@ static void ucc_grad_impl(const Space& s, const Program& p, const UccWork& u, do
       expm_apply(s, p, u, nu, -ds, u.D, u.D, st);
       prev = node;
       k_gate_dots<<<dgrid, kUB, 0, st>>>(sv(s), p.d_terms, term_fast(p), p.d_gates, ng, u.C, u.D, u.dpart);
-      k_gate_accum<<<(unsigned)((ng + kRows - 1) / kRows), 64 * kRows, 0, st>>>(u.dpart, nb, ng, 2.0 * R.w[q] / m,
-                                                                             grad_dev);
+      k_gate_accum<<<(unsigned)((ng + kRows - 1) / kRows), 64 * kRows, 0, st>>>(u.dpart, nb, ng, 2.0 * R.w[q] / m, 1,
+                                                                             grad_dev, nullptr);
       SQ_HIP(hipGetLastError());
     }
   }
@@ -1402,7 +1510,8 @@ int sq_ucc_energy_grad(const sq_space* sp, const sq_program* pr, const sq_hamilt
     double* gdev = scal + 64;              // ng
     double* rest = gdev + std::max(ng, 1) + 64;
     if (UccT* T = ucc_t(s, p, st)) {
-      cheb_energy_grad(s, p, *T, H->h, theta, psi0, psi, lam, scal, grad && ng ? gdev : nullptr, rest, st);
+      cheb_energy_grad(s, p, *T, H->h, theta, psi0, psi, lam, gdev, energy, grad && ng ? grad : nullptr, rest, st);
+      return;
     } else {
       const UccWork u = carve_ucc(s, p, rest);
       const std::vector<double> th = theta_host(p, theta, st);
