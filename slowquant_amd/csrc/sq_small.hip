@@ -6,16 +6,20 @@
 // A gate outside the brick-wall layouts (factorised UCC: excitations between
 // any orbitals) touches a few hundred determinant pairs of a small space, far
 // too few to fill a launch: one launch per gate and direction is launch
-// latency and nothing else ((8e,8o) fUCCSD: 361 gates, 1080 launches of
-// 2-4 us, 4.0 ms per energy and gradient).  Here one block of 1024 threads
+// latency and nothing else ((8e,8o) fUCCSD: 360 gates, 1078 launches of
+// 2-4 us, 4.0 ms per energy and gradient).  Here one block of 512 threads
 // holds psi (and lambda in the reverse sweep) in LDS and runs every gate, one
 // barrier per gate.
 //
 //   * A rotation (GC_ROT, each half of GC_SA_SINGLE) is a list of determinant
 //     pairs, built once per program on the host: 13-bit indices i, j and the
 //     sign, one 32-bit word per pair.  The words of a gate are loaded two
-//     gates ahead into registers and the barrier waits for LDS only, so their
-//     L2 latency is off the chain.
+//     gates ahead into registers, by every thread on every path, so that the
+//     number in flight is known at each wait and their L2 latency is off the
+//     chain (loaded under a condition, each step waited for the words of the
+//     next: (8e,8o) forward sweep 146 -> 126 us, reverse 260 -> 206).  512
+//     threads: fewer idle waves to issue for (an evaluation 1024: 414 us, 512:
+//     359, 256: 400).
 //   * The other gates are polynomials in T (multi-frequency spin-adapted
 //     doubles).  T couples a determinant to few others: its connected
 //     components have at most kMaxComp members.  Members are ordered by their
@@ -26,15 +30,17 @@
 //       D_f = sum_{k odd} K_kf T_c^k,  C_f = sum_{k even} K_kf T_c^k
 //     with the polynomial's frequencies S_f and coefficients K; D_f and C_f
 //     are summed on the host in long double.  T_c is antisymmetric, so the
-//     inverse gate is the transpose.
-//     (eight to ten passes of every term over every determinant per
-//     polynomial gate and vector before).
+//     inverse gate is the transpose.  The matrices of a chunk of gates are
+//     made at once in the LDS that psi and lambda leave ((6e,6o) spin-adapted:
+//     228 -> 187 us an evaluation; gate by gate their two dependent loads were
+//     half of a step).  (The per-gate kernels take eight to ten passes of every
+//     term over every determinant per polynomial gate and vector.)
 //   * The gradient 2 <lambda|T psi> of a gate is summed per thread, reduced
 //     in each wave and added over the waves by one of them during the next
 //     gate: no extra barrier.
 //
 // Energy and gradient, per-gate kernels -> this sweep: fUCCSD (8e,8o) 3.86 ->
-// 0.46 ms, spin-adapted fUCCSD (6e,6o) 11.1 -> 0.36 ms.
+// 0.36 ms, spin-adapted fUCCSD (6e,6o) 11.1 -> 0.19 ms.
 
 #include <algorithm>
 #include <cmath>
@@ -48,7 +54,7 @@ namespace sq {
 
 namespace {
 
-constexpr int kST = 1024;                 // threads of the one block
+constexpr int kST = 512;                  // threads of the one block
 constexpr int kSW = kST / 64;             // its waves
 constexpr int kSmallDim = 8192;           // 13-bit determinant indices
 constexpr int kMaxComp = 8;               // members of a component of T
@@ -58,10 +64,16 @@ constexpr int kDiag = 1 << 16;            // flag of a diagonal matrix element
 constexpr size_t kSmallLds = 160 * 1024 - 1024;
 
 // One step: a rotation half (nf = 0: pair words [e0, e0 + n)) or a polynomial
-// gate (components [e0, e0 + n), its matrix elements [m0, m0 + mn)).  slot:
-// first trig slot within the step's chunk.
+// gate (components [e0, e0 + n), its matrix elements from m0 in the chunk's).
+// slot: first trig slot within the step's chunk.
 struct SmallStep {
-  int32_t gate, nf, e0, n, slot, m0, mn, pad;
+  int32_t gate, nf, e0, n, slot, m0, pad[2];
+};
+
+// A matrix element of a gate: its place in the type's coefficients, their
+// stride (| kDiag), the gate's first trig slot and its frequencies.
+struct MatElem {
+  int32_t off, stride, slot, nf;
 };
 
 struct TrigSlot {
@@ -70,7 +82,7 @@ struct TrigSlot {
 };
 
 struct SmallChunk {
-  int32_t s0, s1, t0, t1;  // steps [s0, s1), trig slots [t0, t1)
+  int32_t s0, s1, t0, t1, m0, m1;  // steps [s0, s1), trig slots [t0, t1), matrix elements [m0, m1)
 };
 
 }  // namespace
@@ -84,7 +96,7 @@ struct SmallPlan {
   uint32_t* pairs = nullptr;
   uint4* members = nullptr;  // per component kMaxComp x (index | negative << 15)
   uint32_t* meta = nullptr;  // per component: size | matrix offset << 8
-  int2* mel = nullptr;       // per matrix element of a gate: {offset into ctab, stride | kDiag}
+  MatElem* mel = nullptr;
   double* ctab = nullptr;    // per type: T | D_0 | C_0 | D_1 | ...
   uint8_t* nograd = nullptr; // per gate: 1 where the generator is zero (gradient 0)
   int ngates = 0;
@@ -110,7 +122,13 @@ T* put(const std::vector<T>& v) {
 
 size_t small_lds(int64_t dim, int maxmat, bool rev) {
   return (size_t)(dim + 1) / 2 * 16 * (rev ? 2 : 1) + (size_t)kChunk * (sizeof(double2) + sizeof(SmallStep) + 8) +
-         (size_t)maxmat * 8 * (rev ? 4 : 2);
+         (size_t)maxmat * 8 * (rev ? 2 : 1);
+}
+
+// Matrix elements per chunk: what the reverse sweep's LDS leaves, at most 64 KB.
+int mat_room(int64_t dim) {
+  const size_t base = small_lds(dim, 0, true);
+  return base >= kSmallLds ? 0 : (int)std::min<size_t>((kSmallLds - base) / 16, 4096);
 }
 
 // A type of component: its size, polynomial and matrix.
@@ -128,7 +146,7 @@ struct Builder {
   std::vector<TrigSlot> slots;
   std::vector<uint32_t> pairs, meta;
   std::vector<uint4> members;
-  std::vector<int2> mel;
+  std::vector<MatElem> mel;
   std::vector<double> ctab;
   std::vector<uint8_t> nograd;
   std::vector<CompType> types;
@@ -153,17 +171,21 @@ struct Builder {
     }
   }
 
-  // Opens a chunk when the running one has no room for a step of nt slots.
-  int open(int nt) {
+  // Opens a chunk when the running one has no room for a step of nt slots and
+  // nm matrix elements.
+  int open(int nt, int nm = 0) {
     if (chunks.empty() || chunks.back().s1 - chunks.back().s0 >= kChunk ||
-        chunks.back().t1 - chunks.back().t0 + nt > kChunk) {
-      const int s = (int)steps.size(), t = (int)slots.size();
-      chunks.push_back(SmallChunk{s, s, t, t});
+        chunks.back().t1 - chunks.back().t0 + nt > kChunk ||
+        chunks.back().m1 - chunks.back().m0 + nm > mat_room(sp.dim)) {
+      const int s = (int)steps.size(), t = (int)slots.size(), m = (int)mel.size();
+      chunks.push_back(SmallChunk{s, s, t, t, m, m});
     }
     SmallChunk& c = chunks.back();
     const int slot = c.t1 - c.t0;
     c.s1 += 1;
     c.t1 += nt;
+    c.m1 += nm;
+    maxmat = std::max(maxmat, c.m1 - c.m0);
     return slot;
   }
 
@@ -173,7 +195,7 @@ struct Builder {
     const int n = (int)pairs.size() - e0;
     const int slot = open(1);
     slots.push_back(TrigSlot{scale, g, 0});
-    steps.push_back(SmallStep{g, 0, e0, n, slot, 0, 0, 0});
+    steps.push_back(SmallStep{g, 0, e0, n, slot, 0, {0, 0}});
   }
 
   int type_of(int m, int slot, const std::vector<double>& T, const GatePoly& poly) {
@@ -298,15 +320,16 @@ struct Builder {
       c.type = type_of(c.m, gd.kind * 16 + gd.poly, S, poly);
     }
     std::stable_sort(comps.begin(), comps.end(), [](const Comp& a, const Comp& b) { return a.type < b.type; });
-    const int m0 = (int)mel.size(), c0 = (int)meta.size();
+    const int c0 = (int)meta.size();
     int moff = -1, last = -1, used = 0;
+    std::vector<MatElem> own;
     for (const Comp& c : comps) {
       const CompType& t = types[c.type];
       if (c.type != last) {
         last = c.type;
         moff = used;
         for (int e = 0; e < t.m * t.m; ++e)
-          mel.push_back(int2{t.off + e, t.m * t.m | (e % (t.m + 1) == 0 ? kDiag : 0)});
+          own.push_back(MatElem{t.off + e, t.m * t.m | (e % (t.m + 1) == 0 ? kDiag : 0), 0, poly.nf});
         used += t.m * t.m;
       }
       uint16_t w[kMaxComp] = {0};
@@ -316,10 +339,12 @@ struct Builder {
       members.push_back(make_uint4(two(0), two(2), two(4), two(6)));
       meta.push_back((uint32_t)c.m | (uint32_t)moff << 8);
     }
-    maxmat = std::max(maxmat, used);
-    const int slot = open(poly.nf);
+    const int slot = open(poly.nf, used);
+    const int m0 = (int)mel.size() - chunks.back().m0;
+    for (MatElem& e : own) e.slot = slot;
+    mel.insert(mel.end(), own.begin(), own.end());
     for (int f = 0; f < poly.nf; ++f) slots.push_back(TrigSlot{poly.S[f], g, 0});
-    steps.push_back(SmallStep{g, poly.nf, c0, (int)comps.size(), slot, m0, used, 0});
+    steps.push_back(SmallStep{g, poly.nf, c0, (int)comps.size(), slot, m0, {0, 0}});
     return true;
   }
 
@@ -352,18 +377,20 @@ struct SmallDev {
   const uint32_t* pairs;
   const uint4* members;
   const uint32_t* meta;
-  const int2* mel;
+  const MatElem* mel;
   const double* ctab;
   const uint8_t* nograd;
   int nchunks, dim, maxmat, ngates;
 };
 
+constexpr int kAhead = 3;  // pairs of a step that a thread loads ahead
+
 // What a thread needs of a step, loaded ahead: the step's record and trig
-// values, and its first two pairs or its first component.
+// values, and its first pairs or its first component.
 struct Ahead {
-  int gate, nf, e0, n;
+  int gate, nf, e0, n, m0;
   double c, sn, scale;
-  uint32_t p0, p1, meta;
+  uint32_t p[kAhead], meta;
   uint4 mem;
 };
 
@@ -374,10 +401,10 @@ __device__ __forceinline__ void lds_barrier() {
   __asm__ volatile("" ::: "memory");
 }
 
-template <int CTRL>
+template <int CTRL, int ROWS = 0xf>
 __device__ __forceinline__ double dpp_add(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, ROWS == 0xf);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, ROWS == 0xf);
   return v + __hiloint2double(hi, lo);
 }
 
@@ -387,6 +414,12 @@ __device__ __forceinline__ double row16_sum(double v) {
   v = dpp_add<0x4e>(v);   // quad_perm [2,3,0,1]
   v = dpp_add<0x114>(v);  // row_shr:4
   return dpp_add<0x118>(v);
+}
+
+// Sum over the wave, in lane 63 (no LDS round trip: shuffles took two).
+__device__ __forceinline__ double wave_sum63(double v) {
+  v = dpp_add<0x142, 0xa>(row16_sum(v));  // row_bcast:15 into rows 1 and 3
+  return dpp_add<0x143, 0xc>(v);          // row_bcast:31 into rows 2 and 3
 }
 
 // The matrix of one component (M: the gate, T: its generator, both m x m at
@@ -460,8 +493,8 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* _
   double2* cs = reinterpret_cast<double2*>(L + dimp);
   SmallStep* steps = reinterpret_cast<SmallStep*>(cs + kChunk);
   double* scales = reinterpret_cast<double*>(steps + kChunk);
-  double* mats = scales + kChunk;  // [2][maxmat] gate matrices | [2][maxmat] generators
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double* mats = scales + kChunk;  // the chunk's gate matrices, [maxmat] | their generators
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool inv = REV || back;
   for (int i = tid; i < S.dim; i += kST) {
     X[i] = src[i];
@@ -473,7 +506,9 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* _
   // the running sum of the gate whose steps are being reduced
   int par = 0;
   int done_gate = -1;   // gate of the previous step
+  int done_waves = 0;   // its waves with pairs or components
   double done_sum = 0.0;
+  SmallStep next{};     // the record of the step after the next but one
   for (int ci = 0; ci < S.nchunks; ++ci) {
     const SmallChunk C = S.chunks[inv ? S.nchunks - 1 - ci : ci];
     __syncthreads();
@@ -483,71 +518,86 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* _
       const double th = theta[t.gate];
       double sn = 0.0, c = 1.0;
       if (fabs(th) >= 1e-28) sincos(t.scale * th, &sn, &c);
-      cs[i] = double2{c, sn};
+      cs[i] = double2{c, !POLY && inv ? -sn : sn};
       scales[i] = t.scale;
     }
     __syncthreads();
+    if (POLY) {
+      const int nm = C.m1 - C.m0;
+      constexpr int U = 4;
+      for (int e0 = tid; e0 < nm; e0 += U * kST) {
+        MatElem me[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) me[u] = S.mel[C.m0 + min(e0 + u * kST, nm - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const double* __restrict__ c = S.ctab + me[u].off;
+          const int mm = me[u].stride & (kDiag - 1);
+          double v = (me[u].stride & kDiag) ? 1.0 : 0.0;
+          for (int f = 0; f < me[u].nf; ++f) {
+            const double2 x = cs[me[u].slot + f];
+            v += x.y * c[(2 * f + 1) * mm] + (x.x - 1.0) * c[(2 * f + 2) * mm];
+          }
+          if (e0 + u * kST < nm) {
+            mats[e0 + u * kST] = v;
+            if (REV) mats[S.maxmat + e0 + u * kST] = c[0];
+          }
+        }
+      }
+    }
     const int ns = C.s1 - C.s0;
     auto step_at = [&](int k) { return inv ? ns - 1 - k : k; };
-    auto load = [&](int k, Ahead& a) {
-      if (k >= ns) return;
-      const SmallStep s = steps[step_at(k)];
-      a.gate = __builtin_amdgcn_readfirstlane(s.gate);
-      a.nf = __builtin_amdgcn_readfirstlane(s.nf);
-      a.e0 = __builtin_amdgcn_readfirstlane(s.e0);
-      a.n = __builtin_amdgcn_readfirstlane(s.n);
-      if (!POLY || a.nf == 0) {
-        const double2 x = cs[s.slot];
-        a.c = x.x;
-        a.sn = inv ? -x.y : x.y;
-        a.scale = scales[s.slot];
-        if (tid < a.n) a.p0 = S.pairs[a.e0 + tid];
-        if (tid + kST < a.n) a.p1 = S.pairs[a.e0 + tid + kST];
-      } else if (tid < a.n) {
-        a.meta = S.meta[a.e0 + tid];
-        a.mem = S.members[a.e0 + tid];
+    // A step's record is read from LDS one step before it is used, and what it
+    // points to is loaded two steps ahead: no LDS round trip but the
+    // amplitudes' own lies between two barriers.  Every load is issued on every
+    // path (the lists are padded, past the last step the last one again), so
+    // that a step waits for its own words and not for those of the next.
+    auto record = [&](int k) { return steps[step_at(min(k, ns - 1))]; };
+    auto load = [&](const SmallStep& r, Ahead& a) {
+      a.gate = __builtin_amdgcn_readfirstlane(r.gate);
+      a.nf = POLY ? __builtin_amdgcn_readfirstlane(r.nf) : 0;
+      a.e0 = __builtin_amdgcn_readfirstlane(r.e0);
+      a.n = __builtin_amdgcn_readfirstlane(r.n);
+      const double2 x = cs[r.slot];
+      a.c = x.x;
+      a.sn = POLY && inv ? -x.y : x.y;
+      if (REV) a.scale = scales[r.slot];
+      const uint32_t* __restrict__ p = S.pairs + (POLY && a.nf != 0 ? 0 : a.e0);
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) a.p[q] = p[tid + q * kST];
+      if (POLY) {
+        a.m0 = __builtin_amdgcn_readfirstlane(r.m0);
+        const int e = (a.nf != 0 ? a.e0 : 0) + tid;
+        a.meta = S.meta[e];
+        a.mem = S.members[e];
       }
     };
-    // the matrices of step k into buffer k & 1
-    auto matrices = [&](int k) {
-      if (!POLY || k >= ns) return;
-      const SmallStep& s = steps[step_at(k)];
-      const int nf = __builtin_amdgcn_readfirstlane(s.nf);
-      if (nf == 0) return;
-      const int mn = __builtin_amdgcn_readfirstlane(s.mn), m0 = __builtin_amdgcn_readfirstlane(s.m0);
-      const int sl = __builtin_amdgcn_readfirstlane(s.slot);
-      for (int e = tid; e < mn; e += kST) {
-        const int2 me = S.mel[m0 + e];
-        const double* c = S.ctab + me.x;
-        const int mm = me.y & (kDiag - 1);
-        double v = (me.y & kDiag) ? 1.0 : 0.0;
-        for (int f = 0; f < nf; ++f) {
-          const double2 x = cs[sl + f];
-          v += x.y * c[(2 * f + 1) * mm] + (x.x - 1.0) * c[(2 * f + 2) * mm];
-        }
-        mats[(k & 1) * S.maxmat + e] = v;
-        if (REV) mats[(2 + (k & 1)) * S.maxmat + e] = c[0];
-      }
+    struct Amps {
+      double xi, xj, li, lj;
     };
-    auto rotate = [&](uint32_t p, double c, double sn, double& dot) {
+    auto fetch = [&](uint32_t p, Amps& v) {
+      const int i = (int)(p & 8191u), j = (int)((p >> 13) & 8191u);
+      v.xi = X[i], v.xj = X[j];
+      if (REV) v.li = L[i], v.lj = L[j];
+    };
+    auto rotate = [&](uint32_t p, const Amps& v, double c, double sn, double& dot) {
       const int i = (int)(p & 8191u), j = (int)((p >> 13) & 8191u);
       const double sg = (p >> 31) ? -sn : sn;
-      const double xi = X[i], xj = X[j];
-      X[i] = c * xi - sg * xj;
-      X[j] = sg * xi + c * xj;
+      X[i] = c * v.xi - sg * v.xj;
+      X[j] = sg * v.xi + c * v.xj;
       if (REV) {
-        const double li = L[i], lj = L[j];
-        L[i] = c * li - sg * lj;
-        L[j] = sg * li + c * lj;
-        const double d = lj * xi - li * xj;
+        L[i] = c * v.li - sg * v.lj;
+        L[j] = sg * v.li + c * v.lj;
+        const double d = v.lj * v.xi - v.li * v.xj;
         dot += (p >> 31) ? -d : d;
       }
     };
-    // one wave adds the previous step's wave sums to its gate's gradient
+    // one wave (the last, which has the fewest pairs) adds the previous step's
+    // wave sums to its gate's gradient
     auto finish = [&](int gate_now) {
       if (!REV || done_gate < 0) return;
-      if (wave == 0) {
-        double v = lane < kSW ? red[par ^ 1][lane & (kSW - 1)] : 0.0;
+      if (wave == kSW - 1) {
+        double v = lane < done_waves ? red[par ^ 1][lane & (kSW - 1)] : 0.0;
         v = row16_sum(v);
         done_sum += v;
         if (gate_now != done_gate) {
@@ -559,36 +609,50 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* _
     auto step = [&](int k, Ahead& cur, Ahead& fill) {
       if (k >= ns) return;
       lds_barrier();
-      load(k + 2, fill);
       const int n = cur.n, gate = cur.gate, e0 = cur.e0;
       double dot = 0.0;
       if (!POLY || cur.nf == 0) {
-        if (tid < n) rotate(cur.p0, cur.c, cur.sn, dot);
-        if (tid + kST < n) rotate(cur.p1, cur.c, cur.sn, dot);
-        for (int i = tid + 2 * kST; i < n; i += kST) rotate(S.pairs[e0 + i], cur.c, cur.sn, dot);
+        Amps v[kAhead];
+        fetch(cur.p[0], v[0]);
+#pragma unroll
+        for (int q = 1; q < kAhead; ++q)
+          if (n > q * kST) fetch(cur.p[q], v[q]);
+        load(next, fill);
+        next = record(k + 3);
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q)
+          if (tid + q * kST < n) rotate(cur.p[q], v[q], cur.c, cur.sn, dot);
+        for (int i = tid + kAhead * kST; i < n; i += kST) {
+          const uint32_t p = S.pairs[e0 + i];
+          fetch(p, v[0]);
+          rotate(p, v[0], cur.c, cur.sn, dot);
+        }
         if (REV) dot *= cur.scale;
       } else {
-        const double* M = mats + (k & 1) * S.maxmat;
-        const double* T = mats + (2 + (k & 1)) * S.maxmat;
+        load(next, fill);
+        next = record(k + 3);
+        const double* M = mats + cur.m0;
+        const double* T = M + S.maxmat;
         if (tid < n) dot += comp_any<REV>(X, L, M, T, cur.meta, cur.mem, inv);
         for (int i = tid + kST; i < n; i += kST)
           dot += comp_any<REV>(X, L, M, T, S.meta[e0 + i], S.members[e0 + i], inv);
       }
-      matrices(k + 1);
       if (REV) {
         finish(gate);
-        dot = row16_sum(dot);
-        dot += __shfl_xor(dot, 16, 64);
-        dot += __shfl_xor(dot, 32, 64);
-        if (lane == 63) red[par][wave] = dot;
+        if (wave * 64 < n) {
+          dot = wave_sum63(dot);
+          if (lane == 63) red[par][wave] = dot;
+        }
         done_gate = gate;
+        done_waves = min((n + 63) >> 6, kSW);
         par ^= 1;
       }
     };
     Ahead a, b, c;
-    load(0, a);
-    load(1, b);
-    matrices(0);
+    load(record(0), a);
+    load(record(1), b);
+    next = record(2);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the loop's waits then count its own loads
     for (int k = 0; k < ns; k += 3) {
       step(k, a, c);
       step(k + 1, b, a);
@@ -597,8 +661,8 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* _
   }
   __syncthreads();
   if (REV) {
-    if (done_gate >= 0 && wave == 0) {
-      double v = lane < kSW ? red[par ^ 1][lane & (kSW - 1)] : 0.0;
+    if (done_gate >= 0 && wave == kSW - 1) {
+      double v = lane < done_waves ? red[par ^ 1][lane & (kSW - 1)] : 0.0;
       v = row16_sum(v);
       if (lane == 15) grad[done_gate] = 2.0 * (done_sum + v);
     }
@@ -626,13 +690,18 @@ const SmallPlan* small_for(const Space& s, const Program& p) {
     if (tiles_cover(s, p)) return nullptr;
     Builder B(s, p);
     if (!B.build()) return nullptr;
+    const bool poly = !B.meta.empty();
+    // a step's loads take whole blocks of words
+    B.pairs.resize(B.pairs.size() + kAhead * kST, 0u);
+    B.meta.resize(B.meta.size() + kST, 0u);
+    B.members.resize(B.members.size() + kST, uint4{0u, 0u, 0u, 0u});
     const size_t lds_rev = small_lds(s.dim, B.maxmat, true);
     if (lds_rev > kSmallLds) return nullptr;
     auto* P = new SmallPlan();
     try {
       P->nchunks = (int)B.chunks.size();
       P->maxmat = B.maxmat;
-      P->poly = !B.meta.empty();
+      P->poly = poly;
       P->steps = put(B.steps);
       P->chunks = put(B.chunks);
       P->slots = put(B.slots);
