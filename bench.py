@@ -18,7 +18,7 @@ The JSON line also carries:
                   on its stream over the timed steps themselves (only that
                   kernel is bracketed there: one event pair per launch)
   rotation        the forward sweep by per-gate rotation kernels and by
-                  the fused tile stages: each kernel's algorithmic bytes per
+                  the fused window stages: each kernel's algorithmic bytes per
                   launch over its average duration, as a fraction of HBM peak
   batch512        the 512-instance batched workload (one hipGraph-replayed
                   persistent launch) in instances/s, against a loop of
@@ -102,7 +102,7 @@ def measured_traffic(kernel_class):
 def rotation_profile(sp, lay, prog, theta, psi0):
     """The forward sweep U(theta) psi0 two ways: per-gate rotation kernels (a
     program built with SQ_TILES=0: one HBM pass per rotation string over the
-    amplitudes it touches) and the fused tile stages; for each, the kernel's
+    amplitudes it touches) and the fused window stages; for each, the kernel's
     algorithmic bytes over its duration as a fraction of HBM peak, and the
     ratio of the two sweep times."""
     from slowquant_amd import engine as E

@@ -133,7 +133,7 @@ int sq_sigma(const sq_space* s, const sq_hamiltonian* H, const double* psi, doub
 
 /* Kernel shape of sq_sigma's row path on space s; no counterpart in the
  * reference (its sigma has no kernel shapes).  rows_per_block: alpha rows per
- * block (0: automatic); nsplit: partial products of the alpha-string GEMM
+ * block (0: automatic); nsplit: partial products of the string products
  * (1..4, 0: automatic); deterministic: 1 selects the staged form whose sums
  * run in a fixed order (bit-identical results run to run), 0 the scatter form
  * (LDS atomics: equal to rounding, faster), -1 the SQ_SIGMA_DETERMINISTIC
@@ -143,7 +143,7 @@ int sq_sigma_configure(sq_space* s, int rows_per_block, int nsplit, int determin
 
 /* sigma = H psi with no allocation: no counterpart in the reference; for
  * callers that cannot allocate (code under HIP graph capture, tight serving
- * loops).  Same kernels as sq_sigma's row path, with its scratch (alpha GEMM
+ * loops).  Same kernels as sq_sigma's row path, with its scratch (string products
  * partials and block partials) in a 64 MiB device array that each GPU the
  * library runs on holds until the process ends; spaces needing more, or
  * above 4096 beta strings, fail with SQ_ERR_ARG.  energy: DEVICE double or
@@ -212,7 +212,7 @@ int sq_ucc_energy_grad(const sq_space* s, const sq_program* p, const sq_hamilton
  * persistent launch computes every instance's energy and adjoint gradient
  * from the HF determinant.  Programs may hold rotation gates only (single,
  * double, sa_single, pair doubles: tUPS / QNP / fUCC-SD layouts); spaces up
- * to 12 orbitals.  n_workgroups <= 0 picks 256.  Instances of 16384 or more
+ * to 12 orbitals.  n_workgroups <= 0 picks 256.  Instances of 4096 or more
  * determinants whose programs are all brick stages run instead in groups
  * of equal (space, gate layout) through the tile-stage, row-sigma and
  * gradient kernels with one grid row per instance (SQ_BATCH_GROUPS=0 keeps

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
 }
 
 // Large instances of one (space, gate layout) run together through the
-// single-instance kernels with an instance grid dimension (tile stages, row
+// single-instance kernels with an instance grid dimension (window stages, row
 // sigma, gradient): one persistent workgroup per instance would leave them
 // bound by one CU each.  Per-instance buffers are contiguous at fixed
 // strides.

@@ -3,7 +3,8 @@
 // one_/two_electron_integral_transform, integralfunctions.py:186-211;
 // get_orbital_gradient, density_matrix.py:181-230).
 //
-// Every contraction is one strided, batched FP64-MFMA GEMM (k_dgemm):
+// The contractions of the first two are strided, batched FP64-MFMA GEMMs
+// (k_dgemm; the gradient is k_kappa_grad, below):
 //   C[b](i,j) = alpha sum_k A[b](i,k) B[b](k,j) + beta C[b](i,j),
 // with element addresses base + b*bs + i*rs + j*cs for each operand, so
 // transposes and index permutations of the quarter transforms are strides.

@@ -479,7 +479,7 @@ __global__ __launch_bounds__(kUB) void k_norms(const double* __restrict__ y, con
 // elements of 12 bytes; without the gathers' misses or the 8-byte numbers it
 // takes as long), and by launch latency below about 10^5 elements.  So a row
 // gets half a wave: 64, 32 and 16 lanes 2464, 2140 and 2200 us an energy and
-// gradient of (10e,10o) UCCSD (U = 6); U = 1, 2, 4, 6: 2448, 2236, 2180, 2140
+// gradient of (10e,10o) UCCSD (U = 6); U = 1, 2, 4, 6: 2448, 2236, 2180, 2140.
 template <int LPR, bool TWO>
 __global__ __launch_bounds__(kUB) void k_spmv(int64_t dim, const int64_t* __restrict__ urow,
                                               const uint32_t* __restrict__ col, const double* __restrict__ val,

@@ -2,9 +2,9 @@
 
 Device counterparts of c_mo = C expm(-kappa) (ups_wavefunction.py:367-385),
 one_/two_electron_integral_transform (integralfunctions.py:186-211) and
-get_orbital_gradient (density_matrix.py:181-230).  Every contraction runs as
-an FP64-MFMA GEMM in libsqhip.so (sq_orbital_rotation, sq_ao2mo,
-sq_orbital_gradient); matrices are float64 CUDA tensors, row-major.
+get_orbital_gradient (density_matrix.py:181-230): sq_orbital_rotation and
+sq_ao2mo (FP64-MFMA GEMMs) and sq_orbital_gradient (one block per rotation) in
+libsqhip.so; matrices are float64 CUDA tensors, row-major.
 """
 
 from __future__ import annotations
