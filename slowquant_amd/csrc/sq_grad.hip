@@ -180,21 +180,24 @@ static void adjoint(const Space& s, const Program& p, const Hamiltonian& H, cons
     const int64_t ne = sigma_partials_dev(s, H, b.psi, b.lam, b.sigw, &epart, zero, st);
     tiles_reverse(s, p, *T, th, b.psi, b.lam, b.t1, b.partial, out + 64, true, st, epart, ne, out);
     slot.wait();
+  } else if (S) {
+    const bool zero = sigma_wants_zero(s, H);
+    small_forward(s, *S, on_host && n > 0 ? slot->theta : theta, psi0, b.psi, false, st, zero ? b.lam : nullptr,
+                  on_host && n > 0 ? slot->dev : nullptr);
+    double* epart = nullptr;
+    const int64_t ne = sigma_partials_dev(s, H, b.psi, b.lam, b.sigw, &epart, zero, st);
+    small_reverse(s, *S, th, b.psi, b.lam, out + 64, st, epart, ne, out);
+    slot.wait();
   } else {
     if (on_host && n > 0)
       SQ_HIP(hipMemcpyAsync(slot->dev, slot->theta, sizeof(double) * n, hipMemcpyHostToDevice, st));
     forward(s, p, th, psi0, b.psi, b, -1, st);
-    if (S) {
-      sigma_energy_dev(s, H, b.psi, b.lam, out, b.sigw, st);
-      small_reverse(s, *S, th, b.psi, b.lam, out + 64, st);
-    } else {
-      sigma_energy_dev(s, H, b.psi, b.lam, b.scal, b.sigw, st);
-      if (T)
-        tiles_reverse(s, p, *T, th, b.psi, b.lam, b.t1, b.partial, b.grad, true, st);  // matrices from forward()
-      else
-        for (int g = n - 1; g >= 0; --g) reverse_step_impl(s, p, g, th, b.psi, b.lam, b.grad, b.t1, b.partial, st);
-      SQ_HIP(hipMemcpyAsync(out, b.scal, sizeof(double) * (64 + (size_t)n), hipMemcpyDeviceToHost, st));
-    }
+    sigma_energy_dev(s, H, b.psi, b.lam, b.scal, b.sigw, st);
+    if (T)
+      tiles_reverse(s, p, *T, th, b.psi, b.lam, b.t1, b.partial, b.grad, true, st);  // matrices from forward()
+    else
+      for (int g = n - 1; g >= 0; --g) reverse_step_impl(s, p, g, th, b.psi, b.lam, b.grad, b.t1, b.partial, st);
+    SQ_HIP(hipMemcpyAsync(out, b.scal, sizeof(double) * (64 + (size_t)n), hipMemcpyDeviceToHost, st));
     slot.wait();
   }
   *energy = out[0];

@@ -305,11 +305,12 @@ bool tiles_cover(const Space& s, const Program& p);  // every gate runs in a til
 
 // Implemented in sq_small.hip: the whole sweep of a small space in one block
 const SmallPlan* small_for(const Space& s, const Program& p);  // nullptr where it does not apply
+// (zero, theta_out: as for tiles_forward; epart, e_out: as for tiles_reverse)
 void small_forward(const Space& s, const SmallPlan& P, const double* theta, const double* psi_in, double* psi,
-                   bool dagger, hipStream_t st);
-// reverse sweep on (psi, lam), left as they are; dE/dtheta to grad (device)
+                   bool dagger, hipStream_t st, double* zero = nullptr, double* theta_out = nullptr);
 void small_reverse(const Space& s, const SmallPlan& P, const double* theta, const double* psi, const double* lam,
-                   double* grad, hipStream_t st);
+                   double* grad, hipStream_t st, const double* epart = nullptr, int64_t n_epart = 0,
+                   double* e_out = nullptr);
 
 // Several instances of one (space, program) evaluated together (batched
 // groups, sq_batch.hip): the tile, gradient and row-sigma kernels run with

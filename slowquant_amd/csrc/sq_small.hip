@@ -477,14 +477,29 @@ __device__ __forceinline__ double comp_any(double* X, double* L, const double* M
   }
 }
 
+// What the launches of an energy and gradient call take along in further
+// blocks, instead of launches and copies of their own ((6e,6o) spin-adapted 186
+// -> 180 us an evaluation, (8e,8o) fUCCSD 358 -> 353): the forward sweep fills
+// zero[0, nzero) with zeros and copies host theta to theta_out, the reverse
+// sweep writes the sum of epart[0, nepart) to *e_out.
+struct SmallExtra {
+  double* zero = nullptr;
+  double* theta_out = nullptr;
+  const double* epart = nullptr;
+  double* e_out = nullptr;
+  int64_t nzero = 0, nepart = 0;
+};
+
+constexpr int kZeroBlocks = 4;
+
 // REV = false: dst = U src (back: U^+ src).  REV = true: the reverse sweep on
 // (src = psi, lam), gradients to grad; back is then true.
 // Bound by the chain of barriers and LDS round trips, one per gate: the block
 // uses one CU, and a gate's arithmetic is a few hundred cycles of it.
 template <bool REV, bool POLY>
-__global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* __restrict__ theta, const double* src,
+__global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* theta, const double* src,
                                                      double* dst, const double* __restrict__ lam,
-                                                     double* __restrict__ grad, int back) {
+                                                     double* __restrict__ grad, int back, SmallExtra ex) {
   extern __shared__ double smem[];
   __shared__ double red[2][kSW];
   double* X = smem;
@@ -496,6 +511,28 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* _
   double* mats = scales + kChunk;  // the chunk's gate matrices, [maxmat] | their generators
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool inv = REV || back;
+  if (blockIdx.x != 0) {
+    if (!REV) {
+      for (int64_t i = (int64_t)(blockIdx.x - 1) * kST + tid; i < ex.nzero; i += (int64_t)(gridDim.x - 1) * kST)
+        ex.zero[i] = 0.0;
+    } else {
+      double e = 0.0;
+      for (int64_t i = tid; i < ex.nepart; i += kST) e += ex.epart[i];
+      e = wave_sum63(e);
+      if (lane == 63) red[0][wave] = e;
+      __syncthreads();
+      if (tid == 0) {
+        e = 0.0;
+        for (int w = 0; w < kSW; ++w) e += red[0][w];
+        *ex.e_out = e;
+      }
+    }
+    return;
+  }
+  if (!REV && ex.theta_out) {
+    for (int g = tid; g < S.ngates; g += kST) ex.theta_out[g] = theta[g];
+    theta = ex.theta_out;  // read again after the barrier below
+  }
   for (int i = tid; i < S.dim; i += kST) {
     X[i] = src[i];
     if (REV) L[i] = lam[i];
@@ -724,21 +761,30 @@ const SmallPlan* small_for(const Space& s, const Program& p) {
 }
 
 void small_forward(const Space& s, const SmallPlan& P, const double* theta, const double* psi_in, double* psi,
-                   bool dagger, hipStream_t st) {
+                   bool dagger, hipStream_t st, double* zero, double* theta_out) {
   const SmallDev D = device_view(s, P);
+  SmallExtra ex;
+  ex.zero = zero;
+  ex.nzero = zero ? s.dim : 0;
+  ex.theta_out = theta_out;
   auto* kernel = P.poly ? k_small_sweep<false, true> : k_small_sweep<false, false>;
   allow_lds(kernel, P.lds_fwd);
   SQ_PROF(PC_SMALL, st, 16.0 * (double)s.dim, 0.0,
-          kernel<<<1, kST, P.lds_fwd, st>>>(D, theta, psi_in, psi, nullptr, nullptr, dagger ? 1 : 0));
+          kernel<<<zero ? 1 + kZeroBlocks : 1, kST, P.lds_fwd, st>>>(D, theta, psi_in, psi, nullptr, nullptr,
+                                                                    dagger ? 1 : 0, ex));
 }
 
 void small_reverse(const Space& s, const SmallPlan& P, const double* theta, const double* psi, const double* lam,
-                   double* grad, hipStream_t st) {
+                   double* grad, hipStream_t st, const double* epart, int64_t n_epart, double* e_out) {
   const SmallDev D = device_view(s, P);
+  SmallExtra ex;
+  ex.epart = epart;
+  ex.nepart = n_epart;
+  ex.e_out = e_out;
   auto* kernel = P.poly ? k_small_sweep<true, true> : k_small_sweep<true, false>;
   allow_lds(kernel, P.lds_rev);
   SQ_PROF(PC_SMALL, st, 16.0 * (double)s.dim, 0.0,
-          kernel<<<1, kST, P.lds_rev, st>>>(D, theta, psi, nullptr, lam, grad, 1));
+          kernel<<<e_out ? 2 : 1, kST, P.lds_rev, st>>>(D, theta, psi, nullptr, lam, grad, 1, ex));
 }
 
 }  // namespace sq
