@@ -25,7 +25,7 @@
 //     components have at most kMaxComp members.  Members are ordered by their
 //     occupation of the gate's orbitals and given signs that make the
 //     component's matrix T_c one of a handful per program, so that the gate
-//     is one small matrix-vector product per component, by one thread:
+//     is one small matrix-vector product per component, a thread per row:
 //       M_c(theta) = 1 + sum_f sin(S_f theta) D_f + (cos(S_f theta) - 1) C_f,
 //       D_f = sum_{k odd} K_kf T_c^k,  C_f = sum_{k even} K_kf T_c^k
 //     with the polynomial's frequencies S_f and coefficients K; D_f and C_f
@@ -33,14 +33,15 @@
 //     inverse gate is the transpose.  The matrices of a chunk of gates are
 //     made at once in the LDS that psi and lambda leave ((6e,6o) spin-adapted:
 //     228 -> 187 us an evaluation; gate by gate their two dependent loads were
-//     half of a step).  (The per-gate kernels take eight to ten passes of every
+//     half of a step; a thread per row instead of one per component, whose m x m
+//     products were one chain: 180 -> 123 us).  (The per-gate kernels take eight to ten passes of every
 //     term over every determinant per polynomial gate and vector.)
 //   * The gradient 2 <lambda|T psi> of a gate is summed per thread, reduced
 //     in each wave and added over the waves by one of them during the next
 //     gate: no extra barrier.
 //
 // Energy and gradient, per-gate kernels -> this sweep: fUCCSD (8e,8o) 3.86 ->
-// 0.36 ms, spin-adapted fUCCSD (6e,6o) 11.1 -> 0.19 ms.
+// 0.35 ms, spin-adapted fUCCSD (6e,6o) 11.1 -> 0.12 ms.
 
 #include <algorithm>
 #include <cmath>
@@ -64,7 +65,7 @@ constexpr int kDiag = 1 << 16;            // flag of a diagonal matrix element
 constexpr size_t kSmallLds = 160 * 1024 - 1024;
 
 // One step: a rotation half (nf = 0: pair words [e0, e0 + n)) or a polynomial
-// gate (components [e0, e0 + n), its matrix elements from m0 in the chunk's).
+// gate (rows of components [e0, e0 + n), its matrix elements from m0 in the chunk's).
 // slot: first trig slot within the step's chunk.
 struct SmallStep {
   int32_t gate, nf, e0, n, slot, m0, pad[2];
@@ -94,8 +95,8 @@ struct SmallPlan {
   SmallChunk* chunks = nullptr;
   TrigSlot* slots = nullptr;
   uint32_t* pairs = nullptr;
-  uint4* members = nullptr;  // per component kMaxComp x (index | negative << 15)
-  uint32_t* meta = nullptr;  // per component: size | matrix offset << 8
+  uint4* members = nullptr;  // per row of a component: its kMaxComp members (index | negative << 15)
+  uint32_t* meta = nullptr;  // and size | row << 4 | matrix offset << 8
   MatElem* mel = nullptr;
   double* ctab = nullptr;    // per type: T | D_0 | C_0 | D_1 | ...
   uint8_t* nograd = nullptr; // per gate: 1 where the generator is zero (gradient 0)
@@ -336,15 +337,22 @@ struct Builder {
       for (int a = 0; a < c.m; ++a)
         w[a] = (uint16_t)((uint32_t)touched[c.x0 + a] | ((c.neg >> a) & 1u) << 15);
       auto two = [&](int a) { return (uint32_t)w[a] | (uint32_t)w[a + 1] << 16; };
-      members.push_back(make_uint4(two(0), two(2), two(4), two(6)));
-      meta.push_back((uint32_t)c.m | (uint32_t)moff << 8);
+      if (c.m < 2) continue;
+      while (((int)meta.size() - c0) % 64 + c.m > 64) {  // the rows of a component stay in one wave
+        members.push_back(uint4{0u, 0u, 0u, 0u});
+        meta.push_back(0u);
+      }
+      for (int a = 0; a < c.m; ++a) {
+        members.push_back(make_uint4(two(0), two(2), two(4), two(6)));
+        meta.push_back((uint32_t)c.m | (uint32_t)a << 4 | (uint32_t)moff << 8);
+      }
     }
     const int slot = open(poly.nf, used);
     const int m0 = (int)mel.size() - chunks.back().m0;
     for (MatElem& e : own) e.slot = slot;
     mel.insert(mel.end(), own.begin(), own.end());
     for (int f = 0; f < poly.nf; ++f) slots.push_back(TrigSlot{poly.S[f], g, 0});
-    steps.push_back(SmallStep{g, poly.nf, c0, (int)comps.size(), slot, m0, {0, 0}});
+    steps.push_back(SmallStep{g, poly.nf, c0, (int)meta.size() - c0, slot, m0, {0, 0}});
     return true;
   }
 
@@ -362,7 +370,7 @@ struct Builder {
       } else if (!polynomial(g)) {
         return false;
       }
-      if (pairs.size() > kSmallEntries || meta.size() > kSmallEntries / 8) return false;
+      if (pairs.size() > kSmallEntries || meta.size() > kSmallEntries / 4) return false;
     }
     return true;
   }
@@ -386,7 +394,7 @@ struct SmallDev {
 constexpr int kAhead = 3;  // pairs of a step that a thread loads ahead
 
 // What a thread needs of a step, loaded ahead: the step's record and trig
-// values, and its first pairs or its first component.
+// values, and its first pairs or its first row of a component.
 struct Ahead {
   int gate, nf, e0, n, m0;
   double c, sn, scale;
@@ -422,58 +430,60 @@ __device__ __forceinline__ double wave_sum63(double v) {
   return dpp_add<0x143, 0xc>(v);          // row_bcast:31 into rows 2 and 3
 }
 
-// The matrix of one component (M: the gate, T: its generator, both m x m at
-// LDS) on its members; the transpose where inv.  Returns <lam|T psi> (REV).
+// One row of a component's matrix (M: the gate, T: its generator, both m x m in
+// LDS) on its members; the transpose where inv.  The rows of a component are
+// lanes of one wave, whose reads of the members all come before its writes.
+// Returns the row's part of <lam|T psi> (REV).
 template <int m, bool REV>
-__device__ __forceinline__ double comp_apply(double* X, double* L, const double* __restrict__ M,
-                                             const double* __restrict__ T, const uint4& mem, bool inv) {
+__device__ __forceinline__ double comp_row(double* X, double* L, const double* __restrict__ M,
+                                           const double* __restrict__ T, const uint4& mem, int row, bool inv) {
   const uint32_t w[4] = {mem.x, mem.y, mem.z, mem.w};
-  int at[m];
-  double s[m], x[m], l[m];
+  double x[m], l[m];
 #pragma unroll
   for (int a = 0; a < m; ++a) {
     const uint32_t h = (w[a >> 1] >> (16 * (a & 1))) & 0xffffu;
-    at[a] = (int)(h & 0x7fffu);
-    s[a] = (h & 0x8000u) ? -1.0 : 1.0;
-    x[a] = s[a] * X[at[a]];
-    if (REV) l[a] = s[a] * L[at[a]];
+    const double s = (h & 0x8000u) ? -1.0 : 1.0;
+    x[a] = s * X[h & 0x7fffu];
+    if (REV) l[a] = s * L[h & 0x7fffu];
   }
-  double dot = 0.0;
+  const uint64_t half = m > 4 && row >= 4 ? (uint64_t)w[2] | (uint64_t)w[3] << 32 : (uint64_t)w[0] | (uint64_t)w[1] << 32;
+  const uint32_t own = (uint32_t)(half >> (16 * (row & 3)));
+  const int at = (int)(own & 0x7fffu);
+  const double s = (own & 0x8000u) ? -1.0 : 1.0;
+  const double mine = REV ? s * L[at] : 0.0;
+  const double* Mr = M + (inv ? row : row * m);
+  const int step = inv ? m : 1;
+  double vx = 0.0, vl = 0.0, vt = 0.0;
 #pragma unroll
-  for (int a = 0; a < m; ++a) {
-    double vx = 0.0, vl = 0.0, vt = 0.0;
-#pragma unroll
-    for (int b = 0; b < m; ++b) {
-      const double e = inv ? M[b * m + a] : M[a * m + b];
-      vx += e * x[b];
-      if (REV) {
-        vl += e * l[b];
-        vt += T[a * m + b] * x[b];
-      }
-    }
-    X[at[a]] = s[a] * vx;
+  for (int b = 0; b < m; ++b) {
+    const double e = Mr[b * step];
+    vx += e * x[b];
     if (REV) {
-      L[at[a]] = s[a] * vl;
-      dot += l[a] * vt;
+      vl += e * l[b];
+      vt += T[row * m + b] * x[b];
     }
   }
-  return dot;
+  X[at] = s * vx;
+  if (REV) L[at] = s * vl;
+  return mine * vt;
 }
 
+// meta: size | row << 4 | matrix offset << 8.
 template <bool REV>
 __device__ __forceinline__ double comp_any(double* X, double* L, const double* M, const double* T, uint32_t meta,
                                            const uint4& mem, bool inv) {
   const double* Mc = M + (meta >> 8);
   const double* Tc = T + (meta >> 8);
-  switch (meta & 255u) {
-    case 2: return comp_apply<2, REV>(X, L, Mc, Tc, mem, inv);
-    case 3: return comp_apply<3, REV>(X, L, Mc, Tc, mem, inv);
-    case 4: return comp_apply<4, REV>(X, L, Mc, Tc, mem, inv);
-    case 5: return comp_apply<5, REV>(X, L, Mc, Tc, mem, inv);
-    case 6: return comp_apply<6, REV>(X, L, Mc, Tc, mem, inv);
-    case 7: return comp_apply<7, REV>(X, L, Mc, Tc, mem, inv);
-    case 8: return comp_apply<8, REV>(X, L, Mc, Tc, mem, inv);
-    default: return 0.0;  // a single member: T = 0
+  const int row = (int)((meta >> 4) & 15u);
+  switch (meta & 15u) {
+    case 2: return comp_row<2, REV>(X, L, Mc, Tc, mem, row, inv);
+    case 3: return comp_row<3, REV>(X, L, Mc, Tc, mem, row, inv);
+    case 4: return comp_row<4, REV>(X, L, Mc, Tc, mem, row, inv);
+    case 5: return comp_row<5, REV>(X, L, Mc, Tc, mem, row, inv);
+    case 6: return comp_row<6, REV>(X, L, Mc, Tc, mem, row, inv);
+    case 7: return comp_row<7, REV>(X, L, Mc, Tc, mem, row, inv);
+    case 8: return comp_row<8, REV>(X, L, Mc, Tc, mem, row, inv);
+    default: return 0.0;  // padding, or a single member: T = 0
   }
 }
 
@@ -543,7 +553,7 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* t
   // the running sum of the gate whose steps are being reduced
   int par = 0;
   int done_gate = -1;   // gate of the previous step
-  int done_waves = 0;   // its waves with pairs or components
+  int done_waves = 0;   // its waves with pairs or rows
   double done_sum = 0.0;
   SmallStep next{};     // the record of the step after the next but one
   for (int ci = 0; ci < S.nchunks; ++ci) {
