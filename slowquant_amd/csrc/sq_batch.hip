@@ -8,8 +8,9 @@
 // assigned on the host, no atomics).  Per instance, inside the workgroup:
 //   psi = HF;  forward rotations;  D build;  G = A.D with FP64 MFMA;
 //   sigma gather + energy;  reverse sweep with fused <lambda|T_i psi> dots.
-// State vectors and D/G live in a per-workgroup slot of global scratch
-// (L2-resident for the small spaces), so instances never interact.
+// psi and lambda live in LDS where all of the launch's instances fit beside A,
+// else, like G, in a per-workgroup slot of global scratch (L2-resident for the
+// small spaces), so instances never interact.
 // The launch can be captured in a hipGraph and replayed.
 
 #include <algorithm>
@@ -24,6 +25,9 @@
 namespace sq {
 
 constexpr int kBT = 512;    // threads per batch workgroup (8 waves)
+constexpr int kBW = kBT / 64;
+constexpr int kBRot = 128;  // rotations whose records and angles are staged in LDS at a time
+constexpr size_t kBatchLds = 160 * 1024 - kBRot * 64 - 1024;  // dynamic LDS of a workgroup
 constexpr int kBatchMT = 5;  // row tiles of the sigma GEMM (kpad <= 80: up to 12 orbitals)
 
 // k -> whether packed pair k = p(p+1)/2 + q is diagonal (p == q), k < 91
@@ -75,6 +79,7 @@ struct BatchDev {
   double* scratch;         // per-workgroup slots
   int64_t slot_doubles;
   int64_t dmax;
+  int64_t vec0;            // psi | lambda in the dynamic LDS from here (in doubles)
   double* energy;          // [ninst]
   double* grad;            // concatenated gradients
   const double* const* psi0;  // [ninst] start states (engine convention), nullptr: HF determinant
@@ -94,17 +99,6 @@ __device__ __forceinline__ void for_each_det(int nsa, int nsb, F&& f) {
 
 __device__ __forceinline__ int2 list_entry(const int2* lists, int off, int i) {
   return off < 0 ? int2{i, i} : lists[off + i];
-}
-
-__device__ double block_reduce(double v, double* red) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  double t = 0.0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
-  return t;  // every thread gets the sum
 }
 
 // One rotation half of the forward (REV = false) or reverse sweep over its
@@ -163,19 +157,28 @@ __device__ __forceinline__ double rotate_lists(const int2* __restrict__ lists, c
 
 // U: rotation pairs per thread in flight; CT: 16-column tiles per wave in the
 // sigma GEMM (sharing each LDS read of A).  Both are picked by the autotuner.
-template <int U, int CT>
+// LDS: psi and lambda at vec0 of the dynamic LDS.  The sweeps are a chain of one
+// rotation after the other; what it waits for is kept short: records and angles
+// of a chunk of rotations are staged at once (a thread-wide sincos per rotation
+// before), one barrier per rotation (four in the reverse sweep before), psi and
+// lambda in LDS.  One 3-layer evaluation of (7: 4,3) 419 -> 238 us, of (8e,8o)
+// 994 -> 608; 38 instances of 4 to 7 orbitals 449 -> 270.
+template <int U, int CT, bool LDS>
 __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
-  __shared__ double red[kBT / 64];
+  __shared__ double red[2][kBW];
+  __shared__ BatchRot recs[kBRot];
+  __shared__ double2 cs[kBRot];
   extern __shared__ double sA[];
   double* slot = B.scratch + (size_t)blockIdx.x * B.slot_doubles;
-  double* psi = slot;
+  double* psi = LDS ? sA + B.vec0 : slot;
   double* lam = psi + B.dmax;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int li = B.wg_off[blockIdx.x]; li < B.wg_off[blockIdx.x + 1]; ++li) {
     const BatchInstance I = B.inst[B.wg_list[li]];
     const BatchSpace S = B.spaces[I.space];
     const int nsb = S.nsb;
     const int dim = S.nsa * nsb;  // < 2^30, checked at creation
-    double* G = lam + B.dmax;
+    double* G = slot + 2 * B.dmax;
     const double* th = B.theta + I.theta0;
     const double* start = B.psi0[B.wg_list[li]];
     if (start) {
@@ -193,16 +196,30 @@ __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
       }
     }
     __syncthreads();
-    // forward sweep
-    for (int r = 0; r < I.ngate; ++r) {
-      const BatchRot& R = B.rots[I.gate0 + r];
-      const double t0 = th[R.theta_idx];
-      if (fabs(t0) >= 1e-28) {
-        double s, c;
-        sincos(R.scale * t0, &s, &c);
-        (void)rotate_lists<U, false>(B.lists, R, nsb, c, s, true, psi, nullptr);
+    // records and angles of rotations [r0, r0 + n); c = 1, s = 0 where theta
+    // vanishes
+    auto stage = [&](int r0, int n, bool rev) {
+      __syncthreads();
+      for (int i = threadIdx.x; i < n; i += kBT) {
+        const BatchRot R = B.rots[I.gate0 + r0 + i];
+        const double t0 = th[R.theta_idx];
+        double s = 0.0, c = 1.0;
+        if (rev ? !(fabs(t0) < 1e-28) : fabs(t0) >= 1e-28) sincos(R.scale * t0, &s, &c);
+        recs[i] = R;
+        cs[i] = double2{c, rev ? -s : s};
       }
       __syncthreads();
+    };
+    // forward sweep
+    for (int r0 = 0; r0 < I.ngate; r0 += kBRot) {
+      const int n = min(kBRot, I.ngate - r0);
+      stage(r0, n, false);
+      for (int r = 0; r < n; ++r) {
+        const double2 x = cs[r];
+        if (x.x != 1.0 || x.y != 0.0)
+          (void)rotate_lists<U, false>(B.lists, recs[r], nsb, x.x, x.y, true, psi, nullptr);
+        __syncthreads();
+      }
     }
     // stage A (K4 x kpad, transposed coefficient matrix) in LDS
     const double* Ag = B.A + I.A_off;
@@ -213,7 +230,7 @@ __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
     // and keeps all kpad/16 row tiles in flight, so D is never stored.
     {
       typedef double double4_t __attribute__((ext_vector_type(4)));
-      const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, kq = lane >> 4, li = lane & 15;
+      const int kq = lane >> 4, li = lane & 15;
       const int nwaves = blockDim.x >> 6;
       const int MT = S.kpad / 16;
       for (int c0 = wave * 16 * CT; c0 < dim; c0 += nwaves * 16 * CT) {
@@ -301,22 +318,44 @@ __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
       lam[x] = v;
       e += v * psi[x];
     });
-    const double energy = block_reduce(e, red);
-    if (threadIdx.x == 0) B.energy[B.wg_list[li]] = energy;
-    // reverse sweep with gradient dots
-    for (int p = threadIdx.x; p < I.nparam; p += blockDim.x) B.grad[I.out0 + p] = 0.0;
+    e = wave_sum63(e);
+    if (lane == 63) red[0][wave] = e;
     __syncthreads();
-    for (int r = I.ngate - 1; r >= 0; --r) {
-      const BatchRot& R = B.rots[I.gate0 + r];
-      const double t0 = th[R.theta_idx];
-      const bool skip = fabs(t0) < 1e-28;
-      double s, c;
-      sincos(-R.scale * t0, &s, &c);
-      const double dot = rotate_lists<U, true>(B.lists, R, nsb, c, s, !skip, psi, lam);
-      const double tot = block_reduce(dot, red);
-      if (threadIdx.x == 0) B.grad[I.out0 + R.grad_idx] += 2.0 * tot;
-      __syncthreads();
+    if (threadIdx.x == 0) {
+      e = 0.0;
+      for (int w = 0; w < kBW; ++w) e += red[0][w];
+      B.energy[B.wg_list[li]] = e;
     }
+    // reverse sweep with gradient dots; the last wave adds the wave sums of one
+    // rotation to its gate's gradient during the next
+    for (int p = threadIdx.x; p < I.nparam; p += blockDim.x) B.grad[I.out0 + p] = 0.0;
+    int par = 0, done = -1;  // grad index of the previous rotation
+    double sum = 0.0;
+    auto finish = [&](int now) {
+      if (wave != kBW - 1 || done < 0) return;
+      sum += row16_sum(lane < kBW ? red[par ^ 1][lane] : 0.0);
+      if (now != done) {
+        if (lane == 15) B.grad[I.out0 + done] = 2.0 * sum;
+        sum = 0.0;
+      }
+    };
+    for (int r1 = I.ngate; r1 > 0; r1 -= kBRot) {
+      const int r0 = max(0, r1 - kBRot);
+      stage(r0, r1 - r0, true);
+      for (int r = r1 - r0 - 1; r >= 0; --r) {
+        const double2 x = cs[r];
+        const double dot = wave_sum63(
+            rotate_lists<U, true>(B.lists, recs[r], nsb, x.x, x.y, x.x != 1.0 || x.y != 0.0, psi, lam));
+        const int now = recs[r].grad_idx;
+        finish(now);
+        if (lane == 63) red[par][wave] = dot;
+        done = now;
+        par ^= 1;
+        __syncthreads();
+      }
+    }
+    finish(-1);
+    __syncthreads();
   }
 }
 
@@ -373,10 +412,11 @@ __global__ void k_group_out(const double* __restrict__ spart, int64_t nblk, cons
 }
 
 // Instances this large go to groups (the persistent launch keeps the rest):
-// one workgroup runs a 3-layer (8e,8o) evaluation in 967 us and then bounds the
-// whole batch, a 2-layer (6e,6o) one in 173, less than the launches of another
-// group.  256 instances of 4 to 10 orbitals with groups from 16384 (10
-// orbitals), 4096 (8) and 300 (6) determinants: 1524, 1206, 1358 us.
+// one workgroup runs a 3-layer (8e,8o) evaluation in 590 us, the large kernels
+// in 92, but a 2-layer (6e,6o) one takes 100, less than the launches of another
+// group.  Groups from 16384, 4096 and 1200 determinants: 256 instances of 4 to
+// 10 orbitals 1158, 1136, 1145 us; 100 of 5 to 8 orbitals 801, 365, 424; 12 of 6
+// to 9 orbitals 3030, 375, 377; 38 of 4 to 7 orbitals 272, 271, 244.
 constexpr int64_t kGroupMinDim = 4096;
 
 // Streams the groups run on: one group's short kernels and the ends of its long
@@ -390,6 +430,7 @@ struct Batch {
   int64_t dmax = 0, slot = 0, ngrad = 0;
   double bytes = 0.0, flops = 0.0;  // algorithmic totals of one launch
   size_t lds = 0;
+  bool vec_lds = false;  // psi and lambda of the persistent launch in LDS
   std::vector<void*> allocs;
   BatchDev dev{};
   double* d_theta = nullptr;
@@ -608,7 +649,8 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
       std::map<std::pair<const Space*, std::string>, int> group_of;  // (space, gate layout) -> group
       const char* genv = getenv("SQ_BATCH_GROUPS");
       const bool groups_on = !(genv && genv[0] == '0');
-      int theta_off = 0, grad_off = 0;
+      int theta_off = 0, grad_off = 0, npmax = 0;
+      size_t small_lds = 0;  // A of the persistent launch's largest space
       for (int i = 0; i < n_inst; ++i) {
         const Space& s = spaces[i]->s;
         const Program& p = programs[i]->p;
@@ -694,9 +736,12 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
         Astore.insert(Astore.end(), A.begin(), A.end());
         I.e_core = H.e_core;
         B.inst.push_back(I);
-        B.dmax = std::max<int64_t>(B.dmax, s.dim);
-        B.slot = std::max<int64_t>(B.slot, (int64_t)(2 + bs.npair) * s.dim);
         B.lds = std::max<size_t>(B.lds, sizeof(double) * bs.K4 * bs.kpad);
+        if (!grouped[i]) {
+          B.dmax = std::max<int64_t>(B.dmax, s.dim);
+          npmax = std::max(npmax, bs.npair);
+          small_lds = std::max<size_t>(small_lds, sizeof(double) * bs.K4 * bs.kpad);
+        }
         cost[i] = s.dim * (int64_t)(2 * I.ngate + 4 + 2 * bs.npair + (bs.npair * bs.K4) / 8);
       }
       SQ_CHECK(B.lds <= 65536, SQ_ERR_ARG, "batched spaces limited to 12 orbitals (LDS)");
@@ -726,6 +771,12 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
         wo.push_back((int32_t)wl.size());
       }
       B.nwg = nwg;
+      B.slot = (2 + npmax) * B.dmax;
+      B.lds = small_lds;
+      B.dev.vec0 = (int64_t)(small_lds / sizeof(double));
+      const size_t with_vec = small_lds + 2 * sizeof(double) * (size_t)B.dmax;
+      B.vec_lds = with_vec <= kBatchLds;
+      if (B.vec_lds) B.lds = with_vec;
       B.dev.spaces = bupload(B, bsp);
       B.dev.inst = bupload(B, B.inst);
       B.dev.rots = bupload(B, rots);
@@ -804,11 +855,17 @@ int sq_batch_set_start_states(sq_batch* bo, const double* const* psi0, void* str
 using BatchKernel = void (*)(BatchDev);
 
 static BatchKernel batch_kernel(const Batch& B) {
-  static const BatchKernel table[3][2] = {{k_batch<1, 1>, k_batch<1, 2>},
-                                          {k_batch<2, 1>, k_batch<2, 2>},
-                                          {k_batch<4, 1>, k_batch<4, 2>}};
+  static const BatchKernel table[2][3][2] = {{{k_batch<1, 1, false>, k_batch<1, 2, false>},
+                                              {k_batch<2, 1, false>, k_batch<2, 2, false>},
+                                              {k_batch<4, 1, false>, k_batch<4, 2, false>}},
+                                             {{k_batch<1, 1, true>, k_batch<1, 2, true>},
+                                              {k_batch<2, 1, true>, k_batch<2, 2, true>},
+                                              {k_batch<4, 1, true>, k_batch<4, 2, true>}}};
   const int u = B.rot_pairs == 1 ? 0 : (B.rot_pairs == 2 ? 1 : 2);
-  return table[u][B.gemm_tiles - 1];
+  const BatchKernel k = table[B.vec_lds ? 1 : 0][u][B.gemm_tiles - 1];
+  // with the static part above 64 KB the launch needs the permission too
+  allow_lds(k, B.lds + kBRot * 64 + 1024 > 65536 ? std::max<size_t>(B.lds, 65536 + 8) : B.lds);
+  return k;
 }
 
 // The persistent launch and the groups write disjoint outputs: between a fork

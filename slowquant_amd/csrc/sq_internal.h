@@ -395,4 +395,26 @@ namespace sq {
 // SQ_UCC_CSR=0).
 bool operator_apply_pattern(const Space& s, sq_operator& op, const double* in, double* out, hipStream_t st);
 void operator_pattern_free(sq_operator& op);
+// Sums across lanes in vector registers.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, ROWS == 0xf);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, ROWS == 0xf);
+  return v + __hiloint2double(hi, lo);
+}
+
+// Sum over each row of 16 lanes, in the row's last lane.
+__device__ __forceinline__ double row16_sum(double v) {
+  v = dpp_add<0xb1>(v);   // quad_perm [1,0,3,2]
+  v = dpp_add<0x4e>(v);   // quad_perm [2,3,0,1]
+  v = dpp_add<0x114>(v);  // row_shr:4
+  return dpp_add<0x118>(v);
+}
+
+// Sum over the wave, in lane 63 (no LDS round trip: shuffles took two).
+__device__ __forceinline__ double wave_sum63(double v) {
+  v = dpp_add<0x142, 0xa>(row16_sum(v));  // row_bcast:15 into rows 1 and 3
+  return dpp_add<0x143, 0xc>(v);          // row_bcast:31 into rows 2 and 3
+}
+
 }  // namespace sq
