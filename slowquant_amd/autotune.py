@@ -6,7 +6,7 @@ chosen here by timing on first use and remembered per device and workload:
 
 * single instance (a space and a gate program): the fused rotation stages'
   tile size (sq_program_set_tile_shape: elements and threads per tile) by timing whole energy + gradient
-  evaluations, then the row sigma's rows per block and alpha-GEMM split
+  evaluations, then the row sigma's rows per block and string product split
   (sq_sigma_configure) by timing sigma alone;
 * batched instances: the persistent launch's workgroup count and kernel shape
   (engine.autotune_batch), keyed by the instance list.
