@@ -278,8 +278,8 @@ int sq_operator_matrix(const sq_space* s, const sq_operator* op, int reference_c
                        void* stream);
 
 /* ---- Orbital rotations and integrals ---------------------------------------
- * Matrices are row-major FP64 device arrays; every contraction is an FP64-MFMA
- * GEMM.  work: sq_orbital_work_bytes(n_ao, n_mo, n_inactive, n_active, n_kappa)
+ * Matrices are row-major FP64 device arrays; the rotation and the transforms
+ * are FP64-MFMA GEMMs, the gradient one block per rotation.  work: sq_orbital_work_bytes(n_ao, n_mo, n_inactive, n_active, n_kappa)
  * bytes (the largest of the three calls below for those sizes). */
 int64_t sq_orbital_work_bytes(int n_ao, int n_mo, int n_inactive, int n_active, int n_kappa);
 /* c_mo = C_old expm(-kappa) (ups_wavefunction.py:367-385): c_old and c_new
