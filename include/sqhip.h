@@ -143,8 +143,8 @@ int sq_sigma_configure(sq_space* s, int rows_per_block, int nsplit, int determin
 
 /* sigma = H psi with no allocation: no counterpart in the reference; for
  * callers that cannot allocate (code under HIP graph capture, tight serving
- * loops).  Same kernels as sq_sigma's row path, with its scratch (string products
- * partials and block partials) in a 64 MiB device array that each GPU the
+ * loops).  Same kernels as sq_sigma's row path, with its scratch (string
+ * product partials and block partials) in a 64 MiB device array that each GPU the
  * library runs on holds until the process ends; spaces needing more, or
  * above 4096 beta strings, fail with SQ_ERR_ARG.  energy: DEVICE double or
  * NULL; nothing is synchronised.  Calls that overlap on one GPU share the
@@ -279,8 +279,8 @@ int sq_operator_matrix(const sq_space* s, const sq_operator* op, int reference_c
 
 /* ---- Orbital rotations and integrals ---------------------------------------
  * Matrices are row-major FP64 device arrays; the rotation and the transforms
- * are FP64-MFMA GEMMs, the gradient one block per rotation.  work: sq_orbital_work_bytes(n_ao, n_mo, n_inactive, n_active, n_kappa)
- * bytes (the largest of the three calls below for those sizes). */
+ * are FP64-MFMA GEMMs, the gradient one block per rotation.  work:
+ * sq_orbital_work_bytes(n_ao, n_mo, n_inactive, n_active, n_kappa) bytes (the largest of the three calls below for those sizes). */
 int64_t sq_orbital_work_bytes(int n_ao, int n_mo, int n_inactive, int n_active, int n_kappa);
 /* c_mo = C_old expm(-kappa) (ups_wavefunction.py:367-385): c_old and c_new
  * are n_ao x n device arrays, kappa the n x n antisymmetric HOST matrix of the
