@@ -315,8 +315,7 @@ __global__ __launch_bounds__(256) void k_kappa_grad(int N, int ni, int na, const
     if (m < o) t += g[n * N3 + p * N2 + qr] * G2(m, p, q, r) + g[p * N3 + n * N2 + qr] * G2(p, m, q, r);
     if (n < o) t -= g[m * N3 + p * N2 + qr] * G2(n, p, q, r) + g[p * N3 + m * N2 + qr] * G2(p, n, q, r);
   }
-  if ((int)threadIdx.x < o) {
-    const int p = threadIdx.x;
+  for (int p = threadIdx.x; p < o; p += 256) {
     if (m < o) t += 2.0 * h[(int64_t)n * N + p] * G1(m, p);
     if (n < o) t -= 2.0 * h[(int64_t)p * N + m] * G1(p, n);
   }
