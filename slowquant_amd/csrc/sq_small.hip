@@ -543,7 +543,7 @@ __global__ __launch_bounds__(kST) void k_small_sweep(SmallDev S, const double* t
       const TrigSlot t = S.slots[C.t0 + i];
       const double th = theta[t.gate];
       double sn = 0.0, c = 1.0;
-      if (fabs(th) >= 1e-28) sincos(t.scale * th, &sn, &c);
+      if (!(fabs(th) < 1e-28)) sincos(t.scale * th, &sn, &c);  // NaN passes through
       cs[i] = double2{c, !POLY && inv ? -sn : sn};
       scales[i] = t.scale;
     }
