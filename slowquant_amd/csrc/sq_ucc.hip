@@ -470,9 +470,13 @@ __global__ __launch_bounds__(kUB) void k_norms(const double* __restrict__ y, con
   }
 }
 
+// A row sum of |T| below this is zero to the exponential, and its reciprocal
+// may overflow.
+constexpr double kTinyBound = 1e-300;
+
 // nxt[I] = f (T cur)[I] + prev[I] (prev: nullptr for none), LPR lanes per row;
 // TWO: nxt2 = f T cur2 in the same pass.  With bound, f is divided by
-// bound[0] (0 where that is 0).  U rounds of a row's elements are loaded before
+// bound[0] (0 where that vanishes).  U rounds of a row's elements are loaded before
 // any is used, the next U during the gathers of those.
 // Bound by the chain row pointer -> elements -> gathers -> sum of a row, some
 // 3 us that the waves of a SIMD overlap, not by bytes ((10e,10o): 9.1 M
@@ -491,7 +495,7 @@ __global__ __launch_bounds__(kUB) void k_spmv(int64_t dim, const int64_t* __rest
   const int lane = threadIdx.x & (LPR - 1);
   const int64_t I = (int64_t)blockIdx.x * (kUB / LPR) + threadIdx.x / LPR;
   if (I >= dim) return;
-  if (bound) f = bound[0] > 0.0 ? f / bound[0] : 0.0;
+  if (bound) f = bound[0] > kTinyBound ? f / bound[0] : 0.0;
   const int64_t e = urow[I + 1];
   int64_t u0 = urow[I] + lane;
   double a[U], v = 0.0, v2 = 0.0;
@@ -1333,7 +1337,7 @@ static Series series_start(const Space& s, const Program& p, const UccT& T, cons
   const double r = S.nu * tmax;
   *m = std::max(1, (int)std::ceil(std::min(r / nu_limit(s), 1e9)));
   *done = 0;
-  if (r == 0.0) {
+  if (r == 0.0 || S.bound <= kTinyBound) {  // K = 0: the identity
     S.taylor = true;
   } else if (r <= 2.0 && S.bound < 1e6) {
     S.taylor = true;
