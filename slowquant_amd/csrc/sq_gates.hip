@@ -823,6 +823,7 @@ int sq_program_set_tile_shape(sq_program* pr, int target, int threads) {
   return guarded([&] {
     SQ_CHECK(pr && target >= 0 && (threads == 0 || threads == 256 || threads == 512), SQ_ERR_ARG,
              "tile target must be >= 0 and threads 0, 256 or 512");
+    std::lock_guard<std::recursive_mutex> lock(pr->p.plan_mu);
     if (pr->p.tile_target == target && pr->p.tile_threads == threads) return;
     SQ_HIP(hipDeviceSynchronize());  // the old plan's buffers may be in use by queued kernels
     for (TilePlan** t : {&pr->p.tiles, &pr->p.group_tiles}) {

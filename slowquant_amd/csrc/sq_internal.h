@@ -158,6 +158,9 @@ void small_plan_free(SmallPlan* P);
 
 struct Program {
   const Space* space;
+  // Held while a plan below is looked up or built, so that the first calls of
+  // several threads wait for one plan and all take its route.
+  mutable std::recursive_mutex plan_mu;
   mutable TilePlan* tiles = nullptr;  // built on first use (sq_tiles.hip)
   mutable bool tiles_built = false;
   mutable TilePlan* group_tiles = nullptr;  // the plan of batched groups

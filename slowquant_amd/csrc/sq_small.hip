@@ -709,6 +709,7 @@ SmallDev device_view(const Space& s, const SmallPlan& P) {
 // components, or programs that run in tile stages from the first gate to the
 // last (a stage spreads over many CUs and takes about 1 us per orbital pair).
 const SmallPlan* small_for(const Space& s, const Program& p) {
+  std::lock_guard<std::recursive_mutex> lock(p.plan_mu);
   if (!p.small_tried) {
     p.small_tried = true;
     const char* env = getenv("SQ_SMALL_SWEEP");

@@ -712,6 +712,7 @@ static bool usable(const TilePlan* T) { return T && T->nops > 0; }
 // have a plan of their own: with many instances per launch the widest window
 // is the best one.
 static const TilePlan* plan_of(const Space& s, const Program& p, TilePlan*& slot, bool& built, int instances) {
+  std::lock_guard<std::recursive_mutex> lock(p.plan_mu);
   if (!built) {
     built = true;
     const char* env = getenv("SQ_TILES");
