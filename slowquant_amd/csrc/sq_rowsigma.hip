@@ -1066,7 +1066,10 @@ int string_gemm_split(const Space& s) {
 // staging of A per row: 10 orbitals in groups 1600 -> 1506 us, (11e,11o) 205 ->
 // 186, (12e,12o) 437 -> 424 (energy and gradient); more rows gain no more.  A
 // launch of many instances has blocks enough: four rows and the string products
-// unsplit (a quarter of the atomic adds), 256 instances 1283 -> 1206 us.
+// unsplit (a quarter of the atomic adds), 256 instances 1283 -> 1206 us.  But no
+// more rows than leave two blocks on a CU where the single instance has two
+// ((12e,12o): three), so that the fused form, which groups need, does not depend
+// on n.
 constexpr int kManyInst = 8;
 
 bool row_plan(const Space& s, RowPlan* out, int n = 1) {
@@ -1083,9 +1086,17 @@ bool row_plan(const Space& s, RowPlan* out, int n = 1) {
   const int tpr = (s.nsb + 15) / 16;
   int bestR = 0;
   if (scatter) {
-    bestR = std::max(list ? (n >= kManyInst ? 4 : 2) : 1, (kRowWaves + tpr - 1) / tpr);
-    bestR = std::max(1, std::min(s.nsa, bestR));
-    while (bestR > 1 && row_lds(s, mt, bestR, true, list) > kLdsMax) --bestR;
+    auto rows = [&](int least) {
+      int R = std::max(1, std::min(s.nsa, std::max(least, (kRowWaves + tpr - 1) / tpr)));
+      while (R > 1 && row_lds(s, mt, R, true, list) > kLdsMax) --R;
+      return R;
+    };
+    bestR = rows(list ? 2 : 1);
+    if (list && n >= kManyInst) {
+      const int one = bestR;
+      bestR = rows(4);
+      while (bestR > one && 2 * row_lds(s, mt, bestR, true, list) > kLdsMax) --bestR;
+    }
   } else {
     int64_t best = -1;
     for (int R = 1; R <= 64 && R <= s.nsa; ++R) {
