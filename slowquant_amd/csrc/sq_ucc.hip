@@ -257,14 +257,19 @@ __global__ __launch_bounds__(64 * kCsrRows) void k_tapply_csr(int64_t dim, const
 constexpr int kGateBits = 24, kCoefBits = 7;
 constexpr int kSortRow = 8192;  // longest row sorted in LDS (64 KB of keys); longer rows merge neighbours only
 
-// Sorts row I's entries by (source, term) in place (bitonic, keys
-// source << 32 | term << 1 | sign) and counts the distinct sources.
-__global__ __launch_bounds__(kUB) void k_row_sort(const int64_t* __restrict__ rowp, uint2* __restrict__ ent,
-                                                  int32_t* __restrict__ ucnt) {
+// Sorts a row's entries by (source, term) in place (bitonic, keys
+// source << 32 | term << 1 | sign) and counts the distinct sources.  A block
+// per row, on two grid dimensions: 256 threads per row would pass the limit of
+// 2^32 in one from 2^24 rows.
+constexpr int64_t kSortGrid = (int64_t)1 << 20;
+__global__ __launch_bounds__(kUB) void k_row_sort(int64_t dim, const int64_t* __restrict__ rowp,
+                                                  uint2* __restrict__ ent, int32_t* __restrict__ ucnt) {
   extern __shared__ uint64_t key[];
   __shared__ int red[kUB / 64];
-  const int64_t b = rowp[blockIdx.x];
-  const int n = (int)(rowp[blockIdx.x + 1] - b);
+  const int64_t row = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (row >= dim) return;
+  const int64_t b = rowp[row];
+  const int n = (int)(rowp[row + 1] - b);
   const int tid = threadIdx.x;
   int c = 0;
   if (n <= kSortRow) {
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(kUB) void k_row_sort(const int64_t* __restrict__ ro
   if (tid == 0) {
     int tot = 0;
     for (int w = 0; w < kUB / 64; ++w) tot += red[w];
-    ucnt[blockIdx.x] = tot;
+    ucnt[row] = tot;
   }
 }
 
@@ -895,7 +900,8 @@ static UccT* ucc_t(const Space& s, const Program& p, hipStream_t st) {
   int P = 1;
   while (P < std::min<int64_t>(longest, kSortRow)) P <<= 1;
   allow_lds(k_row_sort, (size_t)P * 8 + 1024);
-  k_row_sort<<<(unsigned)s.dim, kUB, (size_t)P * 8, st>>>(c->rowp, c->ent, (int32_t*)ucnt.p);
+  const dim3 sort_grid((unsigned)std::min(s.dim, kSortGrid), (unsigned)((s.dim + kSortGrid - 1) / kSortGrid));
+  k_row_sort<<<sort_grid, kUB, (size_t)P * 8, st>>>(s.dim, c->rowp, c->ent, (int32_t*)ucnt.p);
   SQ_HIP(hipGetLastError());
   std::vector<int32_t> hc((size_t)s.dim);
   SQ_HIP(hipMemcpyAsync(hc.data(), ucnt.p, sizeof(int32_t) * hc.size(), hipMemcpyDeviceToHost, st));
