@@ -5,7 +5,8 @@
 // the pair ops inside a window of w consecutive orbitals a determinant keeps
 // its occupation outside the window and its electron count inside it, per
 // spin: strings fall into groups of C(w, k) strings, in the canonical order of
-// their window occupations.  A tile = (one alpha group) x (one beta group) is
+// their window occupations.  A tile = (some alpha groups of one electron count)
+// x (some beta groups of one count) is
 // closed under every gate of the window, so one launch (a stage) loads each
 // tile into LDS once, applies all the pair ops that are ready inside the
 // window, whatever their depth in the brick wall, and writes it back.  The
@@ -52,7 +53,8 @@
 
 namespace sq {
 
-constexpr int kMaxWin = 8;          // orbitals per window: at most C(8,4)^2 = 4900 amplitudes per tile
+constexpr int kMaxWin = 8;          // orbitals per window
+constexpr int kTileElems = 4900;    // amplitudes per tile: C(8,4)^2
 constexpr int kMaxPairEntries = 8;  // entries per pair op (sa_single counts twice)
 constexpr int kMaxOps = 64;         // pair ops per stage
 constexpr int kTypes = 9;           // orbit types (alpha kind x beta kind)
@@ -91,9 +93,9 @@ constexpr int kQVals = 10;
 // op: T_g annihilates them); padded to 36.
 constexpr int kMatVals = 36;
 
-// One dispatch slot: alpha group rows arows[r0, r0 + R), beta group columns
-// bcol[c0, c0 + W), electrons in the window, the orbit words of (ka, kb).
-// R = 0 marks an empty slot.
+// One dispatch slot: rows arows[r0, r0 + R) of its alpha groups, columns
+// bcol[c0, c0 + W) of its beta groups, electrons in the window and groups of
+// each side (k | groups << 8), their orbit words.  R = 0 marks an empty slot.
 struct TileRec {
   int32_t r0, R, c0, W, ka, kb, items, pad;
 };
@@ -104,6 +106,11 @@ struct TileRec {
 struct KInfo {
   int32_t n4, ne, nd;
 };
+// The same over a tile side's groups (g = k | groups << 8).
+__host__ __device__ inline KInfo side_info(const KInfo* k, int g) {
+  const KInfo i = k[g & 255];
+  return KInfo{i.n4 * (g >> 8), i.ne * (g >> 8), i.nd * (g >> 8)};
+}
 
 // Orbit words of one pair position: five ranges and a sixth (alpha list x
 // beta list), each filled up to whole waves of 64 words with kNone, so that a
@@ -117,7 +124,7 @@ struct KInfo {
 // (in waves; m0: first member, in doubles from the tile's first, which is
 // preceded by a zero that kNone points to; dr, dc, d: distance of the others;
 // swapping neighbouring orbitals moves a string by at most C(6, 3) = 20
-// places).
+// places within its group).
 struct OpItems {
   int c1, c2, c3, c4, c5, c6;
 };
@@ -133,7 +140,7 @@ __host__ __device__ inline OpItems op_items(const KInfo& A, const KInfo& B) {
   return o;
 }
 constexpr uint32_t kNone = 0u;  // the zero before the tile
-constexpr int kMaxWaves = 27;   // c5 at most: k = 4 of 8 on both sides
+constexpr int kMaxWaves = 27;   // c5 at most: k = 4 of 8 on both sides; merged tiles stay within it
 
 struct OpRef {
   int32_t op, pos;  // program-wide pair op, pair position within the window
@@ -177,13 +184,19 @@ struct Window {
   int32_t *arows = nullptr, *bcol = nullptr;
   TileRec* tiles = nullptr;
   int nb = 0;
-  int maxR = 0, maxW = 0;
+  size_t lds_fwd = 0, lds_rev = 0;
 };
 
-// What the windows of one width need on one space: the orbit words of the
-// (ka, kb) that occur, and the window positions used so far.
+// Groups of k electrons per tile side, at most (0: none occurs).
+struct Merge {
+  int a[kMaxWin + 1] = {}, b[kMaxWin + 1] = {};
+};
+
+// What the windows of one width and tile target need on one space: the orbit
+// words of the sides that occur, and the window positions used so far.
 struct WidthTables {
   KInfo k[kMaxWin + 1] = {};
+  Merge merge;
   uint32_t* items = nullptr;
   std::map<std::pair<int, int>, int> off;
   std::map<int, Window> at;
@@ -191,7 +204,7 @@ struct WidthTables {
 
 // Kept by the space (a space's programs share them) and freed with it.
 struct WinCache {
-  std::map<int, WidthTables> width;
+  std::map<std::pair<int, int>, WidthTables> width;
   std::vector<void*> allocs;
   ~WinCache() {
     for (void* p : allocs) (void)hipFree(p);
@@ -405,22 +418,137 @@ static void spread_banks(std::vector<uint32_t>& items, size_t from, bool four) {
   std::copy(out.begin(), out.end(), items.begin() + from);
 }
 
-// Orbit words of the electron counts that occur in windows of width w.
-static void build_width(const Space& sp, int w, WidthTables& T, std::vector<void*>& allocs) {
+static int binomial(int n, int k) {
+  if (k < 0 || k > n) return 0;
+  int b = 1;
+  for (int i = 0; i < k; ++i) b = b * (n - i) / (i + 1);
+  return b;
+}
+
+static KInfo window_info(int w, int k) {
+  return KInfo{binomial(w - 2, k - 1), binomial(w - 2, k), binomial(w - 2, k - 2)};
+}
+
+// Windows of width w on a space: per electron count k inside, the strings of a
+// group, the pair counts and the alpha and beta groups.
+struct WinCounts {
+  int w, len[kMaxWin + 1], a[kMaxWin + 1], b[kMaxWin + 1];
+  KInfo info[kMaxWin + 1];
+  WinCounts(const Space& sp, int width) : w(width) {
+    for (int k = 0; k <= w; ++k) {
+      len[k] = binomial(w, k);
+      info[k] = window_info(w, k);
+      a[k] = binomial(sp.n - w, sp.na - k);
+      b[k] = binomial(sp.n - w, sp.nb - k);
+    }
+  }
+};
+
+// Group counts of the tile sides that hold all groups of k electrons, at most
+// m a side, as evenly as they go: the larger count and how many sides have it,
+// the others one less.
+struct Split {
+  int sides, big, nbig;
+};
+static Split split_groups(int groups, int m) {
+  Split s;
+  s.sides = (groups + m - 1) / m;
+  s.big = (groups + s.sides - 1) / s.sides;
+  s.nbig = groups - s.sides * (s.big - 1);
+  return s;
+}
+
+// Groups per tile side for tiles of up to about target amplitudes.  With few
+// electrons the groups are small and many ((16: 3,3), windows of 8: 93 of 1 to
+// 56 strings per spin, 8649 pairs), and a block takes each pair op of its
+// tile behind a barrier, 0.5 us however small the tile.
+static Merge merge_groups(const WinCounts& C, int target) {
+  Merge M;
+  auto side = [&](const int* groups, int limit, int* m) {  // returns the longest side
+    int most = 1;
+    for (int k = 0; k <= C.w; ++k) {
+      m[k] = 0;
+      if (groups[k] == 0) continue;
+      m[k] = split_groups(groups[k], std::max(1, std::min(limit / C.len[k], groups[k]))).big;
+      most = std::max(most, m[k] * C.len[k]);
+    }
+    return most;
+  };
+  for (int e = std::min(target, kTileElems);; e = e * 3 / 4) {
+    int rows = side(C.a, (int)std::sqrt((double)e), M.a);
+    const int cols = side(C.b, e / rows, M.b);
+    rows = side(C.a, e / cols, M.a);
+    bool fits = true;
+    for (int ka = 0; ka <= C.w && fits; ++ka)
+      for (int kb = 0; kb <= C.w && fits; ++kb) {
+        if (M.a[ka] * M.b[kb] <= 1) continue;
+        const OpItems o = op_items(side_info(C.info, ka | M.a[ka] << 8), side_info(C.info, kb | M.b[kb] << 8));
+        fits = M.a[ka] * C.len[ka] * M.b[kb] * C.len[kb] <= kTileElems && o.c5 <= kMaxWaves;
+      }
+    if (fits || e < 4) return M;
+  }
+}
+
+// Tiles of one window of width w and the amplitudes of the largest.
+struct Tiling {
+  int64_t tiles;
+  int most;
+};
+static Tiling merged_tiles(const WinCounts& C, const Merge& M) {
+  auto sides = [&](const int* groups, const int* m, int& most) {
+    int64_t c = 0;
+    for (int k = 0; k <= C.w; ++k) {
+      if (m[k] == 0) continue;
+      c += split_groups(groups[k], m[k]).sides;
+      most = std::max(most, m[k] * C.len[k]);
+    }
+    return std::max<int64_t>(c, 1);
+  };
+  int rows = 1, cols = 1;
+  const int64_t a = sides(C.a, M.a, rows), b = sides(C.b, M.b, cols);
+  return Tiling{a * b, rows * cols};
+}
+
+// Orbit words of the tile sides that occur in windows of width w.
+static void build_width(const Space& sp, int w, int target, WidthTables& T, std::vector<void*>& allocs) {
   std::vector<std::vector<PairLists>> L(w + 1);
+  const WinCounts C(sp, w);
   for (int k = 0; k <= w; ++k) {
     L[k] = pair_lists(w, k);
-    T.k[k] = KInfo{(int)L[k][0].lo.size(), (int)L[k][0].em.size(), (int)L[k][0].db.size()};
+    T.k[k] = C.info[k];
   }
-  auto occurs = [&](int k, int ne) { return k <= ne && ne - k <= sp.n - w; };
+  T.merge = merge_groups(C, target);
+  // the sides (k | groups << 8) of one spin
+  auto sides = [&](const int* groups, const int* m) {
+    std::vector<int> out;
+    for (int k = 0; k <= w; ++k) {
+      if (m[k] == 0) continue;
+      const Split s = split_groups(groups[k], m[k]);
+      out.push_back(k | s.big << 8);
+      if (s.nbig < s.sides) out.push_back(k | (s.big - 1) << 8);
+    }
+    return out;
+  };
+  // a pair position's lists over all groups of a side
+  auto over_groups = [&](int g, int j) {
+    const PairLists& P = L[g & 255][j];
+    const int len = C.len[g & 255];
+    PairLists out;
+    for (int i = 0; i < (g >> 8); ++i) {
+      for (int x : P.lo) out.lo.push_back(x + i * len);
+      for (int x : P.up) out.up.push_back(x + i * len);
+      for (int x : P.em) out.em.push_back(x + i * len);
+      for (int x : P.db) out.db.push_back(x + i * len);
+    }
+    return out;
+  };
   std::vector<uint32_t> items;
-  for (int ka = 0; ka <= w; ++ka)
-    for (int kb = 0; kb <= w; ++kb) {
-      if (!occurs(ka, sp.na) || !occurs(kb, sp.nb)) continue;
-      T.off[{ka, kb}] = (int)items.size();
-      const int W = (int)local_strings(w, kb).size();
+  for (int ga : sides(C.a, T.merge.a))
+    for (int gb : sides(C.b, T.merge.b)) {
+      T.off[{ga, gb}] = (int)items.size();
+      const int W = (gb >> 8) * C.len[gb & 255];
       for (int j = 0; j + 1 < w; ++j) {
-        const PairLists &A = L[ka][j], &B = L[kb][j];
+        const PairLists A = over_groups(ga, j), B = over_groups(gb, j);
         auto at = [&](int r, int c) { return (uint32_t)(1 + r * W + c); };
         size_t from = items.size();
         auto fill = [&](bool four) {
@@ -454,46 +582,50 @@ static void build_width(const Space& sp, int w, WidthTables& T, std::vector<void
   T.items = upload(allocs, items);
 }
 
-struct Group {
-  int k;
+// A tile side: electrons in the window and groups (k | groups << 8), strings.
+struct Side {
+  int g;
   std::vector<int32_t> str;
 };
 
-// Strings by occupation outside [lo, lo + w) and electrons inside; canonical
-// order within a group.
-static std::vector<Group> window_groups(const std::vector<uint32_t>& strs, int lo, int w) {
+// Strings by electrons inside [lo, lo + w) and occupation outside (a group, in
+// canonical order), the groups of one count dealt to tile sides.
+static std::vector<Side> window_sides(const std::vector<uint32_t>& strs, int lo, int w, const int* m) {
   const uint32_t in = ((1u << w) - 1u) << lo;
-  std::map<uint64_t, Group> g;
-  for (size_t i = 0; i < strs.size(); ++i) {
-    const int k = __builtin_popcount(strs[i] & in);
-    Group& G = g[(uint64_t)(strs[i] & ~in) << 8 | (uint64_t)k];
-    G.k = k;
-    G.str.push_back((int32_t)i);
+  std::map<uint32_t, std::vector<int32_t>> g[kMaxWin + 1];
+  for (size_t i = 0; i < strs.size(); ++i)
+    g[__builtin_popcount(strs[i] & in)][strs[i] & ~in].push_back((int32_t)i);
+  std::vector<Side> out;
+  for (int k = 0; k <= w; ++k) {
+    if (g[k].empty()) continue;
+    const Split s = split_groups((int)g[k].size(), m[k]);
+    auto it = g[k].begin();
+    for (int x = 0; x < s.sides; ++x) {
+      const int n = x < s.nbig ? s.big : s.big - 1;
+      out.push_back(Side{k | n << 8, {}});
+      for (int i = 0; i < n; ++i, ++it) out.back().str.insert(out.back().str.end(), it->second.begin(), it->second.end());
+    }
   }
-  std::vector<Group> out;
-  for (auto& x : g) out.push_back(std::move(x.second));
   return out;
 }
 
 // Tables and dispatch order of one window position.  Workgroups go to the
 // XCDs round robin (slot b on XCD b % 8), each XCD with its own L2: tiles of
-// one alpha group read the same rows of the state, so whole groups are given
+// one alpha side read the same rows of the state, so whole sides are given
 // to one XCD (largest first, each to the XCD with the fewest elements so
 // far), largest tiles first there.  Empty slots have R = 0.
 static Window make_window(const Space& sp, int lo, int w, const WidthTables& T, std::vector<void*>& allocs) {
-  const std::vector<Group> A = window_groups(sp.h_astr, lo, w), B = window_groups(sp.h_bstr, lo, w);
+  const std::vector<Side> A = window_sides(sp.h_astr, lo, w, T.merge.a), B = window_sides(sp.h_bstr, lo, w, T.merge.b);
   Window W;
   std::vector<int32_t> arows, bcol;
   std::vector<int> a0, b0;
-  for (const Group& g : A) {
+  for (const Side& g : A) {
     a0.push_back((int)arows.size());
     arows.insert(arows.end(), g.str.begin(), g.str.end());
-    W.maxR = std::max(W.maxR, (int)g.str.size());
   }
-  for (const Group& g : B) {
+  for (const Side& g : B) {
     b0.push_back((int)bcol.size());
     bcol.insert(bcol.end(), g.str.begin(), g.str.end());
-    W.maxW = std::max(W.maxW, (int)g.str.size());
   }
   constexpr int kXcds = 8;
   std::vector<int> ao(A.size()), bo(B.size());
@@ -503,14 +635,17 @@ static Window make_window(const Space& sp, int lo, int w, const WidthTables& T, 
   std::stable_sort(bo.begin(), bo.end(), [&](int x, int y) { return B[x].str.size() > B[y].str.size(); });
   std::vector<std::vector<TileRec>> bins(kXcds);
   std::vector<int64_t> load(kXcds, 0);
-  // few alpha groups: single tiles are spread instead
+  // few alpha sides: single tiles are spread instead
   const bool whole = A.size() >= 2 * kXcds;
   for (int a : ao) {
     int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     for (int b : bo) {
       if (!whole) x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-      bins[x].push_back(TileRec{a0[a], (int)A[a].str.size(), b0[b], (int)B[b].str.size(), A[a].k, B[b].k, T.off.at({A[a].k, B[b].k}), 0});
-      load[x] += (int64_t)A[a].str.size() * (int64_t)B[b].str.size();
+      const int R = (int)A[a].str.size(), C = (int)B[b].str.size();
+      bins[x].push_back(TileRec{a0[a], R, b0[b], C, A[a].g, B[b].g, T.off.at({A[a].g, B[b].g}), 0});
+      load[x] += (int64_t)R * C;
+      W.lds_fwd = std::max(W.lds_fwd, tile_lds(R, C, 1));
+      W.lds_rev = std::max(W.lds_rev, tile_lds(R, C, 2));
     }
   }
   size_t len = 0;
@@ -541,21 +676,23 @@ struct PairOp {
 static std::vector<std::pair<int, std::vector<int>>> schedule(const std::vector<PairOp>& ops, int n, int w) {
   std::vector<std::pair<int, std::vector<int>>> out;
   std::vector<char> done(ops.size(), 0);
-  size_t left = ops.size();
+  std::vector<int> t;
+  size_t left = ops.size(), first = 0;
   while (left > 0) {
     int best = -1;
     std::vector<int> take;
+    while (done[first]) ++first;
     for (int lo = 0; lo + w <= n; ++lo) {
       uint32_t blocked = ~(((1u << w) - 1u) << lo);
-      std::vector<int> t;
-      for (size_t i = 0; i < ops.size() && t.size() < kMaxOps; ++i) {
+      t.clear();
+      for (size_t i = first; i < ops.size() && t.size() < kMaxOps && blocked != ~0u; ++i) {
         if (done[i]) continue;
         const uint32_t m = 3u << ops[i].p;
         if (blocked & m) blocked |= m;
         else t.push_back((int)i);
       }
       if (t.size() > take.size()) {
-        take = t;
+        take.swap(t);
         best = lo;
       }
     }
@@ -566,47 +703,51 @@ static std::vector<std::pair<int, std::vector<int>>> schedule(const std::vector<
   return out;
 }
 
-// Window width.  A program's tile target (or SQ_TILE_TARGET) gives the widest
-// window whose mean tile stays below it.  Otherwise the cheapest by a model of the sweep fitted
-// to launches at 8 to 14 orbitals (us, mean of forward and reverse): a stage
-// costs 8 and 0.3 per round of 256 tiles; a pair op 0.55 and 1 more per 9400
-// amplitudes of a tile, or 1 per 3000 amplitudes that a CU has to work through
-// where there are many tiles.  Narrow windows need more stages, wide ones
-// leave small spaces with fewer tiles than CUs.  Measured, energy and
-// gradient with w = 6, 7, 8: (8e,8o) 125, 118, 123; (10e,10o) 142, 134, 147;
-// (11e,11o) 370, 224, 240; (12e,12o) 1536, 674, 496 us; 256 instances of
-// (4e,4o)..(10e,10o) 3.41, 2.19, 1.83 ms.
-static int window_width(const Space& sp, const std::vector<PairOp>& ops, int target, int instances) {
+// Window width and tile target.  A program's tile target (or SQ_TILE_TARGET)
+// gives the widest window whose mean unmerged tile stays below it.  Otherwise
+// the cheapest of a model of the sweep (us, mean of forward and reverse),
+// fitted to 1- to 4-layer sweeps at 4 to 16 orbitals and all fillings: a stage
+// costs 5.5 and 8.5 per million amplitudes (its passes over memory); a pair op
+// 0.8 and 1 more per 11600 amplitudes of the largest tile and 34000 of the mean
+// one, as often as the tiles go round the 256 CUs.  Narrow windows need more
+// stages, small tiles more rounds, large ones leave CUs idle.  Its choices take
+// 0.8 % more than the best ones on average, 7 % at most.  Measured, forward and
+// reverse sweep of 4 layers with w = 6, 7, 8: (8e,8o) 110, 114, 114; (10e,10o)
+// 145, 131, 157; (12e,12o) 1242, 384, 207 us.  Tiles of one pair of groups
+// against merged ones: (16: 3,3) 3400 -> 270 us, (14: 3,7) 1510 -> 480,
+// (14e,14o) 2450 -> 2350 (energy and gradient of (16: 3,3) 3550 -> 415, with
+// stages of one brick column each 713).
+struct WinShape {
+  int width, target;  // target: of merge_groups
+};
+static WinShape window_shape(const Space& sp, const std::vector<PairOp>& ops, int target, int instances) {
   const int most = std::min(kMaxWin, sp.n);
   if (target <= 0)
     if (const char* env = getenv("SQ_TILE_TARGET")) target = atoi(env);
-  auto groups = [&](int w) {
-    auto count = [&](int k) {
-      int64_t c = 0, b = 1;  // outside strings that leave 0..w electrons inside
-      for (int o = 0; o <= sp.n - w; ++o) {
-        if (k - o >= 0 && k - o <= w) c += b;
-        b = b * (sp.n - w - o) / (o + 1);
-      }
-      return std::max<int64_t>(c, 1);
-    };
-    return count(sp.na) * count(sp.nb);
-  };
   if (target > 0) {
     int w = 2;
-    while (w < most && sp.dim <= groups(w + 1) * (int64_t)target) ++w;
-    return w;
+    auto pairs = [&](int width) {  // of groups
+      const WinCounts C(sp, width);
+      return merged_tiles(C, merge_groups(C, 1)).tiles;
+    };
+    while (w < most && sp.dim <= pairs(w + 1) * (int64_t)target) ++w;
+    return WinShape{w, target};
   }
-  int best = most;
+  WinShape best{most, kTileElems};
   double cost = -1.0;
   for (int w = std::min(4, most); w <= most; ++w) {
-    const double tiles = (double)groups(w) * instances;
-    const double tile = (double)sp.dim / (double)groups(w), rounds = std::ceil(tiles / 256.0);
-    const double op = std::max(0.55 + tile / 9400.0, rounds * tile / 3000.0);
-    double c = 0.0;
-    for (auto& st : schedule(ops, sp.n, w)) c += 8.0 + 0.3 * rounds + (double)st.second.size() * op;
-    if (cost < 0.0 || c < cost) {
-      cost = c;
-      best = w;
+    const WinCounts C(sp, w);
+    const double stages = (double)schedule(ops, sp.n, w).size();
+    for (int fill : {512, 1024, 2048, 4096, kTileElems}) {
+      const Tiling t = merged_tiles(C, merge_groups(C, fill));
+      const double mean = (double)sp.dim / (double)t.tiles;
+      const double op = 0.8 + (double)t.most / 11600.0 + mean / 34000.0;
+      const double c = stages * (5.5 + 8.5e-6 * (double)sp.dim * instances) +
+                       (double)ops.size() * op * std::max(1.0, (double)t.tiles * instances / 256.0);
+      if (cost < 0.0 || c < cost) {
+        cost = c;
+        best = WinShape{w, fill};
+      }
     }
   }
   return best;
@@ -642,12 +783,13 @@ TilePlan* build_tile_plan(const Space& sp, const Program& P, int instances) {
           ops.push_back(PairOp{p, ent});
         }
       }
-      const int w = window_width(sp, ops, P.tile_target, instances);
-      auto wt = sp.win->width.find(w);
+      const WinShape shape = window_shape(sp, ops, P.tile_target, instances);
+      const int w = shape.width;
+      auto wt = sp.win->width.find({w, shape.target});
       if (wt == sp.win->width.end()) {
         WidthTables t;
-        build_width(sp, w, t, sp.win->allocs);
-        wt = sp.win->width.emplace(w, std::move(t)).first;
+        build_width(sp, w, shape.target, t, sp.win->allocs);
+        wt = sp.win->width.emplace(std::make_pair(w, shape.target), std::move(t)).first;
       }
       WidthTables& wide = wt->second;
       for (auto& st : schedule(ops, sp.n, w)) {
@@ -682,8 +824,8 @@ TilePlan* build_tile_plan(const Space& sp, const Program& P, int instances) {
         d.ops = upload(T->allocs, refs);
         for (int k = 0; k <= w; ++k) d.k[k] = wide.k[k];
         S.dev = d;
-        S.lds_fwd = tile_lds(W.maxR, W.maxW, 1);
-        S.lds_rev = tile_lds(W.maxR, W.maxW, 2);
+        S.lds_fwd = W.lds_fwd;
+        S.lds_rev = W.lds_rev;
         T->stages.push_back(S);
       }
     }
@@ -1181,7 +1323,7 @@ __global__ __launch_bounds__(NT) void k_win_fwd(StageDev S, const double* __rest
     const TileRec T{tp->r0, tp->R, tp->c0, tp->W, tp->ka, tp->kb, tp->items, 0};
     if (T.R == 0) continue;
     const TileLds m = carve_lds(smem, T.R, T.W, false);
-    const OpItems o = op_items(S.k[T.ka], S.k[T.kb]);
+    const OpItems o = op_items(side_info(S.k, T.ka), side_info(S.k, T.kb));
     const uint32_t* items = S.items + T.items;
     auto at = [&](int j) { return as_const(S.ops) + (DAGGER ? S.nops - 1 - j : j); };
     auto load = [&](int j, Words<NT>& x) {
@@ -1248,7 +1390,7 @@ __global__ __launch_bounds__(NT) void k_win_rev(StageDev S, const double* __rest
     const TileRec T{tp->r0, tp->R, tp->c0, tp->W, tp->ka, tp->kb, tp->items, 0};
     if (T.R == 0) continue;
     const TileLds m = carve_lds(smem, T.R, T.W, true);
-    const OpItems o = op_items(S.k[T.ka], S.k[T.kb]);
+    const OpItems o = op_items(side_info(S.k, T.ka), side_info(S.k, T.kb));
     const uint32_t* items = S.items + T.items;
     double* X = m.X;
     double* L = m.L;
