@@ -216,11 +216,13 @@ int sq_ucc_energy_grad(const sq_space* s, const sq_program* p, const sq_hamilton
  * determinants whose programs are all brick stages run instead in groups
  * of equal (space, gate layout) through the tile-stage, row-sigma and
  * gradient kernels with one grid row per instance (SQ_BATCH_GROUPS=0 keeps
- * them in the persistent launch).  Such a batch uses the programs' tile
- * plans at every launch: the programs must outlive it, and changing a
- * grouped program's tile shape (sq_program_set_tile_shape) or a grouped
- * space's row-sigma shape (sq_sigma_configure) afterwards makes its launches
- * fail with SQ_ERR_ARG (create the batch again). */
+ * them in the persistent launch).  A group keeps the tile plan and row-sigma
+ * shape of the batch's creation.  Programs of 16384 or more determinants must
+ * outlive the batch, and changing such a program's tile shape
+ * (sq_program_set_tile_shape) or its space's row-sigma shape
+ * (sq_sigma_configure) afterwards makes its launches fail with SQ_ERR_ARG
+ * (create the batch again); smaller instances are free of both.  Spaces must
+ * outlive the batch. */
 typedef struct sq_batch sq_batch;
 int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program* const* programs,
                     const sq_hamiltonian* const* hams, int n_workgroups, sq_batch** out);

@@ -367,10 +367,12 @@ __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
 struct BatchGroup {
   const Space* space = nullptr;
   const Program* prog = nullptr;
+  std::shared_ptr<const TilePlan> tiles;  // the program's plan and the space's shape when the batch was made
+  SigmaShape sigma;
   int n = 0, ng = 0;
   int64_t dim = 0, A_stride = 0, Ma_stride = 0, Mb_stride = 0, mats_stride = 0, tpart_stride = 0, spart_stride = 0;
   double hf = 1.0;  // the HF determinant's amplitude in the engine's sign convention
-  int plan_gen = 0;  // the program's tile-plan generation the buffers are sized for
+  int plan_gen = 0;  // the program's tile-plan generation (check_group)
   int32_t *d_inst = nullptr, *d_theta0 = nullptr, *d_out0 = nullptr;  // per member
   double *theta = nullptr, *A = nullptr, *Ma = nullptr, *Mb = nullptr, *psi = nullptr, *lam = nullptr, *mats = nullptr,
          *tpart = nullptr, *spart = nullptr, *grad = nullptr;
@@ -530,9 +532,10 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
     G.A_stride = (int64_t)K4 * H0.kpad;
     G.Ma_stride = (int64_t)s.nsa * s.nsa;
     G.plan_gen = G.prog->plan_gen;
-    G.mats_stride = tiles_mats_doubles(s, *G.prog);
-    G.tpart_stride = tiles_partial_doubles(s, *G.prog);
-    G.spart_stride = row_sigma_group_partials(s, G.n);
+    G.sigma = s.sig;
+    G.mats_stride = tiles_mats_doubles(*G.tiles);
+    G.tpart_stride = tiles_partial_doubles(*G.tiles);
+    G.spart_stride = row_sigma_group_partials(s, G.sigma, G.n);
     SQ_CHECK(G.mats_stride > 0 && G.tpart_stride > 0 && G.spart_stride > 0, SQ_ERR_ARG, "group path unavailable");
     {
       const uint32_t a = s.h_astr[0], b = s.h_bstr[0];
@@ -571,15 +574,18 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
   }
 }
 
-// A grouped program whose tile shape changed after the batch was created has
-// a new tile plan: the group's buffers (and a captured graph) are sized for
-// the old one.
-// The group buffers are sized for the tile plan of each grouped program and
-// the row-sigma block count of each grouped space when the batch was made.
+// A group keeps the tile plan and the sigma shape that its buffers and graph
+// are made for.  Of instances of kKeepMinDim or more determinants the program
+// must outlive the batch, and a later change of its tile shape or of its
+// space's sigma shape is refused, as such groups always did; smaller instances,
+// which the persistent launch also serves, are free of both.
+constexpr int64_t kKeepMinDim = 16384;
+
 static void check_group(const BatchGroup& G) {
+  if (G.dim < kKeepMinDim) return;
   SQ_CHECK(G.prog->plan_gen == G.plan_gen, SQ_ERR_ARG,
            "a batched program's tile shape changed after the batch was created; create the batch again");
-  SQ_CHECK(row_sigma_group_partials(*G.space, G.n) == G.spart_stride, SQ_ERR_ARG,
+  SQ_CHECK(row_sigma_group_partials(*G.space, G.space->sig, G.n) == G.spart_stride, SQ_ERR_ARG,
            "a batched space's sigma shape changed after the batch was created; create the batch again");
 }
 
@@ -604,9 +610,9 @@ static void group_launch(const Batch& B, const BatchGroup& G, hipStream_t st) {
   const unsigned ib = (unsigned)std::min<int64_t>((G.dim + 255) / 256, 64);
   k_group_init<<<dim3(ib, (unsigned)G.n), 256, 0, st>>>(B.dev.psi0, G.d_inst, G.dim, G.hf, G.psi);
   SQ_HIP(hipGetLastError());
-  tiles_forward_group(s, *G.prog, G.theta, G.psi, G.mats, M, G.lam, st);
-  row_sigma_group(s, G.A, G.A_stride, G.Ma, G.Ma_stride, G.Mb, G.Mb_stride, G.psi, G.lam, G.spart, G.n, true, st);
-  tiles_reverse_group(s, *G.prog, G.theta, G.psi, G.lam, G.mats, G.tpart, G.grad, M, st);
+  tiles_forward_group(s, *G.tiles, G.theta, G.psi, G.mats, M, G.lam, st);
+  row_sigma_group(s, G.sigma, G.A, G.A_stride, G.Ma, G.Ma_stride, G.Mb, G.Mb_stride, G.psi, G.lam, G.spart, G.n, true, st);
+  tiles_reverse_group(s, *G.tiles, G.theta, G.psi, G.lam, G.mats, G.tpart, G.grad, M, st);
   k_group_out<<<(unsigned)G.n, 256, 0, st>>>(G.spart, G.spart_stride, G.grad, G.ng, G.d_inst, G.d_out0,
                                              B.dev.energy, B.dev.grad);
   SQ_HIP(hipGetLastError());
@@ -657,7 +663,9 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
         const Hamiltonian& H = hams[i]->h;
         SQ_CHECK(p.space == &s && H.space == &s, SQ_ERR_ARG, "program / Hamiltonian built for another space");
         SQ_CHECK(s.dim < (int64_t)1 << 30, SQ_ERR_ARG, "batched spaces must have fewer than 2^30 determinants");
-        if (groups_on && s.dim >= kGroupMinDim && H.d_Ma && row_sigma_group_ok(s) && tiles_group_ok(s, p)) {
+        std::shared_ptr<const TilePlan> tiles;
+        if (groups_on && s.dim >= kGroupMinDim && H.d_Ma && row_sigma_group_ok(s)) tiles = group_tiles_for(s, p);
+        if (tiles) {
           // a large instance: grouped with the instances of the same space and gate layout
           for (const GateDev& gd : p.gates)
             SQ_CHECK(gd.kind == GC_ROT || gd.kind == GC_SA_SINGLE, SQ_ERR_ARG,
@@ -669,6 +677,7 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
             BatchGroup G;
             G.space = &s;
             G.prog = &p;
+            G.tiles = tiles;
             G.ng = (int)p.gates.size();
             B.groups.push_back(G);
           }

@@ -810,7 +810,6 @@ int sq_program_destroy(sq_program* pr) {
     if (pr->p.d_term_fast) (void)hipFree(pr->p.d_term_fast);
     if (pr->p.ucc_t) ucc_t_free(pr->p.ucc_t);
     if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
-    if (pr->p.group_tiles) destroy_tile_plan(pr->p.group_tiles);
     if (pr->p.small) small_plan_free(pr->p.small);
     host_slots_free(pr->p);
     delete pr;
@@ -826,10 +825,9 @@ int sq_program_set_tile_shape(sq_program* pr, int target, int threads) {
     std::lock_guard<std::recursive_mutex> lock(pr->p.plan_mu);
     if (pr->p.tile_target == target && pr->p.tile_threads == threads) return;
     SQ_HIP(hipDeviceSynchronize());  // the old plan's buffers may be in use by queued kernels
-    for (TilePlan** t : {&pr->p.tiles, &pr->p.group_tiles}) {
-      if (*t) destroy_tile_plan(*t);
-      *t = nullptr;
-    }
+    if (pr->p.tiles) destroy_tile_plan(pr->p.tiles);
+    pr->p.tiles = nullptr;
+    pr->p.group_tiles.reset();
     pr->p.tiles_built = pr->p.group_tiles_built = false;
     ++pr->p.plan_gen;
     pr->p.tile_target = target;

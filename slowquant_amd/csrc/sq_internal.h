@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -107,6 +108,11 @@ struct GatePoly {
 };
 GatePoly gate_poly(const GateDev& g);
 
+// Row sigma shape (sq_sigma_configure): 0 / -1 = automatic.
+struct SigmaShape {
+  int R = 0, nsplit = 0, det = -1;
+};
+
 struct Space {
   int n, na, nb;
   int nsa, nsb;
@@ -132,8 +138,7 @@ struct Space {
   uint32_t* d_nbr = nullptr;
   int32_t* d_nbr_off = nullptr;
   uint8_t* d_nbr_tile = nullptr;
-  // row sigma shape (sq_sigma_configure): 0 / -1 = automatic
-  int sig_R = 0, sig_nsplit = 0, sig_det = -1;
+  SigmaShape sig;
   std::vector<uint32_t> h_astr, h_bstr;
   // RDM tables (sq_rdm.hip), built on first use
   mutable std::mutex rdm_mu;
@@ -163,7 +168,7 @@ struct Program {
   mutable std::recursive_mutex plan_mu;
   mutable TilePlan* tiles = nullptr;  // built on first use (sq_tiles.hip)
   mutable bool tiles_built = false;
-  mutable TilePlan* group_tiles = nullptr;  // the plan of batched groups
+  mutable std::shared_ptr<TilePlan> group_tiles;  // the plan of batched groups, which share it
   mutable bool group_tiles_built = false;
   mutable SmallPlan* small = nullptr;  // one-block sweep, built on first use (sq_small.hip)
   mutable bool small_tried = false;
@@ -323,22 +328,23 @@ struct Multi {
   int n = 1;
   int64_t theta = 0, mats = 0, vec = 0, part = 0, grad = 0;
 };
-// Group path of a program: every stage tiled, no side launches.
-bool tiles_group_ok(const Space& s, const Program& p);
-int64_t tiles_mats_doubles(const Space& s, const Program& p);     // pair matrices per instance
-int64_t tiles_partial_doubles(const Space& s, const Program& p);  // gradient partials per instance
+// Group plan of a program: every stage tiled (else nullptr).
+std::shared_ptr<const TilePlan> group_tiles_for(const Space& s, const Program& p);
+int64_t tiles_mats_doubles(const TilePlan& T);     // pair matrices per instance
+int64_t tiles_partial_doubles(const TilePlan& T);  // gradient partials per instance
 // psi (in place, start states already there) = U(theta) psi for every instance
-void tiles_forward_group(const Space& s, const Program& p, const double* theta, double* psi, double* mats,
+void tiles_forward_group(const Space& s, const TilePlan& T, const double* theta, double* psi, double* mats,
                          const Multi& M, double* zero, hipStream_t st);
 // reverse sweep on (psi, lam) with dE/dtheta into grad (n x gates)
-void tiles_reverse_group(const Space& s, const Program& p, const double* theta, double* psi, double* lam,
+void tiles_reverse_group(const Space& s, const TilePlan& T, const double* theta, double* psi, double* lam,
                          const double* mats, double* partial, double* grad, const Multi& M, hipStream_t st);
 // sigma = H psi for n instances of one space (row form with the string
 // products' tiles in the launch); A, Ma and Mb per instance at the given strides; energy
 // partials per instance (row_sigma_group_partials of them) at partial.
+// shape: the space's, or an earlier one of it.
 bool row_sigma_group_ok(const Space& s);
-int64_t row_sigma_group_partials(const Space& s, int n);
-void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
+int64_t row_sigma_group_partials(const Space& s, const SigmaShape& shape, int n);
+void row_sigma_group(const Space& s, const SigmaShape& shape, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
                      const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
                      bool zeroed, hipStream_t st);
 // tiles_whole: every stage is tiled, so theta is read by the first and last

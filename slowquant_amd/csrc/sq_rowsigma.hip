@@ -1035,8 +1035,8 @@ size_t row_lds(const Space& s, int mt, int R, bool scatter, bool list = false) {
 // The space's kernel shape choices (sq_sigma_configure) override these
 // defaults: rows per block, string product split, and the deterministic (staged)
 // form instead of the scatter form (default: SQ_SIGMA_DETERMINISTIC, else 0).
-bool row_deterministic(const Space& s) {
-  if (s.sig_det >= 0) return s.sig_det != 0;
+bool row_deterministic(const SigmaShape& shape) {
+  if (shape.det >= 0) return shape.det != 0;
   static int v = -1;
   if (v < 0) v = env_int("SQ_SIGMA_DETERMINISTIC", 0) != 0 ? 1 : 0;
   return v == 1;
@@ -1072,9 +1072,9 @@ int string_gemm_split(const Space& s) {
 // on n.
 constexpr int kManyInst = 8;
 
-bool row_plan(const Space& s, RowPlan* out, int n = 1) {
+bool row_plan(const Space& s, const SigmaShape& shape, RowPlan* out, int n) {
   if (s.dim == 0 || s.nsb > 16384 || s.npair + 1 > 255 || s.dim >= ((int64_t)1 << 31)) return false;
-  const bool scatter = !row_deterministic(s);
+  const bool scatter = !row_deterministic(shape);
   const int kpad = rup(s.npair + 1, 16);
   if (row_lds(s, 1, 1, scatter) > kLdsMax) return false;
   const bool list = scatter && list_form(s);
@@ -1111,8 +1111,8 @@ bool row_plan(const Space& s, RowPlan* out, int n = 1) {
     }
   }
   if (bestR == 0) return false;
-  if (s.sig_R > 0) {
-    const int R = s.sig_R;
+  if (shape.R > 0) {
+    const int R = shape.R;
     if (R <= s.nsa && row_lds(s, mt, R, scatter, list) <= kLdsMax &&
         (scatter || (int64_t)R * s.nsb <= (int64_t)kMaxTargets * kRowThreads))
       bestR = R;
@@ -1130,7 +1130,7 @@ bool row_plan(const Space& s, RowPlan* out, int n = 1) {
     nsplit = std::max(1, std::min({nsplit, kMaxSplit, (len + 15) / 16}));
     return rup((len + nsplit - 1) / nsplit, 16);
   };
-  int nsplit = s.sig_nsplit;
+  int nsplit = shape.nsplit;
   if (nsplit <= 0) nsplit = list ? string_gemm_split(s) : (s.nsa >= 2048 ? 1 : 2);
   out->kchunk = chunk(joined, nsplit);
   out->nsplit = (joined + out->kchunk - 1) / out->kchunk;
@@ -1145,7 +1145,7 @@ bool row_plan(const Space& s, RowPlan* out, int n = 1) {
   out->fused = list && fuse_env != 0 && 2 * out->lds <= kLdsMax && mt <= kMaxFusedMt;
   out->ngemm_a = out->ngemm_b = out->kchunk_b = 0;
   if (out->fused) {
-    const int split = s.sig_nsplit > 0 ? s.sig_nsplit : n >= kManyInst ? 1 : 4;
+    const int split = shape.nsplit > 0 ? shape.nsplit : n >= kManyInst ? 1 : 4;
     out->kchunk = chunk(s.nsa, split);
     out->kchunk_b = chunk(s.nsb, split);
     const int tiles = ((s.nsa + kGemmRows - 1) / kGemmRows) * ((s.nsb + kGemmCols - 1) / kGemmCols);
@@ -1157,6 +1157,8 @@ bool row_plan(const Space& s, RowPlan* out, int n = 1) {
   }
   return true;
 }
+
+bool row_plan(const Space& s, RowPlan* out) { return row_plan(s, s.sig, out, 1); }
 
 bool rows_enabled() {
   static int v = -1;
@@ -1464,7 +1466,7 @@ int64_t row_sigma_used_doubles(const Space& s) {
   if (pl.fused) return (int64_t)pl.ngroups + pl.ngemm_a + pl.ngemm_b;
   // at least two partial products are asked for below 2048 alpha strings, so
   // that the spaces the no-allocation entry point takes do not depend on the form
-  const int least = s.sig_nsplit > 0 ? pl.nsplit : s.nsa >= 2048 ? 1 : 2;
+  const int least = s.sig.nsplit > 0 ? pl.nsplit : s.nsa >= 2048 ? 1 : 2;
   return (int64_t)std::max(pl.nsplit, least) * s.dim + pl.ngroups;
 }
 
@@ -1478,17 +1480,17 @@ bool row_sigma_group_ok(const Space& s) {
   return rows_enabled() && s.d_rtb != nullptr && row_plan(s, &pl) && pl.scatter && pl.fused;
 }
 
-int64_t row_sigma_group_partials(const Space& s, int n) {
+int64_t row_sigma_group_partials(const Space& s, const SigmaShape& shape, int n) {
   RowPlan pl;
-  if (!row_plan(s, &pl, n) || !pl.fused) return 0;
+  if (!row_plan(s, shape, &pl, n) || !pl.fused) return 0;
   return (int64_t)pl.ngroups + pl.ngemm_a + pl.ngemm_b;
 }
 
-void row_sigma_group(const Space& s, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
+void row_sigma_group(const Space& s, const SigmaShape& shape, const double* A, int64_t A_stride, const double* Ma, int64_t Ma_stride,
                      const double* Mb, int64_t Mb_stride, const double* psi, double* sigma, double* partial, int n,
                      bool zeroed, hipStream_t st) {
   RowPlan pl;
-  SQ_CHECK(row_sigma_group_ok(s) && row_plan(s, &pl, n) && n > 0 && n <= 65535, SQ_ERR_ARG,
+  SQ_CHECK(row_plan(s, shape, &pl, n) && pl.fused && n > 0 && n <= 65535, SQ_ERR_ARG,
            "the grouped row sigma does not apply to this space");
   rows_list_launch(s, pl, A, A_stride, rup(s.npair + 1, 16), Ma, Ma_stride, Mb, Mb_stride, psi, nullptr, 0, sigma,
                    partial, n, zeroed, st);
@@ -1504,14 +1506,12 @@ extern "C" int sq_sigma_configure(sq_space* sp, int rows_per_block, int nsplit, 
     sq::Space& s = sp->s;
     sq::RowPlan pl;
     const bool before = sq::row_plan(s, &pl);
-    const int old[3] = {s.sig_R, s.sig_nsplit, s.sig_det};
-    s.sig_R = rows_per_block;
-    s.sig_nsplit = nsplit;
-    s.sig_det = deterministic < 0 ? -1 : (deterministic != 0);
+    const sq::SigmaShape old = s.sig;
+    s.sig.R = rows_per_block;
+    s.sig.nsplit = nsplit;
+    s.sig.det = deterministic < 0 ? -1 : (deterministic != 0);
     if (before && !sq::row_plan(s, &pl)) {  // the workspace sizes assume the row path
-      s.sig_R = old[0];
-      s.sig_nsplit = old[1];
-      s.sig_det = old[2];
+      s.sig = old;
       throw sq::Error{SQ_ERR_ARG, "this sigma form does not fit the space"};
     }
   });

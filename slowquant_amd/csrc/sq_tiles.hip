@@ -848,30 +848,35 @@ TilePlan* build_tile_plan(const Space& sp, const Program& P, int instances) {
 
 void destroy_tile_plan(TilePlan* T) { delete T; }
 
-static bool usable(const TilePlan* T) { return T && T->nops > 0; }
-
-// Tiled stages are used unless SQ_TILES=0.  Groups of instances (sq_batch.hip)
-// have a plan of their own: with many instances per launch the widest window
-// is the best one.
-static const TilePlan* plan_of(const Space& s, const Program& p, TilePlan*& slot, bool& built, int instances) {
-  std::lock_guard<std::recursive_mutex> lock(p.plan_mu);
-  if (!built) {
-    built = true;
-    const char* env = getenv("SQ_TILES");
-    bool enabled = !(env && env[0] == '0');
-    if (enabled && s.dim > 0 && s.nsb <= 65535) slot = build_tile_plan(s, p, instances);
-    if (slot && !usable(slot)) {
-      destroy_tile_plan(slot);
-      slot = nullptr;
-    }
-  }
-  return slot;
+// A plan with tiled stages, or nullptr.  They are used unless SQ_TILES=0.
+static TilePlan* make_plan(const Space& s, const Program& p, int instances) {
+  const char* env = getenv("SQ_TILES");
+  if ((env && env[0] == '0') || s.dim == 0 || s.nsb > 65535) return nullptr;
+  TilePlan* T = build_tile_plan(s, p, instances);
+  if (T->nops > 0) return T;
+  destroy_tile_plan(T);
+  return nullptr;
 }
 
-const TilePlan* tiles_for(const Space& s, const Program& p) { return plan_of(s, p, p.tiles, p.tiles_built, 1); }
+const TilePlan* tiles_for(const Space& s, const Program& p) {
+  std::lock_guard<std::recursive_mutex> lock(p.plan_mu);
+  if (!p.tiles_built) {
+    p.tiles_built = true;
+    p.tiles = make_plan(s, p, 1);
+  }
+  return p.tiles;
+}
 
-static const TilePlan* group_tiles_for(const Space& s, const Program& p) {
-  return plan_of(s, p, p.group_tiles, p.group_tiles_built, 64);
+// Groups of instances (sq_batch.hip) have a plan of their own: with many
+// instances per launch the widest window is the best one.
+std::shared_ptr<const TilePlan> group_tiles_for(const Space& s, const Program& p) {
+  std::lock_guard<std::recursive_mutex> lock(p.plan_mu);
+  if (!p.group_tiles_built) {
+    p.group_tiles_built = true;
+    p.group_tiles.reset(make_plan(s, p, 64));
+    if (p.group_tiles && !tiles_whole(*p.group_tiles)) p.group_tiles.reset();
+  }
+  return p.group_tiles;
 }
 
 bool tiles_cover(const Space& s, const Program& p) {
@@ -1611,41 +1616,27 @@ void tiles_reverse(const Space& s, const Program& p, const TilePlan& T, const do
 
 // ---- groups of instances of one program ------------------------------------
 
-bool tiles_group_ok(const Space& s, const Program& p) {
-  const TilePlan* T = group_tiles_for(s, p);
-  return T && tiles_whole(*T);
-}
+int64_t tiles_mats_doubles(const TilePlan& T) { return (int64_t)T.nops * kMatVals; }
 
-int64_t tiles_mats_doubles(const Space& s, const Program& p) {
-  const TilePlan* T = group_tiles_for(s, p);
-  return T ? (int64_t)T->nops * kMatVals : 0;
-}
+int64_t tiles_partial_doubles(const TilePlan& T) { return std::max<int64_t>(T.partial_len, 1); }
 
-int64_t tiles_partial_doubles(const Space& s, const Program& p) {
-  const TilePlan* T = group_tiles_for(s, p);
-  return T ? std::max<int64_t>(T->partial_len, 1) : 0;
-}
-
-void tiles_forward_group(const Space& s, const Program& p, const double* theta, double* psi, double* mats,
+void tiles_forward_group(const Space& s, const TilePlan& T, const double* theta, double* psi, double* mats,
                          const Multi& M, double* zero, hipStream_t st) {
-  const TilePlan* T = group_tiles_for(s, p);
-  SQ_CHECK(T && tiles_group_ok(s, p) && M.n > 0 && M.n <= 65535, SQ_ERR_ARG, "program has no group tile path");
-  launch_mats(*T, theta, -1, mats, M, st, nullptr, zero, s.dim);
-  for (const Stage& S : T->stages)
-    SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1) * M.n, 0.0, launch_fwd(*T, S, mats, false, psi, psi, M, st));
+  SQ_CHECK(M.n > 0 && M.n <= 65535, SQ_ERR_ARG, "too many instances in one batched group");
+  launch_mats(T, theta, -1, mats, M, st, nullptr, zero, s.dim);
+  for (const Stage& S : T.stages)
+    SQ_PROF(PC_TILE_FWD, st, stage_bytes(s, 1) * M.n, 0.0, launch_fwd(T, S, mats, false, psi, psi, M, st));
 }
 
-void tiles_reverse_group(const Space& s, const Program& p, const double* theta, double* psi, double* lam,
+void tiles_reverse_group(const Space& s, const TilePlan& T, const double* theta, double* psi, double* lam,
                          const double* mats, double* partial, double* grad, const Multi& M, hipStream_t st) {
-  const TilePlan* T = group_tiles_for(s, p);
-  SQ_CHECK(T && tiles_group_ok(s, p) && M.n > 0 && M.n <= 65535, SQ_ERR_ARG, "program has no group tile path");
-  for (int i = (int)T->stages.size() - 1; i >= 0; --i) {
-    const Stage& S = T->stages[i];
+  for (int i = (int)T.stages.size() - 1; i >= 0; --i) {
+    const Stage& S = T.stages[i];
     const int wb = i > 0 ? 1 : 0;
     SQ_PROF(PC_TILE_REV, st, stage_bytes(s, wb ? 2 : 1) * M.n, 0.0,
-            launch_rev(*T, S, mats, psi, lam, partial, wb, M, st));
+            launch_rev(T, S, mats, psi, lam, partial, wb, M, st));
   }
-  launch_grad(*T, theta, partial, grad, M, st);
+  launch_grad(T, theta, partial, grad, M, st);
 }
 
 }  // namespace sq
