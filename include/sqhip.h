@@ -215,7 +215,8 @@ int sq_ucc_energy_grad(const sq_space* s, const sq_program* p, const sq_hamilton
  * to 12 orbitals.  n_workgroups <= 0 picks 256.  Instances of 4096 or more
  * determinants whose programs are all brick stages run instead in groups
  * of equal (space, gate layout) through the tile-stage, row-sigma and
- * gradient kernels with one grid row per instance (SQ_BATCH_GROUPS=0 keeps
+ * gradient kernels with one grid row per instance (below 16384 determinants
+ * not where many groups of few would take longer; SQ_BATCH_GROUPS=0 keeps
  * them in the persistent launch).  A group keeps the tile plan and row-sigma
  * shape of the batch's creation.  Programs of 16384 or more determinants must
  * outlive the batch, and changing such a program's tile shape

@@ -421,6 +421,10 @@ __global__ void k_group_out(const double* __restrict__ spart, int64_t nblk, cons
 // to 9 orbitals 3030, 375, 377; 38 of 4 to 7 orbitals 272, 271, 244.
 constexpr int64_t kGroupMinDim = 4096;
 
+// From here on instances are always grouped (one workgroup needs 3 ms and more
+// for an evaluation), and the batch's user keeps their programs (check_group).
+constexpr int64_t kKeepMinDim = 16384;
+
 // Streams the groups run on: one group's short kernels and the ends of its long
 // ones leave CUs idle that another group's fill (256 instances as above on 1,
 // 3 and 4: 1549, 1329, 1206 us; there are four hardware queues).
@@ -506,6 +510,94 @@ static std::string layout_key(const Program& p) {
   return k;
 }
 
+// About how long a group takes on its stream (us): its chain of launches and its
+// work (29 instances of (10e,10o) with three layers: 800).
+static double group_us(int n, const Space& s, int ng) {
+  return 100.0 + 1.3e-6 * (double)n * (double)s.dim * (ng + 4.0 * s.npair);
+}
+
+static size_t a_bytes(const Space& s) {
+  return sizeof(double) * (size_t)((s.npair + 1 + 3) / 4 * 4) * (size_t)((s.npair + 1 + 15) / 16 * 16);
+}
+
+// Work of an instance of the persistent launch, in amplitudes touched.
+static int64_t persistent_cost(const Space& s, int rotations) {
+  const int K4 = (s.npair + 1 + 3) / 4 * 4;
+  return s.dim * (int64_t)(2 * rotations + 4 + 2 * s.npair + (s.npair * K4) / 8);
+}
+
+// About how long one workgroup takes for it (us, vectors in LDS or not): (7: 4,3)
+// with three layers 238, (8e,8o) 608, (9: 5,4) in scratch 3030.
+static double persistent_us(const Space& s, const Program& p, bool vec_lds) {
+  int rotations = 0;
+  for (const GateDev& g : p.gates) rotations += g.kind == GC_SA_SINGLE ? 2 : 1;
+  return (vec_lds ? 1.0 : 1.6) * (1.4 * rotations + 2e-4 * (double)persistent_cost(s, rotations));
+}
+
+// Instances of one space and gate layout that can run as a group.
+struct GroupCand {
+  std::shared_ptr<const TilePlan> tiles;
+  std::vector<int> mem;
+  bool keep = true;
+};
+
+// Many groups of few instances below kKeepMinDim are chains of launches that
+// wait for the four streams, while one persistent launch holds 256 of them: the
+// ones with the fewest members go there (to 12 orbitals) as far as that takes
+// less by a fifth (by the times above).  Sixty instances of (8e,8o) with as many layouts: groups
+// 2550 us, persistent launch 765; 256 instances of 4 to 10 orbitals keep their
+// groups.
+static void drop_small_groups(std::vector<GroupCand>& cands, const std::vector<int>& rest,
+                              const sq_space* const* spaces, const sq_program* const* programs, int n_workgroups) {
+  auto space = [&](int i) -> const Space& { return spaces[i]->s; };
+  auto program = [&](int i) -> const Program& { return programs[i]->p; };
+  double tg = 0.0;
+  std::vector<int> order;
+  auto time = [&](const GroupCand& c) {  // many chains in a graph: 50 us more each
+    return (50.0 + group_us((int)c.mem.size(), space(c.mem[0]), (int)program(c.mem[0]).gates.size())) / kGroupLanes;
+  };
+  for (size_t i = 0; i < cands.size(); ++i) {
+    tg += time(cands[i]);
+    if (space(cands[i].mem[0]).dim < kKeepMinDim && space(cands[i].mem[0]).n <= 12) order.push_back((int)i);
+  }
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int a, int b) { return cands[a].mem.size() < cands[b].mem.size(); });
+  // the persistent launch with the rest and the first k candidates of the order
+  size_t lds = 0, count = 0;
+  int64_t dmax = 0;
+  double longest[2] = {0.0, 0.0}, total[2] = {0.0, 0.0};  // scratch, LDS
+  auto add = [&](int i) {
+    lds = std::max(lds, a_bytes(space(i)));
+    dmax = std::max(dmax, space(i).dim);
+    ++count;
+    for (int l = 0; l < 2; ++l) {
+      const double us = persistent_us(space(i), program(i), l == 1);
+      longest[l] = std::max(longest[l], us);
+      total[l] += us;
+    }
+  };
+  auto persistent = [&] {
+    if (count == 0) return 0.0;
+    const int l = lds + 2 * sizeof(double) * (size_t)dmax <= kBatchLds ? 1 : 0;
+    return std::max(longest[l], total[l] / (double)std::min<size_t>(n_workgroups > 0 ? n_workgroups : 256, count));
+  };
+  for (int i : rest) add(i);
+  auto both = [&] {  // side by side, in each other's way
+    const double tp = persistent();
+    return std::max(tg, tp) + 0.5 * std::min(tg, tp);
+  };
+  double best = 0.8 * both();
+  size_t drop = 0;
+  for (size_t k = 0; k < order.size(); ++k) {
+    const GroupCand& c = cands[order[k]];
+    tg -= time(c);
+    for (int i : c.mem) add(i);
+    const double t = both();
+    if (t < best) best = t, drop = k + 1;
+  }
+  for (size_t k = 0; k < drop; ++k) cands[order[k]].keep = false;
+}
+
 template <class T>
 static T* balloc(Batch& B, size_t n) {
   T* d = nullptr;
@@ -579,8 +671,6 @@ static void build_groups(Batch& B, const sq_hamiltonian* const* hams, const sq_s
 // must outlive the batch, and a later change of its tile shape or of its
 // space's sigma shape is refused, as such groups always did; smaller instances,
 // which the persistent launch also serves, are free of both.
-constexpr int64_t kKeepMinDim = 16384;
-
 static void check_group(const BatchGroup& G) {
   if (G.dim < kKeepMinDim) return;
   SQ_CHECK(G.prog->plan_gen == G.plan_gen, SQ_ERR_ARG,
@@ -652,32 +742,53 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
       std::vector<double> Astore;
       std::vector<int64_t> cost(n_inst, 0);
       std::vector<char> grouped(n_inst, 0);
-      std::map<std::pair<const Space*, std::string>, int> group_of;  // (space, gate layout) -> group
-      const char* genv = getenv("SQ_BATCH_GROUPS");
-      const bool groups_on = !(genv && genv[0] == '0');
+      std::vector<GroupCand> cands;
+      std::vector<int> cand_of(n_inst, -1), cand_group;
+      {
+        const char* genv = getenv("SQ_BATCH_GROUPS");
+        const bool groups_on = !(genv && genv[0] == '0');
+        std::map<std::pair<const Space*, std::string>, int> index;  // (space, gate layout) -> candidate
+        std::vector<int> rest;
+        for (int i = 0; i < n_inst; ++i) {
+          const Space& s = spaces[i]->s;
+          const Program& p = programs[i]->p;
+          SQ_CHECK(p.space == &s && hams[i]->h.space == &s, SQ_ERR_ARG,
+                   "program / Hamiltonian built for another space");
+          std::shared_ptr<const TilePlan> tiles;
+          if (groups_on && s.dim >= kGroupMinDim && hams[i]->h.d_Ma && row_sigma_group_ok(s))
+            tiles = group_tiles_for(s, p);
+          if (!tiles) {
+            rest.push_back(i);
+            continue;
+          }
+          const auto key = std::make_pair(&s, layout_key(p));
+          auto it = index.find(key);
+          if (it == index.end()) {
+            it = index.emplace(key, (int)cands.size()).first;
+            cands.push_back(GroupCand{tiles, {}, true});
+          }
+          cand_of[i] = it->second;
+          cands[it->second].mem.push_back(i);
+        }
+        drop_small_groups(cands, rest, spaces, programs, n_workgroups);
+        cand_group.assign(cands.size(), -1);
+      }
       int theta_off = 0, grad_off = 0, npmax = 0;
       size_t small_lds = 0;  // A of the persistent launch's largest space
       for (int i = 0; i < n_inst; ++i) {
         const Space& s = spaces[i]->s;
         const Program& p = programs[i]->p;
         const Hamiltonian& H = hams[i]->h;
-        SQ_CHECK(p.space == &s && H.space == &s, SQ_ERR_ARG, "program / Hamiltonian built for another space");
         SQ_CHECK(s.dim < (int64_t)1 << 30, SQ_ERR_ARG, "batched spaces must have fewer than 2^30 determinants");
-        std::shared_ptr<const TilePlan> tiles;
-        if (groups_on && s.dim >= kGroupMinDim && H.d_Ma && row_sigma_group_ok(s)) tiles = group_tiles_for(s, p);
-        if (tiles) {
-          // a large instance: grouped with the instances of the same space and gate layout
-          for (const GateDev& gd : p.gates)
-            SQ_CHECK(gd.kind == GC_ROT || gd.kind == GC_SA_SINGLE, SQ_ERR_ARG,
-                     "batched launches support rotation gates (single, double, sa_single, pair doubles) only");
-          const auto key = std::make_pair(&s, layout_key(p));
-          auto it = group_of.find(key);
-          if (it == group_of.end()) {
-            it = group_of.emplace(key, (int)B.groups.size()).first;
+        if (cand_of[i] >= 0 && cands[cand_of[i]].keep) {
+          // grouped with the instances of the same space and gate layout
+          int& group = cand_group[cand_of[i]];
+          if (group < 0) {
+            group = (int)B.groups.size();
             BatchGroup G;
             G.space = &s;
             G.prog = &p;
-            G.tiles = tiles;
+            G.tiles = cands[cand_of[i]].tiles;
             G.ng = (int)p.gates.size();
             B.groups.push_back(G);
           }
@@ -690,7 +801,7 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
           B.grad_off.push_back(grad_off);
           grad_off += I.nparam;
           B.inst.push_back(I);
-          B.group_members.push_back({it->second, i});
+          B.group_members.push_back({group, i});
           continue;
         }
         if (!sp_index.count(spaces[i])) {
@@ -751,7 +862,7 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
           npmax = std::max(npmax, bs.npair);
           small_lds = std::max<size_t>(small_lds, sizeof(double) * bs.K4 * bs.kpad);
         }
-        cost[i] = s.dim * (int64_t)(2 * I.ngate + 4 + 2 * bs.npair + (bs.npair * bs.K4) / 8);
+        cost[i] = persistent_cost(s, I.ngate);
       }
       SQ_CHECK(B.lds <= 65536, SQ_ERR_ARG, "batched spaces limited to 12 orbitals (LDS)");
       for (const auto& bs : bsp)
@@ -894,12 +1005,7 @@ static void batch_launch(Batch& B, hipStream_t st) {
     SQ_PROF(PC_BATCH, B.side, B.bytes, B.flops, batch_kernel(B)<<<B.nwg, kBT, B.lds, B.side>>>(B.dev));
   }
   for (int l = 1; l < nl; ++l) SQ_HIP(hipStreamWaitEvent(B.lane[l], B.ev_fork, 0));
-  // about how long a group takes (us): its chain of launches and its work
-  // (29 instances of (10e,10o) with three layers: 800)
-  auto us = [&](int i) {
-    const BatchGroup& G = B.groups[i];
-    return 100.0 + 1.3e-6 * (double)G.n * (double)G.dim * (G.ng + 4.0 * G.space->npair);
-  };
+  auto us = [&](int i) { return group_us(B.groups[i].n, *B.groups[i].space, B.groups[i].ng); };
   std::vector<int> order(B.groups.size());
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return us(a) > us(b); });
