@@ -7,7 +7,8 @@ chosen here by timing on first use and remembered per device and workload:
 * single instance (a space and a gate program): the fused rotation stages'
   tile size (sq_program_set_tile_shape: elements and threads per tile) by timing whole energy + gradient
   evaluations, then the row sigma's rows per block and string product split
-  (sq_sigma_configure) by timing sigma alone;
+  (sq_sigma_configure) by timing sigma alone; the automatic shapes (0) are
+  among them, and are kept unless whole evaluations with the choice are faster;
 * batched instances: the persistent launch's workgroup count and kernel shape
   (engine.autotune_batch), keyed by the instance list.
 
@@ -32,9 +33,9 @@ from . import _native as N
 from . import engine as E
 
 TILE_TARGETS = (0, 256, 512, 1024, 2048, 4096)
-TILE_THREADS = (512, 256)
+TILE_THREADS = (0, 512, 256)
 SIGMA_ROWS = (0, 1, 2, 3, 4)
-SIGMA_SPLITS = (1, 2, 4)
+SIGMA_SPLITS = (0, 1, 2, 4)
 
 
 def cache_path() -> str:
@@ -72,7 +73,7 @@ def _device_key() -> str:
 
 def program_key(space: E.Space, prog: E.Program) -> str:
     h = hashlib.sha1(json.dumps([prog.types, prog.indices]).encode()).hexdigest()[:16]
-    return f"{_device_key()}|ups|{space.n_orb},{space.n_alpha},{space.n_beta}|{h}"
+    return f"{_device_key()}|ups2|{space.n_orb},{space.n_alpha},{space.n_beta}|{h}"
 
 
 def _time(fn, reps: int) -> float:
@@ -131,10 +132,18 @@ def tune(space: E.Space, prog: E.Program, H: E.Hamiltonian, theta, psi0: torch.T
             dt = _time(lambda: H.sigma(psi, want_energy=False), 4 * reps)
             if dt < best_st:
                 best_sig, best_st = (r, ns), dt
-    space.configure_sigma(*best_sig)
-    ms = 1e3 * _time(evaluate, reps)
+    default = dict.fromkeys(("tile_target", "tile_threads", "rows_per_block", "nsplit"), 0)
     choice = {"tile_target": best_tile[0], "tile_threads": best_tile[1], "rows_per_block": best_sig[0],
-              "nsplit": best_sig[1], "ms_per_eval": ms}
+              "nsplit": best_sig[1]}
+    t = {False: float("inf"), True: float("inf")}
+    for _ in range(3):
+        for tuned in t:
+            apply(space, prog, choice if tuned else default)
+            t[tuned] = min(t[tuned], _time(evaluate, reps))
+    if t[True] >= t[False]:
+        choice = default
+        apply(space, prog, choice)
+    choice["ms_per_eval"] = 1e3 * min(t.values())
     if use_cache:
         _store(key, choice)
     return {**choice, "cached": False}
