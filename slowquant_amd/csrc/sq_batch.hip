@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kBT) void k_batch(BatchDev B) {
     const BatchSpace S = B.spaces[I.space];
     const int nsb = S.nsb;
     const int dim = S.nsa * nsb;  // < 2^30, checked at creation
-    double* G = slot + 2 * B.dmax;
+    double* G = LDS ? slot : slot + 2 * B.dmax;
     const double* th = B.theta + I.theta0;
     const double* start = B.psi0[B.wg_list[li]];
     if (start) {
@@ -773,8 +773,8 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
         drop_small_groups(cands, rest, spaces, programs, n_workgroups);
         cand_group.assign(cands.size(), -1);
       }
-      int theta_off = 0, grad_off = 0, npmax = 0;
-      size_t small_lds = 0;  // A of the persistent launch's largest space
+      int theta_off = 0, grad_off = 0;
+      int64_t gmax = 0;  // G of the persistent launch's instances, at most
       for (int i = 0; i < n_inst; ++i) {
         const Space& s = spaces[i]->s;
         const Program& p = programs[i]->p;
@@ -856,12 +856,9 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
         Astore.insert(Astore.end(), A.begin(), A.end());
         I.e_core = H.e_core;
         B.inst.push_back(I);
-        B.lds = std::max<size_t>(B.lds, sizeof(double) * bs.K4 * bs.kpad);
-        if (!grouped[i]) {
-          B.dmax = std::max<int64_t>(B.dmax, s.dim);
-          npmax = std::max(npmax, bs.npair);
-          small_lds = std::max<size_t>(small_lds, sizeof(double) * bs.K4 * bs.kpad);
-        }
+        B.lds = std::max(B.lds, a_bytes(s));
+        B.dmax = std::max<int64_t>(B.dmax, s.dim);
+        gmax = std::max<int64_t>(gmax, bs.npair * s.dim);
         cost[i] = persistent_cost(s, I.ngate);
       }
       SQ_CHECK(B.lds <= 65536, SQ_ERR_ARG, "batched spaces limited to 12 orbitals (LDS)");
@@ -891,12 +888,11 @@ int sq_batch_create(int n_inst, const sq_space* const* spaces, const sq_program*
         wo.push_back((int32_t)wl.size());
       }
       B.nwg = nwg;
-      B.slot = (2 + npmax) * B.dmax;
-      B.lds = small_lds;
-      B.dev.vec0 = (int64_t)(small_lds / sizeof(double));
-      const size_t with_vec = small_lds + 2 * sizeof(double) * (size_t)B.dmax;
+      B.dev.vec0 = (int64_t)(B.lds / sizeof(double));
+      const size_t with_vec = B.lds + 2 * sizeof(double) * (size_t)B.dmax;
       B.vec_lds = with_vec <= kBatchLds;
       if (B.vec_lds) B.lds = with_vec;
+      B.slot = gmax + (B.vec_lds ? 0 : 2 * B.dmax);
       B.dev.spaces = bupload(B, bsp);
       B.dev.inst = bupload(B, B.inst);
       B.dev.rots = bupload(B, rots);
