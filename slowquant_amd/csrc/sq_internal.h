@@ -404,6 +404,17 @@ namespace sq {
 // SQ_UCC_CSR=0).
 bool operator_apply_pattern(const Space& s, sq_operator& op, const double* in, double* out, hipStream_t st);
 void operator_pattern_free(sq_operator& op);
+// Barrier that waits for this wave's LDS operations only: global loads issued
+// ahead stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// x with its sign flipped where bit 31 of s is set.
+__device__ __forceinline__ double flip(double x, int s) {
+  return __hiloint2double(__double2hiint(x) ^ (s & (int)0x80000000), __double2loint(x));
+}
+
 // Sums across lanes in vector registers.
 template <int CTRL, int ROWS = 0xf>
 __device__ __forceinline__ double dpp_add(double v) {

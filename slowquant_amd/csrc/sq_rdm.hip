@@ -43,14 +43,6 @@ static inline int rup(int x, int m) { return (x + m - 1) / m * m; }
 
 namespace {
 
-__device__ __forceinline__ void lds_barrier() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-__device__ __forceinline__ double flip(double x, int s) {
-  return __hiloint2double(__double2hiint(x) ^ (s & (int)0x80000000), __double2loint(x));
-}
-
 // alist[s][w] (w a multiple of 16): the Ea_x that do not vanish on alpha
 // string s, {partner row * nsb, x | negative << 31}; the rest {own row, n^2}.
 __global__ void k_rdm_alist(int n, int nsa, int nsb, int w, const int32_t* __restrict__ full,

@@ -227,10 +227,6 @@ __global__ void k_string_ham(int nstr, int npair, int kpad, const int32_t* __res
 // Blocks take tiles in strips of 8 tile rows, contiguous per XCD.
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void lds_barrier() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 struct GemmArgs {
   const double *L0, *R0, *L1, *R1;
   double* out;
@@ -775,11 +771,6 @@ __global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(MT 
 // instance of a group (zero strides: one instance).
 constexpr int kAhead = 4;
 constexpr int kTrash = 64;  // doubles past each sigma row in LDS: targets of outputs that vanish
-
-// x with its sign flipped where bit 31 of s is set
-__device__ __forceinline__ double flip(double x, int s) {
-  return __hiloint2double(__double2hiint(x) ^ (s & (int)0x80000000), __double2loint(x));
-}
 
 struct RowArgs {
   const double *At, *psi, *sin, *Ma, *Mb;

@@ -402,13 +402,6 @@ struct Ahead {
   uint4 mem;
 };
 
-// Waits for this wave's LDS operations only: loads issued ahead stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  __asm__ volatile("" ::: "memory");
-}
-
 // One row of a component's matrix (M: the gate, T: its generator, both m x m in
 // LDS) on its members; the transpose where inv.  The rows of a component are
 // lanes of one wave, whose reads of the members all come before its writes.

@@ -1152,14 +1152,6 @@ __device__ __forceinline__ ConstPtr<T> as_const(const T* p) {
   return (ConstPtr<T>)(uintptr_t)p;
 }
 
-// Waits for this wave's LDS operations only: orbit words loaded ahead stay in
-// flight.
-__device__ __forceinline__ void lds_barrier() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  __asm__ volatile("" ::: "memory");
-}
-
 // A thread's orbit words of one pair op: wave v takes the wave-sized groups
 // v, v + NT / 64, ...
 template <int NT>
@@ -1283,23 +1275,6 @@ __device__ __forceinline__ void fwd_op(const OpItems& o, const Words<NT>& x, dou
   }
   if (deriv)  // T_g annihilates the amplitudes no gate moves
     for (int i = o.c5 * 64 + threadIdx.x; i < o.c6 * 64; i += NT) X[items[i]] = 0.0;
-}
-
-// DPP lane moves of a double (bound_ctrl: lanes without a source read 0).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_move(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-
-// Sum over each row of 16 lanes, in the row's last lane.
-__device__ __forceinline__ double row_sum(double v) {
-  v += dpp_move<0xb1, 0xf>(v);   // quad_perm [1,0,3,2]
-  v += dpp_move<0x4e, 0xf>(v);   // quad_perm [2,3,0,1]
-  v += dpp_move<0x114, 0xf>(v);  // row_shr:4
-  v += dpp_move<0x118, 0xf>(v);  // row_shr:8
-  return v;
 }
 
 // Wave sums of four values on the matrix cores.  v_mfma_f64_4x4x4 contracts
@@ -1472,14 +1447,14 @@ __global__ __launch_bounds__(NT) void k_win_rev(StageDev S, const double* __rest
         for (int q = 0; q < 4; ++q) s0 = rows_of(s0, sel[q], Q[q]);
         s1 = rows_of(s1, sel[0], Q[4]);
         s1 = rows_of(s1, sel[1], Q[5]);
-        s0 = row_sum(s0);
+        s0 = row16_sum(s0);
       }
       s1 = rows_of(s1, sel[2], Q[6]);
       s1 = rows_of(s1, sel[3], Q[7]);
       s2 = rows_of(s2, sel[0], Qe);
       s2 = rows_of(s2, sel[1], Qd);
-      s1 = row_sum(s1);
-      s2 = row_sum(s2);
+      s1 = row16_sum(s1);
+      s2 = row16_sum(s2);
       if ((lane & 15) == 15) {
         const int q = lane >> 4;
         red[j & 1][q][wave] = s0;

@@ -220,17 +220,16 @@ __global__ void k_csr_fill(SV v, const Term* __restrict__ terms, const TermFast*
   }
 }
 
-// nxt[I] = f sum_{entries (J, t, sign) of row I} sign w[t] coef[t] cur[J] and
-// acc[I] += nxt[I] (acc != nullptr), one wave per row: lane l takes entries
-// l, l + 64, ... and the wave sums in a fixed shuffle order.
+// out[I] = sum over the entries (J, t, sign) of row I of sign coef[t] in[J], one
+// wave per row: lane l takes entries l, l + 64, ... and the wave sums in a
+// fixed shuffle order.
 constexpr int kCsrRows = 4;  // rows (waves) per block
 
 __global__ __launch_bounds__(64 * kCsrRows) void k_tapply_csr(int64_t dim, const int64_t* __restrict__ rowp,
                                                               const uint2* __restrict__ ent,
                                                               const double* __restrict__ coef,
-                                                              const double* __restrict__ w,
-                                                              const double* __restrict__ cur, double f,
-                                                              double* __restrict__ nxt, double* __restrict__ acc) {
+                                                              const double* __restrict__ in,
+                                                              double* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const int64_t I = (int64_t)blockIdx.x * kCsrRows + (threadIdx.x >> 6);
   if (I >= dim) return;  // uniform per wave; no block barrier below
@@ -239,15 +238,11 @@ __global__ __launch_bounds__(64 * kCsrRows) void k_tapply_csr(int64_t dim, const
   for (int64_t k = b + lane; k < e; k += 64) {
     const uint2 x = ent[k];
     const uint32_t t = x.y & 0x7fffffffu;
-    const double c = (w ? w[t] : 1.0) * coef[t] * cur[x.x];
+    const double c = coef[t] * in[x.x];
     val += (x.y >> 31) ? -c : c;
   }
   for (int off = 32; off > 0; off >>= 1) val += __shfl_down(val, off, 64);
-  if (lane == 0) {
-    const double r = f * val;
-    nxt[I] = r;
-    if (acc) acc[I] += r;
-  }
+  if (lane == 0) out[I] = val;
 }
 
 // ---- merged pattern -------------------------------------------------------
@@ -946,7 +941,7 @@ bool operator_apply_pattern(const Space& s, sq_operator& op, const double* in, d
   if (!c) return false;
   SQ_PROF(PC_TAPPLY, st, 16.0 * (double)s.dim + 8.0 * (double)c->nnz, 0.0,
           k_tapply_csr<<<(unsigned)((s.dim + kCsrRows - 1) / kCsrRows), 64 * kCsrRows, 0, st>>>(
-              s.dim, c->rowp, c->ent, c->coef, nullptr, in, 1.0, out, nullptr));
+              s.dim, c->rowp, c->ent, c->coef, in, out));
   return true;
 }
 
