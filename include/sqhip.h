@@ -90,9 +90,9 @@ int sq_state_to_reference(const sq_space* s, const double* internal, double* ref
 int sq_program_create(const sq_space* s, const sq_gate_desc* gates, int n_gates, sq_program** out);
 int sq_program_destroy(sq_program* p);
 int sq_program_ngates(const sq_program* p);
-/* Tile shape of the fused rotation stages: elements per tile (0: automatic,
- * 256..2048 by the space's dimension; at most 4096) and threads per tile block
- * (256 or 512; 0: 512).  No counterpart in the reference (its gates have no
+/* Tile shape of the fused rotation stages: mean elements per tile (it sets the
+ * window width and the groups per tile; 0: both by a cost model) and threads
+ * per tile block (256 or 512; 0: 1024 where all tiles run at once, else 512).  No counterpart in the reference (its gates have no
  * tiles).  Synchronises the device and drops the program's tile plan, which
  * the next call rebuilds. */
 int sq_program_set_tile_shape(sq_program* p, int target, int threads);
@@ -195,12 +195,13 @@ int sq_rdm12(const sq_space* s, const double* psi, double* rdm1, double* rdm2, d
  * its generators T_k (G1_sa for "sa_single_ucc", G2_sa, G1..G6 anti-Hermitian)
  * form T(theta) = sum_k theta_k T_k.  work: sq_ucc_work_bytes(). */
 int64_t sq_ucc_work_bytes(const sq_space* s, const sq_program* p);
-/* out = exp(t T(theta)) in, matrix-free scaled Taylor series (in != out). */
+/* out = exp(t T(theta)) in, matrix-free, by a Taylor or Chebyshev series
+ * (in != out). */
 int sq_ucc_expm(const sq_space* s, const sq_program* p, const double* theta, double t, const double* in,
                 double* out, void* work, void* stream);
 /* energy = <psi|H|psi>, psi = exp(T(theta)) psi0, and (if grad != NULL) the
  * analytic dE/dtheta_i = 2 int_0^1 <e^{-sT} lam|T_i|e^{-sT} psi> ds (lam = H psi),
- * by composite 8-point Gauss-Legendre quadrature over s. */
+ * by Gauss-Legendre quadrature over s. */
 int sq_ucc_energy_grad(const sq_space* s, const sq_program* p, const sq_hamiltonian* H, const double* theta,
                        const double* psi0, double* energy, double* grad, void* work, void* stream);
 

@@ -173,7 +173,7 @@ struct Program {
   mutable SmallPlan* small = nullptr;  // one-block sweep, built on first use (sq_small.hip)
   mutable bool small_tried = false;
   int tile_target = 0;   // elements per tile (0: automatic; sq_program_set_tile_shape)
-  int tile_threads = 0;  // threads per tile block, 256 or 512 (0: 512)
+  int tile_threads = 0;  // threads per tile block, 256 or 512 (0: automatic)
   int plan_gen = 0;      // bumped whenever the tile plan is dropped (batched groups check it)
   std::vector<GateDev> gates;
   std::vector<Term> terms;

@@ -133,7 +133,7 @@ class Program:
 
     def set_tile_shape(self, target: int = 0, threads: int = 0) -> None:
         """Elements per tile (0: automatic) and threads per tile block (256 or
-        512; 0: 512) of the fused rotation stages."""
+        512; 0: automatic) of the fused rotation stages."""
         N.check(N.lib().sq_program_set_tile_shape(self._h, int(target), int(threads)))
 
     def theta_tensor(self, theta) -> torch.Tensor:
