@@ -222,6 +222,7 @@ struct Hamiltonian {
 
 // Row sigma (sq_rowsigma.hip)
 bool row_sigma_applies(const Space& s);
+bool sigma_deterministic(const Space& s);  // sums in a fixed order are asked for
 int64_t row_sigma_work_doubles(const Space& s);
 int64_t row_sigma_used_doubles(const Space& s);
 void build_string_hams(const Space& s, Hamiltonian& H);

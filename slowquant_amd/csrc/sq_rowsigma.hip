@@ -1161,6 +1161,8 @@ bool rows_enabled() {
 
 }  // namespace
 
+bool sigma_deterministic(const Space& s) { return row_deterministic(s.sig); }
+
 void string_grams(const double* C, const double* Ct, double* rho_a, double* rho_b, int nsa, int nsb, hipStream_t st) {
   const GemmArgs A{C, Ct, nullptr, nullptr, rho_a, nsa, nsa, nsb, 0, nsb};
   const GemmArgs B{Ct, C, nullptr, nullptr, rho_b, nsb, nsb, nsa, 0, nsa};

@@ -568,22 +568,26 @@ __global__ __launch_bounds__(kCB) void k_combine(int64_t dim, int K, Combine C, 
 
 // Gate dots: per merged element (I, J) r = sum_q V[I][q] U[J][q] over NQ
 // nodes (V carries the weights), added with sign |coef| to every
-// contribution's gate.  Gate sums in LDS per block, then to dpart[block][ng];
-// with more gates than LDS holds (lds = 0) to dpart[0][ng] by global atomics
-// (zeroed before).  One wave per row; a node row is 64 to 128 contiguous
-// bytes.
+// contribution's gate g in [g0, g0 + ng).  Gate sums in LDS, copies of them per
+// block, then to dpart[block][ng]; with more gates than LDS holds (copies = 0)
+// to dpart[0][ng] by global atomics (zeroed before).  One wave per row; a node
+// row is 64 to 128 contiguous bytes.
+// A copy per wave gives every sum a fixed order (a wave's LDS adds run in
+// program order, and those of one instruction by lane), so that the gradient is
+// the same bit for bit where lambda is.
 template <int NQ>
 __global__ __launch_bounds__(64 * kRows) void k_gate_dots_rows(
     int64_t dim, const int64_t* __restrict__ urow, const uint32_t* __restrict__ col,
     const uint32_t* __restrict__ first, const uint32_t* __restrict__ con, const double* __restrict__ coefs, int ncoef,
-    const double* __restrict__ U, const double* __restrict__ V, int ng, int lds, double* __restrict__ dpart) {
+    const double* __restrict__ U, const double* __restrict__ V, int g0, int ng, int copies,
+    double* __restrict__ dpart) {
   extern __shared__ double sg[];
   __shared__ double sc[1 << kCoefBits];
-  if (lds)
-    for (int i = threadIdx.x; i < ng; i += 64 * kRows) sg[i] = 0.0;
+  for (int i = threadIdx.x; i < copies * ng; i += 64 * kRows) sg[i] = 0.0;
   for (int i = threadIdx.x; i < ncoef; i += 64 * kRows) sc[i] = coefs[i];
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double* own = sg + (copies > 1 ? wave * ng : 0);
   for (int64_t I = (int64_t)blockIdx.x * kRows + wave; I < dim; I += (int64_t)gridDim.x * kRows) {
     const int64_t e = urow[I + 1];
     double v[NQ];
@@ -598,15 +602,20 @@ __global__ __launch_bounds__(64 * kRows) void k_gate_dots_rows(
       for (uint32_t c = first[u]; c < c1; ++c) {
         const uint32_t w = con[c];
         const double d = r * sc[(w >> kGateBits) & ((1u << kCoefBits) - 1u)];
-        const uint32_t g = w & ((1u << kGateBits) - 1u);
-        if (lds) atomicAdd(sg + g, (w >> 31) ? -d : d);
+        const uint32_t g = (w & ((1u << kGateBits) - 1u)) - (uint32_t)g0;
+        if (g >= (uint32_t)ng) continue;
+        if (copies) atomicAdd(own + g, (w >> 31) ? -d : d);
         else unsafeAtomicAdd(dpart + g, (w >> 31) ? -d : d);
       }
     }
   }
-  if (!lds) return;
+  if (!copies) return;
   __syncthreads();
-  for (int i = threadIdx.x; i < ng; i += 64 * kRows) dpart[(size_t)blockIdx.x * ng + i] = sg[i];
+  for (int i = threadIdx.x; i < ng; i += 64 * kRows) {
+    double sum = sg[i];
+    for (int c = 1; c < copies; ++c) sum += sg[c * ng + i];
+    dpart[(size_t)blockIdx.x * ng + i] = sum;
+  }
 }
 
 // nxt[I] = f * sum_g part[g][I]; acc[I] += nxt[I] when acc != nullptr.
@@ -1010,11 +1019,10 @@ struct ChebWork {
 
 constexpr int kAsmBlocks = 2048;
 static int64_t row_blocks(const Space& s, int64_t cap) { return std::min<int64_t>((s.dim + kRows - 1) / kRows, cap); }
-static int64_t gate_blocks(const Space& s, int64_t ng) { return ng <= kLdsGates ? row_blocks(s, 1024) : 1; }
 
 static int64_t cheb_head(const Space& s) { return (int64_t)max_nodes(s) * s.dim + 64 + kAsmBlocks; }
 static int64_t cheb_tail(const Space& s, int64_t ng) {
-  return (int64_t)(max_basis(s) + max_nodes(s) + 2) * s.dim + gate_blocks(s, ng) * ng;
+  return (int64_t)(max_basis(s) + max_nodes(s) + 2) * s.dim + std::max(ng, row_blocks(s, 1024) * std::min<int64_t>(ng, kLdsGates));
 }
 
 static ChebWork carve_cheb(const Space& s, double* work) {
@@ -1362,15 +1370,24 @@ static void series_expm(const Space& s, const UccT& T, const Series& S, int m, i
 
 static void gate_dots(const Space& s, const UccT& T, int n, int ng, const ChebWork& u, bool add, double* grad_dev,
                       double* grad_host, hipStream_t st) {
-  const bool lds = ng <= kLdsGates;
+  // a copy of the sums per wave where two blocks fit a CU, or where a fixed order
+  // is asked for, then at most kLdsGates gates per launch
+  const bool det = sigma_deterministic(s);
+  const int copies = det || ng <= kLdsGates / 2 ? kRows : ng <= kLdsGates ? 1 : 0;
   const unsigned nb = (unsigned)row_blocks(s, 1024);
   auto* kernel = n == 8 ? k_gate_dots_rows<8> : n == 12 ? k_gate_dots_rows<12> : k_gate_dots_rows<16>;
-  if (!lds) k_zero<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(u.dpart, ng);
-  SQ_PROF(PC_OTHER, st, 12.0 * (double)T.nu, 0.0,
-          kernel<<<nb, 64 * kRows, lds ? 8 * (size_t)ng : 0, st>>>(s.dim, T.urow, T.col, T.first, T.con, T.coefs, T.ncoef,
-                                                                 u.U, u.V, ng, lds ? 1 : 0, u.dpart));
-  k_gate_accum<<<(unsigned)((ng + kRows - 1) / kRows), 64 * kRows, 0, st>>>(u.dpart, lds ? (int)nb : 1, ng, 1.0,
-                                                                          add ? 1 : 0, grad_dev, grad_host);
+  const int per = copies ? std::min(ng, kLdsGates) : ng;
+  const size_t lds = 8 * (size_t)copies * per;
+  allow_lds(kernel, lds + 2048);
+  if (!copies) k_zero<<<(unsigned)((ng + kUB - 1) / kUB), kUB, 0, st>>>(u.dpart, ng);
+  for (int g0 = 0; g0 < ng; g0 += per) {
+    const int m = std::min(per, ng - g0);
+    SQ_PROF(PC_OTHER, st, 12.0 * (double)T.nu, 0.0,
+            kernel<<<nb, 64 * kRows, lds, st>>>(s.dim, T.urow, T.col, T.first, T.con, T.coefs, T.ncoef, u.U, u.V, g0, m,
+                                               copies, u.dpart));
+    k_gate_accum<<<(unsigned)((m + kRows - 1) / kRows), 64 * kRows, 0, st>>>(
+        u.dpart, copies ? (int)nb : 1, m, 1.0, add ? 1 : 0, grad_dev + g0, grad_host ? grad_host + g0 : nullptr);
+  }
   SQ_HIP(hipGetLastError());
 }
 
