@@ -135,9 +135,9 @@ int sq_sigma(const sq_space* s, const sq_hamiltonian* H, const double* psi, doub
  * reference (its sigma has no kernel shapes).  rows_per_block: alpha rows per
  * block (0: automatic); nsplit: partial products of the string products
  * (1..4, 0: automatic); deterministic: 1 selects the staged form whose sums
- * run in a fixed order (bit-identical results run to run), 0 the scatter form
+ * run in a fixed order (bit-identical results run to run), 0 the list form
  * (LDS atomics: equal to rounding, faster), -1 the SQ_SIGMA_DETERMINISTIC
- * environment default (scatter).  Takes effect at the next call; workspace
+ * environment default (list).  Takes effect at the next call; workspace
  * sizes do not change. */
 int sq_sigma_configure(sq_space* s, int rows_per_block, int nsplit, int deterministic);
 

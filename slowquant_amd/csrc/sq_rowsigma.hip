@@ -27,14 +27,14 @@
 // operand (no Mb):
 //     sigma = Ma C + e_core / 2 C + sum_k E+b_k G_k,
 //     G_k   = h'_k psi + sum_k' A(k,k') (2 E+a_k' + E+b_k') psi.
-// It takes 1.4 ((12e,12o)) to 1.2 ((14e,14o)) times the products of the list
+// It takes 1.4 ((12e,12o)) to 1.03 ((15e,15o)) times the products of the list
 // form and more vector instructions per product: (12e,12o) 271 -> 200 us a
 // sigma, (14e,14o) 7.07 -> 5.40 ms (rows 5.89 -> 2.76, string products 1.18 ->
-// 2.64), 10 orbitals in groups 325 -> 245 us.  It serves the larger spaces
-// (k_sigma_rows_scatter: the beta string product would cost more than it
-// saves) and, with a fixed order of every sum, deterministic runs
-// (k_sigma_rows: each wave's tile of G is staged in LDS and every target adds
-// the staged values of its beta neighbours in list order).
+// 2.64), (15: 7,7) 43.9 -> 28.9, (16: 6,6) 165 -> 55 (one 16-row tile of A at a
+// time beside two rows of 8008 in LDS), 10 orbitals in groups 325 -> 245 us.  It
+// serves deterministic runs, with a fixed order of every sum (k_sigma_rows: each
+// wave's tile of G is staged in LDS and every target adds the staged values of
+// its beta neighbours in list order).
 
 #include <algorithm>
 #include <cmath>
@@ -371,15 +371,11 @@ __global__ __launch_bounds__(256, 2) void k_string_grams(GemmArgs A, GemmArgs B)
 // unrolled by two with ping-pong registers: step s issues the alpha
 // amplitude and beta table loads of later steps before its MFMAs.
 
-template <int MT, int NSTEPS = 0>
+template <int MT>
 __device__ __forceinline__ void row_tile(double4_t (&acc)[MT], const double* __restrict__ sA,
                                          const double* __restrict__ ps, const int2* __restrict__ ra,
                                          const double* __restrict__ psi, const int2* __restrict__ rtb, int nsb,
-                                         int ib, int kq, int li, int nsteps_rt) {
-  // NSTEPS > 0: the step count is known at compile time and the loop is
-  // unrolled, so the loads issued ahead stay in flight across steps (a loop
-  // header makes the compiler wait for every outstanding load)
-  const int nsteps = NSTEPS > 0 ? NSTEPS : nsteps_rt;
+                                         int ib, int kq, int li, int nsteps) {
   constexpr int W = MT * 16;
   const uint32_t ibc = (uint32_t)(ib < nsb ? ib : nsb - 1);
 #pragma unroll
@@ -654,116 +650,14 @@ __device__ __forceinline__ double string_gemm_tile(int i0, int j0, int kb, int k
   return tsum;
 }
 
-// Row kernel, scatter form: LDS = A slice [K8][W] | sigma rows [R][nsb] |
-// psi rows [R][nsb] | alpha operand rows [R][K8 + 16] (small enough for two
-// blocks per CU).  Waves take tiles independently; each output G_k[I_a, J_b]
-// goes to the sigma row at P_k(J_b) (E+b_k is symmetric, so the partner and
-// coefficient are rtb[k][J_b]) by an LDS atomic add.  The order of those
-// adds varies between runs, so results agree to rounding, not bit for bit.
-template <int MT>
-__global__ __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(MT <= 5 ? 4 : 2, 8))) void k_sigma_rows_scatter(
-    const double* __restrict__ At, int kpad, int K4, int K8, int mgroups, int npair, const double* __restrict__ psi,
-    const double* __restrict__ sin, int nsplit, double* __restrict__ sigma, double* __restrict__ partial,
-    const int2* __restrict__ rta, const int2* __restrict__ rtb, int nsa, int nsb, int R, int xcd, double e0) {
-  constexpr int W = MT * 16;
-  extern __shared__ double smem[];
-  __shared__ double red[kRowWaves];
-  const int tpr = (nsb + 15) >> 4;
-  const int RA = K8 + 16;
-  double* sA = smem;
-  double* sAcc = sA + (size_t)K8 * W;
-  double* sPsi = sAcc + (size_t)R * nsb;
-  int2* sRA = reinterpret_cast<int2*>(sPsi + (size_t)R * nsb);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, kq = lane >> 4, li = lane & 15;
-  // with xcd, XCD x (workgroups go to the eight XCDs round robin) takes a
-  // contiguous range of row groups, whose alpha partner rows overlap in its L2
-  int blk = blockIdx.x;
-  const int nrb = (int)gridDim.x;
-  if (xcd && blk < (nrb & ~7)) {  // the remainder past a multiple of 8 keeps its order
-    const int q = nrb >> 3, x = blk & 7;
-    blk = x * q + (blk >> 3);
-  }
-  const int row0 = blk * R;
-  const int nr = min(R, nsa - row0);
-  const int ntg = nr * nsb;
-  const size_t base = (size_t)row0 * nsb;
-  for (int i = tid; i < ntg; i += kRowThreads) {
-    sPsi[i] = psi[base + i];
-    sAcc[i] = 0.0;
-  }
-  for (int i = tid; i < nr * RA; i += kRowThreads) {
-    const int r = i / RA, k = i - r * RA;
-    sRA[i] = rta[(size_t)k * nsa + row0 + r];
-  }
-  const int ntiles = nr * tpr;
-  const int nsteps = K8 / 4;
-  for (int mg = 0; mg < mgroups; ++mg) {
-    const int m0 = mg * W;
-    __syncthreads();  // the previous m-group's reads of sA are done
-    for (int i = tid; i < K8 * W; i += kRowThreads) {
-      const int k = i / W, m = m0 + (i - k * W);
-      sA[i] = (k < K4 && m < kpad) ? At[(size_t)k * kpad + m] : 0.0;
-    }
-    __syncthreads();
-    for (int f = wave; f < ntiles; f += kRowWaves) {
-      const int r = f / tpr, c = f - r * tpr;
-      const int ib = c * 16 + li;
-      double4_t acc[MT];
-      // one m-group: the step count is 4 MT
-      if (K8 == 16 * MT)
-        row_tile<MT, 4 * MT>(acc, sA, sPsi + (size_t)r * nsb, sRA + (size_t)r * RA, psi, rtb, nsb, ib, kq, li, nsteps);
-      else
-        row_tile<MT>(acc, sA, sPsi + (size_t)r * nsb, sRA + (size_t)r * RA, psi, rtb, nsb, ib, kq, li, nsteps);
-      // partners and coefficients of all 4 MT outputs first (rows m >= npair
-      // and columns past nsb read row 0 / the last column and add zero), then
-      // the LDS adds, with no branch between the loads
-      const uint32_t ibc = (uint32_t)(ib < nsb ? ib : nsb - 1);
-      int2 tb[MT][4];
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int m = m0 + t * 16 + kq + 4 * q;
-          tb[t][q] = rtb[(uint32_t)(m < npair ? m : 0) * (uint32_t)nsb + ibc];
-        }
-      double* acc_row = sAcc + (size_t)r * nsb;
-      const bool col_ok = ib < nsb;
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int m = m0 + t * 16 + kq + 4 * q;
-          const double c = (col_ok && m < npair) ? (double)tb[t][q].y : 0.0;
-          atomicAdd(acc_row + tb[t][q].x, c * acc[t][q]);
-        }
-    }
-  }
-  __syncthreads();
-  const size_t dim = (size_t)nsa * nsb;
-  double e = 0.0;
-  for (int tau = tid; tau < ntg; tau += kRowThreads) {
-    double v = sAcc[tau] + e0 * sPsi[tau];
-    for (int z = 0; z < nsplit; ++z) v += sin[(size_t)z * dim + base + tau];
-    sigma[base + tau] = v;
-    e += v * sPsi[tau];
-  }
-  for (int off = 32; off > 0; off >>= 1) e += __shfl_down(e, off, 64);
-  if (lane == 0) red[wave] = e;
-  __syncthreads();
-  if (tid == 0) {
-    double tsum = 0.0;
-    for (int w = 0; w < kRowWaves; ++w) tsum += red[w];
-    partial[blockIdx.x] = tsum;
-  }
-}
-
 // Row kernel over the alpha excitations that do not vanish: LDS = A slice
 // [npair + 1][W] (doubled, the operand's factor 2; row npair is zero) | sigma
 // rows [R][nsb] | lists [R][KA] of the row's nonzero E+a_k' (k_alpha_list).
 // Waves take 16-column tiles independently.  The amplitudes of a step are
 // loaded kAhead steps before its products, those of a tile's first steps before
-// the LDS adds of the previous tile.  Outputs go to the sigma rows as in
-// k_sigma_rows_scatter.
+// the LDS adds of the previous tile.  Each output G_k[I_a, J_b] goes to the sigma
+// row at P_k(J_b) (E+b_k is symmetric) by an LDS atomic add.  The order of those
+// adds varies between runs, so results agree to rounding, not bit for bit.
 // FUSED: the launch also holds the tiles of Ma C and C Mb as extra blocks after
 // the row blocks (they fill the CUs the last row blocks leave idle); every
 // block adds its part to sigma (zeroed beforehand) by global atomics.  Else the
@@ -979,8 +873,8 @@ k_sigma_rows_list(RowArgs P) {
 
 struct RowPlan {
   int mt, mgroups, R, ngroups, nsplit, kchunk;
-  bool scatter, fused;
-  bool list;  // k_sigma_rows_list
+  bool fused;
+  bool list;  // k_sigma_rows_list, else k_sigma_rows
   int ngemm_a, ngemm_b, kchunk_b;  // fused: tile blocks of Ma C and C Mb after the row blocks
   size_t lds;
 };
@@ -996,38 +890,35 @@ size_t string_ham_lds(const Space& s, int nstr, int nel) {
          8 * (size_t)s.npair * (1 + nel * (s.n - nel));
 }
 
-// Whether the contraction over the nonvanishing alpha excitations, with the
-// beta part of H as a string product beside it, takes fewer MFMA products per
-// amplitude than the contraction over all npair + 1 rows: (12e,12o) 78 * 44 +
-// 924 against 78 * 79, (14e,14o) 105 * 56 + 3432 against 105 * 106.  At half
-// filling the string product costs more than it saves from 16 orbitals (from
-// 15, less than a tenth is left).  The constant takes in the spaces of one and
-// two orbitals, whose time is launches: one here, two in the full form (8.0
-// against 11.3 us a sigma).
+// Whether the list form can run: 32-bit byte offsets into psi, and the matrix of
+// Hb built in LDS.
 bool list_form(const Space& s) {
-  const int64_t full = (int64_t)s.npair * (s.npair + 1);
-  return ((int64_t)s.npair * 4 * list_steps(s) + s.nsb) * 10 <= full * 9 + 300 &&
-         s.dim < ((int64_t)1 << 29) &&  // 32-bit byte offsets into psi
-         string_ham_lds(s, s.nsb, s.nb) <= kLdsMax;
+  return s.dim < ((int64_t)1 << 29) && string_ham_lds(s, s.nsb, s.nb) <= kLdsMax;
 }
 
 int row_k8(const Space& s) { return rup(s.npair + 1, 8); }  // contraction rows: two 4-deep k-steps per iteration
 
-// Dynamic LDS of one block (bytes): staged form A slice | G tiles | psi rows |
-// alpha operand rows; scatter form A slice | sigma rows | psi rows | alpha
-// operand rows; list form A slice | sigma rows | lists.
-size_t row_lds(const Space& s, int mt, int R, bool scatter, bool list = false) {
+// Dynamic LDS of one block (bytes): list form A slice | sigma rows | lists;
+// staged form A slice | G tiles | psi rows | alpha operand rows.
+size_t row_lds(const Space& s, int mt, int R, bool list) {
   if (list)
     return 8 * ((size_t)(s.npair + 1) * mt * 16 + (size_t)R * (s.nsb + kTrash) + (size_t)R * list_entries(s));
   const int K8 = row_k8(s);
   const size_t W = (size_t)mt * 16;
-  const size_t mid = scatter ? (size_t)R * s.nsb : (size_t)kRowWaves * W * 16;
-  return 8 * ((size_t)K8 * W + mid + (size_t)R * s.nsb + (size_t)R * (K8 + 16));
+  return 8 * ((size_t)K8 * W + (size_t)kRowWaves * W * 16 + (size_t)R * s.nsb + (size_t)R * (K8 + 16));
+}
+
+// Spaces the list form takes: a row of psi and one of sigma fit a block's LDS
+// beside a 16-row tile of A (to 15 orbitals, and 16 with up to 6 or from 10 beta
+// electrons; the rest runs the two-kernel path).
+bool list_fits(const Space& s) {
+  const int K8 = row_k8(s);
+  return list_form(s) && 8 * ((size_t)K8 * 16 + 2 * (size_t)s.nsb + K8 + 16) <= kLdsMax;
 }
 
 // The space's kernel shape choices (sq_sigma_configure) override these
 // defaults: rows per block, string product split, and the deterministic (staged)
-// form instead of the scatter form (default: SQ_SIGMA_DETERMINISTIC, else 0).
+// form instead of the list form (default: SQ_SIGMA_DETERMINISTIC, else 0).
 bool row_deterministic(const SigmaShape& shape) {
   if (shape.det >= 0) return shape.det != 0;
   static int v = -1;
@@ -1054,9 +945,9 @@ int string_gemm_split(const Space& s) {
 
 // Kernel shape: the m-tile group (largest that fits, then balanced) and the
 // rows per block R.  Staged form: R with the fewest block-rounds on 256 CUs
-// (one block per CU).  Scatter form: the smallest R that gives every wave a
-// tile (more, smaller blocks).  List form: two rows at least, which halves the
-// staging of A per row: 10 orbitals in groups 1600 -> 1506 us, (11e,11o) 205 ->
+// (one block per CU).  List form: the smallest R that gives every wave a tile
+// (more, smaller blocks), but two rows at least, which halves the staging of A
+// per row: 10 orbitals in groups 1600 -> 1506 us, (11e,11o) 205 ->
 // 186, (12e,12o) 437 -> 424 (energy and gradient); more rows gain no more.  A
 // launch of many instances has blocks enough: four rows and the string products
 // unsplit (a quarter of the atomic adds), 256 instances 1283 -> 1206 us.  But no
@@ -1067,28 +958,26 @@ constexpr int kManyInst = 8;
 
 bool row_plan(const Space& s, const SigmaShape& shape, RowPlan* out, int n) {
   if (s.dim == 0 || s.nsb > 16384 || s.npair + 1 > 255 || s.dim >= ((int64_t)1 << 31)) return false;
-  const bool scatter = !row_deterministic(shape);
-  const int kpad = rup(s.npair + 1, 16);
-  if (row_lds(s, 1, 1, scatter) > kLdsMax) return false;
-  const bool list = scatter && list_form(s);
-  const int mt_total = list ? rup(s.npair, 16) / 16 : kpad / 16;
+  const bool list = !row_deterministic(shape);
+  if (!(list ? list_fits(s) : row_lds(s, 1, 1, false) <= kLdsMax)) return false;
+  const int mt_total = rup(list ? s.npair : s.npair + 1, 16) / 16;
   int mt = std::min(mt_total, kMaxMt);
-  while (mt > 1 && row_lds(s, mt, 1, scatter, list) > kLdsMax) --mt;
+  while (mt > 1 && row_lds(s, mt, 1, list) > kLdsMax) --mt;
   const int mgroups = (mt_total + mt - 1) / mt;
   mt = (mt_total + mgroups - 1) / mgroups;
   const int tpr = (s.nsb + 15) / 16;
   int bestR = 0;
-  if (scatter) {
+  if (list) {
     auto rows = [&](int least) {
       int R = std::max(1, std::min(s.nsa, std::max(least, (kRowWaves + tpr - 1) / tpr)));
-      while (R > 1 && row_lds(s, mt, R, true, list) > kLdsMax) --R;
+      while (R > 1 && row_lds(s, mt, R, true) > kLdsMax) --R;
       return R;
     };
-    bestR = rows(list ? 2 : 1);
-    if (list && n >= kManyInst) {
+    bestR = rows(2);
+    if (n >= kManyInst) {
       const int one = bestR;
       bestR = rows(4);
-      while (bestR > one && 2 * row_lds(s, mt, bestR, true, list) > kLdsMax) --bestR;
+      while (bestR > one && 2 * row_lds(s, mt, bestR, true) > kLdsMax) --bestR;
     }
   } else {
     int64_t best = -1;
@@ -1106,14 +995,13 @@ bool row_plan(const Space& s, const SigmaShape& shape, RowPlan* out, int n) {
   if (bestR == 0) return false;
   if (shape.R > 0) {
     const int R = shape.R;
-    if (R <= s.nsa && row_lds(s, mt, R, scatter, list) <= kLdsMax &&
-        (scatter || (int64_t)R * s.nsb <= (int64_t)kMaxTargets * kRowThreads))
+    if (R <= s.nsa && row_lds(s, mt, R, list) <= kLdsMax &&
+        (list || (int64_t)R * s.nsb <= (int64_t)kMaxTargets * kRowThreads))
       bestR = R;
   }
   out->mt = mt;
   out->mgroups = mgroups;
   out->R = bestR;
-  out->scatter = scatter;
   out->list = list;
   out->ngroups = (s.nsa + bestR - 1) / bestR;
   // contraction split of the string products (Ma C and, in the list form, C Mb
@@ -1127,7 +1015,7 @@ bool row_plan(const Space& s, const SigmaShape& shape, RowPlan* out, int n) {
   if (nsplit <= 0) nsplit = list ? string_gemm_split(s) : (s.nsa >= 2048 ? 1 : 2);
   out->kchunk = chunk(joined, nsplit);
   out->nsplit = (joined + out->kchunk - 1) / out->kchunk;
-  out->lds = row_lds(s, mt, bestR, scatter, list);
+  out->lds = row_lds(s, mt, bestR, list);
   // fused form: the tiles of the string products (128 x 64, each contraction
   // split in four: (12e,12o) 481, 441, 432, 424 us an energy and gradient for
   // 1 to 4, 450 for 8) as extra blocks of the row launch, where two row blocks
@@ -1366,7 +1254,6 @@ int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, doubl
   SQ_CHECK(pl.nsplit <= kMaxSplit && pl.ngroups <= s.nsa, SQ_ERR_ARG, "row sigma shape exceeds its workspace");
   SQ_CHECK(!pl.fused || pl.ngroups + pl.ngemm_a + pl.ngemm_b <= row_sigma_work_doubles(s) - 64, SQ_ERR_ARG,
            "row sigma shape exceeds its workspace");
-  static const int xcd = env_int("SQ_ROWS_XCD", 1) != 0 ? 1 : 0;
   const double* Mb = H.d_Mb ? H.d_Mb : H.d_Ma;
   if (pl.fused) {
     *partial_out = work;
@@ -1419,23 +1306,6 @@ int64_t row_sigma(const Space& s, const Hamiltonian& H, const double* psi, doubl
   const double e0 = 0.5 * H.e_core;  // the other half is on Ma's diagonal
   // algorithmic traffic: psi read (rows and alpha partners through the cache), the alpha partials read, sigma written
   const double bytes = 8.0 * (double)s.dim * (2 + nsplit);
-  if (pl.scatter) {
-    switch (pl.mt) {
-#define SQ_RSS(MT)                                                                                              \
-  case MT:                                                                                                      \
-    allow_lds(k_sigma_rows_scatter<MT>, pl.lds);                                                                \
-    SQ_PROF(PC_SIGMA_ROWS, st, bytes, flops,                                                                    \
-            k_sigma_rows_scatter<MT><<<pl.ngroups, kRowThreads, pl.lds, st>>>(                                  \
-                H.d_A, H.kpad, K4, K8, pl.mgroups, s.npair, psi, sinp, nsplit, sigma, partial, s.d_rta,         \
-                s.d_rtb, s.nsa, s.nsb, pl.R, xcd, e0));                                                         \
-    break;
-      SQ_RSS(1) SQ_RSS(2) SQ_RSS(3) SQ_RSS(4) SQ_RSS(5) SQ_RSS(6) SQ_RSS(7) SQ_RSS(8) SQ_RSS(9)
-#undef SQ_RSS
-      default:
-        throw Error{SQ_ERR_ARG, "unsupported orbital count for the row sigma"};
-    }
-    return pl.ngroups;
-  }
   switch (pl.mt) {
 #define SQ_RS(MT)                                                                                               \
   case MT:                                                                                                      \
@@ -1472,7 +1342,7 @@ bool row_sigma_wants_zero(const Space& s) {
 
 bool row_sigma_group_ok(const Space& s) {
   RowPlan pl;
-  return rows_enabled() && s.d_rtb != nullptr && row_plan(s, &pl) && pl.scatter && pl.fused;
+  return rows_enabled() && s.d_rtb != nullptr && row_plan(s, &pl) && pl.fused;
 }
 
 int64_t row_sigma_group_partials(const Space& s, const SigmaShape& shape, int n) {
