@@ -244,11 +244,11 @@ int sq_batch_set_start_states(sq_batch* b, const double* const* psi0, void* stre
 /* Kernel shape picked by the autotuner: rotation pairs of determinants per
  * thread in flight (1, 2 or 4) and sigma GEMM 16-column tiles per wave (1 or
  * 2); no counterpart in the reference (its batching has no kernel shapes).
- * Drops a captured graph. */
+ * Every shape keeps its captured graph until the batch is destroyed. */
 int sq_batch_configure(sq_batch* b, int rot_pairs, int gemm_tiles);
 /* One launch on stream. */
 int sq_batch_run(sq_batch* b, void* stream);
-/* Same launch captured once into a hipGraph, then replayed. */
+/* Same launch captured once per kernel shape into a hipGraph, then replayed. */
 int sq_batch_run_graph(sq_batch* b, void* stream);
 /* Host copies: energies[n_inst] (electronic + core), grads[num_params]. */
 int sq_batch_results(const sq_batch* b, double* energies, double* grads, void* stream);

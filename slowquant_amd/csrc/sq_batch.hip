@@ -429,6 +429,7 @@ constexpr int64_t kKeepMinDim = 16384;
 // ones leave CUs idle that another group's fill (256 instances as above on 1,
 // 3 and 4: 1549, 1329, 1206 us; there are four hardware queues).
 constexpr int kGroupLanes = 4;
+constexpr int kBatchShapes = 6;  // of the persistent launch: 1, 2 or 4 rotation pairs, 1 or 2 column tiles
 
 struct Batch {
   std::vector<BatchInstance> inst;
@@ -443,8 +444,9 @@ struct Batch {
   const double** d_psi0 = nullptr;  // start-state pointer table [inst]
   std::vector<BatchGroup> groups;   // instances run through the tile and row-sigma kernels
   std::vector<std::pair<int, int>> group_members;  // (group, instance), in instance order
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  // a captured launch per kernel shape (kernel_shape), kept until the batch goes
+  hipGraph_t graph[kBatchShapes] = {};
+  hipGraphExec_t exec[kBatchShapes] = {};
   std::vector<int32_t> grad_off;
   double* host_out = nullptr;  // pinned: energies | gradients on their way to the caller
   mutable std::mutex host_mu;
@@ -454,15 +456,15 @@ struct Batch {
   hipEvent_t ev_lane[kGroupLanes] = {};
   int rot_pairs = 2;    // rotation pairs per thread in flight (1, 2, 4)
   int gemm_tiles = 1;   // sigma GEMM column tiles per wave (1, 2)
-  void drop_graph() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    exec = nullptr;
-    graph = nullptr;
+  // 0 to kBatchShapes - 1; one when the persistent launch holds no instance
+  int kernel_shape() const {
+    return nwg == 0 ? 0 : (rot_pairs == 1 ? 0 : rot_pairs == 2 ? 1 : 2) * 2 + gemm_tiles - 1;
   }
   ~Batch() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
+    for (hipGraphExec_t e : exec)
+      if (e) (void)hipGraphExecDestroy(e);
+    for (hipGraph_t g : graph)
+      if (g) (void)hipGraphDestroy(g);
     if (host_out) (void)hipHostFree(host_out);
     if (side) (void)hipStreamDestroy(side);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
@@ -1022,14 +1024,13 @@ static void batch_launch(Batch& B, hipStream_t st) {
 }
 
 /* Kernel shape: rotation pairs per thread in flight (1, 2 or 4) and sigma
- * GEMM column tiles per wave (1 or 2); drops a captured graph. */
+ * GEMM column tiles per wave (1 or 2).  Every shape keeps its captured graph. */
 int sq_batch_configure(sq_batch* bo, int rot_pairs, int gemm_tiles) {
   return guarded([&] {
     SQ_CHECK(bo, SQ_ERR_ARG, "NULL argument");
     SQ_CHECK(rot_pairs == 1 || rot_pairs == 2 || rot_pairs == 4, SQ_ERR_ARG, "rot_pairs must be 1, 2 or 4");
     SQ_CHECK(gemm_tiles == 1 || gemm_tiles == 2, SQ_ERR_ARG, "gemm_tiles must be 1 or 2");
     Batch& B = bo->b;
-    if (B.rot_pairs != rot_pairs || B.gemm_tiles != gemm_tiles) B.drop_graph();
     B.rot_pairs = rot_pairs;
     B.gemm_tiles = gemm_tiles;
   });
@@ -1042,13 +1043,14 @@ int sq_batch_run(sq_batch* bo, void* stream) {
   });
 }
 
-/* Capture the launch in a hipGraph (once) and replay it. */
+/* Capture the launch in a hipGraph (once per kernel shape) and replay it. */
 int sq_batch_run_graph(sq_batch* bo, void* stream) {
   return guarded([&] {
     Batch& B = bo->b;
     hipStream_t st = as_stream(stream);
     check_groups(B);
-    if (!B.exec) {
+    const int shape = B.kernel_shape();
+    if (!B.exec[shape]) {
       // the groups' kernels take their shared-memory attributes on an eager
       // launch first (not a stream operation, so kept out of the capture)
       if (!B.groups.empty()) {
@@ -1076,10 +1078,11 @@ int sq_batch_run_graph(sq_batch* bo, void* stream) {
       (void)hipStreamDestroy(cap);
       prof_resume(prof_was);
       SQ_CHECK(e == hipSuccess && e2 == hipSuccess, SQ_ERR_HIP, "graph capture failed");
-      B.graph = g;
-      SQ_HIP(hipGraphInstantiate(&B.exec, B.graph, nullptr, nullptr, 0));
+      if (B.graph[shape]) (void)hipGraphDestroy(B.graph[shape]);  // of a failed instantiation
+      B.graph[shape] = g;
+      SQ_HIP(hipGraphInstantiate(&B.exec[shape], g, nullptr, nullptr, 0));
     }
-    SQ_HIP(hipGraphLaunch(B.exec, st));
+    SQ_HIP(hipGraphLaunch(B.exec[shape], st));
   });
 }
 
